@@ -376,7 +376,8 @@ int ts_logprob_grad_weight(const void* dlogits, int64_t ld_dlogits, const void* 
  * The reference keeps FP32/FP64 hidden states and heads at their precision
  * (accel/fused_logprob.py:27-58: `_accum_dtype` widens only bf16/fp16); these
  * entry points compute logits, softmax statistics, dlogits and both VJP
- * products in the input type T (dtype TS_F32 or TS_F64) on the vector ALUs.
+ * products in the input type T (dtype TS_F32 or TS_F64; fp32 on the fp32
+ * matrix instruction, fp64 on the vector ALUs).
  * hidden [rows, dim] (row stride ld_hidden), weight [vocab, dim]
  * (ld_weight), target int64 [rows]; every other array is of T.  No
  * alignment or stride-multiple requirements.  A target outside [0, vocab)
@@ -415,6 +416,15 @@ int ts_logprob_dlogits_exact(const void* hidden, int64_t ld_hidden, const void* 
  * inputs (accel/fused_logprob.py:167-193, :297-306). */
 int ts_matmul_exact(const void* a, int64_t a_m, int64_t a_k, const void* b, int64_t b_k, int64_t b_n, int64_t m,
                     int64_t n, int64_t k, void* c, int64_t ldc, int accumulate, int dtype, void* stream);
+
+/* ts_matmul_exact with a workspace of ts_matmul_exact_workspace bytes (0: none
+ * wanted) for the partial sums of contraction ranges, which it takes when the
+ * output tiles alone leave part of the device idle; they are added in range
+ * order.  A null workspace: one range. */
+int64_t ts_matmul_exact_workspace(int64_t m, int64_t n, int64_t k, int dtype);
+int ts_matmul_exact_ws(const void* a, int64_t a_m, int64_t a_k, const void* b, int64_t b_k, int64_t b_n, int64_t m,
+                       int64_t n, int64_t k, void* c, int64_t ldc, int accumulate, void* workspace,
+                       int64_t workspace_bytes, int dtype, void* stream);
 
 /* ------------------------------------------------------------------------
  * Merged-weight LoRA linear (bf16 or fp16 operands, fp32 accumulation)

@@ -63,6 +63,9 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
         _INT,
         [_P, _I64, _P, _I64, _P, _P, _P, _P, _P, _I64, _I64, _I64, _P, _I64, _INT, _P],
     ),
+    "ts_matmul_exact_workspace": (_I64, [_I64, _I64, _I64, _INT]),
+    "ts_matmul_exact_ws": (
+        _INT, [_P, _I64, _I64, _P, _I64, _I64, _I64, _I64, _I64, _P, _I64, _INT, _P, _I64, _INT, _P]),
     "ts_matmul_exact": (_INT, [_P, _I64, _I64, _P, _I64, _I64, _I64, _I64, _I64, _P, _I64, _INT, _INT, _P]),
     "ts_lora_fwd": (_INT, [_P, _I64, _P, _I64, _I64, _I64, _I64, _P, _I64, _INT, _P]),
     "ts_lora_bwd_workspace": (_I64, [_I64, _I64, _I64, _I64]),

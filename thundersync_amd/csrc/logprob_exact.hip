@@ -2,9 +2,8 @@
 // fp64 hidden states and head): logits, softmax statistics, dlogits and the
 // two VJP products all in that type, as the reference keeps FP32/FP64 inputs
 // at their precision (accel/fused_logprob.py:27-58, `_accum_dtype`: only
-// bf16/fp16 widen).  The bf16/fp16 operators run on MFMA (logprob.hip);
-// these take the vector ALUs, which give fp32 and fp64 FMAs with no operand
-// rounding.
+// bf16/fp16 widen).  The entry points of both, and the fp64 kernels, on the
+// vector ALUs; fp32 runs on the fp32 matrix instruction (logprob_f32.hip).
 //
 // One tile product serves every kernel: a 256-thread work-group forms a
 // 64 x 64 tile of C(m, n) = sum_k A(m, k) B(k, n) over operands given by
@@ -25,9 +24,11 @@
 //             dlogits = -p (g_lp + g_H (log p + H)) + g_lp [v == t] in the
 //             input type; grad_hidden = dlogits . W and grad_weight +=
 //             dlogits^T . hidden are two more tile products.
+#include <algorithm>
 #include <cmath>
 
 #include "common.h"
+#include "logprob_f32.h"
 #include "timing.h"
 #include "../../include/thundersync_hip.h"
 
@@ -40,9 +41,7 @@ constexpr int kThreads = 256;
 constexpr int kMaxGroups = 64;  // vocabulary groups of the forward (partials per row)
 
 template <typename T> __device__ __forceinline__ T inf_of() { return (T)__builtin_huge_val(); }
-__device__ __forceinline__ float exp_of(float x) { return expf(x); }
 __device__ __forceinline__ double exp_of(double x) { return exp(x); }
-__device__ __forceinline__ float log_of(float x) { return logf(x); }
 __device__ __forceinline__ double log_of(double x) { return log(x); }
 
 // C tile (m0, n0) of sum_k A(m, k) B(k, n) into acc[i][j] (row 4 ty + i,
@@ -284,8 +283,6 @@ int groups_of(int64_t vocab) {
   return (int)std::min<int64_t>(tiles, kMaxGroups);
 }
 
-int elem_bytes(int dtype) { return dtype == TS_F64 ? 8 : 4; }
-
 template <typename T>
 int fwd_t(const void* hidden, int64_t ld_h, const void* weight, int64_t ld_w, const int64_t* target, int64_t rows,
           int64_t dim, int64_t vocab, void* logprob, void* entropy, void* lse, void* workspace, hipStream_t s) {
@@ -336,7 +333,8 @@ extern "C" {
 
 int64_t ts_logprob_fwd_exact_workspace(int64_t rows, int64_t vocab, int dtype) {
   if (rows < 0 || vocab < 1 || (dtype != TS_F32 && dtype != TS_F64)) return -1;
-  return 3 * (int64_t)groups_of(vocab) * rows * elem_bytes(dtype);
+  const int64_t groups = dtype == TS_F32 ? ts::lpf::fwd_groups(rows, vocab) : groups_of(vocab);
+  return 3 * groups * rows * (dtype == TS_F32 ? 4 : 8);
 }
 
 int ts_logprob_fwd_exact(const void* hidden, int64_t ld_hidden, const void* weight, int64_t ld_weight,
@@ -356,8 +354,9 @@ int ts_logprob_fwd_exact(const void* hidden, int64_t ld_hidden, const void* weig
   hipStream_t s = (hipStream_t)stream;
   return dtype == TS_F64 ? fwd_t<double>(hidden, ld_hidden, weight, ld_weight, target, rows, dim, vocab, logprob,
                                          entropy, lse, workspace, s)
-                         : fwd_t<float>(hidden, ld_hidden, weight, ld_weight, target, rows, dim, vocab, logprob,
-                                        entropy, lse, workspace, s);
+                         : ts::lpf::fwd((const float*)hidden, ld_hidden, (const float*)weight, ld_weight, target, rows,
+                                        dim, vocab, (float*)logprob, (float*)entropy, (float*)lse, (float*)workspace,
+                                        s);
 }
 
 int ts_logprob_dlogits_exact(const void* hidden, int64_t ld_hidden, const void* weight, int64_t ld_weight,
@@ -376,20 +375,35 @@ int ts_logprob_dlogits_exact(const void* hidden, int64_t ld_hidden, const void* 
   hipStream_t s = (hipStream_t)stream;
   return dtype == TS_F64 ? dlogits_t<double>(hidden, ld_hidden, weight, ld_weight, target, lse, entropy, grad_lp,
                                              grad_ent, rows, dim, vocab, dlogits, ld_dlogits, s)
-                         : dlogits_t<float>(hidden, ld_hidden, weight, ld_weight, target, lse, entropy, grad_lp,
-                                            grad_ent, rows, dim, vocab, dlogits, ld_dlogits, s);
+                         : ts::lpf::dlogits((const float*)hidden, ld_hidden, (const float*)weight, ld_weight, target,
+                                            (const float*)lse, (const float*)entropy, (const float*)grad_lp,
+                                            (const float*)grad_ent, rows, dim, vocab, (float*)dlogits, ld_dlogits, s);
 }
 
-int ts_matmul_exact(const void* a, int64_t a_m, int64_t a_k, const void* b, int64_t b_k, int64_t b_n, int64_t m,
-                    int64_t n, int64_t k, void* c, int64_t ldc, int accumulate, int dtype, void* stream) {
+int64_t ts_matmul_exact_workspace(int64_t m, int64_t n, int64_t k, int dtype) {
+  return dtype == TS_F32 && m > 0 && n > 0 && k > 0 ? ts::lpf::matmul_workspace(m, n, k) : 0;
+}
+
+int ts_matmul_exact_ws(const void* a, int64_t a_m, int64_t a_k, const void* b, int64_t b_k, int64_t b_n, int64_t m,
+                       int64_t n, int64_t k, void* c, int64_t ldc, int accumulate, void* workspace,
+                       int64_t workspace_bytes, int dtype, void* stream) {
   TS_CHECK_ARG(dtype == TS_F32 || dtype == TS_F64, "ts_matmul_exact: dtype must be TS_F32 or TS_F64");
   TS_CHECK_ARG(m >= 0 && n >= 0 && k >= 0 && ldc >= n, "ts_matmul_exact: bad shape");
   TS_CHECK_ARG(((m + BT - 1) / BT) * ((n + BT - 1) / BT) < (int64_t)1 << 31, "ts_matmul_exact: too large");
   if (m == 0 || n == 0) return TS_OK;
   TS_CHECK_ARG(c && (k == 0 || (a && b)), "ts_matmul_exact: null pointer");
+  TS_CHECK_ARG(!workspace || workspace_bytes >= ts_matmul_exact_workspace(m, n, k, dtype),
+               "ts_matmul_exact: workspace of %lld bytes, need %lld", (long long)workspace_bytes,
+               (long long)ts_matmul_exact_workspace(m, n, k, dtype));
   hipStream_t s = (hipStream_t)stream;
   return dtype == TS_F64 ? matmul_t<double>(a, a_m, a_k, b, b_k, b_n, m, n, k, c, ldc, accumulate, s)
-                         : matmul_t<float>(a, a_m, a_k, b, b_k, b_n, m, n, k, c, ldc, accumulate, s);
+                         : ts::lpf::matmul((const float*)a, a_m, a_k, (const float*)b, b_k, b_n, m, n, k, (float*)c,
+                                           ldc, accumulate, (float*)workspace, s);
+}
+
+int ts_matmul_exact(const void* a, int64_t a_m, int64_t a_k, const void* b, int64_t b_k, int64_t b_n, int64_t m,
+                    int64_t n, int64_t k, void* c, int64_t ldc, int accumulate, int dtype, void* stream) {
+  return ts_matmul_exact_ws(a, a_m, a_k, b, b_k, b_n, m, n, k, c, ldc, accumulate, nullptr, 0, dtype, stream);
 }
 
 }  // extern "C"

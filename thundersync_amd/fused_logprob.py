@@ -24,9 +24,9 @@ and the fp32 ``[V, D]`` accumulator when the weight gradient is needed.
 
 bf16 or fp16 (one element type per call) on the MFMA kernels above; fp32
 and fp64 at their own precision, as the reference keeps them (FL:27-58):
-logits, statistics, dlogits and both VJP products in the input type on the
-vector-ALU kernels (``ts_logprob_fwd_exact``, ``ts_logprob_dlogits_exact``,
-``ts_matmul_exact``), with the same O(chunk * V) dlogits block and outputs
+logits, statistics, dlogits and both VJP products in the input type
+(``ts_logprob_fwd_exact``, ``ts_logprob_dlogits_exact``,
+``ts_matmul_exact_ws``), with the same O(chunk * V) dlogits block and outputs
 in the input type.  GPU only: other dtypes and CPU tensors raise.
 """
 
@@ -128,13 +128,20 @@ def _backward_exact(hidden, weight, target, lse, ent, grad_lp, grad_ent, chunk, 
     v = w.shape[0]
     dt, dev = h.dtype, h.device
     grad_hidden = torch.empty(n, d, dtype=dt, device=dev)
-    grad_weight = torch.zeros(v, d, dtype=dt, device=dev) if needs_weight_grad else None
     if n == 0:
-        return grad_hidden, grad_weight
+        return grad_hidden, torch.zeros(v, d, dtype=dt, device=dev) if needs_weight_grad else None
+    # the first block writes the weight gradient, the others add to it
+    grad_weight = torch.empty(v, d, dtype=dt, device=dev) if needs_weight_grad else None
     code, stream = _lib.dtype_code(dt), _lib.stream_of(h)
     ldh, ldw = max(h.stride(0), d), max(w.stride(0), d)
     block = min(max(1, int(chunk)), n)
-    dl = torch.empty(block, v, dtype=dt, device=dev)
+    vp = (v + 3) // 4 * 4  # rows of whole 16-byte vectors
+    dl = torch.empty(block, vp, dtype=dt, device=dev)
+    # the contraction ranges' partial sums, for whichever product and block size wants most
+    products = [s for rows in {block, n % block or block}
+                for s in ((rows, d, v), *([(v, d, rows)] if needs_weight_grad else []))]
+    ws_bytes = max(int(lib.ts_matmul_exact_workspace(*s, code)) for s in products)
+    ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=dev)
     g_lp = grad_lp.to(dt).contiguous()
     g_ent = grad_ent.to(dt).contiguous() if grad_ent is not None else None
     esize = h.element_size()
@@ -146,24 +153,24 @@ def _backward_exact(hidden, weight, target, lse, ent, grad_lp, grad_ent, chunk, 
                 lib.ts_logprob_dlogits_exact(
                     h_i, ldh, w.data_ptr(), ldw, t[i:].data_ptr(), lse[i:].data_ptr(),
                     ent[i:].data_ptr() if g_ent is not None else None, g_lp[i:].data_ptr(),
-                    g_ent[i:].data_ptr() if g_ent is not None else None, rows, d, v, dl.data_ptr(), v, code, stream,
+                    g_ent[i:].data_ptr() if g_ent is not None else None, rows, d, v, dl.data_ptr(), vp, code, stream,
                 ),
                 f"ts_logprob_dlogits_exact(rows={rows}, dim={d}, vocab={v})",
             )
         with operator_range("logprob_head_hidden_vjp", role=device_role(dev), rows=rows, hidden=d, vocab=v):
             # grad_hidden[i:i+rows] = dl . W
             _lib.check(
-                lib.ts_matmul_exact(dl.data_ptr(), v, 1, w.data_ptr(), ldw, 1, rows, d, v,
-                                    grad_hidden[i:].data_ptr(), d, 0, code, stream),
-                f"ts_matmul_exact(dlogits . weight, rows={rows}, dim={d}, vocab={v})",
+                lib.ts_matmul_exact_ws(dl.data_ptr(), vp, 1, w.data_ptr(), ldw, 1, rows, d, v,
+                                       grad_hidden[i:].data_ptr(), d, 0, ws.data_ptr(), ws_bytes, code, stream),
+                f"ts_matmul_exact_ws(dlogits . weight, rows={rows}, dim={d}, vocab={v})",
             )
         if grad_weight is not None:
             with operator_range("logprob_head_weight_vjp", role=device_role(dev), rows=rows, hidden=d, vocab=v):
                 # grad_weight += dl^T . h[i:i+rows]
                 _lib.check(
-                    lib.ts_matmul_exact(dl.data_ptr(), 1, v, h_i, ldh, 1, v, d, rows,
-                                        grad_weight.data_ptr(), d, 1, code, stream),
-                    f"ts_matmul_exact(dlogits^T . hidden, rows={rows}, dim={d}, vocab={v})",
+                    lib.ts_matmul_exact_ws(dl.data_ptr(), 1, vp, h_i, ldh, 1, v, d, rows, grad_weight.data_ptr(), d,
+                                           int(i > 0), ws.data_ptr(), ws_bytes, code, stream),
+                    f"ts_matmul_exact_ws(dlogits^T . hidden, rows={rows}, dim={d}, vocab={v})",
                 )
     return grad_hidden, grad_weight
 
