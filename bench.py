@@ -623,7 +623,7 @@ def bench_logprob(args, device, gate: bool = True):
         lp, ent = fused_logprob.fused_logprob_entropy(h, weight, t)
         lp.backward(a)
 
-    kernels = ["logprob.fwd_stats_kernel", "logprob.target_logit_kernel", "logprob.combine_kernel",
+    kernels = ["logprob.fwd_stats_kernel", "logprob.combine_kernel",
                "logprob.dlogits_kernel", "logprob.grad_hidden_kernel", "logprob.grad_hidden_reduce_kernel"]
     ms, per, mem = timed(step, args.steps, args.warmup, kernels)
     gemm = 2 * rows * v * d
@@ -632,7 +632,6 @@ def bench_logprob(args, device, gate: bool = True):
         "logprob.dlogits_kernel": gemm,
         "logprob.grad_hidden_kernel": gemm,
         "logprob.combine_kernel": 0,
-        "logprob.target_logit_kernel": 0,
         "logprob.grad_hidden_reduce_kernel": 0,
     }
     flop = 3 * gemm
@@ -986,7 +985,7 @@ def bench_c5(args, device):
         opt.zero_grad(set_to_none=True)
 
     kernels = ["attention.fwd_kernel", "attention.delta_kernel", "attention.dq_kernel", "attention.dkdv_kernel",
-               "logprob.fwd_stats_kernel", "logprob.target_logit_kernel", "logprob.combine_kernel",
+               "logprob.fwd_stats_kernel", "logprob.combine_kernel",
                "logprob.dlogits_kernel", "logprob.grad_hidden_kernel", "logprob.grad_hidden_reduce_kernel",
                "rmsnorm.rmsnorm_fwd_lanes", "rmsnorm.rmsnorm_fwd_rowwave", "rmsnorm.rmsnorm_bwd_vec",
                "rmsnorm.rmsnorm_bwd_scalar", "rmsnorm.rmsnorm_dw_reduce",

@@ -7,9 +7,9 @@
 //
 //   forward   logits^T tile = W_tile . H_tile^T on MFMA (A = vocab rows of W,
 //             B = token rows of H, both K-contiguous).  The epilogue reduces
-//             each token column of the tile to (max, sum exp, sum exp*(l-max))
-//             and picks the target logit; a combine kernel merges the per-tile
-//             partials into logprob, entropy and lse.  HBM traffic: W once,
+//             each token column of the tile to (max, sum exp, sum exp*(l-max));
+//             a combine kernel merges the per-tile partials into logprob,
+//             entropy and lse and takes the target logit as a dot product.  HBM traffic: W once,
 //             H once per vocab super-tile, partials (12 bytes/token/tile).
 //   backward  the same tile GEMM recomputes the logits; the epilogue forms
 //             dlogits = -p (g_lp + g_H (log p + H)) + g_lp [v == t] in
@@ -72,7 +72,6 @@ struct FwdArgs {
   float* part_m;   // [n_vtiles][rows]
   float* part_s;
   float* part_e;
-  float* tgt;      // [rows] target logit
 };
 
 template <typename E>
@@ -164,70 +163,79 @@ __global__ __launch_bounds__(kGemmThreads, 1) void fwd_stats_kernel(FwdArgs p) {
   }
 }
 
-// target logit l[n, t] = sum_d h[n, d] W[t, d] (fp32 sum of exact bf16
-// products), one wave per row; rows with t outside [0, vocab) are skipped
-// (the combine kernel writes NaN for them)
-template <typename E>
-__global__ __launch_bounds__(kThreads) void target_logit_kernel(const bf16* __restrict__ h, int64_t ldh,
-                                                                const bf16* __restrict__ w, int64_t ldw,
-                                                                const int64_t* __restrict__ target, int rows,
-                                                                int dim, int vocab, float* __restrict__ tgt) {
-  const int lane = threadIdx.x & 63;
-  const int n = blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6);
-  if (n >= rows) return;
-  const int64_t t = target[n];
-  if (t < 0 || t >= vocab) return;
-  const bf16* hr = h + (int64_t)n * ldh;
-  const bf16* wr = w + t * ldw;
-  float acc = 0.f;
-  for (int d = 8 * lane; d < dim; d += 512) {
-    const u32x4 a = ld16(hr + d), b = ld16(wr + d);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      acc = fmaf(bits_to_f<E>(a[i] & 0xffffu), bits_to_f<E>(b[i] & 0xffffu), acc);
-      acc = fmaf(bits_to_f<E>(a[i] >> 16), bits_to_f<E>(b[i] >> 16), acc);
-    }
-  }
-  acc = wave_sum(acc);
-  if (lane == 0) tgt[n] = acc;
-}
+// Merge the per-vocab-tile partials of each token and form its target logit
+// l[n, t] = sum_d h[n, d] W[t, d] (fp32 sum of exact 16-bit products; NaN logprob
+// for t outside [0, vocab)).  A work-group of 16 waves owns 16 tokens: its 64
+// slots of 16 lanes merge the tiles t = slot, slot + 64, ... (a slot reads 64
+// consecutive bytes of one tile's row of partials), then the 4 slots of a wave
+// and the 16 waves meet in a fixed order, while wave w takes token w's dot
+// product.  Bound by the latency of the tile loop, so the tiles are cut over as
+// many slots as a work-group holds and the rows over 16-token work-groups: 64
+// tokens per four-wave work-group walked 149 tiles one after another (400 rows of
+// 594 tiles: 131 us and a target-logit launch of 7 us, now 21 us).
+constexpr int kCombineTokens = 16;
+constexpr int kCombineThreads = 64 * kCombineTokens;
 
-// merge the per-vocab-tile partials of each token: a work-group owns 64 tokens;
-// its 4 waves merge the tiles t = wave, wave + 4, ... (lanes read 64
-// consecutive tokens of one tile: coalesced), then wave 0 merges the four
-// partial states in wave order
-__global__ __launch_bounds__(kThreads) void combine_kernel(const float* __restrict__ pm,
-                                                           const float* __restrict__ ps,
-                                                           const float* __restrict__ pe,
-                                                           const float* __restrict__ tgt,
-                                                           const int64_t* __restrict__ target,
-                                                           int rows, int n_vtiles, int vocab,
-                                                           float* __restrict__ logprob,
-                                                           float* __restrict__ entropy,
-                                                           float* __restrict__ lse) {
-  __shared__ float sm[4][64], ss[4][64], se[4][64];
+template <typename E>
+__global__ __launch_bounds__(kCombineThreads) void combine_kernel(
+    const float* __restrict__ pm, const float* __restrict__ ps, const float* __restrict__ pe,
+    const bf16* __restrict__ h, int64_t ldh, const bf16* __restrict__ w, int64_t ldw,
+    const int64_t* __restrict__ target, int rows, int dim, int n_vtiles, int vocab, float* __restrict__ logprob,
+    float* __restrict__ entropy, float* __restrict__ lse) {
+  __shared__ float sm[16][16], ss[16][16], se[16][16], st[16];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int n = blockIdx.x * 64 + lane;
-  float M = neg_inf(), S = 0.f, E = 0.f;  // E: sum exp(l - M) (l - M)
+  const int tok = lane & 15, slot = 4 * wave + (lane >> 4);
+  const int n0 = blockIdx.x * kCombineTokens, n = n0 + tok;
+  float M = neg_inf(), S = 0.f, X = 0.f;  // X: sum exp(l - M) (l - M)
   if (n < rows) {
-    for (int t = wave; t < n_vtiles; t += 4) {
+#pragma unroll 4
+    for (int t = slot; t < n_vtiles; t += 64) {
       const int64_t o = (int64_t)t * rows + n;
-      merge_stats(M, S, E, pm[o], ps[o], pe[o]);
+      merge_stats(M, S, X, pm[o], ps[o], pe[o]);
     }
   }
-  sm[wave][lane] = M;
-  ss[wave][lane] = S;
-  se[wave][lane] = E;
-  __syncthreads();
-  if (wave != 0 || n >= rows) return;
 #pragma unroll
-  for (int w = 1; w < 4; ++w) merge_stats(M, S, E, sm[w][lane], ss[w][lane], se[w][lane]);
+  for (int o = 16; o < 64; o <<= 1) {
+    const float mo = shfl_xor(M, o), so = shfl_xor(S, o), xo = shfl_xor(X, o);
+    merge_stats(M, S, X, mo, so, xo);
+  }
+  if (lane < 16) {
+    sm[wave][tok] = M;
+    ss[wave][tok] = S;
+    se[wave][tok] = X;
+  }
+  // wave w: the target logit of token n0 + w
+  if (n0 + wave < rows) {
+    const int64_t t = target[n0 + wave];
+    if (t >= 0 && t < vocab) {
+      const bf16* hr = h + (int64_t)(n0 + wave) * ldh;
+      const bf16* wr = w + t * ldw;
+      float acc = 0.f;
+      for (int d = 8 * lane; d < dim; d += 512) {
+        const u32x4 a = ld16(hr + d), b = ld16(wr + d);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          acc = fmaf(bits_to_f<E>(a[i] & 0xffffu), bits_to_f<E>(b[i] & 0xffffu), acc);
+          acc = fmaf(bits_to_f<E>(a[i] >> 16), bits_to_f<E>(b[i] >> 16), acc);
+        }
+      }
+      acc = wave_sum(acc);
+      if (lane == 0) st[wave] = acc;
+    } else if (lane == 0) {
+      st[wave] = __builtin_nanf("");
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x >= 16 || n >= rows) return;
+  M = sm[0][tok];
+  S = ss[0][tok];
+  X = se[0][tok];
+#pragma unroll
+  for (int v = 1; v < 16; ++v) merge_stats(M, S, X, sm[v][tok], ss[v][tok], se[v][tok]);
   const float logs = logf(S);
-  const int64_t tg = target[n];
-  const bool ok = tg >= 0 && tg < vocab;
-  logprob[n] = ok ? (tgt[n] - M) - logs : __builtin_nanf("");
+  logprob[n] = (st[tok] - M) - logs;
   lse[n] = M + logs;
-  if (entropy) entropy[n] = logs - E / S;
+  if (entropy) entropy[n] = logs - X / S;
 }
 
 // ---------------------------------------------------------------------------
@@ -479,7 +487,7 @@ extern "C" {
 int64_t ts_logprob_fwd_workspace(int64_t rows, int64_t vocab) {
   if (rows <= 0 || vocab <= 0) return 0;
   const int64_t vt = (vocab + ts::lp::BM - 1) / ts::lp::BM;
-  return (3 * vt + 1) * rows * (int64_t)sizeof(float);
+  return 3 * vt * rows * (int64_t)sizeof(float);
 }
 
 int ts_logprob_fwd(const void* hidden, int64_t ld_hidden, const void* weight, int64_t ld_weight,
@@ -517,20 +525,18 @@ int ts_logprob_fwd(const void* hidden, int64_t ld_hidden, const void* weight, in
   a.part_m = ws;
   a.part_s = ws + (int64_t)a.n_vtiles * rows;
   a.part_e = ws + 2 * (int64_t)a.n_vtiles * rows;
-  a.tgt = ws + 3 * (int64_t)a.n_vtiles * rows;
   TS_CHECK_ARG((int64_t)a.n_ttiles * a.n_vtiles < (1ll << 31), "ts_logprob_fwd: grid too large");
   hipStream_t s = (hipStream_t)stream;
   { ts::TimedLaunch timed_("logprob.fwd_stats_kernel", s); TS_LAUNCH_E(dtype, fwd_stats_kernel, dim3((unsigned)(a.n_ttiles * a.n_vtiles)), dim3(kGemmThreads),
                      0, s, a); }
   int st = ts::check_launch("ts_logprob_fwd (tiles)");
   if (st != TS_OK) return st;
-  { ts::TimedLaunch timed_("logprob.target_logit_kernel", s); TS_LAUNCH_E(dtype, target_logit_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(kThreads),
-                     0, s, a.h, a.ldh, a.w, a.ldw, target, (int)rows, (int)dim, (int)vocab, a.tgt); }
-  st = ts::check_launch("ts_logprob_fwd (target logits)");
-  if (st != TS_OK) return st;
-  { ts::TimedLaunch timed_("logprob.combine_kernel", s); hipLaunchKernelGGL(combine_kernel, dim3((unsigned)((rows + 63) / 64)), dim3(kThreads),
-                     0, s, a.part_m, a.part_s, a.part_e, a.tgt, target, (int)rows, a.n_vtiles,
-                     (int)vocab, logprob, entropy, lse); }
+  {
+    ts::TimedLaunch timed_("logprob.combine_kernel", s);
+    TS_LAUNCH_E(dtype, combine_kernel, dim3((unsigned)((rows + kCombineTokens - 1) / kCombineTokens)),
+                dim3(kCombineThreads), 0, s, a.part_m, a.part_s, a.part_e, a.h, a.ldh, a.w, a.ldw, target, (int)rows,
+                (int)dim, a.n_vtiles, (int)vocab, logprob, entropy, lse);
+  }
   return ts::check_launch("ts_logprob_fwd (combine)");
 }
 
