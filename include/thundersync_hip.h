@@ -370,6 +370,17 @@ int ts_logprob_grad_weight(const void* dlogits, int64_t ld_dlogits, const void* 
                            int64_t ld_hidden, int64_t rows, int64_t dim, int64_t vocab,
                            float* grad_weight, int64_t ld_grad, int dtype, void* stream);
 
+/* One block of a weight gradient taken block by block: the fp32 sum of the
+ * earlier blocks (`accumulator`, not read when `first`) plus this block's
+ * dlogits^T . hidden, written to the accumulator, or, for the last block
+ * (`grad_weight` given), rounded to `dtype` into grad_weight [vocab, ld_grad].
+ * A gradient of a single block takes no accumulator (null).  The same sums as
+ * ts_logprob_grad_weight on a zeroed accumulator and one cast. */
+int ts_logprob_grad_weight_block(const void* dlogits, int64_t ld_dlogits, const void* hidden, int64_t ld_hidden,
+                                 int64_t rows, int64_t dim, int64_t vocab, float* accumulator,
+                                 int64_t ld_accumulator, int first, void* grad_weight, int64_t ld_grad, int dtype,
+                                 void* stream);
+
 /* ------------------------------------------------------------------------
  * Fused logprob / entropy at the inputs' precision (fp32 or fp64)
  *

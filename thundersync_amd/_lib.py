@@ -56,6 +56,8 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     ),
     "ts_logprob_grad_hidden_workspace": (_I64, [_I64, _I64, _I64]),
     "ts_logprob_grad_hidden": (_INT, [_P, _I64, _P, _I64, _I64, _I64, _I64, _P, _I64, _P, _I64, _INT, _P]),
+    "ts_logprob_grad_weight_block": (
+        _INT, [_P, _I64, _P, _I64, _I64, _I64, _I64, _P, _I64, _INT, _P, _I64, _INT, _P]),
     "ts_logprob_grad_weight": (_INT, [_P, _I64, _P, _I64, _I64, _I64, _I64, _P, _I64, _INT, _P]),
     "ts_logprob_fwd_exact_workspace": (_I64, [_I64, _I64, _INT]),
     "ts_logprob_fwd_exact": (_INT, [_P, _I64, _P, _I64, _P, _I64, _I64, _I64, _P, _P, _P, _P, _I64, _INT, _P]),

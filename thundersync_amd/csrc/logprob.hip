@@ -419,10 +419,17 @@ __global__ __launch_bounds__(kThreads) void grad_hidden_reduce_kernel(const floa
 }
 
 // ---------------------------------------------------------------------------
-// backward 3 (trainable head): grad_weight[v][d] += sum_n dl[n][v] h[n][d] in
-// fp32, as C = dl^T . h with both operands K-strided (K = the block's rows);
-// the epilogue adds the tile into the fp32 accumulator, so a call per block
-// accumulates across blocks in block order.
+// backward 3 (trainable head): grad_weight[v][d] = sum_n dl[n][v] h[n][d] as
+// C = dl^T . h with both operands K-strided (K = the block's rows), in fp32
+// over the blocks in block order.  The first block writes the fp32
+// accumulator without reading it and the last one adds it to its tile and
+// writes the gradient in the element type, so a gradient of one block needs
+// no accumulator and one of two blocks one write and one read of it, with no
+// zero fill before and no cast pass after.  A tile's epilogue is bound by the
+// accumulator's latency (nothing else runs on the CU meanwhile): it takes 16
+// accumulator values at a time, all loads before the first store.  4096 rows x
+// 2048 x 151936 in two blocks: 4.42 ms, a 0.16 ms fill and a 0.30 ms cast with
+// one read-add-write per value, 2.57 ms in all now (0.99 PFLOP/s).
 // ---------------------------------------------------------------------------
 struct DwArgs {
   const bf16* dl;   // [rows][ldl]
@@ -431,8 +438,11 @@ struct DwArgs {
   int64_t ldh;
   int rows, dim, vocab;
   int n_vtiles, n_dtiles;
-  float* gw;        // [vocab][ldg]
+  const float* gw_in;  // [vocab][ldg] the earlier blocks' sum, or null
+  float* gw;           // [vocab][ldg] the sum with this block, or null:
   int64_t ldg;
+  bf16* out;           // [vocab][ldo] rounded to the element type
+  int64_t ldo;
 };
 
 template <typename E>
@@ -452,12 +462,24 @@ __global__ __launch_bounds__(kGemmThreads, 1) void grad_weight_kernel(DwArgs p) 
     const int d = d0 + b_row(ni, lane, wn);
     if (d >= p.dim) continue;
 #pragma unroll
-    for (int mi = 0; mi < 4; ++mi)
+    for (int mi = 0; mi < 4; ++mi) {
+      // rows past the vocabulary read its last row and store nothing
+      if (p.gw_in) {
+        float g[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          g[i] = p.gw_in[(int64_t)min(v0 + a_row(mi, i, lane, wm), p.vocab - 1) * p.ldg + d];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[mi][ni][i] += g[i];
+      }
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         const int v = v0 + a_row(mi, i, lane, wm);
-        if (v < p.vocab) p.gw[(int64_t)v * p.ldg + d] += acc[mi][ni][i];
+        if (v >= p.vocab) continue;
+        if (p.gw) p.gw[(int64_t)v * p.ldg + d] = acc[mi][ni][i];
+        else reinterpret_cast<E*>(p.out)[(int64_t)v * p.ldo + d] = from_f<E>(acc[mi][ni][i]);
       }
+    }
   }
 }
 
@@ -656,18 +678,22 @@ int ts_logprob_grad_hidden(const void* dlogits, int64_t ld_dlogits, const void* 
                                 "logprob.grad_hidden_reduce_kernel");
 }
 
-int ts_logprob_grad_weight(const void* dlogits, int64_t ld_dlogits, const void* hidden, int64_t ld_hidden,
-                           int64_t rows, int64_t dim, int64_t vocab, float* grad_weight, int64_t ld_grad,
-                           int dtype, void* stream) {
+int ts_logprob_grad_weight_block(const void* dlogits, int64_t ld_dlogits, const void* hidden, int64_t ld_hidden,
+                                 int64_t rows, int64_t dim, int64_t vocab, float* accumulator,
+                                 int64_t ld_accumulator, int first, void* grad_weight, int64_t ld_grad, int dtype,
+                                 void* stream) {
   using namespace ts::lp;
   TS_CHECK_ARG(dtype == ts::kBF16 || dtype == ts::kF16, "ts_logprob_grad_weight: dtype %d (bf16 or fp16)", dtype);
   TS_CHECK_ARG(rows >= 0 && dim > 0 && vocab > 0 && rows < (1 << 30) && dim < (1 << 20) && vocab < (1 << 30),
                "ts_logprob_grad_weight: bad shape");
-  if (rows == 0) return TS_OK;
-  TS_CHECK_ARG(dlogits && hidden && grad_weight && ok16(dlogits) && ok16(hidden) && ld_dlogits % 8 == 0 &&
-                   ld_hidden % 8 == 0 && dim % 8 == 0 && ld_dlogits >= vocab && ld_hidden >= dim &&
-                   ld_grad >= dim,
+  if (rows == 0 && !first && !grad_weight) return TS_OK;
+  TS_CHECK_ARG(rows > 0, "ts_logprob_grad_weight: a first or last block without rows");
+  TS_CHECK_ARG(dlogits && hidden && ok16(dlogits) && ok16(hidden) && ld_dlogits % 8 == 0 && ld_hidden % 8 == 0 &&
+                   dim % 8 == 0 && ld_dlogits >= vocab && ld_hidden >= dim,
                "ts_logprob_grad_weight: alignment or leading dimensions");
+  TS_CHECK_ARG((accumulator || (first && grad_weight)) && (!accumulator || ld_accumulator >= dim) &&
+                   (!grad_weight || ld_grad >= dim),
+               "ts_logprob_grad_weight: no accumulator, or leading dimensions");
   TS_CHECK_ARG(31 * ld_dlogits < (1ll << 30) && 31 * ld_hidden < (1ll << 30),
                "ts_logprob_grad_weight: leading dimensions too large for 32-bit tile offsets");
   DwArgs a;
@@ -680,8 +706,11 @@ int ts_logprob_grad_weight(const void* dlogits, int64_t ld_dlogits, const void* 
   a.vocab = (int)vocab;
   a.n_vtiles = (int)((vocab + TM - 1) / TM);
   a.n_dtiles = (int)((dim + TN - 1) / TN);
-  a.gw = grad_weight;
-  a.ldg = ld_grad;
+  a.gw_in = first ? nullptr : accumulator;
+  a.gw = grad_weight ? nullptr : accumulator;
+  a.ldg = ld_accumulator;
+  a.out = (ts::bf16*)grad_weight;
+  a.ldo = ld_grad;
   TS_CHECK_ARG((int64_t)a.n_vtiles * a.n_dtiles < (1ll << 31), "ts_logprob_grad_weight: grid too large");
   {
     ts::TimedLaunch timed_("logprob.grad_weight_kernel", (hipStream_t)stream);
@@ -689,6 +718,14 @@ int ts_logprob_grad_weight(const void* dlogits, int64_t ld_dlogits, const void* 
                        (hipStream_t)stream, a);
   }
   return ts::check_launch("ts_logprob_grad_weight");
+}
+
+int ts_logprob_grad_weight(const void* dlogits, int64_t ld_dlogits, const void* hidden, int64_t ld_hidden,
+                           int64_t rows, int64_t dim, int64_t vocab, float* grad_weight, int64_t ld_grad,
+                           int dtype, void* stream) {
+  TS_CHECK_ARG(grad_weight || rows == 0, "ts_logprob_grad_weight: null grad_weight");
+  return ts_logprob_grad_weight_block(dlogits, ld_dlogits, hidden, ld_hidden, rows, dim, vocab, grad_weight, ld_grad,
+                                      0, nullptr, 0, dtype, stream);
 }
 
 }  // extern "C"

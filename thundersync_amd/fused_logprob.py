@@ -16,11 +16,11 @@ size of the reference's fp32 logit block of one): ``ts_logprob_dlogits`` recompu
 the logits and writes the block's bf16 dlogits (rounded to bf16 as the
 reference rounds its dlogits to the hidden dtype, FL:165 and :295);
 ``ts_logprob_grad_hidden`` multiplies them by the weight, read in place;
-when the head is trainable ``ts_logprob_grad_weight`` adds ``dl^T h`` into
-an fp32 accumulator, cast once at the end (FL:176-193).  Extra device memory
+when the head is trainable ``ts_logprob_grad_weight_block`` adds ``dl^T h`` into
+an fp32 accumulator, rounded once by the last block (FL:176-193).  Extra device memory
 is the ``[chunk, V]`` bf16 dlogits block plus a workspace of vocabulary-range
 partial sums for grad_hidden when one block's row tiles do not fill the GPU,
-and the fp32 ``[V, D]`` accumulator when the weight gradient is needed.
+and, for a weight gradient of more than one block, the fp32 ``[V, D]`` accumulator.
 
 bf16 or fp16 (one element type per call) on the MFMA kernels above; fp32
 and fp64 at their own precision, as the reference keeps them (FL:27-58):
@@ -227,9 +227,8 @@ def _backward(hidden, weight, target, lse, ent, grad_lp, grad_ent, chunk, needs_
     v = w.shape[0]
     vp = (v + 7) // 8 * 8
     grad_hidden = torch.empty_like(h)
-    grad_weight = torch.zeros(v, d, dtype=torch.float32, device=h.device) if needs_weight_grad else None
     if n == 0:
-        return grad_hidden[:, :d_in], (grad_weight[:, :d_in].to(weight.dtype) if grad_weight is not None else None)
+        return grad_hidden[:, :d_in], torch.zeros_like(weight) if needs_weight_grad else None
     stream = _lib.stream_of(h)
     code = _lib.dtype_code(h.dtype)
     block = backward_block_rows(n, chunk)
@@ -239,6 +238,9 @@ def _backward(hidden, weight, target, lse, ent, grad_lp, grad_ent, chunk, needs_
     tail = n % block
     ws_bytes = max(int(lib.ts_logprob_grad_hidden_workspace(rows, d, v)) for rows in {block, tail or block})
     ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=h.device)
+    # the weight gradient's fp32 sum over the blocks, which one block alone does not need
+    grad_weight = torch.empty(v, d, dtype=w.dtype, device=h.device) if needs_weight_grad else None
+    acc = torch.empty(v, d, dtype=torch.float32, device=h.device) if needs_weight_grad and n > block else None
     g_lp = grad_lp.to(torch.float32).contiguous()
     g_ent = grad_ent.to(torch.float32).contiguous() if grad_ent is not None else None
     for i in range(0, n, block):
@@ -263,19 +265,20 @@ def _backward(hidden, weight, target, lse, ent, grad_lp, grad_ent, chunk, needs_
                 f"ts_logprob_grad_hidden(rows={rows}, dim={d}, vocab={v})",
             )
         if grad_weight is not None:
-            # fp32 accumulation across blocks, cast once (FL:176-193)
+            # fp32 accumulation across blocks, rounded once, by the last (FL:176-193)
+            last = i + rows == n
             with operator_range("logprob_head_weight_vjp", role=device_role(h.device), rows=rows, hidden=d, vocab=v):
                 _lib.check(
-                    lib.ts_logprob_grad_weight(
-                        dl.data_ptr(), vp, hi.data_ptr(), h.stride(0), rows, d, v,
-                        grad_weight.data_ptr(), grad_weight.stride(0), code, stream,
+                    lib.ts_logprob_grad_weight_block(
+                        dl.data_ptr(), vp, hi.data_ptr(), h.stride(0), rows, d, v, _lib.ptr(acc), d, int(i == 0),
+                        grad_weight.data_ptr() if last else None, d, code, stream,
                     ),
-                    f"ts_logprob_grad_weight(rows={rows}, dim={d}, vocab={v})",
+                    f"ts_logprob_grad_weight_block(rows={rows}, dim={d}, vocab={v})",
                 )
     if d != d_in:
         grad_hidden = grad_hidden[:, :d_in].contiguous()
-        grad_weight = grad_weight[:, :d_in] if grad_weight is not None else None
-    return grad_hidden, (grad_weight.to(weight.dtype) if grad_weight is not None else None)
+        grad_weight = grad_weight[:, :d_in].contiguous() if grad_weight is not None else None
+    return grad_hidden, grad_weight
 
 
 class _FusedLinearLogprob(torch.autograd.Function):
