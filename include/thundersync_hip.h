@@ -205,6 +205,43 @@ int ts_attn_q_block(int group);
  * kernel, for launches with few work items). */
 int ts_attn_kv_block(int group, int head_dim);
 
+/* An attention layout as the caller describes it (host arrays) and the sizes
+ * of its tables: offsets in bytes into one blob, entry counts, the launch-order
+ * counts, the dS elements per head. */
+typedef struct ts_attn_layout {
+  int64_t q_rows;
+  int64_t n_spans;
+  int32_t hq, hkv, n_segs, n_runs;
+  int32_t kv_block; /* keys per dK/dV item */
+  int32_t reserved;
+  const int64_t* seg_q;     /* [n_segs][2]: first row, rows */
+  const int64_t* seg_span0; /* [n_segs + 1]: segment s has spans seg_span0[s] .. seg_span0[s + 1] - 1 */
+  const int32_t* spans;     /* [n_spans][2]: run, position of its first key in the segment's keys */
+  const int32_t* run_len;   /* [n_runs] */
+} ts_attn_layout;
+
+typedef struct ts_attn_layout_sizes {
+  int64_t bytes, segs, spans, visits, q_work, kv_work, dq_work, span_ds, visit_ds;
+  int64_t n_q_work, n_kv_work, n_dq_work;
+  int64_t n_q_long, n_kv_long, n_dq_long;
+  int64_t ds_head;
+} ts_attn_layout_sizes;
+
+/* Builds a layout's tables in `blob` (host memory, 8-byte aligned, to be
+ * uploaded as one piece): segments, spans, visits, the forward / dK/dV / dQ work
+ * lists in launch order and ts_attn_ds_layout's offsets, at the offsets in
+ * `sizes`; run_visits [n_runs][2] receives each run's (visit0, nvisit).  With a
+ * null blob only the sizes and counts are computed.  No counterpart in the
+ * reference. */
+int ts_attn_layout_tables(const ts_attn_layout* layout, void* blob, int64_t blob_bytes, int32_t* run_visits,
+                          ts_attn_layout_sizes* sizes);
+
+/* One call's run table (host memory): run r is rows run_offset[r] .. +
+ * run_len[r] of source run_source[r], given as sources [n_sources][12]: for k,
+ * v, dk, dv the address (0: none), row stride and head stride in elements. */
+int ts_attn_run_table(int32_t n_runs, const int32_t* run_len, const int32_t* run_source, const int64_t* run_offset,
+                      const int32_t* run_visits, int32_t n_sources, const int64_t* sources, ts_attn_run* runs);
+
 /* Host-side consistency check of a problem's tables, given as host copies
  * of the arrays the problem's device pointers name (those pointers are not
  * read): segment rows inside [0, q_rows) and kv_len >= q_len; each

@@ -55,5 +55,33 @@ class AttnRows(ctypes.Structure):
     _fields_ = [("ptr", ctypes.c_uint64), ("row_stride", ctypes.c_int64), ("head_stride", ctypes.c_int64)]
 
 
+class AttnLayoutDesc(ctypes.Structure):
+    """ts_attn_layout"""
+
+    _fields_ = [
+        ("q_rows", ctypes.c_int64),
+        ("n_spans", ctypes.c_int64),
+        ("hq", ctypes.c_int32),
+        ("hkv", ctypes.c_int32),
+        ("n_segs", ctypes.c_int32),
+        ("n_runs", ctypes.c_int32),
+        ("kv_block", ctypes.c_int32),
+        ("reserved", ctypes.c_int32),
+        ("seg_q", ctypes.c_void_p),
+        ("seg_span0", ctypes.c_void_p),
+        ("spans", ctypes.c_void_p),
+        ("run_len", ctypes.c_void_p),
+    ]
+
+
+class AttnLayoutSizes(ctypes.Structure):
+    """ts_attn_layout_sizes"""
+
+    _fields_ = [(name, ctypes.c_int64) for name in (
+        "bytes", "segs", "spans", "visits", "q_work", "kv_work", "dq_work", "span_ds", "visit_ds", "n_q_work",
+        "n_kv_work", "n_dq_work", "n_q_long", "n_kv_long", "n_dq_long", "ds_head")]
+
+
 assert SEG_DTYPE.itemsize == 24 and REF_DTYPE.itemsize == 8 and RUN_DTYPE.itemsize == 112
 assert ctypes.sizeof(AttnProblem) == 112 and ctypes.sizeof(AttnRows) == 24
+assert ctypes.sizeof(AttnLayoutDesc) == 72 and ctypes.sizeof(AttnLayoutSizes) == 128

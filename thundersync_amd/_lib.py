@@ -23,7 +23,7 @@ import os
 import threading
 from pathlib import Path
 
-from ._abi import AttnProblem, AttnRows
+from ._abi import AttnLayoutDesc, AttnLayoutSizes, AttnProblem, AttnRows
 
 HIP_ENV = "THUNDERSYNC_HIP"
 HIP_SETTINGS = ("require", "off", "auto")
@@ -83,6 +83,8 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "ts_attn_heads_per_block": (_INT, [_INT]),
     "ts_attn_kv_block": (_INT, [_INT, _INT]),
     "ts_attn_q_block": (_INT, [_INT]),
+    "ts_attn_layout_tables": (_INT, [ctypes.POINTER(AttnLayoutDesc), _P, _I64, _P, ctypes.POINTER(AttnLayoutSizes)]),
+    "ts_attn_run_table": (_INT, [ctypes.c_int32, _P, _P, _P, _P, ctypes.c_int32, _P, _P]),
     "ts_attn_check_tables": (_INT, [ctypes.POINTER(AttnProblem), _P, _P, _I64, _P, _P, _I64, _P, _P]),
     "ts_attn_fwd": (_INT, [ctypes.POINTER(AttnProblem), AttnRows, AttnRows, _P, _I64, _P]),
     "ts_attn_bwd": (

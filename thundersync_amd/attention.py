@@ -53,6 +53,7 @@ import ctypes
 import math
 import os
 import threading
+from array import array
 from collections.abc import Sequence
 from dataclasses import dataclass, field
 
@@ -60,7 +61,7 @@ import numpy as np
 import torch
 
 from . import _lib
-from ._abi import REF_DTYPE, RUN_DTYPE, SEG_DTYPE, AttnProblem, AttnRows
+from ._abi import REF_DTYPE, RUN_DTYPE, SEG_DTYPE, AttnLayoutDesc, AttnLayoutSizes, AttnProblem, AttnRows
 from .dispatch import HIP_BACKWARD_PATH, HIP_PATH, count_attention_path
 from .operator_profiling import operator_range
 
@@ -126,6 +127,7 @@ class AttnLayout:
     seg_kv: tuple[int, ...] = field(init=False)
     _tables: dict = field(default_factory=dict, init=False, repr=False)
     _lock: threading.Lock = field(default_factory=threading.Lock, init=False, repr=False)
+    _desc: dict | None = field(default=None, init=False, repr=False)
 
     def __post_init__(self):
         if self.hq <= 0 or self.hkv <= 0 or self.hq % self.hkv:
@@ -169,173 +171,153 @@ class AttnLayout:
         if max([*self.seg_kv, 0]) >= 2**31 or self.q_rows >= 2**40:
             raise ValueError("attention problem too large")
 
-    # -- work lists ---------------------------------------------------------
+    # -- tables -------------------------------------------------------------
+    def _description(self) -> dict:
+        """The layout as the native table builder takes it (host arrays and
+        their addresses), made once."""
+        d = self._desc
+        if d is None:
+            seg_q = np.array(self.seg_q, np.int64).reshape(-1, 2)
+            seg_span0 = np.zeros(len(self.seg_spans) + 1, np.int64)
+            np.cumsum([len(sp) for sp in self.seg_spans], out=seg_span0[1:])
+            spans = np.array([x for sp in self.seg_spans for x in sp], np.int32).reshape(-1, 2)
+            runs = np.array([(r.source, r.offset, r.length) for r in self.runs], np.int64).reshape(-1, 3)
+            run_len, run_source = runs[:, 2].astype(np.int32), runs[:, 0].astype(np.int32)
+            run_offset = runs[:, 1].copy()
+            nvisit = np.bincount(spans[:, 0], minlength=len(self.runs))
+            # rows of each source that a visited run covers (runs do not overlap)
+            covered = np.bincount(run_source, weights=np.where(nvisit > 0, run_len, 0),
+                                  minlength=len(self.source_rows)).astype(np.int64)
+            d = {
+                "arrays": (seg_q, seg_span0, spans, run_len, run_source, run_offset),
+                "ptrs": tuple(a.ctypes.data for a in (seg_q, seg_span0, spans, run_len, run_source, run_offset)),
+                "n_spans": int(spans.shape[0]),
+                "visited_lengths": run_len[nvisit > 0],
+                # sources with rows that no visited run covers: their gradients are filled with zeros first
+                "uncovered": [i for i, n in enumerate(self.source_rows) if covered[i] != n],
+                "all_rows": int(seg_q[:, 1].sum()) == self.q_rows,
+            }
+            self._desc = d
+        return d
+
+    def _build(self, kvb: int, alloc, extra: int = 0):
+        """(sizes, buffer from ``alloc(bytes)``, its numpy view, run_visits): the
+        layout's tables at the start of the buffer, ``extra`` bytes after them."""
+        lib = _lib.require_library()
+        d = self._description()
+        p = d["ptrs"]
+        desc = AttnLayoutDesc(self.q_rows, d["n_spans"], self.hq, self.hkv, len(self.seg_q), len(self.runs), kvb, 0,
+                              p[0], p[1], p[2], p[3])
+        sizes = AttnLayoutSizes()
+        _lib.check(lib.ts_attn_layout_tables(ctypes.byref(desc), None, 0, None, ctypes.byref(sizes)),
+                   "ts_attn_layout_tables")
+        buf = alloc(sizes.bytes + extra)
+        view = buf if isinstance(buf, np.ndarray) else buf.numpy()
+        run_visits = np.zeros((max(len(self.runs), 1), 2), np.int32)
+        _lib.check(lib.ts_attn_layout_tables(ctypes.byref(desc), view.ctypes.data, sizes.bytes,
+                                             run_visits.ctypes.data, ctypes.byref(sizes)), "ts_attn_layout_tables")
+        return sizes, buf, view, run_visits
+
+    def _views(self, sizes: AttnLayoutSizes, view: np.ndarray):
+        """(segs, spans, visits, q_work, kv_work, dq_work) as views of a table buffer."""
+        n = self._description()["n_spans"]
+
+        def part(offset, count, dtype):
+            return view[offset : offset + count * dtype.itemsize].view(dtype)
+
+        pair = np.dtype(np.int32)
+        return (part(sizes.segs, len(self.seg_q), SEG_DTYPE), part(sizes.spans, n, REF_DTYPE),
+                part(sizes.visits, n, REF_DTYPE), part(sizes.q_work, 2 * sizes.n_q_work, pair).reshape(-1, 2),
+                part(sizes.kv_work, 2 * sizes.n_kv_work, pair).reshape(-1, 2),
+                part(sizes.dq_work, 2 * sizes.n_dq_work, pair).reshape(-1, 2))
+
     def _host_tables(self, kvb: int | None = None):
-        qb = q_block_rows(self.hq, self.hkv)
-        segs = np.zeros(len(self.seg_q), SEG_DTYPE)
-        spans, visits_of = [], [[] for _ in self.runs]
-        q_items = []
-        for s, ((row0, length), sp) in enumerate(zip(self.seg_q, self.seg_spans)):
-            segs[s] = (row0, length, self.seg_kv[s], len(spans), len(sp))
-            for run, kpos in sp:
-                spans.append((run, kpos))
-                visits_of[run].append((s, kpos))
-            off = self.seg_kv[s] - length
-            for q0 in range(0, length, qb):
-                # visible keys of the block's last row: the block's cost
-                last = min(q0 + qb, length) - 1
-                q_items.append((-(off + last + 1), s, q0))
-        visit_rows, visit0 = [], []
-        for run, vis in enumerate(visits_of):
-            visit0.append(len(visit_rows))
-            visit_rows.extend(vis)
-        # dK/dV items: every kvb-key block of every visited run; its cost is
-        # the number of query rows that see its first key, over its visits
         kvb = kv_block_keys(self.hq, self.hkv) if kvb is None else kvb
-        seg_len = np.array([n for _, n in self.seg_q], np.int64)
-        seg_off = np.array(self.seg_kv, np.int64) - seg_len
-        kv_cost, kv_run, kv_k0 = [], [], []
-        for run, vis in enumerate(visits_of):
-            if not vis:
-                continue
-            k0 = np.arange(0, self.runs[run].length, kvb, dtype=np.int64)
-            seg = np.array([s for s, _ in vis], np.int64)
-            kpos = np.array([kp for _, kp in vis], np.int64)
-            q_len, off = seg_len[seg], seg_off[seg]
-            first_row = np.maximum(0, kpos[None, :] + k0[:, None] - off[None, :])
-            kv_cost.append(np.maximum(0, q_len[None, :] - first_row).sum(axis=1))
-            kv_run.append(np.full(k0.shape, run, np.int64))
-            kv_k0.append(k0)
-        # longest cost band first, then segment and row (ORDER_BAND)
-        if q_items:
-            qa = np.array(q_items, np.int64).reshape(-1, 3)
-            q_items = [q_items[i] for i in np.lexsort((qa[:, 2], qa[:, 1], -_cost_band(-qa[:, 0])))]
-        q_work = np.array([(s, q0) for _, s, q0 in q_items], np.int32).reshape(-1, 2)
-        if kv_cost:
-            cost, run_of, k0_of = (np.concatenate(x) for x in (kv_cost, kv_run, kv_k0))
-            order = np.lexsort((k0_of, run_of, -_cost_band(cost)))  # cost band descending, then run, then k0
-            kv_work = np.stack([run_of[order], k0_of[order]], axis=1).astype(np.int32)
-            kv_costs = cost[order].tolist()
-        else:
-            kv_work = np.zeros((0, 2), np.int32)
-            kv_costs = []
-        group = self.hq // self.hkv
-        # rows the forward / dQ work-groups re-read: K and V of every run; the
-        # dK/dV work-groups: Q and dO of every row (2-byte elements, all heads)
-        kv_bytes = sum(run.length for run in self.runs) * self.hkv * HEAD_DIM * 2 * 2
-        q_bytes = self.q_rows * self.hq * HEAD_DIM * 2 * 2
-        q_long = _long_items([-c for c, _, _ in q_items], self.hkv * (group // heads_per_block(group)), kv_bytes)
-        kv_long = _long_items(kv_costs, self.hkv, q_bytes)
-        # the dS route's dQ pass over 64-row items (GQA groups that are a
-        # multiple of 4): a dQ work-group then shares its K tiles between the
-        # two 32-row blocks of its four heads
-        dq_work, dq_long = np.zeros((0, 2), np.int32), 0
-        if group % 4 == 0:
-            dq_items = []
-            for s_, ((_, length), kv) in enumerate(zip(self.seg_q, self.seg_kv)):
-                for q0 in range(0, length, DQ_BLOCK_ROWS):
-                    dq_items.append((-(kv - length + min(q0 + DQ_BLOCK_ROWS, length)), s_, q0))
-            if dq_items:
-                da = np.array(dq_items, np.int64).reshape(-1, 3)
-                dq_items = [dq_items[i] for i in np.lexsort((da[:, 2], da[:, 1], -_cost_band(-da[:, 0])))]
-                dq_work = np.array([(s_, q0) for _, s_, q0 in dq_items], np.int32).reshape(-1, 2)
-                dq_long = _long_items([-c for c, _, _ in dq_items], self.hkv * (group // 4), kv_bytes)
-        seg_spans = np.array(spans, REF_DTYPE) if spans else np.zeros(0, REF_DTYPE)
-        run_visits = np.array(visit_rows, REF_DTYPE) if visit_rows else np.zeros(0, REF_DTYPE)
-        return (segs, seg_spans, run_visits, q_work, kv_work, visit0, [len(v) for v in visits_of],
-                q_long, kv_long, dq_work, dq_long)
+        sizes, _, view, run_visits = self._build(kvb, lambda n: np.zeros(n, np.uint8))
+        segs, spans, visits, q_work, kv_work, dq_work = self._views(sizes, view)
+        rv = run_visits[: len(self.runs)]
+        return (segs, spans, visits, q_work, kv_work, rv[:, 0].tolist(), rv[:, 1].tolist(),
+                int(sizes.n_q_long), int(sizes.n_kv_long), dq_work, int(sizes.n_dq_long))
+
+    def _fill_runs(self, tabs: dict, sources: Sequence[int], out: np.ndarray) -> None:
+        """One call's run table into ``out`` (``sources``: ts_attn_run_table's)."""
+        p = self._description()["ptrs"]
+        src = array("q", sources)
+        _lib.check(
+            _lib.require_library().ts_attn_run_table(
+                len(self.runs), p[3], p[4], p[5], tabs["run_visits_ptr"], len(self.source_rows),
+                src.buffer_info()[0] if len(src) else None, out.ctypes.data if len(self.runs) else None),
+            "ts_attn_run_table",
+        )
+
+    def _upload(self, device: torch.device, kvb: int, sources: Sequence[int] | None):
+        """(tables, run table): the layout's tables on ``device``, built and
+        uploaded once per device and dK/dV item size, and, with ``sources``, one
+        call's run table as (device address, host bytes, tensors to keep).  Both
+        go through pinned memory without blocking, in one piece when the layout
+        is new."""
+        key = (device.type, device.index, kvb)
+        run_bytes = len(self.runs) * RUN_DTYPE.itemsize if sources is not None else 0
+
+        def alloc(n):
+            return torch.empty(max(n, 16), dtype=torch.uint8, pin_memory=device.type == "cuda")
+
+        tabs = self._tables.get(key)
+        if tabs is None:
+            with self._lock:
+                tabs = self._tables.get(key)
+                if tabs is None:
+                    sizes, host, view, run_visits = self._build(kvb, alloc, run_bytes)
+                    segs, spans, visits, q_work, kv_work, _ = self._views(sizes, view)
+                    n = self._description()["n_spans"]
+                    tabs = {
+                        "run_visits": run_visits,
+                        "run_visits_ptr": run_visits.ctypes.data,
+                        "arrays": (segs, spans, visits, q_work, kv_work),
+                        "array_ptrs": tuple(a.ctypes.data if a.size else None
+                                            for a in (segs, spans, visits, q_work, kv_work)),
+                        "visit0": run_visits[: len(self.runs), 0].tolist(),
+                        "nvisit": run_visits[: len(self.runs), 1].tolist(),
+                        "n_q_work": int(sizes.n_q_work), "n_kv_work": int(sizes.n_kv_work),
+                        "n_dq_work": int(sizes.n_dq_work), "n_q_long": int(sizes.n_q_long),
+                        "n_kv_long": int(sizes.n_kv_long), "n_dq_long": int(sizes.n_dq_long),
+                        "head": int(sizes.ds_head),
+                        "span_ds": view[sizes.span_ds : sizes.span_ds + 8 * n].view(np.int64),
+                        "visit_ds": view[sizes.visit_ds : sizes.visit_ds + 8 * n].view(np.int64),
+                    }
+                    if run_bytes:
+                        self._fill_runs(tabs, sources, view[sizes.bytes :])
+                    dev = host.to(device, non_blocking=True)
+                    base = dev.data_ptr()
+                    tabs.update(
+                        blob=dev, host=host, segs=base + sizes.segs, seg_spans=base + sizes.spans,
+                        run_visits_dev=base + sizes.visits, q_work=base + sizes.q_work, kv_work=base + sizes.kv_work,
+                        dq_work=base + sizes.dq_work if sizes.n_dq_work else None,
+                        span=base + sizes.span_ds, visit=base + sizes.visit_ds,
+                    )
+                    self._tables[key] = tabs
+                    if sources is not None:
+                        return tabs, (base + sizes.bytes, view[sizes.bytes : sizes.bytes + run_bytes], (dev, host))
+        if sources is None:
+            return tabs, None
+        host = alloc(run_bytes)
+        view = host.numpy()
+        self._fill_runs(tabs, sources, view)
+        dev = host.to(device, non_blocking=True)
+        return tabs, (dev.data_ptr(), view[:run_bytes], (dev, host))
 
     def device_tables(self, device: torch.device, kv_block: int | None = None):
-        """Upload the layout's integer tables once per device and dK/dV item
-        size (pinned, non-blocking); `kv_block` None: the head-dim-128 size."""
+        """The layout's integer tables on ``device``, uploaded once per device
+        and dK/dV item size (pinned, non-blocking); `kv_block` None: the
+        head-dim-128 size."""
         kvb = kv_block_keys(self.hq, self.hkv) if kv_block is None else int(kv_block)
-        key = (device.type, device.index, kvb)
-        hit = self._tables.get(key)
-        if hit is not None:
-            return hit
-        with self._lock:
-            hit = self._tables.get(key)
-            if hit is None:
-                (segs, spans, visits, q_work, kv_work, visit0, nvisit, q_long, kv_long, dq_work,
-                 dq_long) = self._host_tables(kvb)
-                parts = [segs.view(np.uint8), spans.view(np.uint8), visits.view(np.uint8),
-                         q_work.view(np.uint8).reshape(-1), kv_work.view(np.uint8).reshape(-1),
-                         dq_work.view(np.uint8).reshape(-1)]
-                offsets, total = [], 0
-                for p in parts:
-                    offsets.append(total)
-                    total += (p.size + 255) // 256 * 256
-                blob = np.zeros(max(total, 256), np.uint8)
-                for o, p in zip(offsets, parts):
-                    blob[o : o + p.size] = p
-                host = torch.from_numpy(blob).pin_memory() if device.type == "cuda" else torch.from_numpy(blob)
-                dev = host.to(device, non_blocking=True)
-                base = dev.data_ptr()
-                hit = {
-                    "blob": dev,
-                    "host": host,
-                    "arrays": (segs, spans, visits, q_work, kv_work),
-                    "segs": base + offsets[0],
-                    "seg_spans": base + offsets[1],
-                    "run_visits": base + offsets[2],
-                    "q_work": base + offsets[3],
-                    "kv_work": base + offsets[4],
-                    "dq_work": base + offsets[5] if dq_work.shape[0] else None,
-                    "n_dq_work": int(dq_work.shape[0]),
-                    "n_dq_long": int(dq_long),
-                    "n_q_work": int(q_work.shape[0]),
-                    "n_kv_work": int(kv_work.shape[0]),
-                    "visit0": visit0,
-                    "nvisit": nvisit,
-                    "n_q_long": q_long,
-                    "n_kv_long": kv_long,
-                }
-                self._tables[key] = hit
-        return hit
+        return self._upload(device, kvb, None)[0]
 
-    def ds_tables(self, device: torch.device) -> dict:
-        """The dS route's workspace layout (``ts_attn_ds_layout``): elements per
-        head and the per-span / per-visit offsets, uploaded once per device."""
-        key = ("ds", device.type, device.index)
-        hit = self._tables.get(key)
-        if hit is not None:
-            return hit
-        tabs = self.device_tables(device)
-        with self._lock:
-            hit = self._tables.get(key)
-            if hit is None:
-                segs, spans, visits, _, _ = tabs["arrays"]
-                run_len = np.array([r.length for r in self.runs], np.int32)
-                visit0 = np.array(tabs["visit0"], np.int32)
-                nvisit = np.array(tabs["nvisit"], np.int32)
-                span_ds = np.zeros(max(spans.shape[0], 1), np.int64)
-                visit_ds = np.zeros(max(visits.shape[0], 1), np.int64)
-                head = ctypes.c_int64(0)
-
-                def ptr(a):
-                    return a.ctypes.data if a.size else None
-
-                lib = _lib.require_library()
-                _lib.check(
-                    lib.ts_attn_ds_layout(ptr(segs), len(segs), ptr(spans), spans.shape[0], ptr(run_len),
-                                          len(run_len), ptr(visits), ptr(visit0), ptr(nvisit), visits.shape[0],
-                                          span_ds.ctypes.data, visit_ds.ctypes.data, ctypes.byref(head)),
-                    "ts_attn_ds_layout",
-                )
-                blob = np.concatenate([span_ds, visit_ds])
-                host = torch.from_numpy(blob).pin_memory() if device.type == "cuda" else torch.from_numpy(blob)
-                dev = host.to(device, non_blocking=True)
-                hit = {
-                    "blob": dev,
-                    "host": host,
-                    "head": int(head.value),
-                    "span": dev.data_ptr(),
-                    "visit": dev.data_ptr() + 8 * span_ds.shape[0],
-                    "span_ds": span_ds[: spans.shape[0]],
-                    "visit_ds": visit_ds[: visits.shape[0]],
-                }
-                self._tables[key] = hit
-        return hit
+    def ds_tables(self, device: torch.device, kv_block: int | None = None) -> dict:
+        """The dS route's workspace layout: elements per head ("head") and the
+        per-span / per-visit element offsets on the device ("span", "visit") and
+        the host ("span_ds", "visit_ds"); part of the layout's tables."""
+        return self.device_tables(device, kv_block)
 
     def kv_block_for(self, device, head_dim: int) -> int:
         """Keys per dK/dV work item at `head_dim`: ts_attn_kv_block's, except
@@ -344,8 +326,7 @@ class AttnLayout:
         kernel)."""
         kvb = kv_block_keys(self.hq, self.hkv, head_dim)
         if head_dim == 256:
-            nvisit = self.device_tables(device)["nvisit"]
-            n64 = sum((run.length + 63) // 64 for run, nv in zip(self.runs, nvisit) if nv)
+            n64 = int(((self._description()["visited_lengths"].astype(np.int64) + 63) // 64).sum())
             if n64 * self.hkv < DKDV256_MIN_ITEMS:
                 kvb = 48
         return kvb
@@ -355,7 +336,7 @@ class AttnLayout:
         kvb = self.kv_block_for(device, int(head_dim))
         t = self.device_tables(device, kvb)
         return AttnProblem(
-            t["segs"], t["seg_spans"], runs_ptr, t["run_visits"], t["q_work"], t["kv_work"],
+            t["segs"], t["seg_spans"], runs_ptr, t["run_visits_dev"], t["q_work"], t["kv_work"],
             t["n_q_work"], t["n_kv_work"], len(self.seg_q), len(self.runs), self.hq, self.hkv,
             int(head_dim), float(scale), q_block_rows(self.hq, self.hkv), kvb, self.q_rows,
             t["n_q_long"], t["n_kv_long"], _lib.dtype_code(dtype),
@@ -370,12 +351,6 @@ class AttnLayout:
         return total
 
 
-# MI355X: work-group slots of one launch (256 CUs, one attention work-group
-# each) and the last-level cache shared by the 8 XCDs
-LAUNCH_SLOTS = 256
-SHARED_CACHE_BYTES = 256 << 20
-
-
 # Work items are launched in bands of costs within ORDER_BAND of each other
 # (geometric), longest band first, and within a band by run (dK/dV) or
 # segment (forward, dQ) and position: neighbours in the list, which the
@@ -383,36 +358,16 @@ SHARED_CACHE_BYTES = 256 << 20
 # its L2, while the longest-first order that keeps the end of the launch
 # short changes by at most ORDER_BAND.  (C4: dK/dV 34.3 -> 32.4 ms, forward
 # 11.85 -> 11.62 ms, dQ 10.7 -> 10.0 ms; C2 within noise.)
+#
+# The first n_*_long items of a list run item-major at the head of the launch:
+# when the rows the work-groups re-read (all heads) fit in half the shared
+# last-level cache (256 MB), every item does -- each XCD then serves fixed heads
+# and keeps their rows in its L2 while the shared cache holds the rest.
+# Otherwise only the items long enough to stretch the end of the launch when
+# started late -- a quarter or more of a slot's average share of the whole
+# launch -- and the rest run head by head, all XCDs streaming one head's rows
+# through the shared cache.  (ts_attn_layout_tables builds the lists.)
 ORDER_BAND = 0.05
-
-
-def _cost_band(cost: np.ndarray) -> np.ndarray:
-    """Index of each cost's geometric band of width ORDER_BAND (higher for larger costs)."""
-    return np.floor(np.log(np.maximum(cost, 1)) / np.log(1.0 + ORDER_BAND)).astype(np.int64)
-
-
-def _long_items(costs: Sequence[int], heads: int, reread_bytes: int, slots: int = LAUNCH_SLOTS) -> int:
-    """How many of the (descending) ``costs`` run item-major at the head of the
-    launch (ts_attn_problem.n_*_long).
-
-    When the rows the work-groups re-read (``reread_bytes``, all heads) fit in
-    half the shared last-level cache, every item does: each XCD then serves
-    fixed heads and keeps their rows in its L2 while the shared cache holds
-    the rest.  Otherwise only the items long enough to stretch the end of the
-    launch when started late -- a quarter or more of a slot's average share
-    of the whole launch (``heads`` copies of every item) -- and the rest run
-    head by head, all XCDs streaming one head's rows through the shared cache.
-    """
-    if reread_bytes <= SHARED_CACHE_BYTES // 2:
-        return len(costs)
-    total = sum(costs) * heads
-    if not costs or total == 0:
-        return 0
-    threshold = 0.25 * total / slots
-    n = 0
-    while n < len(costs) and costs[n] >= threshold:
-        n += 1
-    return n
 
 
 def _check_rows_tensor(t: torch.Tensor, name: str, heads: int, head_dim: int, max_row_stride: int = 1 << 24) -> None:
@@ -429,30 +384,6 @@ def _rows(t: torch.Tensor) -> AttnRows:
     return AttnRows(t.data_ptr(), t.stride(0), t.stride(1))
 
 
-def _run_table(layout: AttnLayout, keys, values, dkeys=None, dvalues=None) -> torch.Tensor:
-    visit = layout.device_tables(keys[0].device)
-    table = np.zeros(len(layout.runs), RUN_DTYPE)
-    esz = 2
-    for r, run in enumerate(layout.runs):
-        k, v = keys[run.source], values[run.source]
-        row = table[r]
-        row["k"] = k.data_ptr() + run.offset * k.stride(0) * esz
-        row["v"] = v.data_ptr() + run.offset * v.stride(0) * esz
-        row["k_row_stride"], row["k_head_stride"] = k.stride(0), k.stride(1)
-        row["v_row_stride"], row["v_head_stride"] = v.stride(0), v.stride(1)
-        if dkeys is not None:
-            dk, dv = dkeys[run.source], dvalues[run.source]
-            row["dk"] = dk.data_ptr() + run.offset * dk.stride(0) * esz
-            row["dv"] = dv.data_ptr() + run.offset * dv.stride(0) * esz
-            row["dk_row_stride"], row["dk_head_stride"] = dk.stride(0), dk.stride(1)
-            row["dv_row_stride"], row["dv_head_stride"] = dv.stride(0), dv.stride(1)
-        row["len"] = run.length
-        row["visit0"] = visit["visit0"][r]
-        row["nvisit"] = visit["nvisit"][r]
-    host = torch.from_numpy(table.view(np.uint8)).pin_memory()
-    return host.to(keys[0].device, non_blocking=True), host
-
-
 def check_tables(layout: AttnLayout, problem: AttnProblem, run_table: np.ndarray | torch.Tensor,
                  device: torch.device) -> None:
     """Check the layout's tables for ``device`` and one call's run table on the
@@ -460,18 +391,18 @@ def check_tables(layout: AttnLayout, problem: AttnProblem, run_table: np.ndarray
     spans tile every segment's keys, every visit is a span of its segment,
     the work lists hold every row and key block once, K/V/dK/dV addresses are
     aligned.  Raises RuntimeError naming the first inconsistency."""
-    segs, spans, visits, q_work, kv_work = layout.device_tables(device, problem.kv_block)["arrays"]
+    tabs = layout.device_tables(device, problem.kv_block)
     runs = run_table.numpy() if isinstance(run_table, torch.Tensor) else run_table
     runs = np.ascontiguousarray(runs).view(np.uint8)
     if runs.size != len(layout.runs) * RUN_DTYPE.itemsize:
         raise ValueError(f"run table holds {runs.size} bytes, expected {len(layout.runs)} runs")
-    arrays = (segs, spans, runs, visits, q_work, kv_work)
-    segs_p, spans_p, runs_p, visits_p, q_p, kv_p = (a.ctypes.data if a.size else None for a in arrays)
+    segs, spans, visits, q_work, kv_work = tabs["array_ptrs"]
+    n_spans = layout._description()["n_spans"]
     lib = _lib.require_library()
     _lib.check(
-        lib.ts_attn_check_tables(ctypes.byref(problem), segs_p, spans_p, spans.shape[0], runs_p, visits_p,
-                                 visits.shape[0], q_p, kv_p),
-        f"attention tables (rows={layout.q_rows}, segments={len(layout.seg_q)}, runs={len(layout.runs)})",
+        lib.ts_attn_check_tables(ctypes.byref(problem), segs, spans, n_spans, runs.ctypes.data if runs.size else None,
+                                 visits, n_spans, q_work, kv_work),
+        lambda: f"attention tables (rows={layout.q_rows}, segments={len(layout.seg_q)}, runs={len(layout.runs)})",
     )
 
 
@@ -525,8 +456,17 @@ def _device_free_bytes(device: torch.device) -> int:
     if device.type != "cuda":
         return 0
     free, _total = torch.cuda.mem_get_info(device)
-    cached = torch.cuda.memory_reserved(device) - torch.cuda.memory_allocated(device)
-    return int(free) + max(int(cached), 0)
+    return int(free) + _device_cached_bytes(device)
+
+
+def _device_cached_bytes(device: torch.device) -> int:
+    """Bytes torch's allocator holds on `device` unallocated (0 for a host device)."""
+    if device.type != "cuda":
+        return 0
+    stats = torch.cuda.memory_stats_as_nested_dict(device)
+    if not stats:
+        return 0
+    return max(int(stats["reserved_bytes"]["all"]["current"]) - int(stats["allocated_bytes"]["all"]["current"]), 0)
 
 
 def _ds_route(layout: AttnLayout, query: torch.Tensor, lib):
@@ -537,10 +477,13 @@ def _ds_route(layout: AttnLayout, query: torch.Tensor, lib):
     group = layout.hq // layout.hkv
     if not lib.ts_attn_ds_route(query.shape[2], group):
         return None
-    tabs = layout.ds_tables(query.device)
+    tabs = layout.ds_tables(query.device, layout.kv_block_for(query.device, query.shape[2]))
     # a call over n KV heads needs (n * group * head + 512) elements: every
     # query head's part, then the sink block
     per_kv_head = group * max(tabs["head"], 1)
+    need = (layout.hkv * per_kv_head + 512) * 2
+    if need <= DS_MAX_BYTES and need <= int(_device_cached_bytes(query.device) * DS_AVAILABLE_FRACTION):
+        return tabs, layout.hkv  # the allocator's unused memory alone is enough: the device need not be asked
     available = _device_free_bytes(query.device)
     cap = DS_MAX_BYTES
     if (layout.hkv * per_kv_head + 512) * 2 > cap and DS_FREE_FRACTION > 0:
@@ -557,9 +500,9 @@ def _head_rows(rows: AttnRows, first_head: int) -> AttnRows:
     return AttnRows(rows.ptr + first_head * rows.head_stride * 2, rows.row_stride, rows.head_stride)
 
 
-def _head_runs(host: torch.Tensor, first_kv_head: int, device) -> tuple[torch.Tensor, torch.Tensor]:
+def _head_runs(host: np.ndarray, first_kv_head: int, device) -> tuple[torch.Tensor, torch.Tensor]:
     """A copy of a run table whose K/V/dK/dV addresses start at KV head `first_kv_head`."""
-    table = host.numpy().view(RUN_DTYPE).copy()
+    table = host.view(RUN_DTYPE).copy()
     for name in ("k", "v", "dk", "dv"):
         live = table[name] != 0
         table[name][live] += (first_kv_head * table[f"{name}_head_stride"][live] * 2).astype(np.uint64)
@@ -568,28 +511,134 @@ def _head_runs(host: torch.Tensor, first_kv_head: int, device) -> tuple[torch.Te
     return sub.to(device, non_blocking=True), sub
 
 
+def _gather(layout: AttnLayout, query: torch.Tensor, keys, values) -> list[int]:
+    """Validate a call's tensors and list its K/V sources for the run table
+    (12 numbers a source: k, v, dk, dv as address, row stride, head stride; the
+    gradients zero).  Raises as :func:`_validate_call`, which the tests of one
+    look per tensor below stand for."""
+    if not query.is_cuda or query.dim() != 3 or len(keys) != len(layout.source_rows) or len(values) != len(keys):
+        _validate_call(layout, query, keys, values)
+    dtype, device, hkv, d = query.dtype, query.device, layout.hkv, query.shape[2]
+    qs = query.stride()
+    plain = (dtype in ELEMENT_DTYPES and d in HEAD_DIMS and query.shape == (layout.q_rows, layout.hq, d)
+             and qs[2] == 1 and not (qs[0] | qs[1]) & 7 and not query.data_ptr() & 15 and qs[0] < 1 << 24)
+    out: list[int] = []
+    for n, k, v in zip(layout.source_rows, keys, values):
+        ks, vs, kp, vp = k.stride(), v.stride(), k.data_ptr(), v.data_ptr()
+        shape = (n, hkv, d)
+        if not (plain and k.dtype is dtype and v.dtype is dtype and k.shape == shape and v.shape == shape
+                and k.device == device and v.device == device and ks[2] == 1 and vs[2] == 1
+                and not (ks[0] | ks[1] | vs[0] | vs[1]) & 7 and not (kp | vp) & 15
+                and ks[0] < 1 << 24 and vs[0] < 1 << 24):
+            _validate_call(layout, query, keys, values)
+        out += (kp, ks[0], ks[1], vp, vs[0], vs[1], 0, 0, 0, 0, 0, 0)
+    if not plain:
+        _validate_call(layout, query, keys, values)
+    return out
+
+
+def _attention_forward(query: torch.Tensor, layout: AttnLayout, scale: float, keys, values):
+    """(out, lse, tensors to keep while the launch reads them)."""
+    sources = _gather(layout, query, keys, values)
+    lib = _lib.require_library()
+    device = query.device
+    out = torch.empty(query.shape, dtype=query.dtype, device=device)
+    lse = torch.empty(layout.hq, max(layout.q_rows, 1), dtype=torch.float32, device=device)
+    kvb = layout.kv_block_for(device, query.shape[2])
+    _, (runs, host, keep) = layout._upload(device, kvb, sources)
+    problem = layout.problem(device, runs, scale, query.dtype, query.shape[2])
+    check_tables(layout, problem, host, device)
+    with operator_range("hip_attention_forward", rows=layout.q_rows, segments=len(layout.seg_q)):
+        _lib.check(
+            lib.ts_attn_fwd(ctypes.byref(problem), _rows(query), _rows(out), lse.data_ptr(), lse.shape[1],
+                            _lib.stream_of(query)),
+            lambda: f"ts_attn_fwd(rows={layout.q_rows}, hq={layout.hq}, hkv={layout.hkv})",
+        )
+    count_attention_path(HIP_PATH)
+    return out, lse, keep
+
+
+def _attention_backward(query, out, lse, dout, layout: AttnLayout, scale: float, keys, values):
+    """(dq, dkeys, dvalues, tensors to keep while the launches read them)."""
+    lib = _lib.require_library()
+    device = query.device
+    if dout.stride(2) != 1 or dout.stride(0) % 8 or dout.stride(1) % 8:
+        dout = dout.contiguous()
+    # dQ in the query's own layout where it is dense (a [1, Hq, T, D] query
+    # seen as rows gets its gradient without a copy into that layout)
+    dq = torch.empty_like(query)
+    if dq.stride(2) != 1 or dq.stride(0) % 8 or dq.stride(1) % 8:
+        dq = torch.empty(query.shape, dtype=query.dtype, device=device)
+    desc = layout._description()
+    if not desc["all_rows"]:
+        dq.zero_()
+    dkeys = [torch.empty(k.shape, dtype=k.dtype, device=device) for k in keys]
+    dvalues = [torch.empty(v.shape, dtype=v.dtype, device=device) for v in values]
+    # rows of a source that no run covers, or runs nobody reads, get zeros
+    for i in desc["uncovered"]:
+        dkeys[i].zero_()
+        dvalues[i].zero_()
+    sources = _gather(layout, query, keys, values)
+    d = query.shape[2]
+    for i, (dk, dv) in enumerate(zip(dkeys, dvalues)):  # contiguous [rows, Hkv, D]
+        sources[12 * i + 6 : 12 * i + 12] = (dk.data_ptr(), layout.hkv * d, d, dv.data_ptr(), layout.hkv * d, d)
+    tabs, (runs, host, keep_runs) = layout._upload(device, layout.kv_block_for(device, d), sources)
+    rowstats = torch.empty(layout.hq, max(layout.q_rows, 1), 2, dtype=torch.float32, device=device)
+    problem = layout.problem(device, runs, scale, query.dtype, d)
+    check_tables(layout, problem, host, device)
+    keep = [keep_runs]
+    ds = _ds_route(layout, query, lib)
+    if ds is not None:
+        _, kv_heads = ds
+        group = layout.hq // layout.hkv
+        try:
+            work = torch.empty(kv_heads * group * tabs["head"] + 512, dtype=query.dtype, device=device)
+        except torch.cuda.OutOfMemoryError:
+            ds = None
+    with operator_range("hip_attention_backward", rows=layout.q_rows, segments=len(layout.seg_q),
+                        ds_route=ds is not None):
+        if ds is None:
+            _lib.check(
+                lib.ts_attn_bwd(ctypes.byref(problem), _rows(query), _rows(out), _rows(dout),
+                                lse.data_ptr(), lse.shape[1], rowstats.data_ptr(), _rows(dq),
+                                _lib.stream_of(query)),
+                lambda: f"ts_attn_bwd(rows={layout.q_rows}, hq={layout.hq}, hkv={layout.hkv})",
+            )
+        else:
+            rows = [_rows(t) for t in (query, out, dout, dq)]
+            # the dQ pass's 64-row list where it applies (head dim 128, groups of 4)
+            dq_list, n_dq, n_dq_long = None, 0, 0
+            if d == HEAD_DIM and tabs["dq_work"] is not None:
+                dq_list, n_dq, n_dq_long = tabs["dq_work"], tabs["n_dq_work"], tabs["n_dq_long"]
+            for hk0 in range(0, layout.hkv, kv_heads):
+                n, h0 = min(kv_heads, layout.hkv - hk0), hk0 * group
+                sub = problem
+                if n != layout.hkv:  # KV heads hk0 .. hk0 + n - 1 and their query heads
+                    sub_runs, sub_host = _head_runs(host, hk0, device)
+                    keep.append((sub_runs, sub_host))
+                    sub = AttnProblem.from_buffer_copy(problem)
+                    sub.hq, sub.hkv, sub.runs = n * group, n, sub_runs.data_ptr()
+                    check_tables(layout, sub, sub_host, device)
+                q_r, o_r, do_r, dq_r = (_head_rows(r, h0) for r in rows)
+                _lib.check(
+                    lib.ts_attn_bwd_ds(ctypes.byref(sub), q_r, o_r, do_r, lse.data_ptr() + h0 * lse.shape[1] * 4,
+                                       lse.shape[1], rowstats.data_ptr() + h0 * lse.shape[1] * 8, dq_r,
+                                       tabs["span"], tabs["visit"], tabs["head"], work.data_ptr(),
+                                       work.numel() * 2, dq_list, n_dq, n_dq_long, _lib.stream_of(query)),
+                    lambda: f"ts_attn_bwd_ds(rows={layout.q_rows}, hq={layout.hq}, hkv={layout.hkv}, heads from {h0})",
+                )
+            del work
+    count_attention_path(HIP_BACKWARD_PATH)
+    return dq, dkeys, dvalues, keep
+
+
 class _Attention(torch.autograd.Function):
     """out, lse = attention over `layout`; grads to query and every key source."""
 
     @staticmethod
     def forward(ctx, query, layout, scale, n_sources, *kv):
-        keys, values = list(kv[:n_sources]), list(kv[n_sources:])
-        _validate_call(layout, query, keys, values)
-        lib = _lib.require_library()
-        out = torch.empty(query.shape, dtype=query.dtype, device=query.device)
-        lse = torch.empty(layout.hq, max(layout.q_rows, 1), dtype=torch.float32, device=query.device)
-        runs, host = _run_table(layout, keys, values)
-        problem = layout.problem(query.device, runs.data_ptr(), scale, query.dtype, query.shape[2])
-        check_tables(layout, problem, host, query.device)
-        with operator_range("hip_attention_forward", rows=layout.q_rows, segments=len(layout.seg_q)):
-            _lib.check(
-                lib.ts_attn_fwd(ctypes.byref(problem), _rows(query), _rows(out), lse.data_ptr(),
-                                lse.shape[1], _lib.stream_of(query)),
-                f"ts_attn_fwd(rows={layout.q_rows}, hq={layout.hq}, hkv={layout.hkv})",
-            )
-        count_attention_path(HIP_PATH)
+        out, lse, ctx.keep = _attention_forward(query, layout, scale, kv[:n_sources], kv[n_sources:])
         ctx.layout, ctx.scale, ctx.n_sources = layout, scale, n_sources
-        ctx.keep = (runs, host)
         ctx.save_for_backward(query, out, lse, *kv)
         ctx.mark_non_differentiable(lse)
         ctx.set_materialize_grads(False)  # no zero-filled gradient for lse
@@ -599,82 +648,11 @@ class _Attention(torch.autograd.Function):
     @torch.autograd.function.once_differentiable
     def backward(ctx, dout, _dlse):
         query, out, lse, *kv = ctx.saved_tensors
-        layout, n = ctx.layout, ctx.n_sources
-        keys, values = kv[:n], kv[n:]
-        lib = _lib.require_library()
         if dout is None:
             dout = torch.zeros_like(out)
-        dout = dout.contiguous() if dout.stride(2) != 1 or dout.stride(0) % 8 or dout.stride(1) % 8 else dout
-        # dQ in the query's own layout where it is dense (a [1, Hq, T, D] query
-        # seen as rows gets its gradient without a copy into that layout)
-        dq = torch.empty_like(query)
-        if dq.stride(2) != 1 or dq.stride(0) % 8 or dq.stride(1) % 8:
-            dq = torch.empty(query.shape, dtype=query.dtype, device=query.device)
-        covered = sum(t for _, t in layout.seg_q)
-        if covered != layout.q_rows:
-            dq.zero_()
-        dkeys = [torch.empty(k.shape, dtype=k.dtype, device=k.device) for k in keys]
-        dvalues = [torch.empty(v.shape, dtype=v.dtype, device=v.device) for v in values]
-        # rows of a source that no run covers, or runs nobody reads, get zeros
-        visit = layout.device_tables(query.device)
-        covered_rows = [0] * n
-        for r, run in enumerate(layout.runs):
-            if visit["nvisit"][r]:
-                covered_rows[run.source] += run.length
-        for i in range(n):
-            if covered_rows[i] != layout.source_rows[i]:
-                dkeys[i].zero_()
-                dvalues[i].zero_()
-        runs, host = _run_table(layout, keys, values, dkeys, dvalues)
-        rowstats = torch.empty(layout.hq, max(layout.q_rows, 1), 2, dtype=torch.float32, device=query.device)
-        problem = layout.problem(query.device, runs.data_ptr(), ctx.scale, query.dtype, query.shape[2])
-        check_tables(layout, problem, host, query.device)
-        ds = _ds_route(layout, query, lib)
-        if ds is not None:
-            tabs, kv_heads = ds
-            group = layout.hq // layout.hkv
-            try:
-                work = torch.empty(kv_heads * group * tabs["head"] + 512, dtype=query.dtype,
-                                   device=query.device)
-            except torch.cuda.OutOfMemoryError:
-                ds = None
-        with operator_range("hip_attention_backward", rows=layout.q_rows, segments=len(layout.seg_q),
-                            ds_route=ds is not None):
-            if ds is None:
-                _lib.check(
-                    lib.ts_attn_bwd(ctypes.byref(problem), _rows(query), _rows(out), _rows(dout),
-                                    lse.data_ptr(), lse.shape[1], rowstats.data_ptr(), _rows(dq),
-                                    _lib.stream_of(query)),
-                    f"ts_attn_bwd(rows={layout.q_rows}, hq={layout.hq}, hkv={layout.hkv})",
-                )
-            else:
-                rows = [_rows(t) for t in (query, out, dout, dq)]
-                keep = []
-                # the dQ pass's 64-row list where it applies (head dim 128, groups of 4)
-                dq_list, n_dq, n_dq_long = None, 0, 0
-                if query.shape[2] == HEAD_DIM and visit["dq_work"] is not None:
-                    dq_list, n_dq, n_dq_long = visit["dq_work"], visit["n_dq_work"], visit["n_dq_long"]
-                for hk0 in range(0, layout.hkv, kv_heads):
-                    n, h0 = min(kv_heads, layout.hkv - hk0), hk0 * group
-                    sub = problem
-                    if n != layout.hkv:  # KV heads hk0 .. hk0 + n - 1 and their query heads
-                        sub_runs, sub_host = _head_runs(host, hk0, query.device)
-                        keep.append((sub_runs, sub_host))
-                        sub = AttnProblem.from_buffer_copy(problem)
-                        sub.hq, sub.hkv, sub.runs = n * group, n, sub_runs.data_ptr()
-                        check_tables(layout, sub, sub_host, query.device)
-                    q_r, o_r, do_r, dq_r = (_head_rows(r, h0) for r in rows)
-                    _lib.check(
-                        lib.ts_attn_bwd_ds(ctypes.byref(sub), q_r, o_r, do_r, lse.data_ptr() + h0 * lse.shape[1] * 4,
-                                           lse.shape[1], rowstats.data_ptr() + h0 * lse.shape[1] * 8, dq_r,
-                                           tabs["span"], tabs["visit"], tabs["head"], work.data_ptr(),
-                                           work.numel() * 2, dq_list, n_dq, n_dq_long, _lib.stream_of(query)),
-                        f"ts_attn_bwd_ds(rows={layout.q_rows}, hq={layout.hq}, hkv={layout.hkv}, heads from {h0})",
-                    )
-                ctx.keep_bwd_heads = keep
-                del work
-        count_attention_path(HIP_BACKWARD_PATH)
-        ctx.keep_bwd = (runs, host)
+        n = ctx.n_sources
+        dq, dkeys, dvalues, ctx.keep_bwd = _attention_backward(query, out, lse, dout, ctx.layout, ctx.scale, kv[:n],
+                                                               kv[n:])
         return (dq, None, None, None, *dkeys, *dvalues)
 
 
@@ -711,21 +689,39 @@ def attention(query: torch.Tensor, layout: AttnLayout, keys: Sequence[torch.Tens
     return _Attention.apply(query, layout, float(scale), len(keys), *keys, *values)
 
 
+def _pad_heads(t: torch.Tensor, head_dim: int) -> torch.Tensor:
+    return torch.nn.functional.pad(t, (0, head_dim - t.shape[-1])) if t.shape[-1] != head_dim else t
+
+
+def _save_attention(ctx, query: torch.Tensor, layout: AttnLayout, scale: float, keys, values) -> torch.Tensor:
+    """The forward of an autograd function that differentiates the core op
+    itself (no graph inside it): out ``[R, Hq, D]``, with everything
+    :func:`_saved_gradients` needs saved on ``ctx``.  Head dims as in
+    :func:`attention`."""
+    d = query.shape[-1]
+    dk = kernel_head_dim(d) or d
+    query, keys, values = _pad_heads(query, dk), [_pad_heads(k, dk) for k in keys], [_pad_heads(v, dk) for v in values]
+    out, lse, ctx.keep = _attention_forward(query, layout, float(scale), keys, values)
+    ctx.layout, ctx.scale = layout, float(scale)
+    ctx.save_for_backward(query, out, lse, *keys, *values)
+    return out[..., :d] if dk != d else out
+
+
+def _saved_gradients(ctx, dout: torch.Tensor):
+    """(dq, dkeys, dvalues) of a call saved by :func:`_save_attention`, for the
+    gradient ``[R, Hq, D]`` of its output."""
+    query, out, lse, *kv = ctx.saved_tensors
+    d, n = dout.shape[-1], len(kv) // 2
+    dq, dkeys, dvalues, ctx.keep_bwd = _attention_backward(query, out, lse, _pad_heads(dout, query.shape[-1]),
+                                                           ctx.layout, ctx.scale, kv[:n], kv[n:])
+    if query.shape[-1] != d:
+        dq, dkeys, dvalues = dq[..., :d], [g[..., :d] for g in dkeys], [g[..., :d] for g in dvalues]
+    return dq, dkeys, dvalues
+
+
 # ---------------------------------------------------------------------------
 # layouts for the reference's call shapes
 # ---------------------------------------------------------------------------
-def _dedupe(tensors: Sequence[torch.Tensor]):
-    """Distinct tensors (by identity) and, per input position, its source index."""
-    sources, index, where = [], {}, []
-    for t in tensors:
-        key = id(t)
-        if key not in index:
-            index[key] = len(sources)
-            sources.append(t)
-        where.append(index[key])
-    return sources, where
-
-
 def chain_layout(query_len: int, chunk_lengths: Sequence[int], hq: int, hkv: int) -> AttnLayout:
     """One segment of `query_len` rows over the concatenation of chunks."""
     runs = tuple(Run(i, 0, n) for i, n in enumerate(chunk_lengths) if n > 0)
@@ -752,7 +748,8 @@ def _query_rows(query: torch.Tensor) -> torch.Tensor:
 
 def _as_rows(t: torch.Tensor) -> torch.Tensor:
     """A [rows, heads, D] view usable by the kernels (copy only if it must)."""
-    if t.stride(2) == 1 and t.stride(0) % 8 == 0 and t.stride(1) % 8 == 0 and t.data_ptr() % 16 == 0:
+    s = t.stride()
+    if s[2] == 1 and not (s[0] | s[1]) & 7 and not t.data_ptr() & 15:
         return t
     return t.contiguous()
 
@@ -765,17 +762,17 @@ def causal_attention(query: torch.Tensor, ks: Sequence[torch.Tensor], vs: Sequen
     query row i sees keys ``0 .. S - T + i`` of their concatenation, which is
     never materialised (engine/streaming.py:1080-1162).
     """
-    q = _as_rows(_query_rows(query))
-    keys, kw = _dedupe(ks)
-    values, vw = _dedupe(vs)
-    if kw != vw or len(keys) != len(ks):
-        # distinct chunk objects per position keep one run per chunk
-        keys, values = list(ks), list(vs)
-    keys = [_as_rows(k) for k in keys]
-    values = [_as_rows(v) for v in values]
-    layout = chain_layout(q.shape[0], [k.shape[0] for k in keys], q.shape[1], keys[0].shape[1])
+    q, layout, keys, values = _chain_call(query, ks, vs)
     out, _ = attention(q, layout, keys, values, scale)
     return out.transpose(0, 1).unsqueeze(0)
+
+
+def _chain_call(query, ks, vs):
+    """(query rows, layout, keys, values) of a chunk-list call, one run per chunk."""
+    q = _as_rows(_query_rows(query))
+    keys = [_as_rows(k) for k in ks]
+    values = [_as_rows(v) for v in vs]
+    return q, chain_layout(q.shape[0], [k.shape[0] for k in keys], q.shape[1], keys[0].shape[1]), keys, values
 
 
 class ChunkedCausalAttention(torch.autograd.Function):
@@ -803,24 +800,20 @@ class ChunkedCausalAttention(torch.autograd.Function):
         ks, vs = list(chunks[:n_chunks]), list(chunks[n_chunks:])
         ctx.n_chunks, ctx.scale, ctx.backend = n_chunks, scale, backend
         if callable(backend):
-            ctx.graph = None
             ctx.save_for_backward(query, *chunks)
             return backend(query, ks, vs, scale)
         if backend not in ("auto", "cudnn"):
             raise ValueError(f"unknown source attention backend: {backend!r}")
-        with torch.enable_grad():
-            leaves = [c.detach().requires_grad_(c.requires_grad) for c in chunks]
-            q = query.detach().requires_grad_(query.requires_grad)
-            out = causal_attention(q, leaves[:n_chunks], leaves[n_chunks:], scale)
-        ctx.graph = (q, leaves, out)
-        return out.detach()
+        q, layout, keys, values = _chain_call(query, ks, vs)
+        out = _save_attention(ctx, q, layout, scale, keys, values)
+        return out.transpose(0, 1).unsqueeze(0).detach()
 
     @staticmethod
     @torch.autograd.function.once_differentiable
     def backward(ctx, grad_out):
         need = ctx.needs_input_grad
         n = ctx.n_chunks
-        if ctx.graph is None:
+        if callable(ctx.backend):
             query, *chunks = ctx.saved_tensors
             q = query.detach().requires_grad_(True)
             leaves = [c.detach().requires_grad_(True) for c in chunks]
@@ -829,12 +822,9 @@ class ChunkedCausalAttention(torch.autograd.Function):
             grads = torch.autograd.grad(out, [q, *leaves], grad_out, allow_unused=True)
             dq, rest = grads[0], list(grads[1:])
         else:
-            q, leaves, out = ctx.graph
-            inputs = [t for t in (q, *leaves) if t.requires_grad]
-            grads = torch.autograd.grad(out, inputs, grad_out, allow_unused=True) if inputs else []
-            it = iter(grads)
-            dq = next(it) if q.requires_grad else None
-            rest = [next(it) if c.requires_grad else None for c in leaves]
+            dq, dkeys, dvalues = _saved_gradients(ctx, grad_out[0].transpose(0, 1))
+            dq = dq.transpose(0, 1).unsqueeze(0)
+            rest = [*dkeys, *dvalues]
         return (
             dq if need[0] else None, None, None, None, None,
             *(g if need[5 + i] else None for i, g in enumerate(rest)),
@@ -938,43 +928,35 @@ class PackedAttention(torch.autograd.Function):
             source_rows=tuple(t.shape[0] for t in srcs_k), runs=tuple(runs),
             seg_q=tuple(seg_q), seg_spans=tuple(seg_spans),
         )
-        with torch.enable_grad():
-            qd = q.detach().requires_grad_(query.requires_grad)
-            kd = [t.detach().requires_grad_(True) for t in srcs_k]
-            vd = [t.detach().requires_grad_(True) for t in srcs_v]
-            out, _ = attention(qd, att_layout, kd, vd, scale)
-        ctx.graph = (qd, kd, vd, out, src_index, layout, a_keys, a_vals)
+        out = _save_attention(ctx, q, att_layout, scale, srcs_k, srcs_v)
+        # per ancestor input, in input order: its source, or None for an empty
+        # chunk (zeros) or a repeated one (whose gradient the first carries)
+        order, seen = [], set()
+        for ks, vs in zip(reversed(a_keys), reversed(a_vals)):
+            for kc, vc in zip(ks, vs):
+                ident = (id(kc), id(vc))
+                source = src_index.get(ident) if kc.shape[0] and ident not in seen else None
+                order.append((source, kc.shape[0] == 0, kc.shape, vc.shape))
+                seen.add(ident)
+        ctx.order = order
         return out.detach().transpose(0, 1).unsqueeze(0)
 
     @staticmethod
     @torch.autograd.function.once_differentiable
     def backward(ctx, grad_out):
-        qd, kd, vd, out, src_index, layout, a_keys, a_vals = ctx.graph
-        g = grad_out[0].transpose(0, 1)
-        inputs = ([qd] if qd.requires_grad else []) + kd + vd
-        grads = torch.autograd.grad(out, inputs, g)
-        it = iter(grads)
-        dq = next(it).transpose(0, 1).unsqueeze(0) if qd.requires_grad else None
-        dks = [next(it) for _ in kd]
-        dvs = [next(it) for _ in vd]
+        dq, dks, dvs = _saved_gradients(ctx, grad_out[0].transpose(0, 1))
         # ancestor grads in input order; a chunk object appearing several
         # times receives its summed gradient once (autograd adds per input)
-        seen = set()
         anc_k, anc_v = [], []
-        for ks, vs in zip(reversed(a_keys), reversed(a_vals)):
-            for kc, vc in zip(ks, vs):
-                ident = (id(kc), id(vc))
-                if kc.shape[0] == 0:
-                    anc_k.append(torch.zeros_like(kc))
-                    anc_v.append(torch.zeros_like(vc))
-                elif ident in seen:
-                    anc_k.append(None)
-                    anc_v.append(None)
-                else:
-                    seen.add(ident)
-                    anc_k.append(dks[src_index[ident]])
-                    anc_v.append(dvs[src_index[ident]])
-        return (dq, dks[0], dvs[0], None, None, *anc_k, *anc_v)
+        for source, empty, k_shape, v_shape in ctx.order:
+            if source is not None:
+                anc_k.append(dks[source])
+                anc_v.append(dvs[source])
+            else:
+                anc_k.append(torch.zeros(k_shape, dtype=dq.dtype, device=dq.device) if empty else None)
+                anc_v.append(torch.zeros(v_shape, dtype=dq.dtype, device=dq.device) if empty else None)
+        return (dq.transpose(0, 1).unsqueeze(0) if ctx.needs_input_grad[0] else None, dks[0], dvs[0], None, None,
+                *anc_k, *anc_v)
 
 
 def _ragged_layout(lengths: Sequence[int], key_rows: Sequence[int], hq: int, hkv: int) -> AttnLayout:
