@@ -103,6 +103,21 @@ def kv_block_keys(hq: int, hkv: int, head_dim: int = HEAD_DIM) -> int:
 DKDV256_MIN_ITEMS = 512
 
 
+# At head dim 128, 48-key dK/dV items run the kernel whose waves take steps
+# (a query head, 32 rows) of their own, 64-key items the key-split kernel, whose
+# waves take 16 keys each of every step.  The first does each step in fewer LDS
+# reads and without a barrier, the second starts and ends cheaper (16 keys'
+# operands to load, no partials to sum over the waves) and holds two
+# work-groups a CU.  So items of many steps are dealt out, and so are launches
+# that one work-group a CU holds, down to two steps a wave.  Key-split against
+# dealt out, us: 6 steps, 696 items 30 / 44 (24/8 heads, 64 rows over 4160 keys);
+# 16 steps, 348 items 33 / 38 (32/4, 64 over 4160); 16 steps, 704 items 52 / 53
+# (32/8, 128 over 4224); 8 steps, 96 items 17 / 16 (32/8, 64 over 576); 16 steps,
+# 216 items 26 / 22 (16/8, 256 over 1280); 40 steps, 216 items 51 / 35 (40/8,
+# 256 over 1280); 320 steps and more 1.3 to 2.5 times faster dealt out.
+DEALT_STEPS, DEALT_STEPS_ONE_ROUND, ONE_ROUND_ITEMS = 20, 8, 256
+
+
 # ---------------------------------------------------------------------------
 # layout
 # ---------------------------------------------------------------------------
@@ -192,9 +207,11 @@ class AttnLayout:
                 "arrays": (seg_q, seg_span0, spans, run_len, run_source, run_offset),
                 "ptrs": tuple(a.ctypes.data for a in (seg_q, seg_span0, spans, run_len, run_source, run_offset)),
                 "n_spans": int(spans.shape[0]),
-                "visited_lengths": run_len[nvisit > 0],
+                "visited_lengths": runs[nvisit > 0, 2],
                 # sources with rows that no visited run covers: their gradients are filled with zeros first
                 "uncovered": [i for i, n in enumerate(self.source_rows) if covered[i] != n],
+                # query rows that see a visited key, on average
+                "rows_per_key": self.visible_pairs() / max(int(run_len[nvisit > 0].sum()), 1),
                 "all_rows": int(seg_q[:, 1].sum()) == self.q_rows,
             }
             self._desc = d
@@ -326,14 +343,25 @@ class AttnLayout:
         kernel)."""
         kvb = kv_block_keys(self.hq, self.hkv, head_dim)
         if head_dim == 256:
-            n64 = int(((self._description()["visited_lengths"].astype(np.int64) + 63) // 64).sum())
+            n64 = int(((self._description()["visited_lengths"] + 63) // 64).sum())
             if n64 * self.hkv < DKDV256_MIN_ITEMS:
                 kvb = 48
         return kvb
 
+    def call_kv_block(self, device, head_dim: int) -> int:
+        """Keys per dK/dV work item of this package's own calls: kv_block_for's,
+        except that at head dim 128 every GQA group takes either kernel, by the
+        steps of an item and the items of the launch (DEALT_STEPS)."""
+        if head_dim != HEAD_DIM:
+            return self.kv_block_for(device, head_dim)
+        d = self._description()
+        steps = (self.hq // self.hkv) * d["rows_per_key"] / 32
+        items = int(((d["visited_lengths"] + 47) // 48).sum()) * self.hkv
+        return 48 if steps >= (DEALT_STEPS_ONE_ROUND if items <= ONE_ROUND_ITEMS else DEALT_STEPS) else 64
+
     def problem(self, device, runs_ptr: int, scale: float, dtype: torch.dtype = torch.bfloat16,
-                head_dim: int = HEAD_DIM) -> AttnProblem:
-        kvb = self.kv_block_for(device, int(head_dim))
+                head_dim: int = HEAD_DIM, kv_block: int | None = None) -> AttnProblem:
+        kvb = self.kv_block_for(device, int(head_dim)) if kv_block is None else kv_block
         t = self.device_tables(device, kvb)
         return AttnProblem(
             t["segs"], t["seg_spans"], runs_ptr, t["run_visits_dev"], t["q_work"], t["kv_work"],
@@ -477,7 +505,7 @@ def _ds_route(layout: AttnLayout, query: torch.Tensor, lib):
     group = layout.hq // layout.hkv
     if not lib.ts_attn_ds_route(query.shape[2], group):
         return None
-    tabs = layout.ds_tables(query.device, layout.kv_block_for(query.device, query.shape[2]))
+    tabs = layout.ds_tables(query.device, layout.call_kv_block(query.device, query.shape[2]))
     # a call over n KV heads needs (n * group * head + 512) elements: every
     # query head's part, then the sink block
     per_kv_head = group * max(tabs["head"], 1)
@@ -544,9 +572,9 @@ def _attention_forward(query: torch.Tensor, layout: AttnLayout, scale: float, ke
     device = query.device
     out = torch.empty(query.shape, dtype=query.dtype, device=device)
     lse = torch.empty(layout.hq, max(layout.q_rows, 1), dtype=torch.float32, device=device)
-    kvb = layout.kv_block_for(device, query.shape[2])
+    kvb = layout.call_kv_block(device, query.shape[2])
     _, (runs, host, keep) = layout._upload(device, kvb, sources)
-    problem = layout.problem(device, runs, scale, query.dtype, query.shape[2])
+    problem = layout.problem(device, runs, scale, query.dtype, query.shape[2], kvb)
     check_tables(layout, problem, host, device)
     with operator_range("hip_attention_forward", rows=layout.q_rows, segments=len(layout.seg_q)):
         _lib.check(
@@ -582,9 +610,10 @@ def _attention_backward(query, out, lse, dout, layout: AttnLayout, scale: float,
     d = query.shape[2]
     for i, (dk, dv) in enumerate(zip(dkeys, dvalues)):  # contiguous [rows, Hkv, D]
         sources[12 * i + 6 : 12 * i + 12] = (dk.data_ptr(), layout.hkv * d, d, dv.data_ptr(), layout.hkv * d, d)
-    tabs, (runs, host, keep_runs) = layout._upload(device, layout.kv_block_for(device, d), sources)
+    kvb = layout.call_kv_block(device, d)
+    tabs, (runs, host, keep_runs) = layout._upload(device, kvb, sources)
     rowstats = torch.empty(layout.hq, max(layout.q_rows, 1), 2, dtype=torch.float32, device=device)
-    problem = layout.problem(device, runs, scale, query.dtype, d)
+    problem = layout.problem(device, runs, scale, query.dtype, d, kvb)
     check_tables(layout, problem, host, device)
     keep = [keep_runs]
     ds = _ds_route(layout, query, lib)

@@ -53,8 +53,9 @@ int validate(const ts_attn_problem* p, const char* what) {
   const int gc = heads_per_block(p->hq / p->hkv);
   TS_CHECK_ARG(p->q_block == q_block_rows(p->hq / p->hkv), "%s: q_block %d, expected %d for group %d",
                what, p->q_block, q_block_rows(p->hq / p->hkv), p->hq / p->hkv);
-  // head dim 256 also takes 48-key items (the key-split kernel: few work items)
-  TS_CHECK_ARG(p->kv_block == kv_block_keys(p->hq / p->hkv, p->head_dim) || (p->head_dim == 256 && p->kv_block == 48),
+  // the DMA-staged kernels (head dims 128 and 256) take items of either size
+  TS_CHECK_ARG(p->kv_block == kv_block_keys(p->hq / p->hkv, p->head_dim) ||
+                   (ds_route(p->head_dim, p->hq / p->hkv) && (p->kv_block == 48 || p->kv_block == 64)),
                "%s: kv_block %d, expected %d", what, p->kv_block, kv_block_keys(p->hq / p->hkv, p->head_dim));
   TS_CHECK_ARG(p->n_q_work >= 0 && p->n_kv_work >= 0 && p->n_segs >= 0 && p->n_runs >= 0,
                "%s: negative table size", what);

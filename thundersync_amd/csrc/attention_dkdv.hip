@@ -150,8 +150,8 @@ __global__ __launch_bounds__(kThreads, HD > 128 ? 1 : 2) void dkdv_kernel(ts_att
 }
 
 // ---------------------------------------------------------------------------
-// backward dK / dV with the keys split over the waves (head dim 128: GQA
-// groups that are not a multiple of 4; head dim 256: 48-key work items, which
+// backward dK / dV with the keys split over the waves (head dim 128: 64-key
+// work items, for items of few steps; head dim 256: 48-key work items, which
 // launches with few 64-key items take)
 //
 // A work-group owns P.kv_block keys (48 or 64) of one run and one KV head;
@@ -492,13 +492,12 @@ void launch_dkdv_generic(dim3 grid, const ts_attn_problem& P, ts_attn_rows q, ts
 template <typename E, bool DS>
 void launch_dkdv_tuned(dim3 grid, const ts_attn_problem& P, ts_attn_rows q, ts_attn_rows dout,
                        const float* rowstats, int64_t lse_ld, const DsArgs& S, hipStream_t s) {
-  const int group = P.hq / P.hkv;
   ts::TimedLaunch timed_("attention.dkdv_kernel", s);
   if (P.head_dim == 256 && P.kv_block == 64)
     launch_dkdv256<E, DS>(grid, P, q, dout, rowstats, lse_ld, S, s);
   else if (P.head_dim == 256)
     hipLaunchKernelGGL((dkdv_split_kernel<E, 256, DS>), grid, dim3(kThreads), 0, s, P, q, dout, rowstats, lse_ld, S);
-  else if (group % 4 == 0)
+  else if (P.kv_block == 48)
     launch_dkdv_wave<E, DS>(grid, P, q, dout, rowstats, lse_ld, S, s);
   else
     hipLaunchKernelGGL((dkdv_split_kernel<E, D, DS>), grid, dim3(kThreads), 0, s, P, q, dout, rowstats, lse_ld, S);

@@ -1,5 +1,5 @@
-// Attention backward: dK / dV, one wave per query head (GQA groups that are
-// a multiple of 4, head dim 128).  A translation unit of its own so that it
+// Attention backward: dK / dV over 48-key work items, each wave on a (query
+// head, row block) stream of its own (head dim 128).  A translation unit of its own so that it
 // can take its own code-generation flags.
 #include "attention_impl.h"
 
@@ -44,11 +44,21 @@ struct WaveCursor {
 };
 
 // ---------------------------------------------------------------------------
-// backward dK / dV, one wave per query head (GQA groups that are a multiple of 4)
+// backward dK / dV, one (query head, 32-row block) step per wave at a time
 //
-// A work-group owns 16 KB keys of one run and one KV head; wave w handles query
-// heads w, w + 4, ... of the group over all of them, so a wave's LDS reads of
-// its head's Q/dO tile feed 16 KB keys of MFMA work.  The K^T and V^T
+// A work-group owns 16 KB keys of one run and one KV head, and each of its
+// four waves covers all of them, so a wave's LDS reads of a Q/dO tile feed
+// 16 KB keys of MFMA work.  The group's steps -- every query head, then every
+// visible row block -- are dealt out to the waves: for groups that are a
+// multiple of 4 (STR 1) wave w takes heads w, w + 4, ... whole; for the others
+// (STR 4) it takes every fourth step of the one sequence over all heads, so the
+// waves end within a step of each other whatever the group.  Any deal gives
+// the same sums up to their order, since dK and dV add over heads and rows and
+// the waves' partials meet at the end.  (STR 4 against the key-split kernel,
+// whose waves share each tile for 16 keys each with a barrier per step: C2-like
+// pack of 6 turns at 40/8 heads 1280 -> 900 us, 4096 rows over 8192 keys at
+// 40/8, 16/8 and 24/4 heads 1373 -> 1072, 573 -> 440 and 951 -> 651 us; items of
+// few steps keep the key-split kernel, attention.py DEALT_STEPS)  The K^T and V^T
 // operands stay in registers.  Each wave streams its head's 32-row
 // Q/dO tiles and their 32 (lse * log2 e, delta) pairs into its own
 // double-buffered LDS region with buffer_load ... lds: the buffer resource of
@@ -72,7 +82,7 @@ struct WaveCursor {
 // blocks right after computing them (the kernel has no registers for a
 // deferred copy), through a per-lane pointer that follows the visit cursor.
 // ---------------------------------------------------------------------------
-template <typename E, int KB, bool DS = false>
+template <typename E, int KB, bool DS, int STR>
 __global__ __launch_bounds__(kThreads, 1) void dkdv_wave_kernel(ts_attn_problem P, ts_attn_rows Q,
                                                                 ts_attn_rows dO,
                                                                 const float* __restrict__ rowstats,
@@ -126,7 +136,7 @@ __global__ __launch_bounds__(kThreads, 1) void dkdv_wave_kernel(ts_attn_problem 
     qoff[t] = (int)(((4 * t + g4) * Q.row_stride + dchunk[t]) * 2) - 1024 * t;
     doff[t] = (int)(((4 * t + g4) * dO.row_stride + dchunk[t]) * 2) - 1024 * t;
   }
-  const int64_t q32 = 32 * Q.row_stride, d32 = 32 * dO.row_stride;  // one block of rows
+  const int64_t q32 = 32 * STR * Q.row_stride, d32 = 32 * STR * dO.row_stride;  // to the wave's next block
   const int64_t q16 = 16 * Q.row_stride, d16 = 16 * dO.row_stride;  // its upper half
   const uint32_t qrow_bytes = (uint32_t)(Q.row_stride * 2), drow_bytes = (uint32_t)(dO.row_stride * 2);
 
@@ -155,11 +165,13 @@ __global__ __launch_bounds__(kThreads, 1) void dkdv_wave_kernel(ts_attn_problem 
       dv[mb][kb] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
 
-  int hh = 0;  // the wave's current head
+  int hh = 0;        // the wave's current head
+  int phase = wave;  // STR 4: blocks to skip from the start of the next head's sequence
   // enter visit c.vi (< nvisit): cache its segment's fields and start at the
-  // first 32-row block whose rows can see key k0, with that block's Q, dO and
-  // statistics rows of head hh
-  auto enter = [&](WaveCursor& c) {
+  // first 32-row block whose rows can see key k0 (STR 4: `skip` blocks after
+  // it, which may lie past the visit), with that block's Q, dO and statistics
+  // rows of head hh
+  auto enter = [&](WaveCursor& c, int skip) {
     const ts_attn_ref ref = load_uniform(P.run_visits, run.visit0 + c.vi);
     const ts_attn_segment seg = load_uniform(P.segs, ref.index);
     c.q_len = seg.q_len;
@@ -167,22 +179,29 @@ __global__ __launch_bounds__(kThreads, 1) void dkdv_wave_kernel(ts_attn_problem 
     c.kpos = ref.kpos;
     const int rs = ref.kpos + k0 - c.off;
     c.r0 = (rs < 0 ? 0 : rs) & ~31;
+    if constexpr (STR > 1) c.r0 = min(c.r0, (c.q_len + 31) & ~31) + 32 * skip;
     const int64_t row0 = seg.q_row0 + c.r0;
     c.q = (const bf16*)Q.ptr + row0 * Q.row_stride + (int64_t)hh * Q.head_stride;
     c.d = (const bf16*)dO.ptr + row0 * dO.row_stride + (int64_t)hh * dO.head_stride;
     c.st = rowstats + 2 * ((int64_t)hh * lse_ld + row0);
   };
-  // first block at or after c; skips visits with no visible rows
+  // first block at or after c; skips visits with no visible rows.  STR 4: the
+  // blocks by which c passed its visit's last one carry over to the next
+  // visit, and past the last visit to the next head
   auto settle = [&](WaveCursor c) -> WaveCursor {
     while (c.r0 >= c.q_len) {
-      if (++c.vi >= run.nvisit) break;
-      enter(c);
+      const int over = STR > 1 ? (c.r0 - ((c.q_len + 31) & ~31)) >> 5 : 0;
+      if (++c.vi >= run.nvisit) {
+        if (STR > 1 && c.vi == run.nvisit) phase = over;
+        break;
+      }
+      enter(c, over);
     }
     return c;
   };
   auto first = [&]() -> WaveCursor {
     WaveCursor c{0, 0, 0, 0, 0, nullptr, nullptr, nullptr};
-    if (run.nvisit > 0) enter(c);
+    if (run.nvisit > 0) enter(c, phase);
     return settle(c);
   };
   // dS route: this lane's element of block k0 / 16 of c's row block in head
@@ -196,20 +215,23 @@ __global__ __launch_bounds__(kThreads, 1) void dkdv_wave_kernel(ts_attn_problem 
     return ds_lane + (int64_t)hh * ds_head + blk * kDsBlock;
   };
   // the block after c (settled: past its visit's rows, the next visit's
-  // first): within a visit the DMA sources advance by 32 rows; dS route:
-  // `at` follows it, advanced by c's row block's block count within a visit,
-  // located afresh on entering the next
+  // first): within a visit the DMA sources advance by 32 STR rows; dS route:
+  // `at` follows it, advanced by the passed row blocks' block counts within a
+  // visit, located afresh on entering the next
   auto next_block = [&](WaveCursor c, bf16*& at) -> WaveCursor {
     int inc = 0;
     if constexpr (DS) {
-      const int last = c.off - c.kpos + min(c.r0 + 31, c.q_len - 1);
-      inc = last < 0 ? 0 : min(nkb, (last >> 4) + 1);
+#pragma unroll
+      for (int u = 0; u < STR; ++u) {
+        const int last = c.off - c.kpos + min(c.r0 + 32 * u + 31, c.q_len - 1);
+        inc += last < 0 ? 0 : min(nkb, (last >> 4) + 1);
+      }
     }
     const int vi0 = c.vi;
-    c.r0 += 32;
+    c.r0 += 32 * STR;
     c.q += q32;
     c.d += d32;
-    c.st += 64;
+    c.st += 64 * STR;
     if (c.r0 >= c.q_len) c = settle(c);  // tables are read only here
     if constexpr (DS) {
       if (c.vi == vi0)
@@ -395,7 +417,7 @@ __global__ __launch_bounds__(kThreads, 1) void dkdv_wave_kernel(ts_attn_problem 
       nxt = next_block(nxt, nxt_at);
   };
 
-  for (int g = wave; g < group; g += 4) {
+  for (int g = STR > 1 ? 0 : wave; g < group; g += STR > 1 ? 1 : 4) {
     hh = hk * group + g;
     WaveCursor cur = first();
     bf16* cur_at = ds_lane;
@@ -466,7 +488,10 @@ __global__ __launch_bounds__(kThreads, 1) void dkdv_wave_kernel(ts_attn_problem 
 template <typename E, bool DS>
 void launch_dkdv_wave(dim3 grid, const ts_attn_problem& P, ts_attn_rows q, ts_attn_rows dout,
                       const float* rowstats, int64_t lse_ld, const DsArgs& S, hipStream_t s) {
-  hipLaunchKernelGGL((dkdv_wave_kernel<E, 3, DS>), grid, dim3(kThreads), 0, s, P, q, dout, rowstats, lse_ld, S);
+  if ((P.hq / P.hkv) % 4 == 0)
+    hipLaunchKernelGGL((dkdv_wave_kernel<E, 3, DS, 1>), grid, dim3(kThreads), 0, s, P, q, dout, rowstats, lse_ld, S);
+  else
+    hipLaunchKernelGGL((dkdv_wave_kernel<E, 3, DS, 4>), grid, dim3(kThreads), 0, s, P, q, dout, rowstats, lse_ld, S);
 }
 
 template void launch_dkdv_wave<bf16, false>(dim3, const ts_attn_problem&, ts_attn_rows, ts_attn_rows,
