@@ -291,6 +291,19 @@ int ts_attn_bwd(const ts_attn_problem* problem, ts_attn_rows q, ts_attn_rows out
                 ts_attn_rows dout, const float* lse, int64_t lse_ld, float* rowstats,
                 ts_attn_rows dq, void* stream);
 
+/* ts_attn_fwd with each work item's keys cut into `parts` work-groups, for
+ * launches whose items leave much of the device idle (a short turn over a long
+ * context: two row blocks a KV head).  The workspace (16-byte aligned, parts *
+ * hq * q_rows * (head_dim + 2) floats) takes each part's unnormalised fp32 rows
+ * and their (m, l); a second kernel combines them in part order.  parts 1: no
+ * workspace, ts_attn_fwd's launch.  ts_attn_fwd_parts and ts_attn_dq_parts give
+ * the parts worth taking for a problem whose longest item sees max_keys keys
+ * (n_dq_work: items of the dQ pass's own list, 0 without one). */
+int ts_attn_fwd_parts(const ts_attn_problem* problem, int64_t max_keys);
+int ts_attn_dq_parts(const ts_attn_problem* problem, int32_t n_dq_work, int64_t max_keys);
+int ts_attn_fwd_split(const ts_attn_problem* problem, ts_attn_rows q, ts_attn_rows out, float* lse, int64_t lse_ld,
+                      int parts, void* workspace, int64_t workspace_bytes, void* stream);
+
 /* dS route of the backward.  ts_attn_bwd's dQ kernel recomputes S = Q K^T
  * and dP = dO V^T, which its dK/dV kernels also compute; on this route the
  * dK/dV kernels store dS = P (dP - delta) (in the element type, as rounded
@@ -336,6 +349,14 @@ int ts_attn_bwd_ds(const ts_attn_problem* problem, ts_attn_rows q, ts_attn_rows 
                    ts_attn_rows dq, const int64_t* span_ds, const int64_t* visit_ds,
                    int64_t ds_head, void* ds, int64_t ds_bytes, const int32_t* dq_work,
                    int32_t n_dq_work, int32_t n_dq_long, void* stream);
+
+/* ts_attn_bwd_ds with the dQ pass's items cut into dq_parts (workspace: parts *
+ * hq * q_rows * head_dim floats), as ts_attn_fwd_split. */
+int ts_attn_bwd_ds_split(const ts_attn_problem* problem, ts_attn_rows q, ts_attn_rows out, ts_attn_rows dout,
+                         const float* lse, int64_t lse_ld, float* rowstats, ts_attn_rows dq, const int64_t* span_ds,
+                         const int64_t* visit_ds, int64_t ds_head, void* ds, int64_t ds_bytes,
+                         const int32_t* dq_work, int32_t n_dq_work, int32_t n_dq_long, int dq_parts, void* workspace,
+                         int64_t workspace_bytes, void* stream);
 
 /* ------------------------------------------------------------------------
  * Fused chunked-vocab logprob / entropy (bf16 or fp16 operands, fp32 results)

@@ -87,6 +87,14 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "ts_attn_run_table": (_INT, [ctypes.c_int32, _P, _P, _P, _P, ctypes.c_int32, _P, _P]),
     "ts_attn_check_tables": (_INT, [ctypes.POINTER(AttnProblem), _P, _P, _I64, _P, _P, _I64, _P, _P]),
     "ts_attn_fwd": (_INT, [ctypes.POINTER(AttnProblem), AttnRows, AttnRows, _P, _I64, _P]),
+    "ts_attn_fwd_parts": (_INT, [ctypes.POINTER(AttnProblem), _I64]),
+    "ts_attn_dq_parts": (_INT, [ctypes.POINTER(AttnProblem), ctypes.c_int32, _I64]),
+    "ts_attn_fwd_split": (_INT, [ctypes.POINTER(AttnProblem), AttnRows, AttnRows, _P, _I64, _INT, _P, _I64, _P]),
+    "ts_attn_bwd_ds_split": (
+        _INT,
+        [ctypes.POINTER(AttnProblem), AttnRows, AttnRows, AttnRows, _P, _I64, _P, AttnRows, _P, _P, _I64, _P,
+         _I64, _P, ctypes.c_int32, ctypes.c_int32, _INT, _P, _I64, _P],
+    ),
     "ts_attn_bwd": (
         _INT,
         [ctypes.POINTER(AttnProblem), AttnRows, AttnRows, AttnRows, _P, _I64, _P, AttnRows, _P],

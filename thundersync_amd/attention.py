@@ -56,6 +56,8 @@ import threading
 from array import array
 from collections.abc import Sequence
 from dataclasses import dataclass, field
+from itertools import chain
+from typing import NamedTuple
 
 import numpy as np
 import torch
@@ -121,8 +123,7 @@ DEALT_STEPS, DEALT_STEPS_ONE_ROUND, ONE_ROUND_ITEMS = 20, 8, 256
 # ---------------------------------------------------------------------------
 # layout
 # ---------------------------------------------------------------------------
-@dataclass(frozen=True)
-class Run:
+class Run(NamedTuple):
     source: int  # index into the call's key sources
     offset: int  # first row within the source
     length: int
@@ -147,43 +148,46 @@ class AttnLayout:
     def __post_init__(self):
         if self.hq <= 0 or self.hkv <= 0 or self.hq % self.hkv:
             raise ValueError(f"query heads {self.hq} are not a multiple of KV heads {self.hkv}")
+        runs, sources = self.runs, self.source_rows
+        n_runs, n_sources = len(runs), len(sources)
         kv = []
         for s, spans in enumerate(self.seg_spans):
             pos = 0
             for run, kpos in spans:
-                if not 0 <= run < len(self.runs):
-                    raise ValueError(f"segment {s} names run {run} of {len(self.runs)}")
+                if not 0 <= run < n_runs:
+                    raise ValueError(f"segment {s} names run {run} of {n_runs}")
                 if kpos != pos:
                     raise ValueError(f"segment {s}: spans must tile its keys in order (kpos {kpos} != {pos})")
-                pos += self.runs[run].length
+                pos += runs[run][2]
             kv.append(pos)
-        object.__setattr__(self, "seg_kv", tuple(kv))
+        self.seg_kv = tuple(kv)
         if len(self.seg_q) != len(self.seg_spans):
             raise ValueError("one span list per segment")
         for s, (row0, length) in enumerate(self.seg_q):
             if length < 0 or row0 < 0 or row0 + length > self.q_rows:
                 raise ValueError(f"segment {s} rows [{row0}, {row0 + length}) outside [0, {self.q_rows})")
-            if length > 0 and self.seg_kv[s] < length:
+            if length > 0 and kv[s] < length:
                 raise ValueError(
-                    f"segment {s} has {length} query rows but only {self.seg_kv[s]} keys; "
+                    f"segment {s} has {length} query rows but only {kv[s]} keys; "
                     "bottom-right causal attention needs kv_len >= q_len"
                 )
-        for r, run in enumerate(self.runs):
-            if not 0 <= run.source < len(self.source_rows):
-                raise ValueError(f"run {r} names source {run.source}")
-            if run.length <= 0 or run.offset < 0 or run.offset + run.length > self.source_rows[run.source]:
+        for r, (source, offset, length) in enumerate(runs):
+            if not 0 <= source < n_sources:
+                raise ValueError(f"run {r} names source {source}")
+            if length <= 0 or offset < 0 or offset + length > sources[source]:
                 raise ValueError(f"run {r} rows outside its source")
         # the backward writes each run's dK/dV through its own rows, without
         # atomics: two runs may not share a row of a source
-        by_source: dict[int, list[tuple[int, int, int]]] = {}
-        for r, run in enumerate(self.runs):
-            by_source.setdefault(run.source, []).append((run.offset, run.offset + run.length, r))
-        for source, spans in by_source.items():
-            spans.sort()
-            for (a0, a1, ra), (b0, _b1, rb) in zip(spans, spans[1:]):
-                if b0 < a1:
-                    raise ValueError(f"runs {ra} and {rb} overlap in source {source} (rows {b0}..{a1 - 1})")
-        if max([*self.seg_kv, 0]) >= 2**31 or self.q_rows >= 2**40:
+        if len({r[0] for r in runs}) != n_runs:
+            by_source: dict[int, list[tuple[int, int, int]]] = {}
+            for r, (source, offset, length) in enumerate(runs):
+                by_source.setdefault(source, []).append((offset, offset + length, r))
+            for source, spans in by_source.items():
+                spans.sort()
+                for (a0, a1, ra), (b0, _b1, rb) in zip(spans, spans[1:]):
+                    if b0 < a1:
+                        raise ValueError(f"runs {ra} and {rb} overlap in source {source} (rows {b0}..{a1 - 1})")
+        if max([*kv, 0]) >= 2**31 or self.q_rows >= 2**40:
             raise ValueError("attention problem too large")
 
     # -- tables -------------------------------------------------------------
@@ -192,27 +196,35 @@ class AttnLayout:
         their addresses), made once."""
         d = self._desc
         if d is None:
-            seg_q = np.array(self.seg_q, np.int64).reshape(-1, 2)
-            seg_span0 = np.zeros(len(self.seg_spans) + 1, np.int64)
-            np.cumsum([len(sp) for sp in self.seg_spans], out=seg_span0[1:])
-            spans = np.array([x for sp in self.seg_spans for x in sp], np.int32).reshape(-1, 2)
-            runs = np.array([(r.source, r.offset, r.length) for r in self.runs], np.int64).reshape(-1, 3)
-            run_len, run_source = runs[:, 2].astype(np.int32), runs[:, 0].astype(np.int32)
-            run_offset = runs[:, 1].copy()
-            nvisit = np.bincount(spans[:, 0], minlength=len(self.runs))
+            span0, at = array("q", (0,)), 0
+            for spans in self.seg_spans:
+                at += len(spans)
+                span0.append(at)
+            spans = array("i", chain.from_iterable(chain.from_iterable(self.seg_spans)))
+            arrays = (array("q", chain.from_iterable(self.seg_q)), span0, spans, array("i", (r[2] for r in self.runs)),
+                      array("i", (r[0] for r in self.runs)), array("q", (r[1] for r in self.runs)))
+            visited = set(spans[::2])
             # rows of each source that a visited run covers (runs do not overlap)
-            covered = np.bincount(run_source, weights=np.where(nvisit > 0, run_len, 0),
-                                  minlength=len(self.source_rows)).astype(np.int64)
+            covered, key_rows, items48, items64 = [0] * len(self.source_rows), 0, 0, 0
+            for r in visited:
+                source, _, length = self.runs[r]
+                covered[source] += length
+                key_rows += length
+                items48 += (length + 47) // 48
+                items64 += (length + 63) // 64
             d = {
-                "arrays": (seg_q, seg_span0, spans, run_len, run_source, run_offset),
-                "ptrs": tuple(a.ctypes.data for a in (seg_q, seg_span0, spans, run_len, run_source, run_offset)),
-                "n_spans": int(spans.shape[0]),
-                "visited_lengths": runs[nvisit > 0, 2],
+                "arrays": arrays,
+                "ptrs": tuple(a.buffer_info()[0] if len(a) else None for a in arrays),
+                "n_spans": at,
+                # dK/dV items of one KV head, by their size
+                "items48": items48,
+                "items64": items64,
                 # sources with rows that no visited run covers: their gradients are filled with zeros first
                 "uncovered": [i for i, n in enumerate(self.source_rows) if covered[i] != n],
                 # query rows that see a visited key, on average
-                "rows_per_key": self.visible_pairs() / max(int(run_len[nvisit > 0].sum()), 1),
-                "all_rows": int(seg_q[:, 1].sum()) == self.q_rows,
+                "rows_per_key": self.visible_pairs() / max(key_rows, 1),
+                "max_keys": max((kv for kv, (_, n) in zip(self.seg_kv, self.seg_q) if n), default=0),
+                "all_rows": sum(n for _, n in self.seg_q) == self.q_rows,
             }
             self._desc = d
         return d
@@ -343,8 +355,7 @@ class AttnLayout:
         kernel)."""
         kvb = kv_block_keys(self.hq, self.hkv, head_dim)
         if head_dim == 256:
-            n64 = int(((self._description()["visited_lengths"] + 63) // 64).sum())
-            if n64 * self.hkv < DKDV256_MIN_ITEMS:
+            if self._description()["items64"] * self.hkv < DKDV256_MIN_ITEMS:
                 kvb = 48
         return kvb
 
@@ -356,7 +367,7 @@ class AttnLayout:
             return self.kv_block_for(device, head_dim)
         d = self._description()
         steps = (self.hq // self.hkv) * d["rows_per_key"] / 32
-        items = int(((d["visited_lengths"] + 47) // 48).sum()) * self.hkv
+        items = d["items48"] * self.hkv
         return 48 if steps >= (DEALT_STEPS_ONE_ROUND if items <= ONE_ROUND_ITEMS else DEALT_STEPS) else 64
 
     def problem(self, device, runs_ptr: int, scale: float, dtype: torch.dtype = torch.bfloat16,
@@ -546,7 +557,7 @@ def _gather(layout: AttnLayout, query: torch.Tensor, keys, values) -> list[int]:
     look per tensor below stand for."""
     if not query.is_cuda or query.dim() != 3 or len(keys) != len(layout.source_rows) or len(values) != len(keys):
         _validate_call(layout, query, keys, values)
-    dtype, device, hkv, d = query.dtype, query.device, layout.hkv, query.shape[2]
+    dtype, device, hkv, d = query.dtype, query.get_device(), layout.hkv, query.shape[2]
     qs = query.stride()
     plain = (dtype in ELEMENT_DTYPES and d in HEAD_DIMS and query.shape == (layout.q_rows, layout.hq, d)
              and qs[2] == 1 and not (qs[0] | qs[1]) & 7 and not query.data_ptr() & 15 and qs[0] < 1 << 24)
@@ -555,7 +566,7 @@ def _gather(layout: AttnLayout, query: torch.Tensor, keys, values) -> list[int]:
         ks, vs, kp, vp = k.stride(), v.stride(), k.data_ptr(), v.data_ptr()
         shape = (n, hkv, d)
         if not (plain and k.dtype is dtype and v.dtype is dtype and k.shape == shape and v.shape == shape
-                and k.device == device and v.device == device and ks[2] == 1 and vs[2] == 1
+                and k.get_device() == device and v.get_device() == device and ks[2] == 1 and vs[2] == 1
                 and not (ks[0] | ks[1] | vs[0] | vs[1]) & 7 and not (kp | vp) & 15
                 and ks[0] < 1 << 24 and vs[0] < 1 << 24):
             _validate_call(layout, query, keys, values)
@@ -563,6 +574,11 @@ def _gather(layout: AttnLayout, query: torch.Tensor, keys, values) -> list[int]:
     if not plain:
         _validate_call(layout, query, keys, values)
     return out
+
+
+def _parts_workspace(parts: int, hq: int, q_rows: int, floats: int, device) -> torch.Tensor | None:
+    """fp32 rows for the partial sums of work items cut into ``parts`` (None for whole items)."""
+    return torch.empty(parts * hq * q_rows * floats, dtype=torch.float32, device=device) if parts > 1 else None
 
 
 def _attention_forward(query: torch.Tensor, layout: AttnLayout, scale: float, keys, values):
@@ -576,10 +592,14 @@ def _attention_forward(query: torch.Tensor, layout: AttnLayout, scale: float, ke
     _, (runs, host, keep) = layout._upload(device, kvb, sources)
     problem = layout.problem(device, runs, scale, query.dtype, query.shape[2], kvb)
     check_tables(layout, problem, host, device)
+    # few work items over many keys: each item's keys in several work-groups
+    parts = lib.ts_attn_fwd_parts(ctypes.byref(problem), layout._description()["max_keys"])
+    work = _parts_workspace(parts, layout.hq, layout.q_rows, query.shape[2] + 2, device)
     with operator_range("hip_attention_forward", rows=layout.q_rows, segments=len(layout.seg_q)):
         _lib.check(
-            lib.ts_attn_fwd(ctypes.byref(problem), _rows(query), _rows(out), lse.data_ptr(), lse.shape[1],
-                            _lib.stream_of(query)),
+            lib.ts_attn_fwd_split(ctypes.byref(problem), _rows(query), _rows(out), lse.data_ptr(), lse.shape[1],
+                                  parts, _lib.ptr(work), 0 if work is None else work.numel() * 4,
+                                  _lib.stream_of(query)),
             lambda: f"ts_attn_fwd(rows={layout.q_rows}, hq={layout.hq}, hkv={layout.hkv})",
         )
     count_attention_path(HIP_PATH)
@@ -639,6 +659,8 @@ def _attention_backward(query, out, lse, dout, layout: AttnLayout, scale: float,
             dq_list, n_dq, n_dq_long = None, 0, 0
             if d == HEAD_DIM and tabs["dq_work"] is not None:
                 dq_list, n_dq, n_dq_long = tabs["dq_work"], tabs["n_dq_work"], tabs["n_dq_long"]
+            # the whole problem's parts for every group of KV heads: the same sums either way
+            parts = lib.ts_attn_dq_parts(ctypes.byref(problem), n_dq, desc["max_keys"])
             for hk0 in range(0, layout.hkv, kv_heads):
                 n, h0 = min(kv_heads, layout.hkv - hk0), hk0 * group
                 sub = problem
@@ -649,11 +671,13 @@ def _attention_backward(query, out, lse, dout, layout: AttnLayout, scale: float,
                     sub.hq, sub.hkv, sub.runs = n * group, n, sub_runs.data_ptr()
                     check_tables(layout, sub, sub_host, device)
                 q_r, o_r, do_r, dq_r = (_head_rows(r, h0) for r in rows)
+                sums = _parts_workspace(parts, sub.hq, layout.q_rows, d, device)
                 _lib.check(
-                    lib.ts_attn_bwd_ds(ctypes.byref(sub), q_r, o_r, do_r, lse.data_ptr() + h0 * lse.shape[1] * 4,
+                    lib.ts_attn_bwd_ds_split(ctypes.byref(sub), q_r, o_r, do_r, lse.data_ptr() + h0 * lse.shape[1] * 4,
                                        lse.shape[1], rowstats.data_ptr() + h0 * lse.shape[1] * 8, dq_r,
                                        tabs["span"], tabs["visit"], tabs["head"], work.data_ptr(),
-                                       work.numel() * 2, dq_list, n_dq, n_dq_long, _lib.stream_of(query)),
+                                       work.numel() * 2, dq_list, n_dq, n_dq_long, parts, _lib.ptr(sums),
+                                       0 if sums is None else sums.numel() * 4, _lib.stream_of(query)),
                     lambda: f"ts_attn_bwd_ds(rows={layout.q_rows}, hq={layout.hq}, hkv={layout.hkv}, heads from {h0})",
                 )
             del work
@@ -753,16 +777,14 @@ def _saved_gradients(ctx, dout: torch.Tensor):
 # ---------------------------------------------------------------------------
 def chain_layout(query_len: int, chunk_lengths: Sequence[int], hq: int, hkv: int) -> AttnLayout:
     """One segment of `query_len` rows over the concatenation of chunks."""
-    runs = tuple(Run(i, 0, n) for i, n in enumerate(chunk_lengths) if n > 0)
-    spans, pos = [], 0
-    run_index = 0
+    runs, spans, pos = [], [], 0
     for i, n in enumerate(chunk_lengths):
         if n > 0:
-            spans.append((run_index, pos))
-            run_index += 1
+            spans.append((len(runs), pos))
+            runs.append(Run(i, 0, n))
             pos += n
     return AttnLayout(
-        q_rows=query_len, hq=hq, hkv=hkv, source_rows=tuple(chunk_lengths), runs=runs,
+        q_rows=query_len, hq=hq, hkv=hkv, source_rows=tuple(chunk_lengths), runs=tuple(runs),
         seg_q=((0, query_len),), seg_spans=(tuple(spans),),
     )
 

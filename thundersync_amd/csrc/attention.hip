@@ -72,7 +72,7 @@ int validate(const ts_attn_problem* p, const char* what) {
 // null), or storing dS in the dK/dV kernels and forming dQ = dS K from it
 int backward(const ts_attn_problem* problem, ts_attn_rows q, ts_attn_rows out, ts_attn_rows dout,
              const float* lse, int64_t lse_ld, float* rowstats, ts_attn_rows dq, const DsArgs* ds,
-             const char* what, void* stream) {
+             const char* what, void* stream, int dq_parts = 1, float* dq_part = nullptr) {
   int st = validate(problem, what);
   if (st != TS_OK) return st;
   const ts_attn_problem& P = *problem;
@@ -92,7 +92,7 @@ int backward(const ts_attn_problem* problem, ts_attn_rows q, ts_attn_rows out, t
   if (st != TS_OK) return st;
   if (ds) {
     st = launch_dkdv(P, q, dout, rowstats, lse_ld, ds, s);
-    if (st == TS_OK && P.n_q_work > 0) st = launch_dq_ds(P, *ds, dq, s);
+    if (st == TS_OK && P.n_q_work > 0) st = launch_dq_ds(P, *ds, dq, dq_parts, dq_part, s);
     return st;
   }
   if (P.n_q_work > 0) {
@@ -101,6 +101,58 @@ int backward(const ts_attn_problem* problem, ts_attn_rows q, ts_attn_rows out, t
   }
   if (P.n_kv_work > 0) st = launch_dkdv(P, q, dout, rowstats, lse_ld, nullptr, s);
   return st;
+}
+
+// Parts per work item of a launch of `items` work-groups over up to `max_keys`
+// keys each: the count with the least estimated time.  A part takes `tile_us`
+// per tile of its keys and 1.5 tiles to start, as long as at most `full`
+// work-groups run; beyond that the launch's throughput no longer grows (or,
+// with `rounds`, the work-groups run in rounds of `full`).  Parts cost a merge
+// launch and the fp32 rows it reads, which the main kernel wrote.  Fitted to
+// sweeps over 1 to 48 parts at 1 to 1024 rows over 1k to 33k keys and 32/8,
+// 40/8 (head dim 128) and 24/4 heads (256), where it picks a count within 15 %
+// of the best but for a few short launches; whole items against parts, us, with
+// the merge: forward 48 rows over 4144 keys at 32/8 heads 93 / 29, 512 over
+// 8192 171 / 92, 16 over 32784 662 / 52, 24/4 heads at head dim 256 48 over 4144
+// 131 / 37; dQ 108 / 27, 205 / 80, 752 / 47, 125 / 29; 512 rows over 1024 keys
+// stay whole (30 / 33).
+struct SplitModel {
+  double tile_us;
+  int tile_keys;
+  double full;
+  bool rounds;
+};
+constexpr int kMaxParts = 32;       // the merge walks an item's parts one after another
+constexpr double kMergeUs = 9.0;    // the merge launch
+constexpr double kMergeItemUs = 0.028;  // per item and part: 128 fp32 rows written and read
+int parts_of(int64_t items, int64_t max_keys, const SplitModel& m) {
+  // launches of more than one round of whole items balance by themselves
+  if (items <= 0 || (double)items >= (m.rounds ? m.full : 2 * m.full)) return 1;
+  const int64_t tiles = (max_keys + m.tile_keys - 1) / m.tile_keys;
+  int best = 1;
+  double least = 0.0;
+  for (int p = 1; p <= kMaxParts && p <= tiles; ++p) {
+    const double groups = (double)items * p;
+    const double load = groups <= m.full ? 1.0 : m.rounds ? (double)(int64_t)((groups + m.full - 1) / m.full)
+                                                          : groups / m.full;
+    const double us = m.tile_us * ((double)tiles / p + 1.5) * load + (p > 1 ? kMergeUs + kMergeItemUs * groups : 0.0);
+    if (p == 1 || us < least) {
+      least = us;
+      best = p;
+    }
+  }
+  return best;
+}
+
+int check_parts(const ts_attn_problem& P, int parts, const void* part, int64_t bytes, int64_t row_floats,
+                const char* what) {
+  TS_CHECK_ARG(parts >= 1 && parts < 65536 && (parts == 1 || ds_route(P.head_dim, P.hq / P.hkv)),
+               "%s: %d parts (head dims 128 and 256 split their items)", what, parts);
+  TS_CHECK_ARG(parts == 1 || (part && (uint64_t)part % 16 == 0 &&
+                              bytes / 4 / row_floats >= (int64_t)parts * P.hq * P.q_rows),
+               "%s: a workspace of %lld bytes for %d parts of %d heads x %lld rows", what, (long long)bytes, parts, P.hq,
+               (long long)P.q_rows);
+  return TS_OK;
 }
 
 }  // namespace attn
@@ -113,8 +165,35 @@ int ts_attn_heads_per_block(int group) { return group > 0 ? ts::attn::heads_per_
 int ts_attn_kv_block(int group, int head_dim) { return group > 0 ? ts::attn::kv_block_keys(group, head_dim) : 0; }
 int ts_attn_q_block(int group) { return group > 0 ? ts::attn::q_block_rows(group) : 0; }
 
+int ts_attn_fwd_parts(const ts_attn_problem* problem, int64_t max_keys) {
+  using namespace ts::attn;
+  if (!problem || problem->hkv <= 0 || problem->hq % problem->hkv || !ds_route(problem->head_dim, 1)) return 1;
+  const int group = problem->hq / problem->hkv;
+  const int64_t items = (int64_t)problem->n_q_work * problem->hkv * (group / heads_per_block(group));
+  // three work-groups a CU at head dim 128, one of eight waves at 256
+  return parts_of(items, max_keys, problem->head_dim == 128 ? SplitModel{0.7, 32, 330, false}
+                                                            : SplitModel{2.0, 64, 256, true});
+}
+
+int ts_attn_dq_parts(const ts_attn_problem* problem, int32_t n_dq_work, int64_t max_keys) {
+  using namespace ts::attn;
+  if (!problem || problem->hkv <= 0 || problem->hq % problem->hkv || !ds_route(problem->head_dim, 1)) return 1;
+  const int group = problem->hq / problem->hkv;
+  const int64_t items = (int64_t)(n_dq_work > 0 ? n_dq_work : problem->n_q_work) * problem->hkv *
+                        (group / heads_per_block(group));
+  // eight waves over 64-row items; four waves
+  return parts_of(items, max_keys, n_dq_work > 0 ? SplitModel{0.8, 32, 200, false}
+                                   : problem->head_dim == 128 ? SplitModel{0.75, 32, 450, false}
+                                                              : SplitModel{0.9, 32, 340, false});
+}
+
 int ts_attn_fwd(const ts_attn_problem* problem, ts_attn_rows q, ts_attn_rows out, float* lse,
                 int64_t lse_ld, void* stream) {
+  return ts_attn_fwd_split(problem, q, out, lse, lse_ld, 1, nullptr, 0, stream);
+}
+
+int ts_attn_fwd_split(const ts_attn_problem* problem, ts_attn_rows q, ts_attn_rows out, float* lse, int64_t lse_ld,
+                      int parts, void* workspace, int64_t workspace_bytes, void* stream) {
   using namespace ts::attn;
   int st = validate(problem, "ts_attn_fwd");
   if (st != TS_OK) return st;
@@ -124,7 +203,9 @@ int ts_attn_fwd(const ts_attn_problem* problem, ts_attn_rows q, ts_attn_rows out
                "with strides that are multiples of 8 elements");
   TS_CHECK_ARG(lse && lse_ld >= P.q_rows, "ts_attn_fwd: lse null or lse_ld %lld < rows %lld",
                (long long)lse_ld, (long long)P.q_rows);
-  return launch_fwd(P, q, out, lse, lse_ld, (hipStream_t)stream);
+  st = check_parts(P, parts, workspace, workspace_bytes, P.head_dim + 2, "ts_attn_fwd");
+  if (st != TS_OK) return st;
+  return launch_fwd(P, q, out, lse, lse_ld, parts, (float*)workspace, (hipStream_t)stream);
 }
 
 int ts_attn_bwd(const ts_attn_problem* problem, ts_attn_rows q, ts_attn_rows out, ts_attn_rows dout,
@@ -180,6 +261,15 @@ int ts_attn_bwd_ds(const ts_attn_problem* problem, ts_attn_rows q, ts_attn_rows 
                    const float* lse, int64_t lse_ld, float* rowstats, ts_attn_rows dq, const int64_t* span_ds,
                    const int64_t* visit_ds, int64_t ds_head, void* ds, int64_t ds_bytes, const int32_t* dq_work,
                    int32_t n_dq_work, int32_t n_dq_long, void* stream) {
+  return ts_attn_bwd_ds_split(problem, q, out, dout, lse, lse_ld, rowstats, dq, span_ds, visit_ds, ds_head, ds,
+                              ds_bytes, dq_work, n_dq_work, n_dq_long, 1, nullptr, 0, stream);
+}
+
+int ts_attn_bwd_ds_split(const ts_attn_problem* problem, ts_attn_rows q, ts_attn_rows out, ts_attn_rows dout,
+                         const float* lse, int64_t lse_ld, float* rowstats, ts_attn_rows dq, const int64_t* span_ds,
+                         const int64_t* visit_ds, int64_t ds_head, void* ds, int64_t ds_bytes,
+                         const int32_t* dq_work, int32_t n_dq_work, int32_t n_dq_long, int dq_parts, void* workspace,
+                         int64_t workspace_bytes, void* stream) {
   using namespace ts::attn;
   const char* what = "ts_attn_bwd_ds";
   TS_CHECK_ARG(problem != nullptr, "%s: null problem", what);
@@ -198,7 +288,9 @@ int ts_attn_bwd_ds(const ts_attn_problem* problem, ts_attn_rows q, ts_attn_rows 
   TS_CHECK_ARG(!dq_work || (problem->head_dim == 128 && (problem->hq / problem->hkv) % 4 == 0),
                "%s: a dQ work list is for GQA groups that are a multiple of 4 at head dim 128", what);
   const DsArgs args{span_ds, visit_ds, ds_head, (uint64_t)ds, dq_work, n_dq_work, n_dq_long};
-  return backward(problem, q, out, dout, lse, lse_ld, rowstats, dq, &args, what, stream);
+  const int st = check_parts(*problem, dq_parts, workspace, workspace_bytes, problem->head_dim, what);
+  if (st != TS_OK) return st;
+  return backward(problem, q, out, dout, lse, lse_ld, rowstats, dq, &args, what, stream, dq_parts, (float*)workspace);
 }
 
 int ts_attn_check_tables(const ts_attn_problem* problem, const ts_attn_segment* segs,

@@ -83,10 +83,13 @@ template <int HD, int WV> constexpr int dq_ds_occupancy() {
   return n > cap ? cap : n;
 }
 
-// WV waves (4, or 8 at head dim 128 with GC = 4 over 64-row items)
-template <typename E, int HD, int GC, int WV = 4>
+// WV waves (4, or 8 at head dim 128 with GC = 4 over 64-row items).  SPLIT:
+// the launch's y blocks are parts of each item's keys, which write fp32 partial
+// sums that dq_merge_kernel adds in part order.
+template <typename E, int HD, int GC, int WV = 4, bool SPLIT = false>
 __global__ __launch_bounds__(64 * WV, (dq_ds_occupancy<HD, WV>())) void dq_ds_kernel(ts_attn_problem P, DsArgs S,
-                                                                                     ts_attn_rows dQ) {
+                                                                                     ts_attn_rows dQ,
+                                                                                     float* __restrict__ part) {
   static_assert(HD == 128 || HD == 256, "the K tile swizzle needs 16 or 32 chunks per row");
   constexpr int KT = dq_ds_tile_keys<HD>();      // keys per tile (64 or 32)
   constexpr int NKB = KT / 16;                   // 16-key dS blocks per tile
@@ -113,6 +116,8 @@ __global__ __launch_bounds__(64 * WV, (dq_ds_occupancy<HD, WV>())) void dq_ds_ke
   const int T = seg.q_len;
   const int off = seg.kv_len - seg.q_len;
   const int last = min(q0 + 32 * WV / GC, T) - 1;  // the work-group's last row
+  int begin = 0, stop = visible_end(seg, last);
+  if constexpr (SPLIT) part_of<KT>(stop, (int)blockIdx.y, (int)gridDim.y, begin, stop);
   const bool rows_valid = 32 * rb < T;
 
   int ro[4], to[8];
@@ -189,13 +194,13 @@ __global__ __launch_bounds__(64 * WV, (dq_ds_occupancy<HD, WV>())) void dq_ds_ke
   };
 
   // tiles i .. i + NST - 2 are in flight at the top of step i
-  TileCursor nx = first_kv_tile<KT>(P, seg, hk, last);
+  TileCursor nx = SPLIT ? first_kv_tile_from<KT>(P, seg, hk, begin, stop) : first_kv_tile<KT>(P, seg, hk, stop);
   int issued = 0;
 #pragma unroll
   for (int p = 0; p < NST - 1; ++p) {
     if (nx.sp < seg.nspan) {
       issue(nx, p);
-      nx = next_kv_tile<KT>(P, seg, hk, last, nx);
+      nx = next_kv_tile<KT>(P, seg, hk, stop, nx);
       ++issued;
     }
   }
@@ -212,7 +217,7 @@ __global__ __launch_bounds__(64 * WV, (dq_ds_occupancy<HD, WV>())) void dq_ds_ke
     __syncthreads();  // tile i is in every stage; stage (i - 1) % NST is free
     if (nx.sp < seg.nspan) {
       issue(nx, (i + NST - 1) % NST);
-      nx = next_kv_tile<KT>(P, seg, hk, last, nx);
+      nx = next_kv_tile<KT>(P, seg, hk, stop, nx);
       ++issued;
     }
     compute(i % NST);
@@ -225,6 +230,12 @@ __global__ __launch_bounds__(64 * WV, (dq_ds_occupancy<HD, WV>())) void dq_ds_ke
   for (int mbp = 0; mbp < 2; ++mbp) {
     const int row = 32 * rb + 16 * ((j16 >> 2) & 1) + 4 * (2 * mbp + (j16 >> 3)) + (j16 & 3);
     if (row >= T) continue;
+    if constexpr (SPLIT) {
+      float* prow = part + part_row(P, (int)blockIdx.y, h, seg.q_row0 + row) * HD + 4 * g4;
+#pragma unroll
+      for (int mb = 0; mb < NMB; ++mb) *reinterpret_cast<f32x4*>(prow + 16 * mb) = acc[mb][mbp];
+      continue;
+    }
     bf16* qrow = (bf16*)dQ.ptr + (seg.q_row0 + row) * dQ.row_stride + (int64_t)h * dQ.head_stride + 4 * g4;
 #pragma unroll
     for (int mb = 0; mb < NMB; ++mb) {
@@ -234,46 +245,81 @@ __global__ __launch_bounds__(64 * WV, (dq_ds_occupancy<HD, WV>())) void dq_ds_ke
   }
 }
 
-template <typename E, int HD>
-void launch_dq_ds_hd(const ts_attn_problem& P, int gc, dim3 grid, const DsArgs& S, ts_attn_rows dq,
-                     hipStream_t s) {
-  ts::TimedLaunch timed_("attention.dq_kernel", s);
-  if (gc == 4)
-    hipLaunchKernelGGL((dq_ds_kernel<E, HD, 4>), grid, dim3(kThreads), 0, s, P, S, dq);
-  else if (gc == 2)
-    hipLaunchKernelGGL((dq_ds_kernel<E, HD, 2>), grid, dim3(kThreads), 0, s, P, S, dq);
-  else
-    hipLaunchKernelGGL((dq_ds_kernel<E, HD, 1>), grid, dim3(kThreads), 0, s, P, S, dq);
+// dQ = scale (the parts' sums in order), four columns a thread; the work-groups
+// cover the work items' rows, as in fwd_merge_kernel
+template <typename E, int HD, int GC, int ROWS>
+__global__ __launch_bounds__(kThreads) void dq_merge_kernel(ts_attn_problem P, ts_attn_rows dQ,
+                                                            const float* __restrict__ part, int parts) {
+  constexpr int Q4 = HD / 4;  // threads per (row, head)
+  const int chunks = P.hq / P.hkv / GC;
+  const int heads = P.hkv * chunks;
+  const int item = (int)blockIdx.x / heads, yb = (int)blockIdx.x % heads;
+  const int seg_id = uniform_table(P.q_work)[2 * item];
+  const int q0 = uniform_table(P.q_work)[2 * item + 1];
+  const ts_attn_segment seg = load_uniform(P.segs, seg_id);
+  constexpr int kPairs = ROWS * GC / kMergeBlocks;
+  const int64_t step = (int64_t)P.hq * P.q_rows * HD;
+#pragma unroll 1
+  for (int i = threadIdx.x / Q4; i < kPairs; i += kThreads / Q4) {
+    const int pair = (int)blockIdx.y * kPairs + i;
+    const int row = q0 + pair / GC, h = yb * GC + pair % GC, d = 4 * (threadIdx.x % Q4);
+    if (row >= seg.q_len) break;
+    const float* x = part + part_row(P, 0, h, seg.q_row0 + row) * HD + d;
+    f32x4 v = *reinterpret_cast<const f32x4*>(x);
+#pragma unroll 4
+    for (int p = 1; p < parts; ++p) v += *reinterpret_cast<const f32x4*>(x + p * step);
+    v *= P.scale;
+    *reinterpret_cast<u32x2*>((bf16*)dQ.ptr + (seg.q_row0 + row) * dQ.row_stride + (int64_t)h * dQ.head_stride + d) =
+        u32x2{pack2<E>(v[0], v[1]), pack2<E>(v[2], v[3])};
+  }
+}
+
+template <typename E, int HD, int GC, int WV>
+void launch_dq_ds_items(const ts_attn_problem& P, const DsArgs& S, ts_attn_rows dq, int parts, float* part,
+                        hipStream_t s) {
+  if (P.n_q_work == 0) return;
+  const unsigned grid = (unsigned)(P.n_q_work * P.hkv * (P.hq / P.hkv / GC));
+  if (parts <= 1) {
+    ts::TimedLaunch timed_("attention.dq_kernel", s);
+    hipLaunchKernelGGL((dq_ds_kernel<E, HD, GC, WV>), dim3(grid), dim3(64 * WV), 0, s, P, S, dq, nullptr);
+    return;
+  }
+  {
+    ts::TimedLaunch timed_("attention.dq_kernel", s);
+    hipLaunchKernelGGL((dq_ds_kernel<E, HD, GC, WV, true>), dim3(grid, parts), dim3(64 * WV), 0, s, P, S, dq, part);
+  }
+  ts::TimedLaunch timed_("attention.dq_merge_kernel", s);
+  hipLaunchKernelGGL((dq_merge_kernel<E, HD, GC, 32 * WV / GC>), dim3(grid, kMergeBlocks), dim3(kThreads), 0, s, P, dq,
+                     part, parts);
 }
 
 template <typename E>
-void launch_dq_ds_t(const ts_attn_problem& P, const DsArgs& S, ts_attn_rows dq, hipStream_t s) {
-  const int group = P.hq / P.hkv;
-  const int gc = heads_per_block(group);
+void launch_dq_ds_t(const ts_attn_problem& P, const DsArgs& S, ts_attn_rows dq, int parts, float* part,
+                    hipStream_t s) {
+  const int gc = heads_per_block(P.hq / P.hkv);
   if (S.dq_work && P.head_dim == 128 && gc == 4) {
     // 64-row items: eight waves, two 32-row blocks per head
     ts_attn_problem P2 = P;
     P2.q_work = S.dq_work;
     P2.n_q_work = S.n_dq_work;
     P2.n_q_long = S.n_dq_long;
-    if (P2.n_q_work == 0) return;
-    ts::TimedLaunch timed_("attention.dq_kernel", s);
-    hipLaunchKernelGGL((dq_ds_kernel<E, 128, 4, 8>), dim3((unsigned)(P2.n_q_work * P.hkv * (group / 4))),
-                       dim3(512), 0, s, P2, S, dq);
-    return;
+    launch_dq_ds_items<E, 128, 4, 8>(P2, S, dq, parts, part, s);
+  } else if (P.head_dim == 256) {
+    if (gc == 4) launch_dq_ds_items<E, 256, 4, 4>(P, S, dq, parts, part, s);
+    else if (gc == 2) launch_dq_ds_items<E, 256, 2, 4>(P, S, dq, parts, part, s);
+    else launch_dq_ds_items<E, 256, 1, 4>(P, S, dq, parts, part, s);
+  } else {
+    if (gc == 4) launch_dq_ds_items<E, 128, 4, 4>(P, S, dq, parts, part, s);
+    else if (gc == 2) launch_dq_ds_items<E, 128, 2, 4>(P, S, dq, parts, part, s);
+    else launch_dq_ds_items<E, 128, 1, 4>(P, S, dq, parts, part, s);
   }
-  const dim3 grid((unsigned)(P.n_q_work * P.hkv * (group / gc)));
-  if (P.head_dim == 256)
-    launch_dq_ds_hd<E, 256>(P, gc, grid, S, dq, s);
-  else
-    launch_dq_ds_hd<E, 128>(P, gc, grid, S, dq, s);
 }
 
-int launch_dq_ds(const ts_attn_problem& P, const DsArgs& S, ts_attn_rows dq, hipStream_t s) {
+int launch_dq_ds(const ts_attn_problem& P, const DsArgs& S, ts_attn_rows dq, int parts, float* part, hipStream_t s) {
   if (P.dtype == kF16)
-    launch_dq_ds_t<f16>(P, S, dq, s);
+    launch_dq_ds_t<f16>(P, S, dq, parts, part, s);
   else
-    launch_dq_ds_t<bf16>(P, S, dq, s);
+    launch_dq_ds_t<bf16>(P, S, dq, parts, part, s);
   return ts::check_launch("ts_attn_bwd (dq from dS)");
 }
 

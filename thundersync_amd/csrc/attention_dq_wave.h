@@ -243,7 +243,7 @@ __global__ __launch_bounds__(64 * 8 / (NQB * NP), 1) void dq_wave_kernel(ts_attn
   auto step = [&](auto bsel, TileCursor& cur) {
     const int kpos = cur.kpos;
     const int kt0 = cur.kt0;
-    const TileCursor nxt = next_kv_tile(P, seg, hk, last, cur);
+    const TileCursor nxt = next_kv_tile(P, seg, hk, visible_end(seg, last), cur);
     __builtin_amdgcn_s_waitcnt(0);  // this wave's part of the tile has landed
     __syncthreads();                // every part has, and the other stage is free
     const bf16* tk = bsel.value == 0 ? s_k0 : s_k1;
@@ -258,7 +258,7 @@ __global__ __launch_bounds__(64 * 8 / (NQB * NP), 1) void dq_wave_kernel(ts_attn
     cur = nxt;
   };
 
-  TileCursor cur = first_kv_tile(P, seg, hk, last);
+  TileCursor cur = first_kv_tile(P, seg, hk, visible_end(seg, last));
   if (cur.sp < seg.nspan) issue_kv_tile<kWaves, HD>(wave, lane, cur, s_k0, s_v0);
   while (cur.sp < seg.nspan) {
     step(std::integral_constant<int, 0>{}, cur);

@@ -182,11 +182,13 @@ constexpr float kRescaleBound = 256.f;  // 2^kRescaleSlack
 template <int NQB, int HD, int KT>
 constexpr int fwd_occupancy() { return HD > 128 ? (NQB == 1 ? 2 : 1) : (NQB == 1 ? 4 : (KT == 32 ? 3 : 2)); }
 
-template <typename E, int NQB, int HD = D, int GC = 4, int KT = BK>
-__global__ __launch_bounds__(64 * 8 / NQB, (fwd_occupancy<NQB, HD, KT>())) void fwd_wave_kernel(ts_attn_problem P, ts_attn_rows Q,
-                                                                                  ts_attn_rows O,
-                                                                                  float* __restrict__ lse,
-                                                                                  int64_t lse_ld) {
+// SPLIT: the launch's y blocks are parts of each item's keys (launches whose
+// items leave CUs idle, ts_attn_fwd_parts); a part writes its unnormalised fp32
+// accumulators and (m, l) per row, which fwd_merge_kernel combines.
+template <typename E, int NQB, int HD = D, int GC = 4, int KT = BK, bool SPLIT = false>
+__global__ __launch_bounds__(64 * 8 / NQB, (fwd_occupancy<NQB, HD, KT>())) void fwd_wave_kernel(
+    ts_attn_problem P, ts_attn_rows Q, ts_attn_rows O, float* __restrict__ lse, int64_t lse_ld,
+    float* __restrict__ part) {
   constexpr int kWaves = 8 / NQB;
   constexpr int NKS = HD / 32, NMB = HD / 16;  // k-steps of S; 16-column blocks of O
   static_assert(KT == 64 || KT == 32, "tiles of 64 or 32 keys");
@@ -210,6 +212,8 @@ __global__ __launch_bounds__(64 * 8 / NQB, (fwd_occupancy<NQB, HD, KT>())) void 
   const int T = seg.q_len;
   const int off = seg.kv_len - seg.q_len;
   const int last = min(q0 + 16 * NQB * kWaves / GC, T) - 1;
+  int begin = 0, stop = off + last + 1;
+  if constexpr (SPLIT) part_of<KT>(stop, (int)blockIdx.y, (int)gridDim.y, begin, stop);
   const float c = P.scale * kLog2e;
 
   // Q rows as B operands: qreg[qb][ks] = row qw + 16 qb + j16, columns 32 ks + 8 g4 ..
@@ -232,7 +236,7 @@ __global__ __launch_bounds__(64 * 8 / NQB, (fwd_occupancy<NQB, HD, KT>())) void 
   auto step = [&](auto bsel, TileCursor& cur) {
     const int kpos = cur.kpos, run_len = cur.len;
     const int kt0 = cur.kt0;
-    const TileCursor nxt = next_kv_tile<KT>(P, seg, hk, last, cur);
+    const TileCursor nxt = next_kv_tile<KT>(P, seg, hk, stop, cur);
     __builtin_amdgcn_s_waitcnt(0);  // this wave's part of the tile has landed
     __syncthreads();                // every part has, and the other stage is free
     const bf16* tk = bsel.value == 0 ? s_k0 : s_k1;
@@ -312,7 +316,9 @@ __global__ __launch_bounds__(64 * 8 / NQB, (fwd_occupancy<NQB, HD, KT>())) void 
           const bool move = mt > m[qb] + kRescaleSlack;
           if (__builtin_amdgcn_ballot_w64(move) != 0) {
             const float mnew = move ? mt : m[qb];
-            const float alpha = fast_exp2(m[qb] - mnew);  // 0 on the first visible keys (m = -inf)
+            // 0 on the first visible keys (m = -inf); a part can hold rows that
+            // see none of its keys so far beside rows that do
+            const float alpha = SPLIT && !move ? 1.f : fast_exp2(m[qb] - mnew);
             l[qb] *= alpha;
 #pragma unroll
             for (int mb = 0; mb < NMB; ++mb) acc[mb][qb] *= alpha;
@@ -361,7 +367,7 @@ __global__ __launch_bounds__(64 * 8 / NQB, (fwd_occupancy<NQB, HD, KT>())) void 
     cur = nxt;
   };
 
-  TileCursor cur = first_kv_tile<KT>(P, seg, hk, last);
+  TileCursor cur = SPLIT ? first_kv_tile_from<KT>(P, seg, hk, begin, stop) : first_kv_tile<KT>(P, seg, hk, stop);
   if (cur.sp < seg.nspan) issue_kv_tile<kWaves, HD, KT>(wave, lane, cur, s_k0, s_v0);
   while (cur.sp < seg.nspan) {
     step(std::integral_constant<int, 0>{}, cur);
@@ -375,6 +381,18 @@ __global__ __launch_bounds__(64 * 8 / NQB, (fwd_occupancy<NQB, HD, KT>())) void 
     const float ls = rows_sum4(l[qb]);
     const int row = qw + 16 * qb + j16;
     if (row >= T) continue;
+    if constexpr (SPLIT) {
+      float* prow = part + part_row(P, (int)blockIdx.y, h, seg.q_row0 + row) * HD + 4 * g4;
+#pragma unroll
+      for (int mb = 0; mb < NMB; ++mb) *reinterpret_cast<f32x4*>(prow + 16 * mb) = acc[mb][qb];
+      if (g4 == 0) {
+        float* st = part_stats<HD>(P, part, (int)gridDim.y) +
+                    2 * part_row(P, (int)blockIdx.y, h, seg.q_row0 + row);
+        st[0] = m[qb];
+        st[1] = ls;
+      }
+      continue;
+    }
     const float inv = ls > 0.f ? 1.f / ls : 0.f;
     bf16* orow = (bf16*)O.ptr + (seg.q_row0 + row) * O.row_stride + (int64_t)h * O.head_stride + 4 * g4;
 #pragma unroll
@@ -384,6 +402,53 @@ __global__ __launch_bounds__(64 * 8 / NQB, (fwd_occupancy<NQB, HD, KT>())) void 
     }
     if (g4 == 0)
       lse[(int64_t)h * lse_ld + seg.q_row0 + row] = ls > 0.f ? (m[qb] + fast_log2(ls)) * kLn2 : neg_inf();
+  }
+}
+
+// Out and log-sum-exp of a split launch: with M the largest part's m, O =
+// sum_p acc_p 2^(m_p - M) / sum_p l_p 2^(m_p - M), the parts in order.  A wave
+// takes one (row, head) at a time, HD / 64 consecutive columns a lane; the y
+// blocks cut an item's rows and heads so that few items still fill the CUs.
+template <typename E, int HD, int GC>
+__global__ __launch_bounds__(kThreads) void fwd_merge_kernel(ts_attn_problem P, ts_attn_rows O,
+                                                             float* __restrict__ lse, int64_t lse_ld,
+                                                             const float* __restrict__ part, int parts) {
+  constexpr int NC = HD / 64;  // columns per lane (2 or 4)
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int chunks = P.hq / P.hkv / GC;
+  const int heads = P.hkv * chunks;  // head chunks of an item
+  const int item = (int)blockIdx.x / heads, yb = (int)blockIdx.x % heads;
+  const int seg_id = uniform_table(P.q_work)[2 * item];
+  const int q0 = uniform_table(P.q_work)[2 * item + 1];
+  const ts_attn_segment seg = load_uniform(P.segs, seg_id);
+  const float* stats = part_stats<HD>(P, part, parts);
+  constexpr int kPairs = 128 / kMergeBlocks;  // (row, head) pairs of a work-group
+#pragma unroll 1
+  for (int i = wave; i < kPairs; i += kThreads / 64) {
+    const int pair = (int)blockIdx.y * kPairs + i;
+    const int row = q0 + pair / GC, h = yb * GC + pair % GC;
+    if (row >= seg.q_len) break;
+    const int64_t at = part_row(P, 0, h, seg.q_row0 + row), step = (int64_t)P.hq * P.q_rows;
+    float M = neg_inf();
+    for (int p = 0; p < parts; ++p) M = fmaxf(M, stats[2 * (at + p * step)]);
+    const float ref = M == neg_inf() ? 0.f : M;
+    float acc[NC], L = 0.f;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) acc[c] = 0.f;
+#pragma unroll 4
+    for (int p = 0; p < parts; ++p) {
+      const float w = fast_exp2(stats[2 * (at + p * step)] - ref);
+      L = fmaf(stats[2 * (at + p * step) + 1], w, L);
+      const float* x = part + (at + p * step) * HD + NC * lane;
+#pragma unroll
+      for (int c = 0; c < NC; ++c) acc[c] = fmaf(x[c], w, acc[c]);
+    }
+    const float inv = L > 0.f ? 1.f / L : 0.f;
+    uint32_t* o = reinterpret_cast<uint32_t*>((bf16*)O.ptr + (seg.q_row0 + row) * O.row_stride +
+                                              (int64_t)h * O.head_stride + NC * lane);
+#pragma unroll
+    for (int c = 0; c < NC; c += 2) o[c / 2] = pack2<E>(acc[c] * inv, acc[c + 1] * inv);
+    if (lane == 0) lse[(int64_t)h * lse_ld + seg.q_row0 + row] = L > 0.f ? (M + fast_log2(L)) * kLn2 : neg_inf();
   }
 }
 
@@ -406,9 +471,29 @@ void launch_fwd_generic(const ts_attn_problem& P, int gc, dim3 grid, ts_attn_row
     hipLaunchKernelGGL((fwd_kernel<E, 1, HD>), grid, dim3(kThreads), 0, s, P, q, out, lse, lse_ld);
 }
 
+// the DMA-staged forward (head dims 128 and 256), whole items or parts of them
+template <typename E, int NQB, int HD, int GC, int KT>
+void launch_fwd_wave(const ts_attn_problem& P, dim3 grid, ts_attn_rows q, ts_attn_rows out, float* lse, int64_t lse_ld,
+                     int parts, float* part, hipStream_t s) {
+  if (parts <= 1) {
+    ts::TimedLaunch timed_("attention.fwd_kernel", s);
+    hipLaunchKernelGGL((fwd_wave_kernel<E, NQB, HD, GC, KT>), grid, dim3(64 * 8 / NQB), 0, s, P, q, out, lse, lse_ld,
+                       nullptr);
+    return;
+  }
+  {
+    ts::TimedLaunch timed_("attention.fwd_kernel", s);
+    hipLaunchKernelGGL((fwd_wave_kernel<E, NQB, HD, GC, KT, true>), dim3(grid.x, parts), dim3(64 * 8 / NQB), 0, s, P, q,
+                       out, lse, lse_ld, part);
+  }
+  ts::TimedLaunch timed_("attention.fwd_merge_kernel", s);
+  hipLaunchKernelGGL((fwd_merge_kernel<E, HD, GC>), dim3(grid.x, kMergeBlocks), dim3(kThreads), 0, s, P, out, lse,
+                     lse_ld, part, parts);
+}
+
 template <typename E>
-int launch_fwd_t(const ts_attn_problem& P, ts_attn_rows q, ts_attn_rows out, float* lse, int64_t lse_ld,
-               hipStream_t s) {
+int launch_fwd_t(const ts_attn_problem& P, ts_attn_rows q, ts_attn_rows out, float* lse, int64_t lse_ld, int parts,
+                 float* part, hipStream_t s) {
   const int group = P.hq / P.hkv;
   const int gc = heads_per_block(group);
   const dim3 grid((unsigned)(P.n_q_work * P.hkv * (group / gc)));
@@ -417,35 +502,25 @@ int launch_fwd_t(const ts_attn_problem& P, ts_attn_rows q, ts_attn_rows out, flo
     case 64: launch_fwd_generic<E, 64>(P, gc, grid, q, out, lse, lse_ld, s); break;
     case 96: launch_fwd_generic<E, 96>(P, gc, grid, q, out, lse, lse_ld, s); break;
     case 192: launch_fwd_generic<E, 192>(P, gc, grid, q, out, lse, lse_ld, s); break;
-    case 256: {
-      ts::TimedLaunch timed_("attention.fwd_kernel", s);
-      if (gc == 4)
-        hipLaunchKernelGGL((fwd_wave_kernel<E, 1, 256, 4>), grid, dim3(512), 0, s, P, q, out, lse, lse_ld);
-      else if (gc == 2)
-        hipLaunchKernelGGL((fwd_wave_kernel<E, 1, 256, 2>), grid, dim3(512), 0, s, P, q, out, lse, lse_ld);
-      else
-        hipLaunchKernelGGL((fwd_wave_kernel<E, 1, 256, 1>), grid, dim3(512), 0, s, P, q, out, lse, lse_ld);
+    case 256:
+      if (gc == 4) launch_fwd_wave<E, 1, 256, 4, BK>(P, grid, q, out, lse, lse_ld, parts, part, s);
+      else if (gc == 2) launch_fwd_wave<E, 1, 256, 2, BK>(P, grid, q, out, lse, lse_ld, parts, part, s);
+      else launch_fwd_wave<E, 1, 256, 1, BK>(P, grid, q, out, lse, lse_ld, parts, part, s);
       break;
-    }
     default: {
-      ts::TimedLaunch timed_("attention.fwd_kernel", s);
-      if (gc == 4)
-        hipLaunchKernelGGL((fwd_wave_kernel<E, kFwdRowsPerWave / 16, D, 4, TS_FWD_KT128>), grid,
-                           dim3(64 * 128 / kFwdRowsPerWave), 0, s, P, q, out, lse, lse_ld);
-      else if (gc == 2)
-        hipLaunchKernelGGL((fwd_wave_kernel<E, 2, D, 2, TS_FWD_KT128_GC>), grid, dim3(256), 0, s, P, q, out, lse,
-                           lse_ld);
-      else
-        hipLaunchKernelGGL((fwd_wave_kernel<E, 2, D, 1, TS_FWD_KT128_GC>), grid, dim3(256), 0, s, P, q, out, lse,
-                           lse_ld);
+      constexpr int NQB = kFwdRowsPerWave / 16;
+      if (gc == 4) launch_fwd_wave<E, NQB, D, 4, TS_FWD_KT128>(P, grid, q, out, lse, lse_ld, parts, part, s);
+      else if (gc == 2) launch_fwd_wave<E, 2, D, 2, TS_FWD_KT128_GC>(P, grid, q, out, lse, lse_ld, parts, part, s);
+      else launch_fwd_wave<E, 2, D, 1, TS_FWD_KT128_GC>(P, grid, q, out, lse, lse_ld, parts, part, s);
     }
   }
   return ts::check_launch("ts_attn_fwd");
 }
 
-int launch_fwd(const ts_attn_problem& P, ts_attn_rows q, ts_attn_rows out, float* lse, int64_t lse_ld,
-               hipStream_t s) {
-  return P.dtype == kF16 ? launch_fwd_t<f16>(P, q, out, lse, lse_ld, s) : launch_fwd_t<bf16>(P, q, out, lse, lse_ld, s);
+int launch_fwd(const ts_attn_problem& P, ts_attn_rows q, ts_attn_rows out, float* lse, int64_t lse_ld, int parts,
+               float* part, hipStream_t s) {
+  return P.dtype == kF16 ? launch_fwd_t<f16>(P, q, out, lse, lse_ld, parts, part, s)
+                         : launch_fwd_t<bf16>(P, q, out, lse, lse_ld, parts, part, s);
 }
 
 }  // namespace attn

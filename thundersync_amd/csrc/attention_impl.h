@@ -347,45 +347,92 @@ __device__ __forceinline__ void enter_span(const ts_attn_problem& P, const ts_at
   tc.vt = (const bf16*)run.v + (int64_t)hk * run.v_head_stride;
 }
 
-// `tc` itself if some row up to `last` (segment-local) can see its tile, else
-// the next such tile in the segment's key order; sp == nspan when none is
-// left.  Spans are in key order, so once a tile starts past the last visible
-// key so do all later ones.  Tables are read only on entering a span.
+// `tc` itself if its tile starts before key position `stop` (of the segment's
+// key order), else the next such tile; sp == nspan when none is left.  Spans
+// are in key order, so once a tile starts at or past `stop` so do all later
+// ones.  Tables are read only on entering a span.  A work item stops after the
+// last key that its last row sees (visible_end); a part of one (part_of) at the
+// next part's first tile.
 template <int KT = BK>
 __device__ __forceinline__ TileCursor settle_kv_tile(const ts_attn_problem& P, const ts_attn_segment& seg, int hk,
-                                                     int last, TileCursor tc) {
-  const int off = seg.kv_len - seg.q_len;
+                                                     int stop, TileCursor tc) {
   while (tc.sp < seg.nspan) {
     if (tc.kt0 >= tc.len) {
       if (++tc.sp < seg.nspan) enter_span(P, seg, hk, tc);
       tc.kt0 = 0;
       continue;
     }
-    if (tc.kpos + tc.kt0 > off + last) tc.sp = seg.nspan;
+    if (tc.kpos + tc.kt0 >= stop) tc.sp = seg.nspan;
     break;
   }
   return tc;
 }
 
-// the visible tile after `tc`: the K / V pointers advance by KT rows within a
-// span (no table reads, no 64-bit products)
+// the tile after `tc`: the K / V pointers advance by KT rows within a span (no
+// table reads, no 64-bit products)
 template <int KT = BK>
 __device__ __forceinline__ TileCursor next_kv_tile(const ts_attn_problem& P, const ts_attn_segment& seg, int hk,
-                                                   int last, TileCursor tc) {
+                                                   int stop, TileCursor tc) {
   tc.kt0 += KT;
   tc.kt += KT * tc.k_rs;
   tc.vt += KT * tc.v_rs;
-  return settle_kv_tile<KT>(P, seg, hk, last, tc);
+  return settle_kv_tile<KT>(P, seg, hk, stop, tc);
 }
 
-// the first visible tile of a segment
+// the first tile of a segment
 template <int KT = BK>
 __device__ __forceinline__ TileCursor first_kv_tile(const ts_attn_problem& P, const ts_attn_segment& seg, int hk,
-                                                    int last) {
+                                                    int stop) {
   TileCursor tc{0, 0, 0, 0, nullptr, nullptr, 0, 0};
   if (seg.nspan > 0) enter_span(P, seg, hk, tc);
-  return settle_kv_tile<KT>(P, seg, hk, last, tc);
+  return settle_kv_tile<KT>(P, seg, hk, stop, tc);
 }
+
+// the first tile that starts at or after key position `begin` (tiles start at
+// multiples of KT within their runs, so the parts of an item take the tiles
+// the whole item would): the last span that starts at or before it, found by
+// bisection over the span positions
+template <int KT = BK>
+__device__ __forceinline__ TileCursor first_kv_tile_from(const ts_attn_problem& P, const ts_attn_segment& seg, int hk,
+                                                         int begin, int stop) {
+  TileCursor tc{0, 0, 0, 0, nullptr, nullptr, 0, 0};
+  if (seg.nspan == 0) return tc;
+  int lo = 0, hi = seg.nspan - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (load_uniform(P.seg_spans, seg.span0 + mid).kpos <= begin) lo = mid;
+    else hi = mid - 1;
+  }
+  tc.sp = lo;
+  enter_span(P, seg, hk, tc);
+  tc.kt0 = (begin - tc.kpos + KT - 1) / KT * KT;
+  tc.kt += (int64_t)tc.kt0 * tc.k_rs;
+  tc.vt += (int64_t)tc.kt0 * tc.v_rs;
+  return settle_kv_tile<KT>(P, seg, hk, stop, tc);
+}
+
+// keys that row `last` of a segment sees
+__device__ __forceinline__ int visible_end(const ts_attn_segment& seg, int last) {
+  return seg.kv_len - seg.q_len + last + 1;
+}
+// key positions [begin, end) of part `part` of `parts` of an item of `keys` keys
+template <int KT>
+__device__ __forceinline__ void part_of(int keys, int part, int parts, int& begin, int& end) {
+  const int per = ((keys + parts - 1) / parts + KT - 1) / KT * KT;
+  begin = min(keys, part * per);
+  end = min(keys, begin + per);
+}
+
+// Partial sums of a launch whose items are cut into parts: fp32 rows
+// [parts][hq][q_rows][head dim], then (forward) (m, l) pairs [parts][hq][q_rows][2].
+__host__ __device__ inline int64_t part_row(const ts_attn_problem& P, int part, int h, int64_t row) {
+  return ((int64_t)part * P.hq + h) * P.q_rows + row;
+}
+template <int HD, typename T>
+__device__ __forceinline__ T* part_stats(const ts_attn_problem& P, T* part, int parts) {
+  return part + part_row(P, parts, 0, 0) * HD;
+}
+constexpr int kMergeBlocks = 16;  // work-groups that merge one item's parts
 
 // Row swizzle of the 256-byte-row LDS tiles: 16-byte chunk c of row r sits at
 // slot c ^ tile_swizzle(r & 15).  Measured on the MI355X with a read-rate probe
@@ -484,8 +531,10 @@ inline int q_block_rows(int group) { return 32 * 4 / heads_per_block(group); }
 inline int kv_block_keys(int group, int head_dim) { return group % 4 == 0 && head_dim != 256 ? 48 : BK; }
 
 // launchers (one per kernel family); each returns a TS_* status
-int launch_fwd(const ts_attn_problem& P, ts_attn_rows q, ts_attn_rows out, float* lse, int64_t lse_ld,
-               hipStream_t s);
+// `parts` > 1: each item's keys in that many work-groups, partial sums in
+// `part` (split_part_floats per part), merged by a second kernel
+int launch_fwd(const ts_attn_problem& P, ts_attn_rows q, ts_attn_rows out, float* lse, int64_t lse_ld, int parts,
+               float* part, hipStream_t s);
 int launch_delta(const ts_attn_problem& P, ts_attn_rows out, ts_attn_rows dout, const float* lse,
                  float* rowstats, int64_t lse_ld, hipStream_t s);
 int launch_dq(const ts_attn_problem& P, ts_attn_rows q, ts_attn_rows dout, const float* rowstats,
@@ -505,7 +554,8 @@ template <typename E, bool DS>
 void launch_dkdv256(dim3 grid, const ts_attn_problem& P, ts_attn_rows q, ts_attn_rows dout,
                     const float* rowstats, int64_t lse_ld, const DsArgs& S, hipStream_t s);
 // dQ = scale dS K from the workspace the dK/dV launch filled
-int launch_dq_ds(const ts_attn_problem& P, const DsArgs& ds, ts_attn_rows dq, hipStream_t s);
+int launch_dq_ds(const ts_attn_problem& P, const DsArgs& ds, ts_attn_rows dq, int parts, float* part,
+                 hipStream_t s);
 
 // the dS route: head dims 128 and 256 (the DMA-staged dK/dV kernels), every
 // GQA group size
