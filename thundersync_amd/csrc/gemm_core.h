@@ -20,21 +20,28 @@
 namespace ts {
 namespace gemm {
 
-#ifndef TS_GEMM_WAVES
-#define TS_GEMM_WAVES 8
-#endif
-// waves per work-group: 8 (two per SIMD, wave tile 128 x 64) or 4 (one per
-// SIMD, wave tile 128 x 128); wave w covers A rows 128 (w & 1) .. and B rows
-// 32 NI (w >> 1) ..
-constexpr int kWaves = TS_GEMM_WAVES;
-static_assert(kWaves == 8 || kWaves == 4, "8 or 4 waves per GEMM work-group");
+constexpr int kWaves = 8;  // waves per work-group, two per SIMD
 constexpr int kGemmThreads = 64 * kWaves;
-constexpr int NI = 16 / kWaves;         // 32-column B blocks per wave
-constexpr int kDmaPerWave = 16 / kWaves;  // DMA instructions per operand, wave and stage
 constexpr int TM = 256;  // A rows (vocab rows, or hidden dims) per work-group
 constexpr int TN = 256;  // B rows (tokens) per work-group
 constexpr int TK = 32;   // K per LDS stage
 constexpr int kStageElems = (TM + TN) * TK;  // 32 KB: A [TM][TK], then B [TN][TK]
+
+// How the waves cover a tile of 256 A rows: WM_ x WN_ of them, each MI_ x NI_
+// blocks of 32 x 32 (wave w: A rows 32 MI (w % WM) .., B rows 32 NI (w / WM) ..).
+// Full is the 256 x 256 tile.  Narrow<NI> takes 64 NI B rows (64, 128 or 192), for
+// launches of few B rows, which in Full tiles would do their MFMAs on zeros.  Its
+// waves are 64 x 32 NI blocks, (2 + NI) / 2 NI LDS fragment reads per MFMA against
+// 3 / 4.
+template <int WM_, int WN_, int MI_, int NI_>
+struct Shape {
+  static constexpr int WM = WM_, WN = WN_, MI = MI_, NI = NI_;
+  static constexpr int BN = 32 * WN_ * NI_;  // B rows of the tile
+  static_assert(WM_ * WN_ == kWaves && 32 * WM_ * MI_ == TM && BN <= TN, "eight waves over 256 A rows");
+};
+using Full = Shape<2, 4, 4, 2>;
+template <int NI_> using Narrow = Shape<4, 2, 2, NI_>;
+constexpr int NI = Full::NI;
 
 __device__ __forceinline__ u32x4 ld16(const bf16* p) { return *reinterpret_cast<const u32x4*>(p); }
 
@@ -59,16 +66,20 @@ __device__ __forceinline__ void grouped_tile(int id, int n_a, int n_b, int& ta, 
 }
 
 // One operand's share of a stage: 256 rows x 64 bytes = 16 instructions of 16
-// rows each, issued by the waves as t = wave + kWaves u.  Lane i of an
+// rows each (a narrower B tile fewer), issued by the waves as t = wave + kWaves u
+// modulo their number (a wave past the end repeats another's, with the same
+// bytes, so that every wave counts alike).  Lane i of an
 // instruction fills row 16 t + i / 4, slot i & 3 with the logical 16-byte
 // chunk c = (i & 3) ^ (i >> 4): row r's chunk c sits at slot c ^ ((r >> 2) & 3),
 // so the 16 rows of a fragment read at one chunk hit 16 distinct bank groups.
+template <int ROWS>
 struct Streamer {
+  static constexpr int kInstr = ROWS / 16, kPerWave = (kInstr + kWaves - 1) / kWaves;
   const bf16* base;  // row 0, k 0
   int64_t ld;
   int rows;          // valid rows from base (>= 1)
   int K;
-  int voff[kDmaPerWave];  // byte offset of this lane's row and chunk within a stage, per u
+  int voff[kPerWave];  // byte offset of this lane's row and chunk within a stage, per u
   int kchunk;        // this lane's chunk start within a stage (elements)
   __device__ __forceinline__ void init(const bf16* b, int64_t ld_, int rows_, int K_, int wave, int lane) {
     base = b;
@@ -77,8 +88,8 @@ struct Streamer {
     K = K_;
     kchunk = 8 * ((lane & 3) ^ (lane >> 4));
 #pragma unroll
-    for (int u = 0; u < kDmaPerWave; ++u)
-      voff[u] = (int)(((16 * (wave + kWaves * u) + (lane >> 2)) * ld + kchunk) * 2);
+    for (int u = 0; u < kPerWave; ++u)
+      voff[u] = (int)(((16 * ((wave + kWaves * u) % kInstr) + (lane >> 2)) * ld + kchunk) * 2);
   }
   // descriptor and this lane's chunk validity for K columns [k0, k0 + TK)
   __device__ __forceinline__ u32x4 descriptor(int k0) const {
@@ -87,7 +98,7 @@ struct Streamer {
   // instruction u of this wave's share of the stage into dst (wave-uniform);
   // a chunk past K reads nothing: zeros
   __device__ __forceinline__ void issue(u32x4 r, bool in_k, bf16* dst, int u, int wave) const {
-    buffer_dma16_untracked(r, dst + (wave + kWaves * u) * 512, in_k ? voff[u] : 0x7ffffff0);
+    buffer_dma16_untracked(r, dst + ((wave + kWaves * u) % kInstr) * 512, in_k ? voff[u] : 0x7ffffff0);
   }
 };
 
@@ -102,18 +113,19 @@ struct Streamer {
 // range checking); chunks past M in earlier rows read the next row, which
 // lands in output rows or columns the epilogue discards.
 struct StreamerT {
+  static constexpr int kPerWave = 2;
   const bf16* base;  // k 0, m 0 of the tile
   int64_t ld;        // elements between consecutive K rows
   int mvalid;        // valid M columns from base (>= 1)
   int K;
-  int voff[kDmaPerWave];
+  int voff[kPerWave];
   __device__ __forceinline__ void init(const bf16* b, int64_t ld_, int mvalid_, int K_, int wave, int lane) {
     base = b;
     ld = ld_;
     mvalid = min(mvalid_, TM);
     K = K_;
 #pragma unroll
-    for (int u = 0; u < kDmaPerWave; ++u) {
+    for (int u = 0; u < kPerWave; ++u) {
       const int row = 2 * (wave + kWaves * u) + (lane >> 5);
       const int c = (lane & 31) ^ (4 * (row & 3));
       voff[u] = (int)((row * ld + 8 * c) * 2);
@@ -179,33 +191,36 @@ template <> struct Frag<true> {
   }
 };
 
-// acc[mi][ni]: 32x32 block (A rows 128 wm + 32 mi, B rows 32 NI wn + 32 ni),
-// wm = wave & 1, wn = wave >> 1.  Lane l holds B row b_row(ni, l, wn) and A rows
+// acc[mi][ni]: 32x32 block (A rows 32 (MI wm + mi), B rows 32 (NI wn + ni)),
+// wm = wave % WM, wn = wave / WM.  Lane l holds B row b_row(ni, l, wn) and A rows
 // a_row(mi, i, l, wm), i = 0..15.
+template <class S = Full>
 __device__ __forceinline__ int a_row(int mi, int i, int lane, int wm) {
-  return 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3) + 32 * mi + 128 * wm;
+  return 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3) + 32 * mi + 32 * S::MI * wm;
 }
-__device__ __forceinline__ int b_row(int ni, int lane, int wn) { return 32 * NI * wn + 32 * ni + (lane & 31); }
+template <class S = Full>
+__device__ __forceinline__ int b_row(int ni, int lane, int wn) { return 32 * S::NI * wn + 32 * ni + (lane & 31); }
 
 // The MFMAs of one stage (two k-steps of 16) in a fixed order.  The k-step-0
 // fragments a0 / b0 of `st` arrive already in registers (read during the
-// previous stage); four groups of {two k-step-0 MFMAs, one or two k-step-1
-// fragment reads, one refill DMA instruction}, then the 8 k-step-1 MFMAs,
-// beside which the k-step-0 fragments of the next stage `nx` (if any) are
-// read into a0 / b0.  Spreading the refill over the MFMAs keeps the wave
+// previous stage); MI groups of {the k-step-0 MFMAs of an A block, a share of
+// the k-step-1 fragment reads, a share of the refill DMA}, then the k-step-1
+// MFMAs, beside which the k-step-0 fragments of the next stage `nx` (if any)
+// are read into a0 / b0.  Spreading the refill over the MFMAs keeps the wave
 // issuing MFMAs while the DMA is in flight, and with the next stage's first
 // fragments in registers the MFMAs start right after the stage barrier
 // instead of waiting for LDS reads every wave issues at once.
-template <typename E, bool HAS_NEXT, class FA, class FB, class Dma>
-__device__ __forceinline__ void mma_stage(f32x16 acc[4][NI], const bf16* st, const bf16* nx, const FA& fa,
-                                          const FB& fb, bf16x8 (&a0)[4], bf16x8 (&b0)[NI], Dma&& dma) {
-  bf16x8 a1[4], b1[NI];
+template <typename E, bool HAS_NEXT, class S, int DMA, class FA, class FB, class Dma>
+__device__ __forceinline__ void mma_stage(f32x16 (&acc)[S::MI][S::NI], const bf16* st, const bf16* nx, const FA& fa,
+                                          const FB& fb, bf16x8 (&a0)[S::MI], bf16x8 (&b0)[S::NI], Dma&& dma) {
+  constexpr int MI = S::MI, NI = S::NI, READS = MI + NI;
+  bf16x8 a1[MI], b1[NI];
   const bf16* sb = st + TM * TK;
 #pragma unroll
-  for (int g = 0; g < 4; ++g) {
+  for (int g = 0; g < MI; ++g) {
 #pragma unroll
     for (int ni = 0; ni < NI; ++ni) acc[g][ni] = mma32<E>(a0[g], b0[ni], acc[g][ni]);
-    if constexpr (NI == 2) {
+    if constexpr (MI == 4 && NI == 2) {
       if (g < 2) {
         a1[2 * g] = fa.read(st, 1, 2 * g);
         a1[2 * g + 1] = fa.read(st, 1, 2 * g + 1);
@@ -213,93 +228,103 @@ __device__ __forceinline__ void mma_stage(f32x16 acc[4][NI], const bf16* st, con
         b1[g - 2] = fb.read(sb, 1, g - 2);
       }
     } else {
-      a1[g] = fa.read(st, 1, g);
-      b1[g] = fb.read(sb, 1, g);
+#pragma unroll
+      for (int r = g * READS / MI; r < (g + 1) * READS / MI; ++r) {
+        if (r < MI) a1[r] = fa.read(st, 1, r);
+        else b1[r - MI] = fb.read(sb, 1, r - MI);
+      }
     }
-    dma(g);
+#pragma unroll
+    for (int d = g * DMA / MI; d < (g + 1) * DMA / MI; ++d) dma(d);
     __builtin_amdgcn_sched_barrier(0);
   }
 #pragma unroll
-  for (int mi = 0; mi < 4; ++mi) {
+  for (int mi = 0; mi < MI; ++mi) {
 #pragma unroll
     for (int ni = 0; ni < NI; ++ni) acc[mi][ni] = mma32<E>(a1[mi], b1[ni], acc[mi][ni]);
     if (HAS_NEXT || nx != nullptr) {
       a0[mi] = fa.read(nx, 0, mi);
-      if (mi < NI) b0[mi] = fb.read(nx + TM * TK, 0, mi);
+      if constexpr (MI == 4 && NI == 2) {
+        if (mi < NI) b0[mi] = fb.read(nx + TM * TK, 0, mi);
+      } else {
+#pragma unroll
+        for (int ni = mi * NI / MI; ni < (mi + 1) * NI / MI; ++ni) b0[ni] = fb.read(nx + TM * TK, 0, ni);
+      }
     }
     __builtin_amdgcn_sched_barrier(0);
   }
 }
 
-// wait until at most `ahead` stages of this wave's DMA instructions are in
-// flight (2 kDmaPerWave instructions per stage)
+// wait until at most `ahead` stages of this wave's DMA instructions (PER each)
+// are in flight
+template <int PER>
 __device__ __forceinline__ void wait_dma(int ahead) {
-  if constexpr (kDmaPerWave == 2) {
-    if (ahead >= 2) __builtin_amdgcn_s_waitcnt(0x0F78);       // vmcnt(8)
-    else if (ahead == 1) __builtin_amdgcn_s_waitcnt(0x0F74);  // vmcnt(4)
-    else __builtin_amdgcn_s_waitcnt(0x0F70);                  // vmcnt(0)
-  } else {
-    if (ahead >= 2) __builtin_amdgcn_s_waitcnt(0x4F70);       // vmcnt(16)
-    else if (ahead == 1) __builtin_amdgcn_s_waitcnt(0x0F78);  // vmcnt(8)
-    else __builtin_amdgcn_s_waitcnt(0x0F70);                  // vmcnt(0)
-  }
+  static_assert(2 * PER < 16, "the low four bits of vmcnt");
+  if (ahead >= 2) __builtin_amdgcn_s_waitcnt(0x0F70 | (2 * PER));
+  else if (ahead == 1) __builtin_amdgcn_s_waitcnt(0x0F70 | PER);
+  else __builtin_amdgcn_s_waitcnt(0x0F70);
 }
 
 // C tile = A . B^T over K through the LDS ring s0..s3 (distinct arrays, so the
 // compiler sees that a refill and the reads of another stage never alias);
 // the ring is free on return.  AKS / BKS: the operand is K-strided (A is then
 // given as its [K][M] storage from the tile's first column, B likewise);
-// otherwise K-contiguous (a_rows / b_rows valid rows of 256 from A / B).
-template <typename E, bool AKS, bool BKS>
-__device__ __forceinline__ void gemm_tile(f32x16 acc[4][NI], const bf16* A, int64_t lda, int a_rows,
+// otherwise K-contiguous (a_rows / b_rows valid rows from A / B).  S: the tile's
+// B rows and how the waves cover it.
+template <typename E, bool AKS, bool BKS, class S = Full>
+__device__ __forceinline__ void gemm_tile(f32x16 (&acc)[S::MI][S::NI], const bf16* A, int64_t lda, int a_rows,
                                           const bf16* B, int64_t ldb, int b_rows, int K, bf16* s0,
                                           bf16* s1, bf16* s2, bf16* s3) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave & 1, wn = wave >> 1;
+  constexpr int MI = S::MI, NI = S::NI;
+  static_assert(!BKS || S::BN == TN, "a K-strided B operand is staged as whole 256-column rows");
+  const int wm = wave % S::WM, wn = wave / S::WM;
 #pragma unroll
-  for (int mi = 0; mi < 4; ++mi)
+  for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
     for (int ni = 0; ni < NI; ++ni)
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc[mi][ni][i] = 0.f;
-  std::conditional_t<AKS, StreamerT, Streamer> sa;
-  std::conditional_t<BKS, StreamerT, Streamer> sb;
+  using SA = std::conditional_t<AKS, StreamerT, Streamer<TM>>;
+  using SB = std::conditional_t<BKS, StreamerT, Streamer<S::BN>>;
+  constexpr int PA = SA::kPerWave, PB = SB::kPerWave;  // DMA instructions per wave and stage
+  SA sa;
+  SB sb;
   sa.init(A, lda, a_rows, K, wave, lane);
   sb.init(B, ldb, b_rows, K, wave, lane);
   Frag<AKS> fa;
   Frag<BKS> fb;
-  fa.init(lane, 128 * wm);
+  fa.init(lane, 32 * MI * wm);
   fb.init(lane, 32 * NI * wn);
   const int nk = (K + TK - 1) / TK;
   // operand s of stage kt: descriptor, and per lane whether its chunk is in K
   // (K-strided operands bound K by the descriptor's row count instead)
   auto in_k = [&](const auto& s, int k0) {
-    if constexpr (std::is_same_v<std::decay_t<decltype(s)>, Streamer>) return k0 + s.kchunk < K;
-    else return true;
+    if constexpr (std::is_same_v<std::decay_t<decltype(s)>, StreamerT>) return true;
+    else return k0 + s.kchunk < K;
   };
   auto put = [&](const auto& s, u32x4 r, bool ik, bf16* dst, int u) {
-    if constexpr (std::is_same_v<std::decay_t<decltype(s)>, Streamer>) s.issue(r, ik, dst, u, wave);
-    else s.issue(r, dst, u, wave);
+    if constexpr (std::is_same_v<std::decay_t<decltype(s)>, StreamerT>) s.issue(r, dst, u, wave);
+    else s.issue(r, ik, dst, u, wave);
   };
   auto issue = [&](bf16* st, int kt) {
     const u32x4 ra = sa.descriptor(kt * TK), rb = sb.descriptor(kt * TK);
     const bool ka = in_k(sa, kt * TK), kb = in_k(sb, kt * TK);
 #pragma unroll
-    for (int u = 0; u < kDmaPerWave; ++u) {
-      put(sa, ra, ka, st, u);
-      put(sb, rb, kb, st + TM * TK, u);
-    }
+    for (int u = 0; u < PA; ++u) put(sa, ra, ka, st, u);
+#pragma unroll
+    for (int u = 0; u < PB; ++u) put(sb, rb, kb, st + TM * TK, u);
   };
   issue(s0, 0);
   if (nk > 1) issue(s1, 1);
   if (nk > 2) issue(s2, 2);
   // stage 0 landed everywhere: its k-step-0 fragments into registers
-  bf16x8 a0[4], b0[NI];
-  wait_dma(min(nk - 1, 2));
+  bf16x8 a0[MI], b0[NI];
+  wait_dma<PA + PB>(min(nk - 1, 2));
   __builtin_amdgcn_s_barrier();
 #pragma unroll
-  for (int mi = 0; mi < 4; ++mi) a0[mi] = fa.read(s0, 0, mi);
+  for (int mi = 0; mi < MI; ++mi) a0[mi] = fa.read(s0, 0, mi);
 #pragma unroll
   for (int ni = 0; ni < NI; ++ni) b0[ni] = fb.read(s0 + TM * TK, 0, ni);
   // step kt: this wave's DMA of stages kt and kt + 1 has landed (stage kt + 2
@@ -314,23 +339,18 @@ __device__ __forceinline__ void gemm_tile(f32x16 acc[4][NI], const bf16* A, int6
   auto step = [&](auto full, const bf16* cur, const bf16* nxt, bf16* refill, int kt) {
     constexpr bool FULL = decltype(full)::value;
     __builtin_amdgcn_sched_barrier(0);  // keep each stage's loads inside its stage
-    if constexpr (FULL) wait_dma(1);
-    else wait_dma(max(min(nk - 2 - kt, 1), 0));
+    if constexpr (FULL) wait_dma<PA + PB>(1);
+    else wait_dma<PA + PB>(max(min(nk - 2 - kt, 1), 0));
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
     __builtin_amdgcn_s_barrier();
     const bool refill_now = FULL || kt + 3 < nk;
     const int k0 = (kt + 3) * TK;
     const u32x4 ra = sa.descriptor(refill_now ? k0 : 0), rb = sb.descriptor(refill_now ? k0 : 0);
     const bool ka = FULL || in_k(sa, k0), kb = FULL || in_k(sb, k0);
-    mma_stage<E, FULL>(acc, cur, (FULL || kt + 1 < nk) ? nxt : nullptr, fa, fb, a0, b0, [&](int g) {
+    mma_stage<E, FULL, S, PA + PB>(acc, cur, (FULL || kt + 1 < nk) ? nxt : nullptr, fa, fb, a0, b0, [&](int d) {
       if (refill_now) {
-        if constexpr (kDmaPerWave == 2) {
-          if (g < 2) put(sa, ra, ka, refill, g);
-          else put(sb, rb, kb, refill + TM * TK, g - 2);
-        } else {
-          put(sa, ra, ka, refill, g);
-          put(sb, rb, kb, refill + TM * TK, g);
-        }
+        if (d < PA) put(sa, ra, ka, refill, d);
+        else put(sb, rb, kb, refill + TM * TK, d - PA);
       }
     });
   };

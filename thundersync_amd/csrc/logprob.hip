@@ -74,38 +74,52 @@ struct FwdArgs {
   float* part_e;
 };
 
-template <typename E>
+// Token rows per tile of a launch: the rows spread evenly over as few tiles as
+// 256-token tiles take.  Rows past the end of a tile are MFMA work on zeros --
+// cheap on a chip whose clock follows its power, so a narrower tile pays only
+// where it is much narrower: 64 or 128 tokens (4096 x 151936: 25 rows forward 279
+// -> 264, dlogits 307 -> 269, grad_hidden 201 -> 188 us, 128 rows 307 -> 288, 337 ->
+// 295, 235 -> 223), and for grad_hidden, whose launch of few rows is one round that
+// ends with its widest tiles, 192 for up to 160 (281 rows 469 -> 427, 320 rows 463 ->
+// 409; at 192 rows a tile 464 -> 478, and forward and dlogits gain nothing).
+inline int token_tile(int64_t rows, bool up_to_192) {
+  const int64_t tiles = (rows + TN - 1) / TN, each = (rows + tiles - 1) / tiles;
+  return each <= 64 ? 64 : each <= 128 ? 128 : up_to_192 && each <= 160 ? 192 : 256;
+}
+
+template <typename E, class S>
 __global__ __launch_bounds__(kGemmThreads, 1) void fwd_stats_kernel(FwdArgs p) {
   GEMM_RING
+  constexpr int MI = S::MI, NI = S::NI;
   const int total = p.n_ttiles * p.n_vtiles;
   int vt, tt;
   grouped_tile(xcd_logical(blockIdx.x, total), p.n_vtiles, p.n_ttiles, vt, tt);
-  const int v0 = vt * TM, n0 = tt * TN;
-  f32x16 acc[4][NI];
-  gemm_tile<E, false, false>(acc, p.w + (int64_t)v0 * p.ldw, p.ldw, min(TM, p.vocab - v0),
-                          p.h + (int64_t)n0 * p.ldh, p.ldh, min(TN, p.rows - n0), p.dim, s0, s1, s2, s3);
+  const int v0 = vt * TM, n0 = tt * S::BN;
+  f32x16 acc[MI][NI];
+  gemm_tile<E, false, false, S>(acc, p.w + (int64_t)v0 * p.ldw, p.ldw, min(TM, p.vocab - v0),
+                          p.h + (int64_t)n0 * p.ldh, p.ldh, min(S::BN, p.rows - n0), p.dim, s0, s1, s2, s3);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave & 1, wn = wave >> 1;
-  float* xm = reinterpret_cast<float*>(s0);  // [TN] per token, from the wm = 1 waves
-  float* xs = xm + TN;
-  float* xe = xs + TN;
+  const int wm = wave % S::WM, wn = wave / S::WM;
+  float* xm = reinterpret_cast<float*>(s0);  // [WM - 1][BN] per token, from the waves wm > 0
+  float* xs = xm + (S::WM - 1) * S::BN;
+  float* xe = xs + (S::WM - 1) * S::BN;
   // rows past the vocabulary (last vocab tile only) take no part
   if (v0 + TM > p.vocab) {
 #pragma unroll
-    for (int mi = 0; mi < 4; ++mi)
+    for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
       for (int ni = 0; ni < NI; ++ni)
 #pragma unroll
         for (int i = 0; i < 16; ++i)
-          if (v0 + a_row(mi, i, lane, wm) >= p.vocab) acc[mi][ni][i] = neg_inf();
+          if (v0 + a_row<S>(mi, i, lane, wm) >= p.vocab) acc[mi][ni][i] = neg_inf();
   }
   float mk[NI], sk[NI], ek[NI];  // this lane's column statistics, kept across the exchange
 #pragma unroll
   for (int ni = 0; ni < NI; ++ni) {
-    const int col = b_row(ni, lane, wn);
+    const int col = b_row<S>(ni, lane, wn);
     float m = neg_inf();
 #pragma unroll
-    for (int mi = 0; mi < 4; ++mi)
+    for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
       for (int i = 0; i < 16; i += 2) m = fmaxf(m, fmaxf(acc[mi][ni][i], acc[mi][ni][i + 1]));
     // sum of q = 2^d2 and of q d2 with d2 = (l - m) log2 e as one FMA per logit; the second
@@ -114,7 +128,7 @@ __global__ __launch_bounds__(kGemmThreads, 1) void fwd_stats_kernel(FwdArgs p) {
     const float m2 = m * kLog2e;
     if (v0 + TM <= p.vocab) {
 #pragma unroll
-      for (int mi = 0; mi < 4; ++mi)
+      for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
           const float d2 = fmaf(acc[mi][ni][i], kLog2e, -m2);
@@ -124,7 +138,7 @@ __global__ __launch_bounds__(kGemmThreads, 1) void fwd_stats_kernel(FwdArgs p) {
         }
     } else if (m != neg_inf()) {
 #pragma unroll
-      for (int mi = 0; mi < 4; ++mi)
+      for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
           const float d2 = fmaf(acc[mi][ni][i], kLog2e, -m2);  // -inf past the vocabulary: q = 0
@@ -139,10 +153,10 @@ __global__ __launch_bounds__(kGemmThreads, 1) void fwd_stats_kernel(FwdArgs p) {
       const float mo = shfl_xor(m, 32), so = shfl_xor(sum, 32), eo = shfl_xor(e, 32);
       merge_stats(m, sum, e, mo, so, eo);
     }
-    if (wm == 1 && lane < 32) {
-      xm[col] = m;
-      xs[col] = sum;
-      xe[col] = e;
+    if (wm > 0 && lane < 32) {
+      xm[(wm - 1) * S::BN + col] = m;
+      xs[(wm - 1) * S::BN + col] = sum;
+      xe[(wm - 1) * S::BN + col] = e;
     }
     mk[ni] = m;
     sk[ni] = sum;
@@ -151,10 +165,12 @@ __global__ __launch_bounds__(kGemmThreads, 1) void fwd_stats_kernel(FwdArgs p) {
   __syncthreads();  // one exchange for both column groups (their columns differ)
 #pragma unroll
   for (int ni = 0; ni < NI; ++ni) {
-    const int col = b_row(ni, lane, wn);
+    const int col = b_row<S>(ni, lane, wn);
     const int n = n0 + col;
     if (wm == 0 && lane < 32 && n < p.rows) {
-      merge_stats(mk[ni], sk[ni], ek[ni], xm[col], xs[col], xe[col]);
+#pragma unroll
+      for (int w = 0; w < S::WM - 1; ++w)
+        merge_stats(mk[ni], sk[ni], ek[ni], xm[w * S::BN + col], xs[w * S::BN + col], xe[w * S::BN + col]);
       const int64_t o = (int64_t)vt * p.rows + n;
       p.part_m[o] = mk[ni];
       p.part_s[o] = sk[ni];
@@ -260,33 +276,60 @@ struct DlArgs {
 constexpr int OPITCH = TM + 8;  // staging pitch (bf16) of [64 tokens][TM vocab] quarter tiles
 static_assert(64 * OPITCH <= kRingElems, "a quarter of the dlogits tile fits one ring stage");
 
-template <typename E>
+// A target lies in one vocabulary tile of 594, so the one-hot term sits behind a
+// wave-wide test of whether any of the wave's tokens has its target among the
+// wave's rows: compared in every element it also spilled 243 scalar registers of
+// comparison masks (dlogits 2.15 -> 2.06 ms per 2048 rows x 4096 x 151936).
+template <typename E, class S>
 __global__ __launch_bounds__(kGemmThreads, 1) void dlogits_kernel(DlArgs p) {
   GEMM_RING
+  constexpr int MI = S::MI, NI = S::NI;
   const int total = p.n_ttiles * p.n_vtiles;
   int vt, tt;
   grouped_tile(xcd_logical(blockIdx.x, total), p.n_vtiles, p.n_ttiles, vt, tt);
-  const int v0 = vt * TM, n0 = tt * TN;
-  f32x16 acc[4][NI];
-  gemm_tile<E, false, false>(acc, p.w + (int64_t)v0 * p.ldw, p.ldw, min(TM, p.vocab - v0),
-                          p.h + (int64_t)n0 * p.ldh, p.ldh, min(TN, p.rows - n0), p.dim, s0, s1, s2, s3);
+  const int v0 = vt * TM, n0 = tt * S::BN;
+  f32x16 acc[MI][NI];
+  gemm_tile<E, false, false, S>(acc, p.w + (int64_t)v0 * p.ldw, p.ldw, min(TM, p.vocab - v0),
+                          p.h + (int64_t)n0 * p.ldh, p.ldh, min(S::BN, p.rows - n0), p.dim, s0, s1, s2, s3);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave & 1, wn = wave >> 1;
+  const int wm = wave % S::WM, wn = wave / S::WM;
   // tokens 64 q .. 64 q + 63 of the tile are staged in ring stage q as [64][OPITCH]
   auto quarter = [&](int q) -> bf16* { return q == 0 ? s0 : q == 1 ? s1 : q == 2 ? s2 : s3; };
   // dl = -p (g_lp + g_H (log p + H)) + g_lp [v = t], with log2 p = l log2 e - lse log2 e as one
   // FMA and the bracket as one FMA in log2 p: A = g_H ln 2, B = g_lp + g_H H per token.  Tiles
   // inside the vocabulary and the row range (all but the last of each) skip the bounds tests.
+  auto column = [&](int ni, auto full_c, auto hot_c, float lse2, float coef_a, float coef_b, float glp, int hot,
+                    bool in_rows) __attribute__((always_inline)) {
+    constexpr bool FULL = decltype(full_c)::value, HOT = decltype(hot_c)::value;
+    const int col = b_row<S>(ni, lane, wn);  // token within the tile
+    bf16* out = quarter(col >> 6) + (col & 63) * OPITCH;
+#pragma unroll
+    for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+      for (int i4 = 0; i4 < 4; ++i4) {
+        float d[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int i = 4 * i4 + j;
+          const float logp2 = fmaf(acc[mi][ni][i], kLog2e, -lse2);
+          d[j] = -fast_exp2(logp2) * fmaf(coef_a, logp2, coef_b);
+          if (HOT && a_row<S>(mi, i, lane, wm) == hot) d[j] += glp;
+          if (!FULL && !(v0 + a_row<S>(mi, i, lane, wm) < p.vocab && in_rows)) d[j] = 0.f;
+        }
+        // vocab rows a_row(mi, 4 i4 .. 4 i4 + 3) are consecutive: one 8-byte write
+        *reinterpret_cast<u32x2*>(out + a_row<S>(mi, 4 * i4, lane, wm)) =
+            u32x2{pack2<E>(d[0], d[1]), pack2<E>(d[2], d[3])};
+      }
+  };
   auto epilogue = [&](auto full_c) __attribute__((always_inline)) {
     constexpr bool FULL = decltype(full_c)::value;
 #pragma unroll
     for (int ni = 0; ni < NI; ++ni) {
-      const int col = b_row(ni, lane, wn);  // token within the tile
-      bf16* out = quarter(col >> 6) + (col & 63) * OPITCH;
-      const int n = n0 + col;
+      const int n = n0 + b_row<S>(ni, lane, wn);
       float lse2 = 0.f, coef_a = 0.f, coef_b = 0.f, glp = 0.f;
-      int t = -1;
-      if (FULL || n < p.rows) {
+      int hot = -1;  // the token's target as a row of the tile (out-of-range targets match none)
+      const bool in_rows = FULL || n < p.rows;
+      if (in_rows) {
         lse2 = p.lse[n] * kLog2e;
         glp = p.g_lp[n];
         coef_b = glp;
@@ -295,41 +338,23 @@ __global__ __launch_bounds__(kGemmThreads, 1) void dlogits_kernel(DlArgs p) {
           coef_a = gent * kLn2;
           coef_b = fmaf(gent, p.ent[n], glp);
         }
-        const int64_t tt = p.target[n];
-        t = (tt >= 0 && tt < p.vocab) ? (int)tt : -1;  // out-of-range targets match no row
+        const int64_t t = p.target[n];
+        if (t >= v0 && t < min(v0 + TM, p.vocab)) hot = (int)(t - v0);
       }
-#pragma unroll
-      for (int mi = 0; mi < 4; ++mi)
-#pragma unroll
-        for (int i4 = 0; i4 < 4; ++i4) {
-          uint32_t packed[2];
-#pragma unroll
-          for (int j = 0; j < 4; j += 2) {
-            float d2[2];
-#pragma unroll
-            for (int jj = 0; jj < 2; ++jj) {
-              const int i = 4 * i4 + j + jj;
-              const int v = v0 + a_row(mi, i, lane, wm);
-              const float logp2 = fmaf(acc[mi][ni][i], kLog2e, -lse2);
-              float d = -fast_exp2(logp2) * fmaf(coef_a, logp2, coef_b);
-              if (v == t) d += glp;
-              if (!FULL && !(v < p.vocab && n < p.rows)) d = 0.f;
-              d2[jj] = d;
-            }
-            packed[j >> 1] = pack2<E>(d2[0], d2[1]);
-          }
-          // vocab rows a_row(mi, 4 i4 .. 4 i4 + 3) are consecutive: one 8-byte write
-          *reinterpret_cast<u32x2*>(out + a_row(mi, 4 * i4, lane, wm)) = u32x2{packed[0], packed[1]};
-        }
+      const int mine = hot - 32 * MI * wm;
+      if (__builtin_amdgcn_ballot_w64(mine >= 0 && mine < 32 * MI) != 0)
+        column(ni, full_c, std::true_type{}, lse2, coef_a, coef_b, glp, hot, in_rows);
+      else
+        column(ni, full_c, std::false_type{}, lse2, coef_a, coef_b, glp, hot, in_rows);
     }
   };
-  if (v0 + TM <= p.vocab && n0 + TN <= p.rows) epilogue(std::true_type{});
+  if (v0 + TM <= p.vocab && n0 + S::BN <= p.rows) epilogue(std::true_type{});
   else epilogue(std::false_type{});
   __syncthreads();
-  // coalesced store of the [TN tokens][TM vocab] tile
+  // coalesced store of the [BN tokens][TM vocab] tile
   const int vmax = min(TM, p.vocab_pad - v0);
 #pragma unroll 4
-  for (int it = 0; it < (TN * TM / 8) / kGemmThreads; ++it) {
+  for (int it = 0; it < (S::BN * TM / 8) / kGemmThreads; ++it) {
     const int c = it * kGemmThreads + tid;
     const int row = c / (TM / 8), chunk = (c % (TM / 8)) * 8;
     const int n = n0 + row;
@@ -358,31 +383,32 @@ struct DhArgs {
   float* part;      // [ksplit][rows][dim] when ksplit > 1
 };
 
-template <typename E>
+template <typename E, class S>
 __global__ __launch_bounds__(kGemmThreads, 1) void grad_hidden_kernel(DhArgs p) {
   GEMM_RING
+  constexpr int MI = S::MI, NI = S::NI;
   const int tiles = p.n_ttiles * p.n_dtiles;
-  const int total = tiles * p.ksplit;
-  const int id = xcd_logical(blockIdx.x, total);
+  const int id = xcd_logical(blockIdx.x, tiles * p.ksplit);
   const int ks = id / tiles;  // vocabulary range: tiles of one range run together
   int dt, tt;
   grouped_tile(id - ks * tiles, p.n_dtiles, p.n_ttiles, dt, tt);
-  const int d0 = dt * TM, n0 = tt * TN;
+  const int d0 = dt * TM, n0 = tt * S::BN;
   const int kb = ks * p.kper, ke = min(p.vocab, kb + p.kper);
-  f32x16 acc[4][NI];
-  gemm_tile<E, true, false>(acc, p.w + (int64_t)kb * p.ldw + d0, p.ldw, p.dim - d0, p.dl + (int64_t)n0 * p.ldl + kb,
-                         p.ldl, min(TN, p.rows - n0), ke - kb, s0, s1, s2, s3);
+  f32x16 acc[MI][NI];
+  gemm_tile<E, true, false, S>(acc, p.w + (int64_t)kb * p.ldw + d0, p.ldw, p.dim - d0,
+                               p.dl + (int64_t)n0 * p.ldl + kb, p.ldl, min(S::BN, p.rows - n0), ke - kb, s0, s1, s2,
+                               s3);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int wm = wave & 1, wn = wave >> 1;
+  const int wm = wave % S::WM, wn = wave / S::WM;
 #pragma unroll
   for (int ni = 0; ni < NI; ++ni) {
-    const int n = n0 + b_row(ni, lane, wn);
+    const int n = n0 + b_row<S>(ni, lane, wn);
     if (n >= p.rows) continue;
 #pragma unroll
-    for (int mi = 0; mi < 4; ++mi)
+    for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
       for (int i4 = 0; i4 < 4; ++i4) {
-        const int d = d0 + a_row(mi, 4 * i4, lane, wm);
+        const int d = d0 + a_row<S>(mi, 4 * i4, lane, wm);
         const float a[4] = {acc[mi][ni][4 * i4], acc[mi][ni][4 * i4 + 1], acc[mi][ni][4 * i4 + 2],
                             acc[mi][ni][4 * i4 + 3]};
         if (p.ksplit > 1) {
@@ -499,6 +525,14 @@ inline void grad_hidden_split(int64_t rows, int64_t dim, int64_t vocab, int& ksp
   kper = (int)per;
 }
 
+// launch kernel<element, tile shape> by a DType code and token_tile's width
+#define TS_LAUNCH_TOKENS(dtype, width, kernel, ...)                               \
+  do {                                                                            \
+    if ((width) == 64) TS_LAUNCH_E_T(dtype, kernel, Narrow<1>, __VA_ARGS__);      \
+    else if ((width) == 128) TS_LAUNCH_E_T(dtype, kernel, Narrow<2>, __VA_ARGS__); \
+    else TS_LAUNCH_E_T(dtype, kernel, Full, __VA_ARGS__);                         \
+  } while (0)
+
 bool ok16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
 }  // namespace lp
@@ -549,7 +583,7 @@ int ts_logprob_fwd(const void* hidden, int64_t ld_hidden, const void* weight, in
   a.part_e = ws + 2 * (int64_t)a.n_vtiles * rows;
   TS_CHECK_ARG((int64_t)a.n_ttiles * a.n_vtiles < (1ll << 31), "ts_logprob_fwd: grid too large");
   hipStream_t s = (hipStream_t)stream;
-  { ts::TimedLaunch timed_("logprob.fwd_stats_kernel", s); TS_LAUNCH_E(dtype, fwd_stats_kernel, dim3((unsigned)(a.n_ttiles * a.n_vtiles)), dim3(kGemmThreads),
+  { ts::TimedLaunch timed_("logprob.fwd_stats_kernel", s); TS_LAUNCH_TOKENS(dtype, token_tile(rows, false), fwd_stats_kernel, dim3((unsigned)(a.n_ttiles * a.n_vtiles)), dim3(kGemmThreads),
                      0, s, a); }
   int st = ts::check_launch("ts_logprob_fwd (tiles)");
   if (st != TS_OK) return st;
@@ -599,7 +633,7 @@ int ts_logprob_dlogits(const void* hidden, int64_t ld_hidden, const void* weight
   a.dl = (ts::bf16*)dlogits;
   a.ldl = ld_dlogits;
   TS_CHECK_ARG(a.vocab_pad <= ld_dlogits, "ts_logprob_dlogits: ld_dlogits below padded vocab");
-  { ts::TimedLaunch timed_("logprob.dlogits_kernel", (hipStream_t)stream); TS_LAUNCH_E(dtype, dlogits_kernel, dim3((unsigned)(a.n_ttiles * a.n_vtiles)), dim3(kGemmThreads),
+  { ts::TimedLaunch timed_("logprob.dlogits_kernel", (hipStream_t)stream); TS_LAUNCH_TOKENS(dtype, token_tile(rows, false), dlogits_kernel, dim3((unsigned)(a.n_ttiles * a.n_vtiles)), dim3(kGemmThreads),
                      0, (hipStream_t)stream, a); }
   return ts::check_launch("ts_logprob_dlogits");
 }
@@ -652,8 +686,10 @@ int grad_hidden_launch(const void* dlogits, int64_t ld_dlogits, const void* weig
   hipStream_t s = (hipStream_t)stream;
   {
     ts::TimedLaunch timed_(label, s);
-    TS_LAUNCH_E(dtype, grad_hidden_kernel, dim3((unsigned)(a.n_ttiles * a.n_dtiles * a.ksplit)), dim3(kGemmThreads),
-                       0, s, a);
+    const int width = token_tile(rows, true);
+    const dim3 grid((unsigned)(a.n_ttiles * a.n_dtiles * a.ksplit));
+    if (width == 192) TS_LAUNCH_E_T(dtype, grad_hidden_kernel, Narrow<3>, grid, dim3(kGemmThreads), 0, s, a);
+    else TS_LAUNCH_TOKENS(dtype, width, grad_hidden_kernel, grid, dim3(kGemmThreads), 0, s, a);
   }
   int st = ts::check_launch("ts_logprob_grad_hidden");
   if (st != TS_OK || a.ksplit == 1) return st;
