@@ -221,6 +221,14 @@ template <> __device__ __forceinline__ void store4<float>(float* p, const float 
   *reinterpret_cast<f32x4*>(p) = f32x4{o[0], o[1], o[2], o[3]};
 }
 
+// store4 with the non-temporal hint
+template <typename T> __device__ __forceinline__ void store4_once(T* p, const float (&o)[4]) {
+  if constexpr (sizeof(T) == 2)
+    __builtin_nontemporal_store((u32x2{pack2<T>(o[0], o[1]), pack2<T>(o[2], o[3])}), reinterpret_cast<u32x2*>(p));
+  else
+    __builtin_nontemporal_store((f32x4{o[0], o[1], o[2], o[3]}), reinterpret_cast<f32x4*>(p));
+}
+
 // y = w * T(x * r): the product rounded to fp32, then to T, then w * that
 // rounded to T, as the module's operations.  The fp32 product is hidden from
 // the optimiser: for fp16 it otherwise folds T(x * r) into one
@@ -239,7 +247,13 @@ template <typename T> __device__ __forceinline__ float primal(float w, float x, 
 //  VEC: the lane's loads are 4-element vectors x + k bw (width % 4 == 0); NV
 //       bounds their number.  Otherwise (width < 128) the lane sums elements
 //       sub and sub + bw, the only ones its loop reaches.
-template <typename T, bool VEC, int NV>
+// Bound by HBM.  The weight's vectors are loaded beside the row's, so that the
+// stores wait for the reduction alone, and an output that no cache can hold
+// (STREAM, kStreamBytes) is stored without displacing the lines the loads
+// bring in.  bf16 from cold caches, us: 16384 x 4096 62 plain, 55.6 with the weight
+// loads, 51.6 with the stores too (5.2 TB/s); 8192 x 5120 43.5, 40.5 with the weight
+// loads, 33.5 with 20 vectors instead of 32.
+template <typename T, bool VEC, int NV, bool STREAM>
 __global__ __launch_bounds__(kThreads) void rmsnorm_fwd_lanes(
     const T* __restrict__ x, const T* __restrict__ w, T* __restrict__ y,
     float* __restrict__ rstd, int64_t rows, int width, int bw, float factor, float eps) {
@@ -256,6 +270,9 @@ __global__ __launch_bounds__(kThreads) void rmsnorm_fwd_lanes(
     Raw4<T> v[NV];
 #pragma unroll
     for (int k = 0; k < NV; ++k) v[k] = load4<T>(xr + min(sub + k * bw, nvec - 1) * 4);
+    Raw4<T> wr[NV];
+#pragma unroll
+    for (int k = 0; k < NV; ++k) wr[k] = load4<T>(w + min(sub + k * bw, nvec - 1) * 4);
     float acc[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
@@ -278,10 +295,11 @@ __global__ __launch_bounds__(kThreads) void rmsnorm_fwd_lanes(
       if (vi < nvec) {
         float f[4], wv[4], o[4];
         unpack4<T>(v[k], f);
-        unpack4<T>(load4<T>(w + vi * 4), wv);
+        unpack4<T>(wr[k], wv);
 #pragma unroll
         for (int i = 0; i < 4; ++i) o[i] = primal<T>(wv[i], f[i], r);
-        store4<T>(yr + vi * 4, o);
+        if constexpr (STREAM) store4_once<T>(yr + vi * 4, o);
+        else store4<T>(yr + vi * 4, o);
       }
     }
   } else {
@@ -394,7 +412,7 @@ __global__ __launch_bounds__(kWave) void rmsnorm_fwd_rowwave(
 template <typename T, int NV, bool FULL> struct BwdShape {
   // prefetch where the compiled kernel then still fits 256 VGPRs unspilled
   static constexpr bool kPrefetch = NV <= 4 || (sizeof(T) == 2 && NV == 8 && FULL);
-  static constexpr int kWaves = NV <= 8 ? 8 : 4;
+  static constexpr int kWaves = NV <= 12 ? 8 : 4;
   static constexpr int kThreads = kWaves * kWave;
 };
 
@@ -622,8 +640,14 @@ Geometry pick(int64_t width, int dtype) {
   int lpr = 64;
   while (lpr > 4 && lpr > nvec) lpr >>= 1;
   const int64_t nv = (nvec + lpr - 1) / lpr;
+  // vectors per lane the kernel is built for: powers of two and, between 8 and
+  // 16, 10 (widths up to 5120) and 12 (6144), which keep eight waves a block where
+  // 16 has registers for four (8192 rows: 5120 73 -> 54 us, 6144 83 -> 64); 12 that
+  // do not fill the row spill (5632: 87 us against 78 through 16)
   int nvp = 1;
   while (nvp < nv) nvp <<= 1;
+  if (nvp == 16 && nv <= 10) nvp = 10;
+  if (nvp == 16 && nvec == 12 * kWave) nvp = 12;
   if (nvp > 16) return g;  // wider than 8192: scalar path
   (void)dtype;
   g.lpr = lpr;
@@ -632,11 +656,15 @@ Geometry pick(int64_t width, int dtype) {
 }
 
 int64_t bwd_parts(int64_t rows, int64_t width) {
-  // at least 32 rows per block, so the partial rows (written and read once)
-  // stay within 8/(6*32) of the kernel's traffic; at most 256 blocks for rows
+  // at least one pass of the block's eight waves per block (8 rows, or 8 64 / LPR
+  // narrow ones up to 32): the partial rows, written and read once, are then at most a
+  // sixth of the kernel's traffic, and short launches fill the CUs (2048 x 4096:
+  // 64 blocks of 32 rows 32 us, 256 of 8 20; 64 x 4096 26 -> 15); at most 256 blocks for rows
   // of 2048 and more elements -- one 8-wave block per CU is enough bytes in
   // flight there -- and up to 1024 for narrower rows, whose blocks carry less
-  int64_t parts = (rows + 31) / 32;
+  const Geometry g = pick(width, 0);
+  const int64_t pass = g.lpr > 16 ? 8 * (kWave / g.lpr) : 32;
+  int64_t parts = (rows + pass - 1) / pass;
   const int64_t max_parts = width >= 2048 ? 256 : 1024;
   if (parts > max_parts) parts = max_parts;
   if (parts < 1) parts = 1;
@@ -655,6 +683,12 @@ int stream_cus(hipStream_t s) {
   return n;
 }
 
+// input and output together fill the Infinity Cache's 256 MB.  Below that the next
+// kernel finds part of the output there, and so does this one its own lines: 8192 x
+// 5120 (84 MB) 33.5 us stored plainly and 35.7 streamed, 8192 x 6144 (101 MB) 41.6
+// and 43.4; 16384 x 4096 (134 MB) 55.6 and 51.7, 32768 x 4096 118 -> 102.
+constexpr int64_t kStreamBytes = 128ll << 20;
+
 template <typename T>
 int launch_fwd(const void* x, const void* w, void* y, float* rstd, int64_t rows, int width,
                float eps, hipStream_t s) {
@@ -671,18 +705,23 @@ int launch_fwd(const void* x, const void* w, void* y, float* rstd, int64_t rows,
     const dim3 grid((unsigned)((rows + rows_per_block - 1) / rows_per_block));
     ts::TimedLaunch timed_("rmsnorm.rmsnorm_fwd_lanes", s);
     if (!c.vec) {
-      hipLaunchKernelGGL((rmsnorm_fwd_lanes<T, false, 1>), grid, dim3(kThreads), 0, s, (const T*)x,
+      hipLaunchKernelGGL((rmsnorm_fwd_lanes<T, false, 1, false>), grid, dim3(kThreads), 0, s, (const T*)x,
                          (const T*)w, (T*)y, rstd, rows, width, c.bw, factor, eps);
       return check_launch("ts_rmsnorm_fwd");
     }
     const int loads = (width / 4 + c.bw - 1) / c.bw;
-#define TS_FWD(NV)                                                                             \
-  if (loads <= NV) {                                                                           \
-    hipLaunchKernelGGL((rmsnorm_fwd_lanes<T, true, NV>), grid, dim3(kThreads), 0, s,           \
-                       (const T*)x, (const T*)w, (T*)y, rstd, rows, width, c.bw, factor, eps); \
-    return check_launch("ts_rmsnorm_fwd");                                                     \
+    const bool stream = rows * (int64_t)width * (int64_t)sizeof(T) >= kStreamBytes;
+#define TS_FWD(NV)                                                                               \
+  if (loads <= NV) {                                                                             \
+    if (stream)                                                                                  \
+      hipLaunchKernelGGL((rmsnorm_fwd_lanes<T, true, NV, true>), grid, dim3(kThreads), 0, s,     \
+                         (const T*)x, (const T*)w, (T*)y, rstd, rows, width, c.bw, factor, eps); \
+    else                                                                                         \
+      hipLaunchKernelGGL((rmsnorm_fwd_lanes<T, true, NV, false>), grid, dim3(kThreads), 0, s,    \
+                         (const T*)x, (const T*)w, (T*)y, rstd, rows, width, c.bw, factor, eps); \
+    return check_launch("ts_rmsnorm_fwd");                                                       \
   }
-    TS_FWD(1) TS_FWD(2) TS_FWD(4) TS_FWD(8) TS_FWD(16) TS_FWD(32)
+    TS_FWD(1) TS_FWD(2) TS_FWD(4) TS_FWD(8) TS_FWD(12) TS_FWD(16) TS_FWD(20) TS_FWD(24) TS_FWD(32)
 #undef TS_FWD
   }
   if (rows > 0x7fffffff) {
@@ -733,7 +772,7 @@ int launch_bwd(const void* dy, const void* x, const void* w, const float* rstd, 
     launched = true;                                                                         \
   }
     TS_BWD(4, 1) TS_BWD(8, 1) TS_BWD(16, 1) TS_BWD(32, 1) TS_BWD(64, 1)
-    TS_BWD(4, 2) TS_BWD(8, 2) TS_BWD(16, 2) TS_BWD(32, 2) TS_BWD(64, 2) TS_BWD(64, 4) TS_BWD(64, 8) TS_BWD(64, 16)
+    TS_BWD(4, 2) TS_BWD(8, 2) TS_BWD(16, 2) TS_BWD(32, 2) TS_BWD(64, 2) TS_BWD(64, 4) TS_BWD(64, 8) TS_BWD(64, 10) TS_BWD(64, 12) TS_BWD(64, 16)
 #undef TS_BWD
     if (!launched) {
       set_error("ts_rmsnorm_bwd: no kernel for width %d", width);
