@@ -179,7 +179,7 @@ typedef struct ts_attn_problem {
   int32_t head_dim; /* 32, 64, 96, 128, 192 or 256 */
   float scale;
   int32_t q_block;  /* rows per q_work item: ts_attn_q_block(hq / hkv) */
-  int32_t kv_block; /* keys per kv_work item: ts_attn_kv_block(hq / hkv, head_dim); head dims 128, 256: 48 or 64 */
+  int32_t kv_block; /* keys per kv_work item: 48 or 64 (ts_attn_kv_block) */
   int64_t q_rows;   /* rows of Q/O/dO/dQ */
   /* Launch order.  The work lists are sorted longest first; their first
    * n_q_long / n_kv_long items run first, item by item across all heads (so

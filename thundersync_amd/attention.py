@@ -39,9 +39,8 @@ Reference entry points mirrored here (same argument meaning):
 Element types: bf16 and fp16 (Q, K, V of one call share one).  Head dims D:
 any from 1 to 256, as the reference's flash paths take
 (engine/streaming.py:532-548, :915-930).  The kernels are built for 32, 64,
-96, 128, 192 and 256 (128 and 256 run the DMA-staged kernels, the others the
-register-staged ones); any other D runs the next larger of them over Q, K
-and V zero-padded to it (see :func:`kernel_head_dim`).  At head dims 128 and
+96, 128, 192 and 256; any other D runs the next larger of them over Q, K and V
+zero-padded to it (see :func:`kernel_head_dim`).  At head dims 128 and
 256 the backward stores dS once in a workspace and forms dQ = dS K from it
 (see ``DS_MAX_BYTES``).  There is no host path: CPU tensors, other dtypes or
 head dims above 256 raise.
@@ -362,9 +361,13 @@ class AttnLayout:
     def call_kv_block(self, device, head_dim: int) -> int:
         """Keys per dK/dV work item of this package's own calls: kv_block_for's,
         except that at head dim 128 every GQA group takes either kernel, by the
-        steps of an item and the items of the launch (DEALT_STEPS)."""
-        if head_dim != HEAD_DIM:
+        steps of an item and the items of the launch (DEALT_STEPS), and at the
+        head dims that only the key-split kernel takes, whose four waves hold 16
+        keys each, every group has 64."""
+        if head_dim == 256:
             return self.kv_block_for(device, head_dim)
+        if head_dim != HEAD_DIM:
+            return 64
         d = self._description()
         steps = (self.hq // self.hkv) * d["rows_per_key"] / 32
         items = d["items48"] * self.hkv

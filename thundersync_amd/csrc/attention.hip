@@ -1,14 +1,14 @@
-// Forest / packed bottom-right-causal GQA attention for gfx950 (bf16, D = 128).
+// Forest / packed bottom-right-causal GQA attention for gfx950 (bf16 and fp16; the kernels in attention_*.hip).
 //
 // One description (segments of query rows, runs of keys read in place, see
 // include/thundersync_hip.h) drives three kernels:
 //
 //   fwd      query-stationary: a work-group owns a block of query rows of one
 //            segment for GC query heads of one GQA group, streams the
-//            segment's key runs through LDS 64 keys at a time (K and V tiles
+//            segment's key runs through LDS 32 or 64 keys at a time (K and V tiles
 //            shared by the GC heads), and keeps an online softmax per row.
 //   dq       query-stationary like fwd, recomputing P from the saved LSE.
-//   dkdv     key-stationary: a work-group owns 64 keys of one run and one KV
+//   dkdv     key-stationary: a work-group owns 48 or 64 keys of one run and one KV
 //            head, visits every segment that reads the run, and accumulates
 //            dK/dV for all query heads of the group in registers -- no
 //            atomics, fixed order, so the gradients are deterministic.
@@ -20,11 +20,12 @@
 //           softmax statistics of a query live in the four lanes that share
 //           (lane & 15) and P^T is already in the B-operand layout of
 //           O^T += V^T P^T.  V^T (and K^T for dQ) are fed from LDS rows
-//           through an 8x8 register transpose.
+//           by transposed LDS reads.
 //   dkdv    S = Q K^T, dP = dO V^T (A from LDS rows, B = K^T/V^T held in
 //           registers); dV^T += dO^T P and dK^T += Q^T dS with dO^T / Q^T
-//           from LDS rows through the register transpose.
+//           from LDS rows by transposed reads.
 // Both sides of every contraction use the same slot permutation of the
+// contracted index, so it cancels.
 #include <vector>
 
 #include "attention_impl.h"
@@ -53,10 +54,9 @@ int validate(const ts_attn_problem* p, const char* what) {
   const int gc = heads_per_block(p->hq / p->hkv);
   TS_CHECK_ARG(p->q_block == q_block_rows(p->hq / p->hkv), "%s: q_block %d, expected %d for group %d",
                what, p->q_block, q_block_rows(p->hq / p->hkv), p->hq / p->hkv);
-  // the DMA-staged kernels (head dims 128 and 256) take items of either size
-  TS_CHECK_ARG(p->kv_block == kv_block_keys(p->hq / p->hkv, p->head_dim) ||
-                   (ds_route(p->head_dim, p->hq / p->hkv) && (p->kv_block == 48 || p->kv_block == 64)),
-               "%s: kv_block %d, expected %d", what, p->kv_block, kv_block_keys(p->hq / p->hkv, p->head_dim));
+  // items of either size run at every head dim
+  TS_CHECK_ARG(p->kv_block == 48 || p->kv_block == 64, "%s: kv_block %d, expected 48 or 64", what,
+               p->kv_block);
   TS_CHECK_ARG(p->n_q_work >= 0 && p->n_kv_work >= 0 && p->n_segs >= 0 && p->n_runs >= 0,
                "%s: negative table size", what);
   TS_CHECK_ARG(p->n_q_long >= 0 && p->n_q_long <= p->n_q_work && p->n_kv_long >= 0 &&

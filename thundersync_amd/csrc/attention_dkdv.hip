@@ -5,161 +5,17 @@ namespace ts {
 namespace attn {
 
 // ---------------------------------------------------------------------------
-// backward dK / dV (key-stationary)
-// ---------------------------------------------------------------------------
-// Register-staged dK/dV for any supported head dim HD and GQA groups that are
-// not a multiple of 4 (and, at head dims other than 128, those that are): a
-// work-group owns P.kv_block keys (48 or 64) of one run and one KV head, wave
-// w keys 16 w .. 16 w + 15 (a wave past the block only helps stage the
-// tiles), and loops over every query head of the group and every visible
-// 32-row block; Q and dO rows pass through registers into padded LDS rows,
-// dO^T and Q^T come from ds_read_b64_tr_b16 (tr_frag).
-template <typename E, int HD>
-__global__ __launch_bounds__(kThreads, HD > 128 ? 1 : 2) void dkdv_kernel(ts_attn_problem P, ts_attn_rows Q,
-                                                           ts_attn_rows dO, const float* __restrict__ rowstats,
-                                                           int64_t lse_ld) {
-  constexpr int NMB = HD / 16;  // 16-column blocks of dK / dV
-  __shared__ __attribute__((aligned(16))) bf16 sq[32 * pitch_of<HD>()];
-  __shared__ __attribute__((aligned(16))) bf16 sd[32 * pitch_of<HD>()];
-  __shared__ float s_lse2[32];
-  __shared__ float s_dlt[32];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  int hk;
-  const int item = task_of(P.n_kv_work, P.n_kv_long, hk);
-  const int run_id = uniform_table(P.kv_work)[2 * item];
-  const int k0 = uniform_table(P.kv_work)[2 * item + 1];
-  const int group = P.hq / P.hkv;
-  const ts_attn_run run = load_uniform(P.runs, run_id);
-  const int wk0 = k0 + 16 * wave;                 // first key (run-local) of this wave
-  const int mykey = wk0 + (lane & 15);            // key column this lane holds
-  const bool in_block = 16 * wave < P.kv_block;   // the wave's keys belong to this work item
-  const bool wave_has_keys = in_block && wk0 < run.len;
-  const bool key_valid = in_block && mykey < run.len;
-  const float c = P.scale * kLog2e;
-
-  // K^T / V^T B operands: key (lane & 15), d = 32 ks + 8 (lane >> 4) .. +7
-  bf16x8 kreg[HD / 32], vreg[HD / 32];
-  {
-    const bf16* kp = (const bf16*)run.k + (int64_t)mykey * run.k_row_stride + (int64_t)hk * run.k_head_stride;
-    const bf16* vp = (const bf16*)run.v + (int64_t)mykey * run.v_row_stride + (int64_t)hk * run.v_head_stride;
-#pragma unroll
-    for (int ks = 0; ks < HD / 32; ++ks) {
-      u32x4 a = u32x4{0u, 0u, 0u, 0u}, b = u32x4{0u, 0u, 0u, 0u};
-      if (key_valid) {
-        a = ld16(kp + 32 * ks + 8 * (lane >> 4));
-        b = ld16(vp + 32 * ks + 8 * (lane >> 4));
-      }
-      kreg[ks] = as_bf16x8(a);
-      vreg[ks] = as_bf16x8(b);
-    }
-  }
-  f32x4 dk[NMB], dv[NMB];
-#pragma unroll
-  for (int mb = 0; mb < NMB; ++mb) {
-    dk[mb] = f32x4{0.f, 0.f, 0.f, 0.f};
-    dv[mb] = f32x4{0.f, 0.f, 0.f, 0.f};
-  }
-
-  for (int vi = 0; vi < run.nvisit; ++vi) {
-    const ts_attn_ref ref = load_uniform(P.run_visits, run.visit0 + vi);
-    const ts_attn_segment seg = load_uniform(P.segs, ref.index);
-    const int T = seg.q_len;
-    const int off = seg.kv_len - seg.q_len;
-    // row r sees key k iff kpos + k <= off + r
-    int r_start = ref.kpos + k0 - off;
-    if (r_start < 0) r_start = 0;
-    r_start &= ~31;
-    for (int r0 = r_start; r0 < T; r0 += 32) {
-      const int nrows = min(32, T - r0);
-      // the wave's keys are all invisible to this block when its first key
-      // is beyond the block's last row
-      const bool wave_active = wave_has_keys && (ref.kpos + wk0 <= off + r0 + nrows - 1);
-      for (int g = 0; g < group; ++g) {
-        const int h = hk * group + g;
-        __syncthreads();
-        const int64_t row0 = seg.q_row0 + r0;
-        rows32_to_lds<HD>(sq, (const bf16*)Q.ptr + row0 * Q.row_stride + (int64_t)h * Q.head_stride,
-                          Q.row_stride, nrows, tid);
-        rows32_to_lds<HD>(sd, (const bf16*)dO.ptr + row0 * dO.row_stride + (int64_t)h * dO.head_stride,
-                          dO.row_stride, nrows, tid);
-        if (tid < 32) {
-          float l2 = __builtin_huge_valf(), dl = 0.f;
-          if (tid < nrows) {
-            const int64_t at = 2 * ((int64_t)h * lse_ld + row0 + tid);
-            l2 = rowstats[at];
-            dl = rowstats[at + 1];
-          }
-          s_lse2[tid] = l2;
-          s_dlt[tid] = dl;
-        }
-        __syncthreads();
-        if (!wave_active) continue;
-
-        // S = Q K^T and dP = dO V^T: [qb] lane holds rows 16 qb + 4 (lane >> 4) + i, key (lane & 15)
-        f32x4 s[2], dp[2];
-#pragma unroll
-        for (int qb = 0; qb < 2; ++qb) {
-          s[qb] = f32x4{0.f, 0.f, 0.f, 0.f};
-          dp[qb] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int ks = 0; ks < HD / 32; ++ks) {
-            const int r = 16 * qb + (lane & 15);
-            const bf16x8 aq = as_bf16x8(ld16(sq + r * pitch_of<HD>() + 32 * ks + 8 * (lane >> 4)));
-            const bf16x8 ad = as_bf16x8(ld16(sd + r * pitch_of<HD>() + 32 * ks + 8 * (lane >> 4)));
-            s[qb] = mma16<E>(aq, kreg[ks], s[qb]);
-            dp[qb] = mma16<E>(ad, vreg[ks], dp[qb]);
-          }
-        }
-        float pv[8], dsv[8];
-#pragma unroll
-        for (int qb = 0; qb < 2; ++qb)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int rl = 16 * qb + 4 * (lane >> 4) + i;
-            float p = fast_exp2(s[qb][i] * c - s_lse2[rl]);
-            if (rl >= nrows || !key_valid || ref.kpos + mykey > off + r0 + rl) p = 0.f;
-            pv[4 * qb + i] = p;
-            dsv[4 * qb + i] = p * (dp[qb][i] - s_dlt[rl]);
-          }
-        const bf16x8 pk = pack8<E>(pv);
-        const bf16x8 dsk = pack8<E>(dsv);
-#pragma unroll
-        for (int mb = 0; mb < NMB; ++mb) {
-          dv[mb] = mma16<E>(tr_frag<HD>(sd, 0, mb, lane), pk, dv[mb]);
-          dk[mb] = mma16<E>(tr_frag<HD>(sq, 0, mb, lane), dsk, dk[mb]);
-        }
-      }
-    }
-  }
-  if (!key_valid) return;
-  // dk[mb] / dv[mb] lane (g4, j16) holds d = 16 mb + 4 g4 + i of key mykey: 8-byte stores
-  if (run.dk) {
-    bf16* p = (bf16*)run.dk + (int64_t)mykey * run.dk_row_stride + (int64_t)hk * run.dk_head_stride + 4 * (lane >> 4);
-#pragma unroll
-    for (int mb = 0; mb < NMB; ++mb) {
-      const f32x4 v = dk[mb] * P.scale;
-      *reinterpret_cast<u32x2*>(p + 16 * mb) = u32x2{pack2<E>(v[0], v[1]), pack2<E>(v[2], v[3])};
-    }
-  }
-  if (run.dv) {
-    bf16* p = (bf16*)run.dv + (int64_t)mykey * run.dv_row_stride + (int64_t)hk * run.dv_head_stride + 4 * (lane >> 4);
-#pragma unroll
-    for (int mb = 0; mb < NMB; ++mb)
-      *reinterpret_cast<u32x2*>(p + 16 * mb) = u32x2{pack2<E>(dv[mb][0], dv[mb][1]), pack2<E>(dv[mb][2], dv[mb][3])};
-  }
-}
-
-// ---------------------------------------------------------------------------
 // backward dK / dV with the keys split over the waves (head dim 128: 64-key
 // work items, for items of few steps; head dim 256: 48-key work items, which
-// launches with few 64-key items take)
+// launches with few 64-key items take; head dims 32, 64, 96 and 192: every
+// launch)
 //
 // A work-group owns P.kv_block keys (48 or 64) of one run and one KV head;
 // wave w owns keys 16 w .. 16 w + 15, their K^T and V^T in registers, and all
 // waves walk the same sequence of steps -- every query head of the group,
 // then every visible 32-row block -- reading one double-buffered LDS stage:
 // the step's Q and dO rows (HD-element rows, 16-byte chunk c of row r at slot
-// c ^ tile_swizzle(r & 15)) and the rows' 32 (lse * log2 e, delta) pairs,
+// c ^ row_swizzle(r & 15)) and the rows' 32 (lse * log2 e, delta) pairs,
 // filled by buffer_load ... lds with each wave issuing its share of the
 // instructions, one work-group barrier per step.  The buffer resource of a
 // tile covers exactly its valid rows, so rows past a segment's end arrive as
@@ -169,25 +25,29 @@ __global__ __launch_bounds__(kThreads, HD > 128 ? 1 : 2) void dkdv_kernel(ts_att
 // (the lane layout of the one-wave-per-head kernel).  A wave past the work
 // item's keys (kv_block 48) only issues its DMA share; only steps that cross
 // the diagonal are masked.
+//
+// Every wave reads the whole step from LDS for 16 of its keys, which bounds the
+// steps (16 KB of LDS reads a wave for 16 MFMAs at head dim 64).  Against
+// staging each step through registers between two barriers, with 48-key items
+// at groups of 4 (8 sequences of 512 to 2048 rows, us): head dim 64 at 16/8 heads
+// 184 -> 131, at 32/8 712 -> 300, 96 at 16/8 310 -> 167, 192 at 24/4 1222 -> 512.
 // ---------------------------------------------------------------------------
 template <typename E, int HD, bool DS = false>
 __global__ __launch_bounds__(kThreads, 1) void dkdv_split_kernel(ts_attn_problem P, ts_attn_rows Q,
                                                                  ts_attn_rows dO,
                                                                  const float* __restrict__ rowstats,
                                                                  int64_t lse_ld, DsArgs S) {
-  static_assert(HD == 128 || HD == 256, "the swizzle needs 16 or 32 chunks per row");
   constexpr int CH = HD / 8;              // 16-byte chunks per row
   constexpr int NKS = HD / 32;            // k-steps of S / dP over the head dim
   constexpr int NMB = HD / 16;            // 16-column blocks of dK / dV
   constexpr int TILE = 32 * HD;           // elements of a 32-row tile
   constexpr int STAGE = 2 * TILE + 512;   // Q, dO, then 1 KB of statistics
-  constexpr int RPI = 64 / CH;            // rows one DMA instruction fills (4 or 2)
-  constexpr int NDMA = 32 / RPI;          // DMA instructions per tile (8 or 16)
-  constexpr int PER_WAVE = NDMA / 4;      // of them issued by each wave
+  constexpr int NDMA = 32 * CH / 64;      // DMA instructions per tile, 64 chunks each
+  constexpr int PER_WAVE = (NDMA + 3) / 4;  // of them issued by each wave (at most)
   // dO^T / Q^T blocks whose transposed reads are issued before the softmax
   // (head dim 256: eight, 4.94 -> 4.83 ms on the branch shape), and the
   // read-ahead distance of the rest
-  constexpr int NPRE = HD == 256 ? 8 : 4;
+  constexpr int NPRE = HD == 256 ? 8 : NMB < 4 ? NMB : 4;
   __shared__ __attribute__((aligned(16))) bf16 s_b0[STAGE];
   __shared__ __attribute__((aligned(16))) bf16 s_b1[STAGE];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -210,16 +70,16 @@ __global__ __launch_bounds__(kThreads, 1) void dkdv_split_kernel(ts_attn_problem
   // the run is put past every row (2^24 rows), so the mask zeroes its P too
   const int mask_key = mykey + (DS && !key_valid ? (1 << 24) : 0);
 
-  int ro[4], to[8];
+  int ro[kRowOffsets<HD>], to[2 * kRowOffsets<HD>];
   swizzled_offsets<HD>(lane, ro, to);
-  // DMA instruction t fills rows RPI t .. RPI t + RPI - 1: lane l the row
-  // RPI t + l / CH, slot l % CH with logical chunk (l % CH) ^ tile_swizzle(row);
+  // DMA instruction t fills the tile's chunk slots 64 t .. 64 t + 63: lane l slot
+  // i = 64 t + l, of row i / CH, with logical chunk (i % CH) ^ row_swizzle(row);
   // this wave issues t = wave + 4 u.  Byte offsets of the lane's row and chunk.
   int qoff[PER_WAVE], doff[PER_WAVE];
 #pragma unroll
   for (int u = 0; u < PER_WAVE; ++u) {
-    const int row = RPI * (wave + 4 * u) + lane / CH;
-    const int chunk = (lane % CH) ^ tile_swizzle(row & 15);
+    const int slot = 64 * (wave + 4 * u) + lane, row = slot / CH;
+    const int chunk = (slot % CH) ^ row_swizzle<HD>(row & 15);
     qoff[u] = (int)((row * Q.row_stride + chunk * 8) * 2);
     doff[u] = (int)((row * dO.row_stride + chunk * 8) * 2);
   }
@@ -338,6 +198,7 @@ __global__ __launch_bounds__(kThreads, 1) void dkdv_split_kernel(ts_attn_problem
     const rsrc_t rd = make_rsrc(db, (uint32_t)(nrows * dO.row_stride * 2));
 #pragma unroll
     for (int u = 0; u < PER_WAVE; ++u) {
+      if (NDMA % 4 != 0 && wave + 4 * u >= NDMA) break;
       buffer_dma16(rq, buf + (wave + 4 * u) * 512, qoff[u]);
       buffer_dma16(rd, buf + TILE + (wave + 4 * u) * 512, doff[u]);
     }
@@ -385,8 +246,8 @@ __global__ __launch_bounds__(kThreads, 1) void dkdv_split_kernel(ts_attn_problem
       for (int ks = 0; ks < NKS; ++ks)
 #pragma unroll
         for (int qb = 0; qb < 2; ++qb) {
-          const bf16x8 aq = as_bf16x8(ld16(tq + ro_of(ro, ks) + 16 * qb * HD));
-          const bf16x8 ad = as_bf16x8(ld16(td + ro_of(ro, ks) + 16 * qb * HD));
+          const bf16x8 aq = as_bf16x8(ld16(tq + ro_of<HD>(ro, ks) + 16 * qb * HD));
+          const bf16x8 ad = as_bf16x8(ld16(td + ro_of<HD>(ro, ks) + 16 * qb * HD));
           sc[qb] = mma16<E>(aq, kreg[ks], sc[qb]);
           dp[qb] = mma16<E>(ad, vreg[ks], dp[qb]);
         }
@@ -400,7 +261,7 @@ __global__ __launch_bounds__(kThreads, 1) void dkdv_split_kernel(ts_attn_problem
       u32x2 fa[NMB][2], fb[NMB][2];  // dO^T / Q^T fragments of block mb
 #pragma unroll
       for (int mb = 0; mb < NPRE; ++mb) {
-        const int o = to_of(to, mb);
+        const int o = to_of<HD>(to, mb);
         fa[mb][0] = tr_read(td + o);
         fa[mb][1] = tr_read(td + o + 16 * HD);
         fb[mb][0] = tr_read(tq + o);
@@ -431,7 +292,7 @@ __global__ __launch_bounds__(kThreads, 1) void dkdv_split_kernel(ts_attn_problem
 #pragma unroll
       for (int mb = 0; mb < NMB; ++mb) {
         if (mb >= NPRE) {
-          const int o = to_of(to, mb);
+          const int o = to_of<HD>(to, mb);
           fa[mb][0] = tr_read(td + o);
           fa[mb][1] = tr_read(td + o + 16 * HD);
           fb[mb][0] = tr_read(tq + o);
@@ -483,10 +344,10 @@ __global__ __launch_bounds__(kThreads, 1) void dkdv_split_kernel(ts_attn_problem
 }
 
 template <typename E, int HD>
-void launch_dkdv_generic(dim3 grid, const ts_attn_problem& P, ts_attn_rows q, ts_attn_rows dout,
-                         const float* rowstats, int64_t lse_ld, hipStream_t s) {
+void launch_dkdv_hd(dim3 grid, const ts_attn_problem& P, ts_attn_rows q, ts_attn_rows dout, const float* rowstats,
+                    int64_t lse_ld, hipStream_t s) {
   ts::TimedLaunch timed_("attention.dkdv_kernel", s);
-  hipLaunchKernelGGL((dkdv_kernel<E, HD>), grid, dim3(kThreads), 0, s, P, q, dout, rowstats, lse_ld);
+  hipLaunchKernelGGL((dkdv_split_kernel<E, HD>), grid, dim3(kThreads), 0, s, P, q, dout, rowstats, lse_ld, DsArgs{});
 }
 
 template <typename E, bool DS>
@@ -508,10 +369,10 @@ int launch_dkdv_t(const ts_attn_problem& P, ts_attn_rows q, ts_attn_rows dout, c
                   int64_t lse_ld, const DsArgs* ds, hipStream_t s) {
   const dim3 grid((unsigned)(P.n_kv_work * P.hkv));
   switch (P.head_dim) {
-    case 32: launch_dkdv_generic<E, 32>(grid, P, q, dout, rowstats, lse_ld, s); break;
-    case 64: launch_dkdv_generic<E, 64>(grid, P, q, dout, rowstats, lse_ld, s); break;
-    case 96: launch_dkdv_generic<E, 96>(grid, P, q, dout, rowstats, lse_ld, s); break;
-    case 192: launch_dkdv_generic<E, 192>(grid, P, q, dout, rowstats, lse_ld, s); break;
+    case 32: launch_dkdv_hd<E, 32>(grid, P, q, dout, rowstats, lse_ld, s); break;
+    case 64: launch_dkdv_hd<E, 64>(grid, P, q, dout, rowstats, lse_ld, s); break;
+    case 96: launch_dkdv_hd<E, 96>(grid, P, q, dout, rowstats, lse_ld, s); break;
+    case 192: launch_dkdv_hd<E, 192>(grid, P, q, dout, rowstats, lse_ld, s); break;
     default:  // 128 and 256
       if (ds)
         launch_dkdv_tuned<E, true>(grid, P, q, dout, rowstats, lse_ld, *ds, s);

@@ -86,7 +86,7 @@ __global__ __launch_bounds__(128, 1) void dkdv256_kernel(ts_attn_problem P, ts_a
   const float c = P.scale * kLog2e;
   const int nkb = (run.len + 15) >> 4;  // 16-key blocks of the run
 
-  int ro[4], to[8];
+  int ro[kRowOffsets<HD>], to[2 * kRowOffsets<HD>];
   swizzled_offsets<HD>(lane, ro, to);
   // DMA: a tile is 16 instructions of two rows (lane l: row 2 t + l / 32, slot
   // l % 32 with logical chunk (l % 32) ^ tile_swizzle(row & 15)); wave w issues
@@ -264,8 +264,8 @@ __global__ __launch_bounds__(128, 1) void dkdv256_kernel(ts_attn_problem P, ts_a
         bf16x8 aq[2], ad[2];
 #pragma unroll
         for (int qb = 0; qb < 2; ++qb) {
-          aq[qb] = as_bf16x8(ld16(tq + ro_of(ro, ks) + 16 * qb * HD));
-          ad[qb] = as_bf16x8(ld16(td + ro_of(ro, ks) + 16 * qb * HD));
+          aq[qb] = as_bf16x8(ld16(tq + ro_of<HD>(ro, ks) + 16 * qb * HD));
+          ad[qb] = as_bf16x8(ld16(td + ro_of<HD>(ro, ks) + 16 * qb * HD));
         }
 #pragma unroll
         for (int kb = 0; kb < KB; ++kb)
@@ -322,7 +322,7 @@ __global__ __launch_bounds__(128, 1) void dkdv256_kernel(ts_attn_problem P, ts_a
       // dV^T += dO^T P, dK^T += Q^T dS: rows d = 16 mb + 4 g4 + i, column key 16 kb + j16
 #pragma unroll
       for (int mb = 0; mb < NMB; ++mb) {
-        const int o = to_of(to, mb);
+        const int o = to_of<HD>(to, mb);
         const u32x2 a0 = tr_read(td + o), a1 = tr_read(td + o + 16 * HD);
         const u32x2 b0 = tr_read(tq + o), b1 = tr_read(tq + o + 16 * HD);
         const bf16x8 a = as_bf16x8(u32x4{a0[0], a0[1], a1[0], a1[1]});

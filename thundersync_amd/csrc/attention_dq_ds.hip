@@ -120,7 +120,7 @@ __global__ __launch_bounds__(64 * WV, (dq_ds_occupancy<HD, WV>())) void dq_ds_ke
   if constexpr (SPLIT) part_of<KT>(stop, (int)blockIdx.y, (int)gridDim.y, begin, stop);
   const bool rows_valid = 32 * rb < T;
 
-  int ro[4], to[8];
+  int ro[kRowOffsets<HD>], to[2 * kRowOffsets<HD>];
   swizzled_offsets<HD>(lane, ro, to);
   // transposed-read offsets into a dS block: key 4 g4 + j16 / 4, slots
   // 16 mb' + 4 (j16 & 3) .. + 3 (logical chunk 2 mb' + (j16 & 3) / 2)
@@ -176,8 +176,8 @@ __global__ __launch_bounds__(64 * WV, (dq_ds_occupancy<HD, WV>())) void dq_ds_ke
       }
 #pragma unroll
       for (int mb = 0; mb < NMB; ++mb) {
-        const u32x2 a0 = tr_read(tk + to_of(to, mb) + 32 * ss * HD);
-        const u32x2 a1 = tr_read(tk + to_of(to, mb) + (32 * ss + 16) * HD);
+        const u32x2 a0 = tr_read(tk + to_of<HD>(to, mb) + 32 * ss * HD);
+        const u32x2 a1 = tr_read(tk + to_of<HD>(to, mb) + (32 * ss + 16) * HD);
         const bf16x8 a = as_bf16x8(u32x4{a0[0], a0[1], a1[0], a1[1]});
         acc[mb][0] = mma16<E>(a, b[0], acc[mb][0]);
         acc[mb][1] = mma16<E>(a, b[1], acc[mb][1]);

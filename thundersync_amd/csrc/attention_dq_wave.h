@@ -1,6 +1,6 @@
 // The dQ kernel that shares K/V tiles among its waves, as a template: compiled
-// at head dim 128 in attention_dq.hip (MFMA results in VGPRs) and at head dim
-// 256 in attention_dq256.hip (MFMA results in the accumulation registers: four
+// at head dims up to 128 in attention_dq.hip (MFMA results in VGPRs) and at 192
+// and 256 in attention_dq256.hip (MFMA results in the accumulation registers: four
 // waves of 32 rows need more than the 256 VGPRs for their dQ accumulators).
 #pragma once
 #include "attention_impl.h"
@@ -9,24 +9,28 @@ namespace ts {
 namespace attn {
 
 // ---------------------------------------------------------------------------
-// backward dQ with the waves sharing K/V tiles (query-stationary; head dim 128
-// with GQA groups that are a multiple of 4 (GC = 4), head dim 256 with any
-// group, GC heads per work-group)
+// backward dQ with the waves sharing K/V tiles (query-stationary; every head
+// dim and GQA group, GC heads per work-group)
 //
 // A work-group owns 128 / GC query rows of one segment for GC query heads of
 // one GQA group; wave w takes head w % GC and 16 NQB of the rows (head dim
 // 128: NQB = 1, eight waves, two per SIMD, so that one wave's LDS and MFMA
-// waits are covered by the other's work; head dim 256: NQB = 2, four waves of
-// 32 rows, one per SIMD).  Q and dO rows stay in registers as B operands, with
+// waits are covered by the other's work; the narrower head dims and 192: NQB =
+// 2, four waves of 32 rows, which read each K and V fragment once for two row
+// blocks: 8 sequences of 512 to 2048 rows at 16/8 heads of 64 72 us against 91
+// with 16 rows a wave; 256: attention_dq256.hip).  Q and dO rows stay in registers as B operands, with
 // the rows' (lse * log2 e, delta) pairs.  The segment's key runs stream
 // through 64-key K/V tiles that all waves share: double-buffered LDS stages
 // filled by buffer_load ... lds (each wave issues its share of a tile's
 // instructions; rows past a run's end arrive as zeros and add nothing,
 // because a zero K row contributes zero to dQ), one work-group barrier per
 // tile.  Tiles use the dK/dV kernel's swizzled rows
-// with chunk c of row r at slot c ^ tile_swizzle(r & 15): K and V rows feed S^T = K Q^T
+// with chunk c of row r at slot c ^ row_swizzle(r & 15): K and V rows feed S^T = K Q^T
 // and dP^T = V dO^T as A operands, K^T for dQ^T += K^T dS^T comes from
-// ds_read_b64_tr_b16.  Only tiles that cross the diagonal are masked.
+// ds_read_b64_tr_b16.  Only tiles that cross the diagonal are masked.  Against
+// tiles passed through registers between two barriers (8 sequences of 512 to 2048
+// rows, us): head dim 64 at 16/8 heads 115 -> 71, 32 75 -> 48, 96 143 -> 98, 192 at
+// 24/4 647 -> 387.
 // ---------------------------------------------------------------------------
 template <typename E, int NQB, int HD = D, int GC = 4, int NP = 1>
 __global__ __launch_bounds__(64 * 8 / (NQB * NP), 1) void dq_wave_kernel(ts_attn_problem P, ts_attn_rows Q, ts_attn_rows dO,
@@ -54,7 +58,7 @@ __global__ __launch_bounds__(64 * 8 / (NQB * NP), 1) void dq_wave_kernel(ts_attn
   const int T = seg.q_len;
   const int off = seg.kv_len - seg.q_len;
   const float c = P.scale * kLog2e;
-  int ro[4], to[8];
+  int ro[kRowOffsets<HD>], to[2 * kRowOffsets<HD>];
   swizzled_offsets<HD>(lane, ro, to);
 
   // the work item's rows in NP passes over its keys (one at head dim 128)
@@ -113,8 +117,8 @@ __global__ __launch_bounds__(64 * 8 / (NQB * NP), 1) void dq_wave_kernel(ts_attn
     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
       for (int ks = 0; ks < NKS; ++ks) {
-        const bf16x8 ak = as_bf16x8(ld16(tk + ro_of(ro, ks) + (32 * ss + 16 * kb) * HD));
-        const bf16x8 av = as_bf16x8(ld16(tv + ro_of(ro, ks) + (32 * ss + 16 * kb) * HD));
+        const bf16x8 ak = as_bf16x8(ld16(tk + ro_of<HD>(ro, ks) + (32 * ss + 16 * kb) * HD));
+        const bf16x8 av = as_bf16x8(ld16(tv + ro_of<HD>(ro, ks) + (32 * ss + 16 * kb) * HD));
 #pragma unroll
         for (int qb = 0; qb < NQB; ++qb) {
           sc[kb][qb] = mma16<E>(ak, qreg[qb][ks], sc[kb][qb]);
@@ -151,8 +155,8 @@ __global__ __launch_bounds__(64 * 8 / (NQB * NP), 1) void dq_wave_kernel(ts_attn
   auto accumulate = [&](const bf16* tk, int ss, const bf16x8 (&dsk)[NQB]) __attribute__((always_inline)) {
 #pragma unroll
     for (int mb = 0; mb < NMB; ++mb) {
-      const u32x2 a0 = tr_read(tk + to_of(to, mb) + 32 * ss * HD);
-      const u32x2 a1 = tr_read(tk + to_of(to, mb) + (32 * ss + 16) * HD);
+      const u32x2 a0 = tr_read(tk + to_of<HD>(to, mb) + 32 * ss * HD);
+      const u32x2 a1 = tr_read(tk + to_of<HD>(to, mb) + (32 * ss + 16) * HD);
       const bf16x8 a = as_bf16x8(u32x4{a0[0], a0[1], a1[0], a1[1]});
 #pragma unroll
       for (int qb = 0; qb < NQB; ++qb) acc[mb][qb] = mma16<E>(a, dsk[qb], acc[mb][qb]);
@@ -282,9 +286,9 @@ __global__ __launch_bounds__(64 * 8 / (NQB * NP), 1) void dq_wave_kernel(ts_attn
 }
 
 
-// dQ at head dim 256 (attention_dq256.hip): the one-wave-per-SIMD instance
-void launch_dq_wave256(const ts_attn_problem& P, int gc, dim3 grid, ts_attn_rows q, ts_attn_rows dout,
-                       const float* rowstats, int64_t lse_ld, ts_attn_rows dq, hipStream_t s);
+// dQ at head dims 192 and 256 (attention_dq256.hip)
+void launch_dq_wide(const ts_attn_problem& P, int gc, dim3 grid, ts_attn_rows q, ts_attn_rows dout,
+                    const float* rowstats, int64_t lse_ld, ts_attn_rows dq, hipStream_t s);
 
 }  // namespace attn
 }  // namespace ts

@@ -5,148 +5,8 @@ namespace ts {
 namespace attn {
 
 // ---------------------------------------------------------------------------
-// forward
-// ---------------------------------------------------------------------------
-// Register-staged forward for any supported head dim HD and GQA groups that
-// are not a multiple of 4 (and, at head dims other than 128, those that are):
-// a work-group owns 32 4 / GC query rows of GC query heads (wave w: head
-// w % GC, rows 32 (w / GC) ..); K/V tiles of 64 keys pass through registers
-// into padded LDS rows; V^T comes from ds_read_b64_tr_b16 (tr_frag).
-template <typename E, int GC, int HD>
-__global__ __launch_bounds__(kThreads, HD > 128 ? 1 : 2) void fwd_kernel(ts_attn_problem P, ts_attn_rows Q,
-                                                          ts_attn_rows O, float* __restrict__ lse,
-                                                          int64_t lse_ld) {
-  constexpr int NMB = HD / 16;  // 16-column blocks of O
-  __shared__ __attribute__((aligned(16))) bf16 sk[BK * pitch_of<HD>()];
-  __shared__ __attribute__((aligned(16))) bf16 sv[BK * pitch_of<HD>()];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  int yb;
-  const int item = task_of(P.n_q_work, P.n_q_long, yb);
-  const int seg_id = uniform_table(P.q_work)[2 * item];
-  const int q0 = uniform_table(P.q_work)[2 * item + 1];
-  const int group = P.hq / P.hkv;
-  const int chunks = group / GC;
-  const int hk = yb / chunks;
-  const int h = hk * group + (yb % chunks) * GC + (wave % GC);
-  const ts_attn_segment seg = load_uniform(P.segs, seg_id);
-  const int T = seg.q_len;
-  const int off = seg.kv_len - seg.q_len;
-  const int wq0 = q0 + 32 * (wave / GC);
-  const int wg_last = min(q0 + P.q_block, T) - 1;
-  const bool active = wq0 < T;
-  const int w_last = min(wq0 + 32, T) - 1;
-  const float c = P.scale * kLog2e;
-
-  bf16x8 qreg[2][HD / 32];
-  const bf16* qbase = (const bf16*)Q.ptr + (seg.q_row0 + wq0) * Q.row_stride + (int64_t)h * Q.head_stride;
-  load_rows_b<2, HD>(qreg, qbase, Q.row_stride, active ? T - wq0 : 0, lane);
-
-  f32x4 o[2][NMB];
-#pragma unroll
-  for (int qb = 0; qb < 2; ++qb)
-#pragma unroll
-    for (int mb = 0; mb < NMB; ++mb) o[qb][mb] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float m[2] = {neg_inf(), neg_inf()};
-  float lsum[2] = {0.f, 0.f};
-
-  for (int sp = 0; sp < seg.nspan; ++sp) {
-    const ts_attn_ref ref = load_uniform(P.seg_spans, seg.span0 + sp);
-    const ts_attn_run run = load_uniform(P.runs, ref.index);
-    const bf16* kb0 = (const bf16*)run.k + (int64_t)hk * run.k_head_stride;
-    const bf16* vb0 = (const bf16*)run.v + (int64_t)hk * run.v_head_stride;
-    for (int kt0 = 0; kt0 < run.len; kt0 += BK) {
-      if (ref.kpos + kt0 > off + wg_last) break;  // later keys are invisible to every row
-      const int nvalid = min(BK, run.len - kt0);
-      stage_kv<HD>(sk, sv, kb0 + (int64_t)kt0 * run.k_row_stride, run.k_row_stride,
-                   vb0 + (int64_t)kt0 * run.v_row_stride, run.v_row_stride, nvalid, tid);
-      if (!active || ref.kpos + kt0 > off + w_last) continue;
-
-      f32x4 s[4][2];
-      tile_scores<E, HD>(s, sk, qreg, lane);
-      const bool need_mask = (kt0 + BK > run.len) || (ref.kpos + kt0 + BK - 1 > off + wq0);
-#pragma unroll
-      for (int kb = 0; kb < 4; ++kb)
-#pragma unroll
-        for (int qb = 0; qb < 2; ++qb)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            float val = s[kb][qb][i] * c;
-            if (need_mask) {
-              const int key = kt0 + 16 * kb + 4 * (lane >> 4) + i;
-              const int row = wq0 + 16 * qb + (lane & 15);
-              if (key >= run.len || ref.kpos + key > off + row) val = neg_inf();
-            }
-            s[kb][qb][i] = val;
-          }
-      // online softmax, one query column per lane (shared by lanes l, l^16, l^32, l^48)
-#pragma unroll
-      for (int qb = 0; qb < 2; ++qb) {
-        float mx = neg_inf();
-#pragma unroll
-        for (int kb = 0; kb < 4; ++kb)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) mx = fmaxf(mx, s[kb][qb][i]);
-        mx = rows_max4(mx);
-        const float mnew = fmaxf(m[qb], mx);
-        const float mref = (mnew == neg_inf()) ? 0.f : mnew;
-        const float alpha = fast_exp2(m[qb] - mref);
-        m[qb] = mnew;
-        float ps = 0.f;
-#pragma unroll
-        for (int kb = 0; kb < 4; ++kb)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const float p = fast_exp2(s[kb][qb][i] - mref);
-            s[kb][qb][i] = p;
-            ps += p;
-          }
-        lsum[qb] = lsum[qb] * alpha + ps;
-#pragma unroll
-        for (int mb = 0; mb < NMB; ++mb) o[qb][mb] *= alpha;
-      }
-      // O^T += V^T P^T, 32 keys per k-step
-#pragma unroll
-      for (int ss = 0; ss < 2; ++ss) {
-        bf16x8 pk[2];
-#pragma unroll
-        for (int qb = 0; qb < 2; ++qb) {
-          float tmp[8];
-#pragma unroll
-          for (int j = 0; j < 8; ++j) tmp[j] = s[2 * ss + (j >> 2)][qb][j & 3];
-          pk[qb] = pack8<E>(tmp);
-        }
-#pragma unroll
-        for (int mb = 0; mb < NMB; ++mb) {
-          const bf16x8 vt = tr_frag<HD>(sv, 32 * ss, mb, lane);
-          o[0][mb] = mma16<E>(vt, pk[0], o[0][mb]);
-          o[1][mb] = mma16<E>(vt, pk[1], o[1][mb]);
-        }
-      }
-    }
-  }
-  if (!active) return;
-#pragma unroll
-  for (int qb = 0; qb < 2; ++qb) {
-    const float l = rows_sum4(lsum[qb]);
-    const int row = wq0 + 16 * qb + (lane & 15);
-    if (row >= T) continue;
-    const float inv = l > 0.f ? 1.f / l : 0.f;
-    // o[qb][mb] lane holds d = 16 mb + 4 g4 + i of this row: 8-byte stores
-    bf16* orow = (bf16*)O.ptr + (seg.q_row0 + row) * O.row_stride + (int64_t)h * O.head_stride + 4 * (lane >> 4);
-#pragma unroll
-    for (int mb = 0; mb < NMB; ++mb) {
-      const f32x4 v = o[qb][mb] * inv;
-      *reinterpret_cast<u32x2*>(orow + 16 * mb) = u32x2{pack2<E>(v[0], v[1]), pack2<E>(v[2], v[3])};
-    }
-    if ((lane >> 4) == 0)
-      lse[(int64_t)h * lse_ld + seg.q_row0 + row] = l > 0.f ? (m[qb] + fast_log2(l)) * kLn2 : neg_inf();
-  }
-}
-
-// ---------------------------------------------------------------------------
-// forward with the waves sharing K/V tiles (head dim 128 with GQA groups that
-// are a multiple of 4 (GC = 4); head dim 256 with any group, GC heads per
-// work-group)
+// forward with the waves sharing K/V tiles (every head dim and GQA group, GC
+// heads per work-group)
 //
 // A work-group owns 128 / GC query rows of one segment for GC query heads of
 // one GQA group; wave w takes head w % GC and 16 NQB rows (at head dim 128
@@ -155,8 +15,10 @@ __global__ __launch_bounds__(kThreads, HD > 128 ? 1 : 2) void fwd_kernel(ts_attn
 // NQB = 1, eight waves, two per SIMD, one work-group per CU for its 128 KB of
 // tiles).  The heads share K/V tiles of KT keys (32 at head dim 128: 32 KB
 // of stages per work-group, three work-groups and three waves per SIMD at 168
-// VGPRs, against two with 64-key tiles: C2 forward 1.20 -> 1.09 ms; 64 at
-// 256), streamed by buffer DMA into double-buffered swizzled LDS stages (one
+// VGPRs, against two with 64-key tiles: C2 forward 1.20 -> 1.09 ms; 32 at 192,
+// where 16 rows a wave over 64-key tiles took 172 us against 136 for 8 sequences
+// of 512 to 2048 rows at 16/8 heads; 64 at the others: 59 us against 63 with 32 at
+// head dim 64 there, 65 with 16 rows a wave), streamed by buffer DMA into double-buffered swizzled LDS stages (one
 // work-group barrier per tile).  Q rows stay in registers as B operands of
 // S^T = K Q^T; V^T for O^T += V^T P^T comes from ds_read_b64_tr_b16.  Per 32
 // keys of a tile each lane owns one query column (16 qb + j16) and 8 of the
@@ -166,7 +28,9 @@ __global__ __launch_bounds__(kThreads, HD > 128 ? 1 : 2) void fwd_kernel(ts_attn
 // more than 8 (a factor of 256): the accumulators are rescaled in the rare
 // tile where that happens (skipped wave-wide otherwise), and since O and the
 // row sum share the same m the result is unchanged.  Only tiles that cross
-// the diagonal or pass a run's end are masked.
+// the diagonal or pass a run's end are masked.  Against K/V tiles passed through
+// registers between two barriers (8 sequences of 512 to 2048 rows, us): head dim
+// 64 at 16/8 heads 92 -> 60, 32 71 -> 48, 96 112 -> 81, 192 at 24/4 584 -> 200.
 // ---------------------------------------------------------------------------
 constexpr float kRescaleSlack = 8.f;    // log2 units
 constexpr float kRescaleBound = 256.f;  // 2^kRescaleSlack
@@ -180,7 +44,10 @@ constexpr float kRescaleBound = 256.f;  // 2^kRescaleSlack
 #endif
 // work-groups per CU: their LDS stages (two K/V stages of KT keys) and registers
 template <int NQB, int HD, int KT>
-constexpr int fwd_occupancy() { return HD > 128 ? (NQB == 1 ? 2 : 1) : (NQB == 1 ? 4 : (KT == 32 ? 3 : 2)); }
+constexpr int fwd_occupancy() {
+  if (HD < 128 || HD == 192) return HD <= 64 ? 4 : HD == 96 ? 3 : 2;
+  return HD > 128 ? (NQB == 1 ? 2 : 1) : (NQB == 1 ? 4 : (KT == 32 ? 3 : 2));
+}
 
 // SPLIT: the launch's y blocks are parts of each item's keys (launches whose
 // items leave CUs idle, ts_attn_fwd_parts); a part writes its unnormalised fp32
@@ -230,7 +97,7 @@ __global__ __launch_bounds__(64 * 8 / NQB, (fwd_occupancy<NQB, HD, KT>())) void 
     m[qb] = neg_inf();
     l[qb] = 0.f;
   }
-  int ro[4], to[8];
+  int ro[kRowOffsets<HD>], to[2 * kRowOffsets<HD>];
   swizzled_offsets<HD>(lane, ro, to);
 
   auto step = [&](auto bsel, TileCursor& cur) {
@@ -260,7 +127,7 @@ __global__ __launch_bounds__(64 * 8 / NQB, (fwd_occupancy<NQB, HD, KT>())) void 
         for (int qb = 0; qb < NQB; ++qb) sc[kb][qb] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int ks = 0; ks < NKS; ++ks) {
-          const bf16x8 ak = as_bf16x8(ld16(tk + ro_of(ro, ks) + (32 * ss + 16 * kb) * HD));
+          const bf16x8 ak = as_bf16x8(ld16(tk + ro_of<HD>(ro, ks) + (32 * ss + 16 * kb) * HD));
 #pragma unroll
           for (int qb = 0; qb < NQB; ++qb) sc[kb][qb] = mma16<E>(ak, qreg[qb][ks], sc[kb][qb]);
         }
@@ -348,8 +215,8 @@ __global__ __launch_bounds__(64 * 8 / NQB, (fwd_occupancy<NQB, HD, KT>())) void 
       __builtin_amdgcn_s_setprio(1);
 #pragma unroll
       for (int mb = 0; mb < NMB; ++mb) {
-        const u32x2 a0 = tr_read(tv + to_of(to, mb) + 32 * ss * HD);
-        const u32x2 a1 = tr_read(tv + to_of(to, mb) + (32 * ss + 16) * HD);
+        const u32x2 a0 = tr_read(tv + to_of<HD>(to, mb) + 32 * ss * HD);
+        const u32x2 a1 = tr_read(tv + to_of<HD>(to, mb) + (32 * ss + 16) * HD);
         const bf16x8 a = as_bf16x8(u32x4{a0[0], a0[1], a1[0], a1[1]});
 #pragma unroll
         for (int qb = 0; qb < NQB; ++qb) acc[mb][qb] = mma16<E>(a, pk[qb], acc[mb][qb]);
@@ -455,23 +322,7 @@ __global__ __launch_bounds__(kThreads) void fwd_merge_kernel(ts_attn_problem P, 
 // query rows per wave of the forward kernel (32: four waves per work-group; 16: eight)
 constexpr int kFwdRowsPerWave = 32;
 
-template <typename E, int HD>
-void launch_fwd_generic(const ts_attn_problem& P, int gc, dim3 grid, ts_attn_rows q, ts_attn_rows out, float* lse,
-                        int64_t lse_ld, hipStream_t s) {
-  ts::TimedLaunch timed_("attention.fwd_kernel", s);
-  if constexpr (HD != D) {
-    if (gc == 4) {
-      hipLaunchKernelGGL((fwd_kernel<E, 4, HD>), grid, dim3(kThreads), 0, s, P, q, out, lse, lse_ld);
-      return;
-    }
-  }
-  if (gc == 2)
-    hipLaunchKernelGGL((fwd_kernel<E, 2, HD>), grid, dim3(kThreads), 0, s, P, q, out, lse, lse_ld);
-  else
-    hipLaunchKernelGGL((fwd_kernel<E, 1, HD>), grid, dim3(kThreads), 0, s, P, q, out, lse, lse_ld);
-}
-
-// the DMA-staged forward (head dims 128 and 256), whole items or parts of them
+// whole items, or parts of them (head dims 128 and 256)
 template <typename E, int NQB, int HD, int GC, int KT>
 void launch_fwd_wave(const ts_attn_problem& P, dim3 grid, ts_attn_rows q, ts_attn_rows out, float* lse, int64_t lse_ld,
                      int parts, float* part, hipStream_t s) {
@@ -481,14 +332,24 @@ void launch_fwd_wave(const ts_attn_problem& P, dim3 grid, ts_attn_rows q, ts_att
                        nullptr);
     return;
   }
-  {
-    ts::TimedLaunch timed_("attention.fwd_kernel", s);
-    hipLaunchKernelGGL((fwd_wave_kernel<E, NQB, HD, GC, KT, true>), dim3(grid.x, parts), dim3(64 * 8 / NQB), 0, s, P, q,
-                       out, lse, lse_ld, part);
+  if constexpr (HD % 128 == 0) {
+    {
+      ts::TimedLaunch timed_("attention.fwd_kernel", s);
+      hipLaunchKernelGGL((fwd_wave_kernel<E, NQB, HD, GC, KT, true>), dim3(grid.x, parts), dim3(64 * 8 / NQB), 0, s, P,
+                         q, out, lse, lse_ld, part);
+    }
+    ts::TimedLaunch timed_("attention.fwd_merge_kernel", s);
+    hipLaunchKernelGGL((fwd_merge_kernel<E, HD, GC>), dim3(grid.x, kMergeBlocks), dim3(kThreads), 0, s, P, out, lse,
+                       lse_ld, part, parts);
   }
-  ts::TimedLaunch timed_("attention.fwd_merge_kernel", s);
-  hipLaunchKernelGGL((fwd_merge_kernel<E, HD, GC>), dim3(grid.x, kMergeBlocks), dim3(kThreads), 0, s, P, out, lse,
-                     lse_ld, part, parts);
+}
+
+template <typename E, int NQB, int HD, int KT>
+void launch_fwd_hd(const ts_attn_problem& P, int gc, dim3 grid, ts_attn_rows q, ts_attn_rows out, float* lse,
+                   int64_t lse_ld, int parts, float* part, hipStream_t s) {
+  if (gc == 4) launch_fwd_wave<E, NQB, HD, 4, KT>(P, grid, q, out, lse, lse_ld, parts, part, s);
+  else if (gc == 2) launch_fwd_wave<E, NQB, HD, 2, KT>(P, grid, q, out, lse, lse_ld, parts, part, s);
+  else launch_fwd_wave<E, NQB, HD, 1, KT>(P, grid, q, out, lse, lse_ld, parts, part, s);
 }
 
 template <typename E>
@@ -498,15 +359,11 @@ int launch_fwd_t(const ts_attn_problem& P, ts_attn_rows q, ts_attn_rows out, flo
   const int gc = heads_per_block(group);
   const dim3 grid((unsigned)(P.n_q_work * P.hkv * (group / gc)));
   switch (P.head_dim) {
-    case 32: launch_fwd_generic<E, 32>(P, gc, grid, q, out, lse, lse_ld, s); break;
-    case 64: launch_fwd_generic<E, 64>(P, gc, grid, q, out, lse, lse_ld, s); break;
-    case 96: launch_fwd_generic<E, 96>(P, gc, grid, q, out, lse, lse_ld, s); break;
-    case 192: launch_fwd_generic<E, 192>(P, gc, grid, q, out, lse, lse_ld, s); break;
-    case 256:
-      if (gc == 4) launch_fwd_wave<E, 1, 256, 4, BK>(P, grid, q, out, lse, lse_ld, parts, part, s);
-      else if (gc == 2) launch_fwd_wave<E, 1, 256, 2, BK>(P, grid, q, out, lse, lse_ld, parts, part, s);
-      else launch_fwd_wave<E, 1, 256, 1, BK>(P, grid, q, out, lse, lse_ld, parts, part, s);
-      break;
+    case 32: launch_fwd_hd<E, 2, 32, BK>(P, gc, grid, q, out, lse, lse_ld, parts, part, s); break;
+    case 64: launch_fwd_hd<E, 2, 64, BK>(P, gc, grid, q, out, lse, lse_ld, parts, part, s); break;
+    case 96: launch_fwd_hd<E, 2, 96, BK>(P, gc, grid, q, out, lse, lse_ld, parts, part, s); break;
+    case 192: launch_fwd_hd<E, 2, 192, 32>(P, gc, grid, q, out, lse, lse_ld, parts, part, s); break;
+    case 256: launch_fwd_hd<E, 1, 256, BK>(P, gc, grid, q, out, lse, lse_ld, parts, part, s); break;
     default: {
       constexpr int NQB = kFwdRowsPerWave / 16;
       if (gc == 4) launch_fwd_wave<E, NQB, D, 4, TS_FWD_KT128>(P, grid, q, out, lse, lse_ld, parts, part, s);

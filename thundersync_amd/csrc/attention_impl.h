@@ -16,7 +16,6 @@ namespace attn {
 constexpr int D = 128;
 constexpr int BK = 64;          // keys per tile (fwd / dq) and per dkdv block
 constexpr int kThreads = 256;   // 4 waves
-constexpr int PITCH = D + 8;    // LDS row pitch in elements (272 bytes)
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
 
@@ -25,93 +24,10 @@ __device__ __forceinline__ float neg_inf() { return -__builtin_huge_valf(); }
 __device__ __forceinline__ u32x4 ld16(const bf16* p) { return *reinterpret_cast<const u32x4*>(p); }
 __device__ __forceinline__ void st16(bf16* p, u32x4 v) { *reinterpret_cast<u32x4*>(p) = v; }
 
-// Head dims the kernels take: a multiple of 32 up to 256.  128 runs the
-// tuned one-wave-per-head kernels (GQA groups that are a multiple of 4); every
-// other head dim, and groups that are not a multiple of 4, run the
-// register-staged kernels below, templated on the head dim HD.
+// Head dims the kernels take.  All of them stage K/V (or Q/dO) tiles by buffer
+// DMA into swizzled LDS rows of the head dim (row_swizzle).
 __host__ __device__ constexpr bool head_dim_supported(int hd) {
   return hd == 32 || hd == 64 || hd == 96 || hd == 128 || hd == 192 || hd == 256;
-}
-
-// LDS row pitch (elements) of the register-staged kernels' tiles: 16 bytes of
-// padding per row
-template <int HD> constexpr int pitch_of() { return HD + 8; }
-
-// A 64 x HD tile of K or V rows moved global -> registers -> LDS by 256
-// threads; HD / 8 consecutive threads read one row.
-template <int HD>
-struct Tile {
-  u32x4 v[HD / 32];
-};
-
-template <int HD>
-__device__ __forceinline__ void tile_load(Tile<HD>& t, const bf16* base, int64_t row_stride, int nvalid,
-                                          int tid) {
-  constexpr int CH = HD / 8;
-#pragma unroll
-  for (int it = 0; it < HD / 32; ++it) {
-    const int idx = it * kThreads + tid;
-    const int row = idx / CH, chunk = idx % CH;
-    if (row < nvalid)
-      t.v[it] = ld16(base + (int64_t)row * row_stride + chunk * 8);
-    else
-      t.v[it] = u32x4{0u, 0u, 0u, 0u};
-  }
-}
-
-template <int HD>
-__device__ __forceinline__ void tile_store(const Tile<HD>& t, bf16* lds, int tid) {
-  constexpr int CH = HD / 8;
-#pragma unroll
-  for (int it = 0; it < HD / 32; ++it) {
-    const int idx = it * kThreads + tid;
-    st16(lds + (idx / CH) * pitch_of<HD>() + (idx % CH) * 8, t.v[it]);
-  }
-}
-
-// One 64-key K tile and V tile into LDS (all threads; the barriers order the
-// stores after every wave's reads of the previous tiles and the reads after
-// the stores).  Up to a head dim of 128 both tiles are in flight at once;
-// above it they go one after the other, halving the staging registers.
-template <int HD>
-__device__ __forceinline__ void stage_kv(bf16* sk, bf16* sv, const bf16* kp, int64_t k_stride, const bf16* vp,
-                                         int64_t v_stride, int nvalid, int tid) {
-  if constexpr (HD <= 128) {
-    Tile<HD> tk, tv;
-    tile_load(tk, kp, k_stride, nvalid, tid);
-    tile_load(tv, vp, v_stride, nvalid, tid);
-    __syncthreads();
-    tile_store(tk, sk, tid);
-    tile_store(tv, sv, tid);
-  } else {
-    Tile<HD> t;
-    tile_load(t, kp, k_stride, nvalid, tid);
-    __syncthreads();
-    tile_store(t, sk, tid);
-    tile_load(t, vp, v_stride, nvalid, tid);
-    tile_store(t, sv, tid);
-  }
-  __syncthreads();
-}
-
-// rows [0, 32) x HD of a per-head query-row tensor -> LDS (256 threads)
-template <int HD = D>
-__device__ __forceinline__ void rows32_to_lds(bf16* lds, const bf16* base, int64_t row_stride,
-                                              int nvalid, int tid) {
-  constexpr int CH = HD / 8;
-#pragma unroll
-  for (int idx = tid; idx < 32 * CH; idx += kThreads) {
-    const int row = idx / CH, chunk = idx % CH;
-    u32x4 v = u32x4{0u, 0u, 0u, 0u};
-    if (row < nvalid) v = ld16(base + (int64_t)row * row_stride + chunk * 8);
-    st16(lds + row * pitch_of<HD>() + chunk * 8, v);
-  }
-}
-
-// the row of slot j for lane group g: 4g + (j & 3) + 16 (j >> 2)
-__device__ __forceinline__ void slot_rows(int g, int base, int rows[8]) {
-#pragma unroll
-  for (int j = 0; j < 8; ++j) rows[j] = base + 4 * g + (j & 3) + 16 * (j >> 2);
 }
 
 // eight floats as eight T values (an operand container; see mma16)
@@ -135,24 +51,6 @@ __device__ __forceinline__ void load_rows_b(bf16x8 (&reg)[NQB][HD / 32], const b
       u32x4 v = u32x4{0u, 0u, 0u, 0u};
       if (row < nvalid) v = ld16(base + (int64_t)row * row_stride + 32 * ks + 8 * (lane >> 4));
       reg[qb][ks] = as_bf16x8(v);
-    }
-  }
-}
-
-// S^T tile (64 keys x 32 rows) = K_lds Q^T: s[kb][qb] lane holds keys
-// 16 kb + 4 (lane >> 4) + i, row 16 qb + (lane & 15).
-template <typename E, int HD = D>
-__device__ __forceinline__ void tile_scores(f32x4 s[4][2], const bf16* sk, const bf16x8 qreg[2][HD / 32],
-                                            int lane) {
-#pragma unroll
-  for (int kb = 0; kb < 4; ++kb) {
-    s[kb][0] = f32x4{0.f, 0.f, 0.f, 0.f};
-    s[kb][1] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int ks = 0; ks < HD / 32; ++ks) {
-      const bf16x8 a = as_bf16x8(ld16(sk + (16 * kb + (lane & 15)) * pitch_of<HD>() + 32 * ks + 8 * (lane >> 4)));
-      s[kb][0] = mma16<E>(a, qreg[0][ks], s[kb][0]);
-      s[kb][1] = mma16<E>(a, qreg[1][ks], s[kb][1]);
     }
   }
 }
@@ -203,21 +101,6 @@ __device__ __forceinline__ u32x2 tr_read(const bf16* p) {
   u32x2 r;
   __builtin_memcpy(&r, &v, 8);
   return r;
-}
-
-// A transposed operand of the register-staged kernels from a padded LDS tile
-// (row pitch HD + 8 elements) by two ds_read_b64_tr_b16: the 16 x 32 A
-// operand X^T[16 mb .. 16 mb + 15][row0 + slot rows], slot j <-> row
-// row0 + 16 (j >> 2) + 4 g4 + (j & 3) (the slot order of slot_rows).  Lane
-// (g4, j16) addresses row row0 + 4 g4 + j16 / 4 and columns
-// 16 mb + 4 (j16 & 3) .. + 3, and receives X[row0 + 4 g4 + t][16 mb + j16],
-// t = 0..3, then the same from 16 rows further.
-template <int HD>
-__device__ __forceinline__ bf16x8 tr_frag(const bf16* lds, int row0, int mb, int lane) {
-  const int g4 = lane >> 4, j16 = lane & 15;
-  const bf16* p = lds + (row0 + 4 * g4 + (j16 >> 2)) * pitch_of<HD>() + 16 * mb + 4 * (j16 & 3);
-  const u32x2 a = tr_read(p), b = tr_read(p + 16 * pitch_of<HD>());
-  return as_bf16x8(u32x4{a[0], a[1], b[0], b[1]});
 }
 
 // A key run's position in its visit list with the visited segment's fields
@@ -446,18 +329,26 @@ constexpr int kMergeBlocks = 16;  // work-groups that merge one item's parts
 // 2.2 clk per transposed read per CU, against 4.2 and 4.1 for s(r) = r).
 __device__ __forceinline__ int tile_swizzle(int r) { return r ^ ((r & 1) ? 12 : 0); }
 
+// The same for rows of HD elements.  Below 256 bytes a 256-byte line of banks
+// holds several rows (or, at 384 bytes, a row and a half), so fewer bits of the
+// chunk are left to permute: at 128 and 384 bytes (8 | chunks) rows of equal
+// parity share 8 slots, and r & 6 gives both kinds of read 16 distinct slots a
+// pass; at 64 and 192 bytes rows 4 apart share 4 slots, and (r >> 1) & 2 does.
+template <int HD>
+__device__ __forceinline__ int row_swizzle(int r) {
+  return HD % 128 == 0 ? tile_swizzle(r) : HD % 64 == 0 ? r & 6 : (r >> 1) & 2;
+}
+
 // DMA of the cursor's K/V tile of KT keys into swizzled LDS tiles (rows of
-// HD elements, chunk c of row r at slot c ^ tile_swizzle(r & 15)).  The WAVES
+// HD elements, chunk c of row r at slot c ^ row_swizzle(r & 15)).  The WAVES
 // waves of a work-group (4 or 8) each issue instructions t = wave + WAVES u;
-// instruction t fills rows RPI t .. RPI t + RPI - 1 (RPI = 4 at HD 128, 2 at
-// 256): lane l the row RPI t + l / (HD / 8), slot l % (HD / 8) with logical
-// chunk (l % (HD / 8)) ^ tile_swizzle(row).  Rows past the run arrive as
-// zeros.
+// instruction t fills the tile's 16-byte slots 64 t .. 64 t + 63: lane l slot
+// i = 64 t + l, the slot i % (HD / 8) of row i / (HD / 8) with logical chunk
+// (i % (HD / 8)) ^ row_swizzle(row).  Rows past the run arrive as zeros.
 template <int WAVES = 4, int HD = D, int KT = BK>
 __device__ __forceinline__ void issue_kv_tile(int wave, int lane, const TileCursor& tc, bf16* sk, bf16* sv) {
   static_assert(WAVES == 4 || WAVES == 8, "a tile is 16 or 32 instructions");
-  static_assert(HD == 128 || HD == 256, "the swizzle needs 16 or 32 chunks per row");
-  constexpr int CH = HD / 8, RPI = 64 / CH, NI = KT / RPI;
+  constexpr int CH = HD / 8, NI = KT * CH / 64;
   static_assert(NI % WAVES == 0, "every wave issues the same number of instructions");
   const int nvalid = min(KT, tc.len - tc.kt0);
   const rsrc_t rk = make_rsrc(tc.kt, (uint32_t)(nvalid * tc.k_rs * 2));
@@ -479,8 +370,8 @@ __device__ __forceinline__ void issue_kv_tile(int wave, int lane, const TileCurs
 #pragma unroll
     for (int u = 0; u < NI / WAVES; ++u) {
       const int t = wave + WAVES * u;
-      const int row = RPI * t + lane / CH;
-      const int chunk = ((lane % CH) ^ tile_swizzle(row & 15)) << 3;
+      const int slot = 64 * t + lane, row = slot / CH;
+      const int chunk = ((slot % CH) ^ row_swizzle<HD>(row & 15)) << 3;
       buffer_dma16(rk, sk + t * 512, (row * tc.k_rs + chunk) * 2);
       buffer_dma16(rv, sv + t * 512, (row * tc.v_rs + chunk) * 2);
     }
@@ -491,25 +382,35 @@ __device__ __forceinline__ void issue_kv_tile(int wave, int lane, const TileCurs
 // ro[ks]: row j16, logical chunk 4 ks + g4 (A-operand row reads of 16 rows);
 // to[mb]: row 4 g4 + j16 / 4, columns 16 mb + 4 (j16 & 3) .. + 3 (the
 // addresses of a ds_read_b64_tr_b16 that yields X[4 g4 + t][16 mb + j16]).
-// The swizzle permutes chunks within aligned groups of 16, so at head dim 256
-// the offsets of k-step ks + 4 and column block mb + 8 are those of ks and mb
-// plus 128 elements: only the first four and eight are kept (the rest fold
-// into the reads' immediate offsets).
+// The swizzle permutes chunks within aligned groups of 4 NRO (16 at head dims
+// 128 and 256, 8 at 64 and 192, 4 at 32 and 96), so the offsets of k-step ks +
+// NRO and column block mb + 2 NRO are those of ks and mb plus 32 NRO elements:
+// only the first NRO and 2 NRO are kept (the rest fold into the reads' immediate
+// offsets).
+template <int HD> constexpr int kRowOffsets = HD % 128 == 0 ? 4 : HD % 64 == 0 ? 2 : 1;
 template <int HD = D>
-__device__ __forceinline__ void swizzled_offsets(int lane, int ro[4], int to[8]) {
+__device__ __forceinline__ void swizzled_offsets(int lane, int (&ro)[kRowOffsets<HD>], int (&to)[2 * kRowOffsets<HD>]) {
   const int g4 = lane >> 4, j16 = lane & 15;
 #pragma unroll
-  for (int ks = 0; ks < 4; ++ks) ro[ks] = j16 * HD + (((4 * ks + g4) ^ tile_swizzle(j16)) << 3);
+  for (int ks = 0; ks < kRowOffsets<HD>; ++ks) ro[ks] = j16 * HD + (((4 * ks + g4) ^ row_swizzle<HD>(j16)) << 3);
 #pragma unroll
-  for (int mb = 0; mb < 8; ++mb) {
+  for (int mb = 0; mb < 2 * kRowOffsets<HD>; ++mb) {
     const int r = 4 * g4 + (j16 >> 2);
     const int col = 16 * mb + 4 * (j16 & 3);
-    to[mb] = r * HD + (((col >> 3) ^ tile_swizzle(r)) << 3) + (col & 7);
+    to[mb] = r * HD + (((col >> 3) ^ row_swizzle<HD>(r)) << 3) + (col & 7);
   }
 }
 // the offsets of k-step ks and column block mb
-__device__ __forceinline__ int ro_of(const int ro[4], int ks) { return ro[ks & 3] + 128 * (ks >> 2); }
-__device__ __forceinline__ int to_of(const int to[8], int mb) { return to[mb & 7] + 128 * (mb >> 3); }
+template <int HD = D>
+__device__ __forceinline__ int ro_of(const int (&ro)[kRowOffsets<HD>], int ks) {
+  constexpr int N = kRowOffsets<HD>;
+  return ro[ks % N] + 32 * N * (ks / N);
+}
+template <int HD = D>
+__device__ __forceinline__ int to_of(const int (&to)[2 * kRowOffsets<HD>], int mb) {
+  constexpr int N = 2 * kRowOffsets<HD>;
+  return to[mb % N] + 16 * N * (mb / N);
+}
 
 
 // ---------------------------------------------------------------------------
@@ -524,10 +425,11 @@ inline int heads_per_block(int group) {
 // query rows per forward / dQ work item: 32 per query head of the work-group
 inline int q_block_rows(int group) { return 32 * 4 / heads_per_block(group); }
 
-// keys per dK/dV work-group: 48 for the one-wave-per-head kernel (GQA groups
-// that are a multiple of 4 below head dim 256: its 192 dK/dV accumulators and
-// 48 S/dP values fill the 256 AGPRs), else 64 (at head dim 256 the two waves
-// of 32 keys of dkdv256_kernel, every group)
+// keys per dK/dV work-group unless the caller chooses (48 and 64 both run): 48
+// at GQA groups that are a multiple of 4 below head dim 256 (at 128 the kernel
+// whose waves take steps of their own: its 192 dK/dV accumulators and 48 S/dP
+// values fill the 256 AGPRs), else 64 (at head dim 256 the two waves of 32 keys
+// of dkdv256_kernel, every group)
 inline int kv_block_keys(int group, int head_dim) { return group % 4 == 0 && head_dim != 256 ? 48 : BK; }
 
 // launchers (one per kernel family); each returns a TS_* status
