@@ -122,7 +122,9 @@ struct StreamerT {
   __device__ __forceinline__ void init(const bf16* b, int64_t ld_, int mvalid_, int K_, int wave, int lane) {
     base = b;
     ld = ld_;
-    mvalid = min(mvalid_, TM);
+    // whole chunks: the range check drops the 16 bytes (of a K row that ends the
+    // descriptor) that straddle its end; storage rows are padded to chunks
+    mvalid = min((mvalid_ + 7) & ~7, TM);
     K = K_;
 #pragma unroll
     for (int u = 0; u < kPerWave; ++u) {
