@@ -32,15 +32,17 @@ constexpr int kStageElems = (TM + TN) * TK;  // 32 KB: A [TM][TK], then B [TN][T
 // Full is the 256 x 256 tile.  Narrow<NI> takes 64 NI B rows (64, 128 or 192), for
 // launches of few B rows, which in Full tiles would do their MFMAs on zeros.  Its
 // waves are 64 x 32 NI blocks, (2 + NI) / 2 NI LDS fragment reads per MFMA against
-// 3 / 4.
+// 3 / 4.  Wide takes 320 in the same way (7 / 10; its four stages fill 144 KB of
+// LDS and its 160 accumulators with two stages' fragments 246 of 256 VGPRs).
 template <int WM_, int WN_, int MI_, int NI_>
 struct Shape {
   static constexpr int WM = WM_, WN = WN_, MI = MI_, NI = NI_;
   static constexpr int BN = 32 * WN_ * NI_;  // B rows of the tile
-  static_assert(WM_ * WN_ == kWaves && 32 * WM_ * MI_ == TM && BN <= TN, "eight waves over 256 A rows");
+  static_assert(WM_ * WN_ == kWaves && 32 * WM_ * MI_ == TM && BN <= 320, "eight waves over 256 A rows");
 };
 using Full = Shape<2, 4, 4, 2>;
 template <int NI_> using Narrow = Shape<4, 2, 2, NI_>;
+using Wide = Narrow<5>;
 constexpr int NI = Full::NI;
 
 __device__ __forceinline__ u32x4 ld16(const bf16* p) { return *reinterpret_cast<const u32x4*>(p); }
@@ -382,11 +384,15 @@ __device__ __forceinline__ void gemm_tile(f32x16 (&acc)[S::MI][S::NI], const bf1
 // that a quarter of a staged output tile fits one stage), reused by the
 // epilogues
 constexpr int kRingElems = kStageElems + 1024;
-#define GEMM_RING                                                    \
-  __shared__ __attribute__((aligned(16))) bf16 s0[kRingElems];     \
-  __shared__ __attribute__((aligned(16))) bf16 s1[kRingElems];     \
-  __shared__ __attribute__((aligned(16))) bf16 s2[kRingElems];     \
-  __shared__ __attribute__((aligned(16))) bf16 s3[kRingElems];
+template <class S> constexpr int ring_elems() {
+  return (TM + S::BN) * TK > kRingElems ? (TM + S::BN) * TK : kRingElems;
+}
+#define GEMM_RING_OF(S)                                                   \
+  __shared__ __attribute__((aligned(16))) bf16 s0[gemm::ring_elems<S>()]; \
+  __shared__ __attribute__((aligned(16))) bf16 s1[gemm::ring_elems<S>()]; \
+  __shared__ __attribute__((aligned(16))) bf16 s2[gemm::ring_elems<S>()]; \
+  __shared__ __attribute__((aligned(16))) bf16 s3[gemm::ring_elems<S>()];
+#define GEMM_RING GEMM_RING_OF(Full)
 
 }  // namespace gemm
 }  // namespace ts

@@ -80,16 +80,35 @@ struct FwdArgs {
 // where it is much narrower: 64 or 128 tokens (4096 x 151936: 25 rows forward 279
 // -> 264, dlogits 307 -> 269, grad_hidden 201 -> 188 us, 128 rows 307 -> 288, 337 ->
 // 295, 235 -> 223), and for grad_hidden, whose launch of few rows is one round that
-// ends with its widest tiles, 192 for up to 160 (281 rows 469 -> 427, 320 rows 463 ->
-// 409; at 192 rows a tile 464 -> 478, and forward and dlogits gain nothing).
+// ends with its widest tiles, 192 for up to 160 (320 rows 463 -> 409; at 192 rows a
+// tile 464 -> 478, and forward and dlogits gain nothing).
 inline int token_tile(int64_t rows, bool up_to_192) {
   const int64_t tiles = (rows + TN - 1) / TN, each = (rows + tiles - 1) / tiles;
   return each <= 64 ? 64 : each <= 128 ? 128 : up_to_192 && each <= 160 ? 192 : 256;
 }
 
+// The 320-token tile (Wide) reads a weight tile once for rows that need two or
+// more 256-token ones, in kWideCost / 256 of a 256-token tile's time (by its MFMAs
+// 320 / 256; set to what the launches below take).  `stride`: the token
+// operand's, for the 32-bit offsets of its rows within a tile.
+constexpr int kWideTokens = Wide::BN;
+constexpr int kWideCost = 352;
+inline bool wide_fits(int64_t rows, int64_t stride) { return rows > TN && (kWideTokens - 1) * stride < (1ll << 30); }
+
+// Forward and dlogits: 320 where the launch then takes less time in rounds of one
+// work-group per CU: 1 tile for 2 at 257 .. 320 rows of 594 vocabulary tiles (3
+// rounds for 5: 281 rows forward 488 -> 434 us, dlogits 500 -> 450), 2 for 3 at 600 (5
+// for 7: 755 -> 698, 778 -> 723), but not at 384 (5 for 5: 520 -> 651) or 2048 (17 for
+// 19: 2157 -> 2286).
+inline int logits_tile(int64_t rows, int64_t vtiles, int64_t stride) {
+  auto rounds = [&](int64_t w) { return ((rows + w - 1) / w * vtiles + 255) / 256; };
+  if (wide_fits(rows, stride) && rounds(kWideTokens) * kWideCost < rounds(TN) * TN) return kWideTokens;
+  return token_tile(rows, false);
+}
+
 template <typename E, class S>
 __global__ __launch_bounds__(kGemmThreads, 1) void fwd_stats_kernel(FwdArgs p) {
-  GEMM_RING
+  GEMM_RING_OF(S)
   constexpr int MI = S::MI, NI = S::NI;
   const int total = p.n_ttiles * p.n_vtiles;
   int vt, tt;
@@ -282,7 +301,7 @@ static_assert(64 * OPITCH <= kRingElems, "a quarter of the dlogits tile fits one
 // comparison masks (dlogits 2.15 -> 2.06 ms per 2048 rows x 4096 x 151936).
 template <typename E, class S>
 __global__ __launch_bounds__(kGemmThreads, 1) void dlogits_kernel(DlArgs p) {
-  GEMM_RING
+  GEMM_RING_OF(S)
   constexpr int MI = S::MI, NI = S::NI;
   const int total = p.n_ttiles * p.n_vtiles;
   int vt, tt;
@@ -293,15 +312,19 @@ __global__ __launch_bounds__(kGemmThreads, 1) void dlogits_kernel(DlArgs p) {
                           p.h + (int64_t)n0 * p.ldh, p.ldh, min(S::BN, p.rows - n0), p.dim, s0, s1, s2, s3);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave % S::WM, wn = wave / S::WM;
-  // tokens 64 q .. 64 q + 63 of the tile are staged in ring stage q as [64][OPITCH]
+  // tokens 64 q .. 64 q + 63 of the tile are staged in ring stage q as [64][OPITCH];
+  // a Wide tile does not fit, its waves' two halves of the tokens take turns
+  constexpr int PASSES = S::BN > TN ? S::WN : 1, PT = S::BN / PASSES;  // tokens per pass
+  static_assert(PT <= 256, "four stages of 64 tokens");
   auto quarter = [&](int q) -> bf16* { return q == 0 ? s0 : q == 1 ? s1 : q == 2 ? s2 : s3; };
   // dl = -p (g_lp + g_H (log p + H)) + g_lp [v = t], with log2 p = l log2 e - lse log2 e as one
   // FMA and the bracket as one FMA in log2 p: A = g_H ln 2, B = g_lp + g_H H per token.  Tiles
-  // inside the vocabulary and the row range (all but the last of each) skip the bounds tests.
-  auto column = [&](int ni, auto full_c, auto hot_c, float lse2, float coef_a, float coef_b, float glp, int hot,
-                    bool in_rows) __attribute__((always_inline)) {
+  // inside the vocabulary (all but the last) skip the bounds test; columns past the rows take
+  // the last row's values and are not stored.
+  auto column = [&](int ni, auto full_c, auto hot_c, float lse2, float coef_a, float coef_b, float glp, int hot)
+                    __attribute__((always_inline)) {
     constexpr bool FULL = decltype(full_c)::value, HOT = decltype(hot_c)::value;
-    const int col = b_row<S>(ni, lane, wn);  // token within the tile
+    const int col = b_row<S>(ni, lane, PASSES > 1 ? 0 : wn);  // token within the pass
     bf16* out = quarter(col >> 6) + (col & 63) * OPITCH;
 #pragma unroll
     for (int mi = 0; mi < MI; ++mi)
@@ -314,7 +337,7 @@ __global__ __launch_bounds__(kGemmThreads, 1) void dlogits_kernel(DlArgs p) {
           const float logp2 = fmaf(acc[mi][ni][i], kLog2e, -lse2);
           d[j] = -fast_exp2(logp2) * fmaf(coef_a, logp2, coef_b);
           if (HOT && a_row<S>(mi, i, lane, wm) == hot) d[j] += glp;
-          if (!FULL && !(v0 + a_row<S>(mi, i, lane, wm) < p.vocab && in_rows)) d[j] = 0.f;
+          if (!FULL && v0 + a_row<S>(mi, i, lane, wm) >= p.vocab) d[j] = 0.f;
         }
         // vocab rows a_row(mi, 4 i4 .. 4 i4 + 3) are consecutive: one 8-byte write
         *reinterpret_cast<u32x2*>(out + a_row<S>(mi, 4 * i4, lane, wm)) =
@@ -322,45 +345,57 @@ __global__ __launch_bounds__(kGemmThreads, 1) void dlogits_kernel(DlArgs p) {
       }
   };
   auto epilogue = [&](auto full_c) __attribute__((always_inline)) {
-    constexpr bool FULL = decltype(full_c)::value;
 #pragma unroll
     for (int ni = 0; ni < NI; ++ni) {
-      const int n = n0 + b_row<S>(ni, lane, wn);
-      float lse2 = 0.f, coef_a = 0.f, coef_b = 0.f, glp = 0.f;
-      int hot = -1;  // the token's target as a row of the tile (out-of-range targets match none)
-      const bool in_rows = FULL || n < p.rows;
-      if (in_rows) {
-        lse2 = p.lse[n] * kLog2e;
-        glp = p.g_lp[n];
-        coef_b = glp;
-        if (p.g_ent) {
-          const float gent = p.g_ent[n];
-          coef_a = gent * kLn2;
-          coef_b = fmaf(gent, p.ent[n], glp);
-        }
-        const int64_t t = p.target[n];
-        if (t >= v0 && t < min(v0 + TM, p.vocab)) hot = (int)(t - v0);
+      const int n = min(n0 + b_row<S>(ni, lane, wn), p.rows - 1);
+      const float lse2 = p.lse[n] * kLog2e, glp = p.g_lp[n];
+      float coef_a = 0.f, coef_b = glp;
+      if (p.g_ent) {
+        const float gent = p.g_ent[n];
+        coef_a = gent * kLn2;
+        coef_b = fmaf(gent, p.ent[n], glp);
       }
+      const int64_t t = p.target[n];
+      // the token's target as a row of the tile (out-of-range targets match none)
+      const int hot = t >= v0 && t < min(v0 + TM, p.vocab) ? (int)(t - v0) : -1;
       const int mine = hot - 32 * MI * wm;
       if (__builtin_amdgcn_ballot_w64(mine >= 0 && mine < 32 * MI) != 0)
-        column(ni, full_c, std::true_type{}, lse2, coef_a, coef_b, glp, hot, in_rows);
+        column(ni, full_c, std::true_type{}, lse2, coef_a, coef_b, glp, hot);
       else
-        column(ni, full_c, std::false_type{}, lse2, coef_a, coef_b, glp, hot, in_rows);
+        column(ni, full_c, std::false_type{}, lse2, coef_a, coef_b, glp, hot);
+      if constexpr (PASSES > 1) __builtin_amdgcn_sched_barrier(0);
     }
   };
-  if (v0 + TM <= p.vocab && n0 + S::BN <= p.rows) epilogue(std::true_type{});
-  else epilogue(std::false_type{});
-  __syncthreads();
-  // coalesced store of the [BN tokens][TM vocab] tile
   const int vmax = min(TM, p.vocab_pad - v0);
+  // coalesced store of the pass's [PT tokens][TM vocab]
+  auto store = [&](int pass) __attribute__((always_inline)) {
 #pragma unroll 4
-  for (int it = 0; it < (S::BN * TM / 8) / kGemmThreads; ++it) {
-    const int c = it * kGemmThreads + tid;
-    const int row = c / (TM / 8), chunk = (c % (TM / 8)) * 8;
-    const int n = n0 + row;
-    if (n < p.rows && chunk < vmax)
-      *reinterpret_cast<u32x4*>(p.dl + (int64_t)n * p.ldl + v0 + chunk) =
-          *reinterpret_cast<const u32x4*>(quarter(row >> 6) + (row & 63) * OPITCH + chunk);
+    for (int it = 0; it < (PT * TM / 8) / kGemmThreads; ++it) {
+      const int c = it * kGemmThreads + tid;
+      const int row = c / (TM / 8), chunk = (c % (TM / 8)) * 8;
+      const int n = n0 + pass * PT + row;
+      if (n < p.rows && chunk < vmax)
+        *reinterpret_cast<u32x4*>(p.dl + (int64_t)n * p.ldl + v0 + chunk) =
+            *reinterpret_cast<const u32x4*>(quarter(row >> 6) + (row & 63) * OPITCH + chunk);
+    }
+  };
+  auto values = [&]() __attribute__((always_inline)) {
+    if (v0 + TM <= p.vocab) epilogue(std::true_type{});
+    else epilogue(std::false_type{});
+  };
+  if constexpr (PASSES == 1) {
+    values();
+    __syncthreads();
+    store(0);
+  } else {
+    static_assert(PASSES <= 2, "two halves");
+    if (wn == 0) values();
+    __syncthreads();
+    store(0);
+    __syncthreads();
+    if (wn == 1) values();
+    __syncthreads();
+    store(1);
   }
 }
 
@@ -385,7 +420,7 @@ struct DhArgs {
 
 template <typename E, class S>
 __global__ __launch_bounds__(kGemmThreads, 1) void grad_hidden_kernel(DhArgs p) {
-  GEMM_RING
+  GEMM_RING_OF(S)
   constexpr int MI = S::MI, NI = S::NI;
   const int tiles = p.n_ttiles * p.n_dtiles;
   const int id = xcd_logical(blockIdx.x, tiles * p.ksplit);
@@ -513,16 +548,30 @@ __global__ __launch_bounds__(kGemmThreads, 1) void grad_weight_kernel(DwArgs p) 
 // launch within one round of 256 work-groups (one per CU) when the row tiles
 // alone do not fill it -- a second, partial round would cost a whole range's
 // time (80 tiles: three ranges of a third, not four of a quarter in two
-// rounds) -- each range at least 4096 vocabulary rows
-inline void grad_hidden_split(int64_t rows, int64_t dim, int64_t vocab, int& ksplit, int& kper) {
-  const int64_t tiles = ((rows + TN - 1) / TN) * ((dim + TM - 1) / TM);
-  int64_t k = 256 / tiles;
-  k = std::min<int64_t>(k, std::max<int64_t>(1, vocab / 4096));
-  k = std::max<int64_t>(1, std::min<int64_t>(k, 16));
+// rounds) -- each range at least 4096 vocabulary rows.  `width`: token rows per
+// tile, 320 where the launch of its tiles and ranges takes less time
+// (4096 x 151936: 281 rows 437 -> 351 us, 600 728 -> 618).  Returns the number of token tiles.
+inline int grad_hidden_split(int64_t rows, int64_t dim, int64_t vocab, int64_t stride, int& width, int& ksplit,
+                             int& kper) {
+  const int64_t dtiles = (dim + TM - 1) / TM;
+  auto ranges = [&](int64_t w) {
+    int64_t k = 256 / ((rows + w - 1) / w * dtiles);
+    k = std::min<int64_t>(k, std::max<int64_t>(1, vocab / 4096));
+    return std::max<int64_t>(1, std::min<int64_t>(k, 16));
+  };
+  // time of a launch: rounds x tile width / ranges
+  auto time = [&](int64_t w, int cost) {
+    const int64_t k = ranges(w), groups = (rows + w - 1) / w * dtiles * k;
+    return (double)((groups + 255) / 256 * cost) / (double)k;
+  };
+  width = token_tile(rows, true);
+  if (wide_fits(rows, stride) && time(kWideTokens, kWideCost) < time(width, width)) width = kWideTokens;
+  const int64_t k = ranges(width);
   int64_t per = (vocab + k - 1) / k;
   per = (per + TK - 1) / TK * TK;
   ksplit = (int)((vocab + per - 1) / per);
   kper = (int)per;
+  return (int)((rows + width - 1) / width);
 }
 
 // launch kernel<element, tile shape> by a DType code and token_tile's width
@@ -530,6 +579,7 @@ inline void grad_hidden_split(int64_t rows, int64_t dim, int64_t vocab, int& ksp
   do {                                                                            \
     if ((width) == 64) TS_LAUNCH_E_T(dtype, kernel, Narrow<1>, __VA_ARGS__);      \
     else if ((width) == 128) TS_LAUNCH_E_T(dtype, kernel, Narrow<2>, __VA_ARGS__); \
+    else if ((width) == kWideTokens) TS_LAUNCH_E_T(dtype, kernel, Wide, __VA_ARGS__); \
     else TS_LAUNCH_E_T(dtype, kernel, Full, __VA_ARGS__);                         \
   } while (0)
 
@@ -575,15 +625,16 @@ int ts_logprob_fwd(const void* hidden, int64_t ld_hidden, const void* weight, in
   a.rows = (int)rows;
   a.dim = (int)dim;
   a.vocab = (int)vocab;
-  a.n_ttiles = (int)((rows + TN - 1) / TN);
   a.n_vtiles = (int)((vocab + BM - 1) / BM);
+  const int width = logits_tile(rows, a.n_vtiles, ld_hidden);
+  a.n_ttiles = (int)((rows + width - 1) / width);
   float* ws = (float*)workspace;
   a.part_m = ws;
   a.part_s = ws + (int64_t)a.n_vtiles * rows;
   a.part_e = ws + 2 * (int64_t)a.n_vtiles * rows;
   TS_CHECK_ARG((int64_t)a.n_ttiles * a.n_vtiles < (1ll << 31), "ts_logprob_fwd: grid too large");
   hipStream_t s = (hipStream_t)stream;
-  { ts::TimedLaunch timed_("logprob.fwd_stats_kernel", s); TS_LAUNCH_TOKENS(dtype, token_tile(rows, false), fwd_stats_kernel, dim3((unsigned)(a.n_ttiles * a.n_vtiles)), dim3(kGemmThreads),
+  { ts::TimedLaunch timed_("logprob.fwd_stats_kernel", s); TS_LAUNCH_TOKENS(dtype, width, fwd_stats_kernel, dim3((unsigned)(a.n_ttiles * a.n_vtiles)), dim3(kGemmThreads),
                      0, s, a); }
   int st = ts::check_launch("ts_logprob_fwd (tiles)");
   if (st != TS_OK) return st;
@@ -628,20 +679,21 @@ int ts_logprob_dlogits(const void* hidden, int64_t ld_hidden, const void* weight
   a.dim = (int)dim;
   a.vocab = (int)vocab;
   a.vocab_pad = (int)((vocab + 7) / 8 * 8);
-  a.n_ttiles = (int)((rows + TN - 1) / TN);
   a.n_vtiles = (int)((a.vocab_pad + BM - 1) / BM);
+  const int width = logits_tile(rows, a.n_vtiles, ld_hidden);
+  a.n_ttiles = (int)((rows + width - 1) / width);
   a.dl = (ts::bf16*)dlogits;
   a.ldl = ld_dlogits;
   TS_CHECK_ARG(a.vocab_pad <= ld_dlogits, "ts_logprob_dlogits: ld_dlogits below padded vocab");
-  { ts::TimedLaunch timed_("logprob.dlogits_kernel", (hipStream_t)stream); TS_LAUNCH_TOKENS(dtype, token_tile(rows, false), dlogits_kernel, dim3((unsigned)(a.n_ttiles * a.n_vtiles)), dim3(kGemmThreads),
+  { ts::TimedLaunch timed_("logprob.dlogits_kernel", (hipStream_t)stream); TS_LAUNCH_TOKENS(dtype, width, dlogits_kernel, dim3((unsigned)(a.n_ttiles * a.n_vtiles)), dim3(kGemmThreads),
                      0, (hipStream_t)stream, a); }
   return ts::check_launch("ts_logprob_dlogits");
 }
 
 int64_t ts_logprob_grad_hidden_workspace(int64_t rows, int64_t dim, int64_t vocab) {
   if (rows <= 0 || dim <= 0 || vocab <= 0) return 0;
-  int ksplit, kper;
-  ts::lp::grad_hidden_split(rows, dim, vocab, ksplit, kper);
+  int width, ksplit, kper;
+  ts::lp::grad_hidden_split(rows, dim, vocab, vocab, width, ksplit, kper);
   return ksplit > 1 ? (int64_t)ksplit * rows * dim * (int64_t)sizeof(float) : 0;
 }
 
@@ -672,9 +724,9 @@ int grad_hidden_launch(const void* dlogits, int64_t ld_dlogits, const void* weig
   a.rows = (int)rows;
   a.dim = (int)dim;
   a.vocab = (int)vocab;
-  a.n_ttiles = (int)((rows + TN - 1) / TN);
   a.n_dtiles = (int)((dim + TM - 1) / TM);
-  grad_hidden_split(rows, dim, vocab, a.ksplit, a.kper);
+  int width;
+  a.n_ttiles = grad_hidden_split(rows, dim, vocab, ld_dlogits, width, a.ksplit, a.kper);
   a.dh = (ts::bf16*)grad_hidden;
   a.ldd = ld_grad;
   a.part = (float*)workspace;
@@ -686,7 +738,6 @@ int grad_hidden_launch(const void* dlogits, int64_t ld_dlogits, const void* weig
   hipStream_t s = (hipStream_t)stream;
   {
     ts::TimedLaunch timed_(label, s);
-    const int width = token_tile(rows, true);
     const dim3 grid((unsigned)(a.n_ttiles * a.n_dtiles * a.ksplit));
     if (width == 192) TS_LAUNCH_E_T(dtype, grad_hidden_kernel, Narrow<3>, grid, dim3(kGemmThreads), 0, s, a);
     else TS_LAUNCH_TOKENS(dtype, width, grad_hidden_kernel, grid, dim3(kGemmThreads), 0, s, a);
