@@ -1,8 +1,7 @@
-"""RMSNorm kernels by vectors per lane and by size of the output.
+"""RMSNorm kernels by vectors per lane.
 
 The forward is built for 12, 20 and 24 vectors a lane beside the powers of two,
-and stores outputs of 128 MiB and more past the caches; the backward for 10 and
-12 vectors.  Each is met full, with its last vector part empty and with one
+the backward for 10 and 12.  Each is met full, with its last vector part empty and with one
 vector more than the variant below it.
 """
 
@@ -19,7 +18,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("rows,width", [
     (1025, 2308), (1025, 3072), (1025, 4100), (1025, 5120), (1025, 5124), (1025, 6144), (1025, 6148),
-    (16383, 4096), (16387, 4096)])  # bf16: one row below 128 MiB, three past it
+    (16387, 4096)])
 def test_forward_bytes(cuda, rows, width, dtype):
     print(f"rmsnorm fwd rows={rows} width={width} {dtype}", flush=True)
     g = torch.Generator(device=cuda).manual_seed(rows + width)

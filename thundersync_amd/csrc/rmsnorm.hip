@@ -221,14 +221,6 @@ template <> __device__ __forceinline__ void store4<float>(float* p, const float 
   *reinterpret_cast<f32x4*>(p) = f32x4{o[0], o[1], o[2], o[3]};
 }
 
-// store4 with the non-temporal hint
-template <typename T> __device__ __forceinline__ void store4_once(T* p, const float (&o)[4]) {
-  if constexpr (sizeof(T) == 2)
-    __builtin_nontemporal_store((u32x2{pack2<T>(o[0], o[1]), pack2<T>(o[2], o[3])}), reinterpret_cast<u32x2*>(p));
-  else
-    __builtin_nontemporal_store((f32x4{o[0], o[1], o[2], o[3]}), reinterpret_cast<f32x4*>(p));
-}
-
 // y = w * T(x * r): the product rounded to fp32, then to T, then w * that
 // rounded to T, as the module's operations.  The fp32 product is hidden from
 // the optimiser: for fp16 it otherwise folds T(x * r) into one
@@ -248,12 +240,12 @@ template <typename T> __device__ __forceinline__ float primal(float w, float x, 
 //       bounds their number.  Otherwise (width < 128) the lane sums elements
 //       sub and sub + bw, the only ones its loop reaches.
 // Bound by HBM.  The weight's vectors are loaded beside the row's, so that the
-// stores wait for the reduction alone, and an output that no cache can hold
-// (STREAM, kStreamBytes) is stored without displacing the lines the loads
-// bring in.  bf16 from cold caches, us: 16384 x 4096 62 plain, 55.6 with the weight
-// loads, 51.6 with the stores too (5.2 TB/s); 8192 x 5120 43.5, 40.5 with the weight
-// loads, 33.5 with 20 vectors instead of 32.
-template <typename T, bool VEC, int NV, bool STREAM>
+// stores wait for the reduction alone.  bf16 from cold caches, us: 16384 x 4096 62
+// -> 55.6 (4.8 TB/s), 8192 x 5120 43.5 -> 40.5 and 33.5 with 20 vectors instead of 32.
+// Non-temporal stores make that first launch 51.7 us in a stream of others, but a
+// pass by itself, forward and backward, 13 us longer (140 -> 153): the last-level
+// cache then takes no part of the output, which the next kernel would find there.
+template <typename T, bool VEC, int NV>
 __global__ __launch_bounds__(kThreads) void rmsnorm_fwd_lanes(
     const T* __restrict__ x, const T* __restrict__ w, T* __restrict__ y,
     float* __restrict__ rstd, int64_t rows, int width, int bw, float factor, float eps) {
@@ -298,8 +290,7 @@ __global__ __launch_bounds__(kThreads) void rmsnorm_fwd_lanes(
         unpack4<T>(wr[k], wv);
 #pragma unroll
         for (int i = 0; i < 4; ++i) o[i] = primal<T>(wv[i], f[i], r);
-        if constexpr (STREAM) store4_once<T>(yr + vi * 4, o);
-        else store4<T>(yr + vi * 4, o);
+        store4<T>(yr + vi * 4, o);
       }
     }
   } else {
@@ -683,12 +674,6 @@ int stream_cus(hipStream_t s) {
   return n;
 }
 
-// input and output together fill the Infinity Cache's 256 MB.  Below that the next
-// kernel finds part of the output there, and so does this one its own lines: 8192 x
-// 5120 (84 MB) 33.5 us stored plainly and 35.7 streamed, 8192 x 6144 (101 MB) 41.6
-// and 43.4; 16384 x 4096 (134 MB) 55.6 and 51.7, 32768 x 4096 118 -> 102.
-constexpr int64_t kStreamBytes = 128ll << 20;
-
 template <typename T>
 int launch_fwd(const void* x, const void* w, void* y, float* rstd, int64_t rows, int width,
                float eps, hipStream_t s) {
@@ -705,21 +690,16 @@ int launch_fwd(const void* x, const void* w, void* y, float* rstd, int64_t rows,
     const dim3 grid((unsigned)((rows + rows_per_block - 1) / rows_per_block));
     ts::TimedLaunch timed_("rmsnorm.rmsnorm_fwd_lanes", s);
     if (!c.vec) {
-      hipLaunchKernelGGL((rmsnorm_fwd_lanes<T, false, 1, false>), grid, dim3(kThreads), 0, s, (const T*)x,
+      hipLaunchKernelGGL((rmsnorm_fwd_lanes<T, false, 1>), grid, dim3(kThreads), 0, s, (const T*)x,
                          (const T*)w, (T*)y, rstd, rows, width, c.bw, factor, eps);
       return check_launch("ts_rmsnorm_fwd");
     }
     const int loads = (width / 4 + c.bw - 1) / c.bw;
-    const bool stream = rows * (int64_t)width * (int64_t)sizeof(T) >= kStreamBytes;
-#define TS_FWD(NV)                                                                               \
-  if (loads <= NV) {                                                                             \
-    if (stream)                                                                                  \
-      hipLaunchKernelGGL((rmsnorm_fwd_lanes<T, true, NV, true>), grid, dim3(kThreads), 0, s,     \
-                         (const T*)x, (const T*)w, (T*)y, rstd, rows, width, c.bw, factor, eps); \
-    else                                                                                         \
-      hipLaunchKernelGGL((rmsnorm_fwd_lanes<T, true, NV, false>), grid, dim3(kThreads), 0, s,    \
-                         (const T*)x, (const T*)w, (T*)y, rstd, rows, width, c.bw, factor, eps); \
-    return check_launch("ts_rmsnorm_fwd");                                                       \
+#define TS_FWD(NV)                                                                             \
+  if (loads <= NV) {                                                                           \
+    hipLaunchKernelGGL((rmsnorm_fwd_lanes<T, true, NV>), grid, dim3(kThreads), 0, s,           \
+                       (const T*)x, (const T*)w, (T*)y, rstd, rows, width, c.bw, factor, eps); \
+    return check_launch("ts_rmsnorm_fwd");                                                     \
   }
     TS_FWD(1) TS_FWD(2) TS_FWD(4) TS_FWD(8) TS_FWD(12) TS_FWD(16) TS_FWD(20) TS_FWD(24) TS_FWD(32)
 #undef TS_FWD
