@@ -22,12 +22,14 @@ namespace attn {
 // the rows' (lse * log2 e, delta) pairs.  The segment's key runs stream
 // through 64-key K/V tiles that all waves share: double-buffered LDS stages
 // filled by buffer_load ... lds (each wave issues its share of a tile's
-// instructions; rows past a run's end arrive as zeros and add nothing,
-// because a zero K row contributes zero to dQ), one work-group barrier per
-// tile.  Tiles use the dK/dV kernel's swizzled rows
+// instructions; rows past a run's end arrive as zeros), one work-group barrier
+// per tile.  Tiles use the dK/dV kernel's swizzled rows
 // with chunk c of row r at slot c ^ row_swizzle(r & 15): K and V rows feed S^T = K Q^T
 // and dP^T = V dO^T as A operands, K^T for dQ^T += K^T dS^T comes from
-// ds_read_b64_tr_b16.  Only tiles that cross the diagonal are masked.  Against
+// ds_read_b64_tr_b16.  Tiles that cross the diagonal or end a run are masked: a
+// key past a run's end has S = 0, so its P = exp2(-lse2) grows without bound where
+// the row's scores are low (dS past the element type's range, times its zero K
+// row: NaN).  Against
 // tiles passed through registers between two barriers (8 sequences of 512 to 2048
 // rows, us): head dim 64 at 16/8 heads 115 -> 71, 32 75 -> 48, 96 143 -> 98, 192 at
 // 24/4 647 -> 387.
@@ -128,19 +130,19 @@ __global__ __launch_bounds__(64 * 8 / (NQB * NP), 1) void dq_wave_kernel(ts_attn
   };
   // dS^T = P^T (dP^T - delta) (dp holds dP^T - delta), P^T = exp2(S^T c - lse2), packed as the B
   // operand of dQ^T += K^T dS^T (slot j <-> key 32 ss + 16 (j >> 2) + 4 g4 +
-  // (j & 3)); DIAG masks keys past each row's diagonal
-  auto dscores = [&](auto diag, int kpos, int kt0, int ss, f32x4 (&sc)[2][NQB], const f32x4 (&dp)[2][NQB],
-                     bf16x8 (&dsk)[NQB]) __attribute__((always_inline)) {
+  // (j & 3)); `masked`: keys past each row's diagonal or past the run's end get P = 0
+  auto dscores = [&](auto masked, int kpos, int kt0, int run_len, int ss, f32x4 (&sc)[2][NQB],
+                     const f32x4 (&dp)[2][NQB], bf16x8 (&dsk)[NQB]) __attribute__((always_inline)) {
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
       for (int qb = 0; qb < NQB; ++qb) {
-        // row qw + 16 qb + j16 sees key kt0 + 32 ss + 16 kb + 4 g4 + i iff i <= lim
-        const int lim = off + qw + 16 * qb + j16 - kpos - kt0 - 32 * ss - 16 * kb - 4 * g4;
+        // row qw + 16 qb + j16 sees key kt0 + 32 ss + 16 kb + 4 g4 + i of the run iff i <= lim
+        const int lim = min(off + qw + 16 * qb + j16 - kpos, run_len - 1) - kt0 - 32 * ss - 16 * kb - 4 * g4;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           float p = fast_exp2(sc[kb][qb][i] * c - lse2[qb]);
-          if (decltype(diag)::value) p = i <= lim ? p : 0.f;
+          if (decltype(masked)::value) p = i <= lim ? p : 0.f;
           sc[kb][qb][i] = p * dp[kb][qb][i];
         }
       }
@@ -164,7 +166,8 @@ __global__ __launch_bounds__(64 * 8 / (NQB * NP), 1) void dq_wave_kernel(ts_attn
   };
   // one tile, the halves software-pipelined: half 1's score MFMAs are issued
   // beside half 0's exponentials, half 0's dQ MFMAs beside half 1's
-  auto tile_body = [&](auto diag, const bf16* tk, const bf16* tv, int kpos, int kt0) __attribute__((always_inline)) {
+  auto tile_body = [&](auto masked, const bf16* tk, const bf16* tv, int kpos, int kt0, int run_len)
+      __attribute__((always_inline)) {
     if constexpr (HD > 128 && kWaves == 8) {
       // at head dim 256 with two waves per SIMD the halves run one after the
       // other: the pipelined form's two halves of S and dP do not fit the
@@ -182,7 +185,7 @@ __global__ __launch_bounds__(64 * 8 / (NQB * NP), 1) void dq_wave_kernel(ts_attn
           if (i + 2 < 2 * NKS) __builtin_amdgcn_sched_group_barrier(0x100, 2, 3);
         }
         __builtin_amdgcn_sched_barrier(0);
-        dscores(diag, kpos, kt0, ss, sc, dp, dsk);
+        dscores(masked, kpos, kt0, run_len, ss, sc, dp, dsk);
         accumulate(tk, ss, dsk);
         // K^T fragment reads kept four blocks ahead of their MFMAs
         __builtin_amdgcn_sched_group_barrier(0x100, 8, 4);
@@ -200,7 +203,7 @@ __global__ __launch_bounds__(64 * 8 / (NQB * NP), 1) void dq_wave_kernel(ts_attn
     scores(tk, tv, 0, sc0, dp0);
     __builtin_amdgcn_sched_barrier(0);
     scores(tk, tv, 1, sc1, dp1);
-    dscores(diag, kpos, kt0, 0, sc0, dp0, dsk0);
+    dscores(masked, kpos, kt0, run_len, 0, sc0, dp0, dsk0);
     // 4 NKS K/V reads and 4 NKS NQB MFMAs of half 1 beside ~40 NQB VALU instructions
     constexpr int v1 = (NQB == 2 ? 5 : 3) * 4 / NKS > 0 ? (NQB == 2 ? 5 : 3) * 4 / NKS : 1;
     constexpr int v2 = (NQB == 2 ? 4 : 3) * 4 / NKS > 0 ? (NQB == 2 ? 4 : 3) * 4 / NKS : 1;
@@ -217,7 +220,7 @@ __global__ __launch_bounds__(64 * 8 / (NQB * NP), 1) void dq_wave_kernel(ts_attn
       __builtin_amdgcn_sched_group_barrier(0x002, v2, 0);
     }
     __builtin_amdgcn_sched_barrier(0);
-    dscores(diag, kpos, kt0, 1, sc1, dp1, dsk1);
+    dscores(masked, kpos, kt0, run_len, 1, sc1, dp1, dsk1);
     accumulate(tk, 0, dsk0);
     constexpr int v3 = (NQB == 2 ? 4 : 5) * 8 / NMB > 0 ? (NQB == 2 ? 4 : 5) * 8 / NMB : 1;
     __builtin_amdgcn_sched_group_barrier(0x100, 8, 1);  // K^T reads for dQ of half 0
@@ -246,7 +249,7 @@ __global__ __launch_bounds__(64 * 8 / (NQB * NP), 1) void dq_wave_kernel(ts_attn
 
   auto step = [&](auto bsel, TileCursor& cur) {
     const int kpos = cur.kpos;
-    const int kt0 = cur.kt0;
+    const int kt0 = cur.kt0, run_len = cur.len;
     const TileCursor nxt = next_kv_tile(P, seg, hk, visible_end(seg, last), cur);
     __builtin_amdgcn_s_waitcnt(0);  // this wave's part of the tile has landed
     __syncthreads();                // every part has, and the other stage is free
@@ -255,10 +258,10 @@ __global__ __launch_bounds__(64 * 8 / (NQB * NP), 1) void dq_wave_kernel(ts_attn
     if (nxt.sp < seg.nspan)
       issue_kv_tile<kWaves, HD>(wave, lane, nxt, bsel.value == 0 ? s_k1 : s_k0, bsel.value == 0 ? s_v1 : s_v0);
 
-    if (kpos + kt0 + BK - 1 > off + qw)
-      tile_body(std::true_type{}, tk, tv, kpos, kt0);
+    if ((kpos + kt0 + BK - 1 > off + qw) | (kt0 + BK > run_len))
+      tile_body(std::true_type{}, tk, tv, kpos, kt0, run_len);
     else
-      tile_body(std::false_type{}, tk, tv, kpos, kt0);
+      tile_body(std::false_type{}, tk, tv, kpos, kt0, run_len);
     cur = nxt;
   };
 
