@@ -183,9 +183,10 @@ __global__ __launch_bounds__(64 * 8 / NQB, (fwd_occupancy<NQB, HD, KT>())) void 
           const bool move = mt > m[qb] + kRescaleSlack;
           if (__builtin_amdgcn_ballot_w64(move) != 0) {
             const float mnew = move ? mt : m[qb];
-            // 0 on the first visible keys (m = -inf); a part can hold rows that
-            // see none of its keys so far beside rows that do
-            const float alpha = SPLIT && !move ? 1.f : fast_exp2(m[qb] - mnew);
+            // 0 on the first finite score (m = -inf); a row whose scores so far are
+            // all -inf (or, in a part, none of whose keys it sees) stays as it is beside
+            // rows that move
+            const float alpha = move ? fast_exp2(m[qb] - mnew) : 1.f;
             l[qb] *= alpha;
 #pragma unroll
             for (int mb = 0; mb < NMB; ++mb) acc[mb][qb] *= alpha;
