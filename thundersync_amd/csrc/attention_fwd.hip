@@ -18,19 +18,27 @@ namespace attn {
 // VGPRs, against two with 64-key tiles: C2 forward 1.20 -> 1.09 ms; 32 at 192,
 // where 16 rows a wave over 64-key tiles took 172 us against 136 for 8 sequences
 // of 512 to 2048 rows at 16/8 heads; 64 at the others: 59 us against 63 with 32 at
-// head dim 64 there, 65 with 16 rows a wave), streamed by buffer DMA into double-buffered swizzled LDS stages (one
-// work-group barrier per tile).  Q rows stay in registers as B operands of
-// S^T = K Q^T; V^T for O^T += V^T P^T comes from ds_read_b64_tr_b16.  Per 32
-// keys of a tile each lane owns one query column (16 qb + j16) and 8 of the
-// keys, the others sitting in the lanes j16 + 16, + 32, + 48.  The softmax runs in the
-// log2 domain with the scale folded into one FMA per score, and the
-// reference point m of a row moves only when the row maximum exceeds it by
-// more than 8 (a factor of 256): the accumulators are rescaled in the rare
-// tile where that happens (skipped wave-wide otherwise), and since O and the
-// row sum share the same m the result is unchanged.  Only tiles that cross
-// the diagonal or pass a run's end are masked.  Against K/V tiles passed through
-// registers between two barriers (8 sequences of 512 to 2048 rows, us): head dim
-// 64 at 16/8 heads 92 -> 60, 32 71 -> 48, 96 112 -> 81, 192 at 24/4 584 -> 200.
+// head dim 64 there, 65 with 16 rows a wave), streamed by buffer DMA into
+// double-buffered swizzled LDS stages (one work-group barrier per tile).  Q rows
+// stay in registers as B operands of S^T = K Q^T; V^T for O^T += V^T P^T comes
+// from ds_read_b64_tr_b16.  Per 32 keys of a tile each lane owns one query column
+// (16 qb + j16) and 8 of the keys, the others sitting in the lanes j16 + 16, + 32,
+// + 48.  The softmax runs in the log2 domain.  Only tiles that cross the diagonal
+// or pass a run's end are masked.
+//
+// The reference point m of a row: at head dims 128 and 256 it moves only when the
+// row maximum exceeds it by more than 8 (a factor of 256), so that the
+// accumulators are rescaled in the rare tile where that happens (skipped wave-wide
+// otherwise), with the scale folded into one FMA per score.  At the other head
+// dims it is the running maximum, exactly, of scores already in log2 units: the
+// largest weight of a row is 1, which the rounding of the weights to 16 bits
+// leaves as it is, and scores and scales of any size and sign keep their softmax.
+// Against 64 bits an fp16 cohort at head dim 64 is off by 3.2e-4, by 3.3e-4 with
+// the other rule, which takes 49 us there against 64.
+//
+// Against K/V tiles passed through registers between two barriers (8 sequences of
+// 512 to 2048 rows, us): head dim 64 at 16/8 heads 72 -> 64, at 32/8 122 -> 104, 32
+// 62 -> 55, 96 93 -> 77, 192 at 24/4 430 -> 184.
 // ---------------------------------------------------------------------------
 constexpr float kRescaleSlack = 8.f;    // log2 units
 constexpr float kRescaleBound = 256.f;  // 2^kRescaleSlack
@@ -49,6 +57,9 @@ constexpr int fwd_occupancy() {
   return HD > 128 ? (NQB == 1 ? 2 : 1) : (NQB == 1 ? 4 : (KT == 32 ? 3 : 2));
 }
 
+// whether the reference point of a row moves only past kRescaleSlack
+template <int HD> constexpr bool fwd_lazy_reference() { return HD % 128 == 0; }
+
 // SPLIT: the launch's y blocks are parts of each item's keys (launches whose
 // items leave CUs idle, ts_attn_fwd_parts); a part writes its unnormalised fp32
 // accumulators and (m, l) per row, which fwd_merge_kernel combines.
@@ -58,6 +69,7 @@ __global__ __launch_bounds__(64 * 8 / NQB, (fwd_occupancy<NQB, HD, KT>())) void 
     float* __restrict__ part) {
   constexpr int kWaves = 8 / NQB;
   constexpr int NKS = HD / 32, NMB = HD / 16;  // k-steps of S; 16-column blocks of O
+  constexpr bool kLazy = fwd_lazy_reference<HD>();
   static_assert(KT == 64 || KT == 32, "tiles of 64 or 32 keys");
   __shared__ __attribute__((aligned(16))) bf16 s_k0[KT * HD];
   __shared__ __attribute__((aligned(16))) bf16 s_v0[KT * HD];
@@ -140,6 +152,14 @@ __global__ __launch_bounds__(64 * 8 / NQB, (fwd_occupancy<NQB, HD, KT>())) void 
         if (st + 3 < 2 * NKS) __builtin_amdgcn_sched_group_barrier(0x100, 1, 1);
       }
       __builtin_amdgcn_s_setprio(0);
+      // at an exact reference point the scores go to log2 units here, and the
+      // largest one of a row to exactly 0 below
+      if constexpr (!kLazy) {
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+          for (int qb = 0; qb < NQB; ++qb) sc[kb][qb] *= c;
+      }
       if (masked) {
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb)
@@ -152,35 +172,41 @@ __global__ __launch_bounds__(64 * 8 / NQB, (fwd_occupancy<NQB, HD, KT>())) void 
               if (i > lim) sc[kb][qb][i] = neg_inf();
           }
       }
-      // Fast path: the exponentials against the current reference point m.
-      // They stand unless some score exceeds m by more than kRescaleSlack, which
-      // a lane detects as a partial sum above 2^kRescaleSlack (every term is
-      // positive), or m is still -inf; then, rarely, the half is redone on the
-      // slow path: column maxima, the move of m with the rescale of O and the
-      // row sum, and the exponentials again.
       float pe[2][NQB][4], ps[NQB];
-      bool redo = false;
-#pragma unroll
-      for (int qb = 0; qb < NQB; ++qb) {
+      auto exponentials = [&](int qb) __attribute__((always_inline)) {
         const float mref = m[qb] == neg_inf() ? 0.f : m[qb];
         ps[qb] = 0.f;
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            pe[kb][qb][i] = fast_exp2(fmaf(sc[kb][qb][i], c, -mref));
+            pe[kb][qb][i] = fast_exp2(kLazy ? fmaf(sc[kb][qb][i], c, -mref) : sc[kb][qb][i] - mref);
             ps[qb] += pe[kb][qb][i];
           }
-        redo |= (m[qb] == neg_inf()) | (ps[qb] > kRescaleBound);
+      };
+      // Fast path: the exponentials against the current reference point m.
+      // They stand unless some score exceeds m by more than kRescaleSlack, which
+      // a lane detects as a partial sum above 2^kRescaleSlack (every term is
+      // positive), or m is still -inf; then, rarely, the half is redone on the
+      // slow path: column maxima, the move of m with the rescale of O and the
+      // row sum, and the exponentials again.
+      bool redo = !kLazy;
+      if constexpr (kLazy) {
+#pragma unroll
+        for (int qb = 0; qb < NQB; ++qb) {
+          exponentials(qb);
+          redo |= (m[qb] == neg_inf()) | (ps[qb] > kRescaleBound);
+        }
       }
-      if (__builtin_amdgcn_ballot_w64(redo) != 0) {
+      if (!kLazy || __builtin_amdgcn_ballot_w64(redo) != 0) {
 #pragma unroll
         for (int qb = 0; qb < NQB; ++qb) {
           float mx = fmaxf(fmaxf(fmaxf(sc[0][qb][0], sc[0][qb][1]), fmaxf(sc[0][qb][2], sc[0][qb][3])),
                            fmaxf(fmaxf(sc[1][qb][0], sc[1][qb][1]), fmaxf(sc[1][qb][2], sc[1][qb][3])));
           mx = rows_max4(mx);
-          const float mt = mx * c;  // maximum in log2 units (-inf if the column sees none of these keys)
-          const bool move = mt > m[qb] + kRescaleSlack;
+          // maximum in log2 units (-inf if the column sees none of these keys)
+          const float mt = kLazy ? mx * c : mx;
+          const bool move = mt > m[qb] + (kLazy ? kRescaleSlack : 0.f);
           if (__builtin_amdgcn_ballot_w64(move) != 0) {
             const float mnew = move ? mt : m[qb];
             // 0 on the first finite score (m = -inf); a row whose scores so far are
@@ -192,15 +218,7 @@ __global__ __launch_bounds__(64 * 8 / NQB, (fwd_occupancy<NQB, HD, KT>())) void 
             for (int mb = 0; mb < NMB; ++mb) acc[mb][qb] *= alpha;
             m[qb] = mnew;
           }
-          const float mref = m[qb] == neg_inf() ? 0.f : m[qb];
-          ps[qb] = 0.f;
-#pragma unroll
-          for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              pe[kb][qb][i] = fast_exp2(fmaf(sc[kb][qb][i], c, -mref));
-              ps[qb] += pe[kb][qb][i];
-            }
+          exponentials(qb);
         }
       }
 #pragma unroll
