@@ -8,6 +8,7 @@ from __future__ import annotations
 import pytest
 import torch
 
+from oracle import attention as ref
 from tests.test_attention_parts_gpu import _Parts
 from thundersync_amd import _lib
 from thundersync_amd import attention as hip
@@ -40,3 +41,26 @@ def test_leading_keys_of_minus_infinity(cuda, monkeypatch, hq, hkv, dim, parts, 
     off = (out.double().cpu() - want).abs()
     assert bool((off <= 2e-2 * max(1.0, want.abs().max().item())).all())
     torch.testing.assert_close(lse.double().cpu(), scores.logsumexp(-1), rtol=1e-5, atol=1e-4)
+
+
+@pytest.mark.parametrize("dim", [32, 64, 96, 192])
+@pytest.mark.parametrize("rows", [1, 40, 64])
+def test_gradients_of_a_key_that_no_row_sees(cuda, dim, rows):
+    """A key of -inf in a component that every query holds positive: its weight is
+    0 in every row, and its own gradients are 0, in row blocks of 32 and in a
+    remainder (whose missing rows are zeros: 0 * -inf is no score)."""
+    print(f"a key of -inf: head dim {dim}, {rows} rows", flush=True)
+    g = torch.Generator().manual_seed(dim + rows)
+    q, do = (torch.randn(rows, 4, dim, generator=g) for _ in range(2))
+    q[:, :, 0] = q[:, :, 0].abs() + 0.1
+    k, v = (torch.randn(90, 2, dim, generator=g) for _ in range(2))
+    k[17, :, 0] = -torch.inf
+    q, do, k, v = (t.bfloat16() for t in (q, do, k, v))
+    qc, kc, vc = (t.to(cuda).requires_grad_() for t in (q, k, v))
+    out, _ = hip.attention(qc, hip.chain_layout(rows, [90], 4, 2), [kc], [vc], dim ** -0.5)
+    out.backward(do.to(cuda))
+    want_o, _, want_k, want_v = ref.attention_with_grads(q, [k], [v], do, dim ** -0.5, dtype=torch.float64)
+    assert bool((want_k[0][17] == 0).all()) and bool((want_v[0][17] == 0).all())
+    for got, want in ((out, want_o), (kc.grad, want_k[0]), (vc.grad, want_v[0])):
+        off = (got.detach().double().cpu() - want).abs()
+        assert bool((off <= 2e-2 * max(1.0, want.abs().max().item())).all())

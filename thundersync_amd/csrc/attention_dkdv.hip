@@ -20,7 +20,8 @@ namespace attn {
 // instructions, one work-group barrier per step.  The buffer resource of a
 // tile covers exactly its valid rows, so rows past a segment's end arrive as
 // zeros and add nothing (S = dP = 0, statistics (0, 0), hence dS = 0 and a
-// zero dO row).  S = Q K^T and dP = dO V^T take the Q/dO rows as A operands;
+// zero dO row; at head dims 32, 64, 96 and 192 their P is also set to 0, which
+// holds beside a key with an infinite component too).  S = Q K^T and dP = dO V^T take the Q/dO rows as A operands;
 // dV^T += dO^T P and dK^T += Q^T dS take dO^T / Q^T from ds_read_b64_tr_b16
 // (the lane layout of the one-wave-per-head kernel).  A wave past the work
 // item's keys (kv_block 48) only issues its DMA share; only steps that cross
@@ -273,14 +274,14 @@ __global__ __launch_bounds__(kThreads, 1) void dkdv_split_kernel(ts_attn_problem
       const int lim = off + r0 - kpos - mask_key;  // row rl sees the key iff rl >= -lim
       // wave-uniform: the keys cross the diagonal (or, when dS is stored, the
       // run's end: P of a key past it, whose K row is zero, is exp2(-lse2))
-      const bool diag = (kpos + wk0 + 15 > off + r0) | (DS && wk0 + 16 > run.len);
+      const bool diag = (kpos + wk0 + 15 > off + r0) | (DS && wk0 + 16 > run.len) | (HD % 128 != 0 && nrows < 32);
 #pragma unroll
       for (int qb = 0; qb < 2; ++qb)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int rl = 16 * qb + 4 * g4 + i;
           float p = fast_exp2(sc[qb][i] * c - sl[2 * rl]);
-          if (diag && rl + lim < 0) p = 0.f;
+          if (diag && (rl + lim < 0 || (HD % 128 != 0 && rl >= nrows))) p = 0.f;
           pv[4 * qb + i] = p;
           dsv[4 * qb + i] = p * (dp[qb][i] - sl[2 * rl + 1]);
         }
