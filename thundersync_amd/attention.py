@@ -109,14 +109,28 @@ DKDV256_MIN_ITEMS = 512
 # waves take 16 keys each of every step.  The first does each step in fewer LDS
 # reads and without a barrier, the second starts and ends cheaper (16 keys'
 # operands to load, no partials to sum over the waves) and holds two
-# work-groups a CU.  So items of many steps are dealt out, and so are launches
-# that one work-group a CU holds, down to two steps a wave.  Key-split against
-# dealt out, us: 6 steps, 696 items 30 / 44 (24/8 heads, 64 rows over 4160 keys);
-# 16 steps, 348 items 33 / 38 (32/4, 64 over 4160); 16 steps, 704 items 52 / 53
-# (32/8, 128 over 4224); 8 steps, 96 items 17 / 16 (32/8, 64 over 576); 16 steps,
-# 216 items 26 / 22 (16/8, 256 over 1280); 40 steps, 216 items 51 / 35 (40/8,
-# 256 over 1280); 320 steps and more 1.3 to 2.5 times faster dealt out.
-DEALT_STEPS, DEALT_STEPS_ONE_ROUND, ONE_ROUND_ITEMS = 20, 8, 256
+# work-groups a CU.  So the first pays where items have many steps, the second
+# where there are many items of few.  A launch takes about
+#     start + round * rounds + step * max(tail * longest item's steps, steps a slot)
+# us, slots being the work-groups the device holds at once and rounds the items
+# over them: fitted to 186 launches (one sequence over a context, cohorts, packs; 16
+# to 9000 rows over up to 14000 keys) at head counts from 32/4 to 8/8, where the
+# choice costs 0.3 % on average and at most 13 % (24/8 heads, 8 sequences of 512 to
+# 2048 rows: 290 us dealt, 258 split).  By the average steps of an item alone it
+# cost 3.6 % and up to 79 %: dealt against split 146 / 101 us for 16 sequences of 256
+# to 1024 rows at 16/8, 130 / 103 for 256 rows over 8448 keys at 24/8, 31 / 41 for 4
+# sequences of 256 to 1024 rows at 8/8.
+class DkdvCost(NamedTuple):
+    keys: int  # of an item
+    slots: int
+    start: float
+    round: float
+    step: float
+    tail: float
+
+
+DEALT_COST = DkdvCost(48, 256, 4.0, 12.0, 0.46, 0.7)
+SPLIT_COST = DkdvCost(64, 512, 10.0, 0.0, 1.8, 0.55)
 
 
 # ---------------------------------------------------------------------------
@@ -202,10 +216,13 @@ class AttnLayout:
             spans = array("i", chain.from_iterable(chain.from_iterable(self.seg_spans)))
             arrays = (array("q", chain.from_iterable(self.seg_q)), span0, spans, array("i", (r[2] for r in self.runs)),
                       array("i", (r[0] for r in self.runs)), array("q", (r[1] for r in self.runs)))
-            visited = set(spans[::2])
+            users: dict[int, int] = {}  # visited runs: query rows of the segments that read them
+            for (_, n), seg in zip(self.seg_q, self.seg_spans):
+                for r, _ in seg:
+                    users[r] = users.get(r, 0) + n
             # rows of each source that a visited run covers (runs do not overlap)
             covered, key_rows, items48, items64 = [0] * len(self.source_rows), 0, 0, 0
-            for r in visited:
+            for r in users:
                 source, _, length = self.runs[r]
                 covered[source] += length
                 key_rows += length
@@ -222,6 +239,8 @@ class AttnLayout:
                 "uncovered": [i for i, n in enumerate(self.source_rows) if covered[i] != n],
                 # query rows that see a visited key, on average
                 "rows_per_key": self.visible_pairs() / max(key_rows, 1),
+                # query rows that read a run, at most
+                "most_rows": max(users.values(), default=0),
                 "max_keys": max((kv for kv, (_, n) in zip(self.seg_kv, self.seg_q) if n), default=0),
                 "all_rows": sum(n for _, n in self.seg_q) == self.q_rows,
             }
@@ -360,18 +379,23 @@ class AttnLayout:
 
     def call_kv_block(self, device, head_dim: int) -> int:
         """Keys per dK/dV work item of this package's own calls: kv_block_for's,
-        except that at head dim 128 every GQA group takes either kernel, by the
-        steps of an item and the items of the launch (DEALT_STEPS), and at the
-        head dims that only the key-split kernel takes, whose four waves hold 16
-        keys each, every group has 64."""
+        except that at head dim 128 every GQA group takes either kernel, whichever
+        is estimated to end sooner (DkdvCost), and at the head dims that only the
+        key-split kernel takes, whose four waves hold 16 keys each, every group has
+        64."""
         if head_dim == 256:
             return self.kv_block_for(device, head_dim)
         if head_dim != HEAD_DIM:
             return 64
         d = self._description()
-        steps = (self.hq // self.hkv) * d["rows_per_key"] / 32
-        items = d["items48"] * self.hkv
-        return 48 if steps >= (DEALT_STEPS_ONE_ROUND if items <= ONE_ROUND_ITEMS else DEALT_STEPS) else 64
+        steps = (self.hq // self.hkv) / 32  # of a row that an item sees
+
+        def us(c: DkdvCost) -> float:
+            rounds = d[f"items{c.keys}"] * self.hkv / c.slots
+            work = max(c.tail * d["most_rows"], d["rows_per_key"] * rounds)
+            return c.start + c.round * max(rounds, 1.0) + c.step * steps * work
+
+        return 48 if us(DEALT_COST) < us(SPLIT_COST) else 64
 
     def problem(self, device, runs_ptr: int, scale: float, dtype: torch.dtype = torch.bfloat16,
                 head_dim: int = HEAD_DIM, kv_block: int | None = None) -> AttnProblem:
