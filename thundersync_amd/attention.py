@@ -120,17 +120,18 @@ DKDV256_MIN_ITEMS = 512
 # cost 3.6 % and up to 79 %: dealt against split 146 / 101 us for 16 sequences of 256
 # to 1024 rows at 16/8, 130 / 103 for 256 rows over 8448 keys at 24/8, 31 / 41 for 4
 # sequences of 256 to 1024 rows at 8/8.
-class DkdvCost(NamedTuple):
-    keys: int  # of an item
-    slots: int
-    start: float
-    round: float
-    step: float
-    tail: float
+# (slots, start, round, step, tail) of the dealt and the key-split kernel
+DKDV_DEALT = (256, 4.0, 12.0, 0.46, 0.7)
+DKDV_SPLIT = (512, 10.0, 0.0, 1.8, 0.55)
 
 
-DEALT_COST = DkdvCost(48, 256, 4.0, 12.0, 0.46, 0.7)
-SPLIT_COST = DkdvCost(64, 512, 10.0, 0.0, 1.8, 0.55)
+def _dkdv_us(kernel, items: int, group: int, mean_rows: float, most_rows: int) -> float:
+    """Estimated us of a dK/dV launch of `items` work items, each seen by
+    `mean_rows` query rows on average and `most_rows` at most."""
+    slots, start, per_round, step, tail = kernel
+    rounds = items / slots
+    work = max(tail * most_rows, mean_rows * rounds)
+    return start + per_round * (rounds if rounds > 1.0 else 1.0) + step * group * work / 32
 
 
 # ---------------------------------------------------------------------------
@@ -216,10 +217,14 @@ class AttnLayout:
             spans = array("i", chain.from_iterable(chain.from_iterable(self.seg_spans)))
             arrays = (array("q", chain.from_iterable(self.seg_q)), span0, spans, array("i", (r[2] for r in self.runs)),
                       array("i", (r[0] for r in self.runs)), array("q", (r[1] for r in self.runs)))
-            users: dict[int, int] = {}  # visited runs: query rows of the segments that read them
-            for (_, n), seg in zip(self.seg_q, self.seg_spans):
-                for r, _ in seg:
-                    users[r] = users.get(r, 0) + n
+            # visited runs: query rows of the segments that read them
+            if len(self.seg_q) == 1:
+                users = dict.fromkeys(spans[::2], self.seg_q[0][1])
+            else:
+                users = {}
+                for (_, n), seg in zip(self.seg_q, self.seg_spans):
+                    for r, _ in seg:
+                        users[r] = users.get(r, 0) + n
             # rows of each source that a visited run covers (runs do not overlap)
             covered, key_rows, items48, items64 = [0] * len(self.source_rows), 0, 0, 0
             for r in users:
@@ -228,19 +233,18 @@ class AttnLayout:
                 key_rows += length
                 items48 += (length + 47) // 48
                 items64 += (length + 63) // 64
+            # the GQA group, and the query rows that see a visited key, on average and at most
+            rows = (self.hq // self.hkv, self.visible_pairs() / max(key_rows, 1), max(users.values(), default=0))
             d = {
                 "arrays": arrays,
                 "ptrs": tuple(a.buffer_info()[0] if len(a) else None for a in arrays),
                 "n_spans": at,
                 # dK/dV items of one KV head, by their size
-                "items48": items48,
                 "items64": items64,
                 # sources with rows that no visited run covers: their gradients are filled with zeros first
                 "uncovered": [i for i, n in enumerate(self.source_rows) if covered[i] != n],
-                # query rows that see a visited key, on average
-                "rows_per_key": self.visible_pairs() / max(key_rows, 1),
-                # query rows that read a run, at most
-                "most_rows": max(users.values(), default=0),
+                "kv_block128": 48 if _dkdv_us(DKDV_DEALT, items48 * self.hkv, *rows)
+                < _dkdv_us(DKDV_SPLIT, items64 * self.hkv, *rows) else 64,
                 "max_keys": max((kv for kv, (_, n) in zip(self.seg_kv, self.seg_q) if n), default=0),
                 "all_rows": sum(n for _, n in self.seg_q) == self.q_rows,
             }
@@ -380,22 +384,14 @@ class AttnLayout:
     def call_kv_block(self, device, head_dim: int) -> int:
         """Keys per dK/dV work item of this package's own calls: kv_block_for's,
         except that at head dim 128 every GQA group takes either kernel, whichever
-        is estimated to end sooner (DkdvCost), and at the head dims that only the
+        is estimated to end sooner (_dkdv_us), and at the head dims that only the
         key-split kernel takes, whose four waves hold 16 keys each, every group has
         64."""
         if head_dim == 256:
             return self.kv_block_for(device, head_dim)
         if head_dim != HEAD_DIM:
             return 64
-        d = self._description()
-        steps = (self.hq // self.hkv) / 32  # of a row that an item sees
-
-        def us(c: DkdvCost) -> float:
-            rounds = d[f"items{c.keys}"] * self.hkv / c.slots
-            work = max(c.tail * d["most_rows"], d["rows_per_key"] * rounds)
-            return c.start + c.round * max(rounds, 1.0) + c.step * steps * work
-
-        return 48 if us(DEALT_COST) < us(SPLIT_COST) else 64
+        return self._description()["kv_block128"]
 
     def problem(self, device, runs_ptr: int, scale: float, dtype: torch.dtype = torch.bfloat16,
                 head_dim: int = HEAD_DIM, kv_block: int | None = None) -> AttnProblem:
