@@ -272,6 +272,7 @@ __global__ __launch_bounds__(kThreads, 1) void dkdv_split_kernel(ts_attn_problem
       // P and dS as B operands: slot j = 4 qb + i  <->  row 16 qb + 4 g4 + i
       float pv[8], dsv[8];
       const int lim = off + r0 - kpos - mask_key;  // row rl sees the key iff rl >= -lim
+      const unsigned seen = max(0, nrows + lim);   // and is one of the block's iff rl + lim < seen, too
       // wave-uniform: the keys cross the diagonal (or, when dS is stored, the
       // run's end: P of a key past it, whose K row is zero, is exp2(-lse2))
       const bool diag = (kpos + wk0 + 15 > off + r0) | (DS && wk0 + 16 > run.len) | (HD % 128 != 0 && nrows < 32);
@@ -281,7 +282,7 @@ __global__ __launch_bounds__(kThreads, 1) void dkdv_split_kernel(ts_attn_problem
         for (int i = 0; i < 4; ++i) {
           const int rl = 16 * qb + 4 * g4 + i;
           float p = fast_exp2(sc[qb][i] * c - sl[2 * rl]);
-          if (diag && (rl + lim < 0 || (HD % 128 != 0 && rl >= nrows))) p = 0.f;
+          if (diag && (HD % 128 != 0 ? (unsigned)(rl + lim) >= seen : rl + lim < 0)) p = 0.f;
           pv[4 * qb + i] = p;
           dsv[4 * qb + i] = p * (dp[qb][i] - sl[2 * rl + 1]);
         }
