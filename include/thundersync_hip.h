@@ -293,14 +293,18 @@ int ts_attn_bwd(const ts_attn_problem* problem, ts_attn_rows q, ts_attn_rows out
 
 /* ts_attn_fwd with each work item's keys cut into `parts` work-groups, for
  * launches whose items leave much of the device idle (a short turn over a long
- * context: two row blocks a KV head).  The workspace (16-byte aligned, parts *
- * hq * q_rows * (head_dim + 2) floats) takes each part's unnormalised fp32 rows
- * and their (m, l); a second kernel combines them in part order.  parts 1: no
- * workspace, ts_attn_fwd's launch.  ts_attn_fwd_parts and ts_attn_dq_parts give
+ * context: two row blocks a KV head).  The workspace (16-byte aligned,
+ * ts_attn_fwd_parts_workspace bytes: parts times head_dim + 2 floats for each of
+ * the hq * q_rows rows or, where these are fewer, of the items' 128 row slots a
+ * head chunk) takes each part's unnormalised fp32 rows and their (m, l); a second
+ * kernel combines them in part order.  parts 1: no workspace, ts_attn_fwd's
+ * launch.  ts_attn_fwd_parts and ts_attn_dq_parts give
  * the parts worth taking for a problem whose longest item sees max_keys keys
  * (n_dq_work: items of the dQ pass's own list, 0 without one). */
 int ts_attn_fwd_parts(const ts_attn_problem* problem, int64_t max_keys);
 int ts_attn_dq_parts(const ts_attn_problem* problem, int32_t n_dq_work, int64_t max_keys);
+int64_t ts_attn_fwd_parts_workspace(const ts_attn_problem* problem, int parts);
+int64_t ts_attn_dq_parts_workspace(const ts_attn_problem* problem, int32_t n_dq_work, int parts);
 int ts_attn_fwd_split(const ts_attn_problem* problem, ts_attn_rows q, ts_attn_rows out, float* lse, int64_t lse_ld,
                       int parts, void* workspace, int64_t workspace_bytes, void* stream);
 
@@ -350,8 +354,8 @@ int ts_attn_bwd_ds(const ts_attn_problem* problem, ts_attn_rows q, ts_attn_rows 
                    int64_t ds_head, void* ds, int64_t ds_bytes, const int32_t* dq_work,
                    int32_t n_dq_work, int32_t n_dq_long, void* stream);
 
-/* ts_attn_bwd_ds with the dQ pass's items cut into dq_parts (workspace: parts *
- * hq * q_rows * head_dim floats), as ts_attn_fwd_split. */
+/* ts_attn_bwd_ds with the dQ pass's items cut into dq_parts (workspace:
+ * ts_attn_dq_parts_workspace bytes), as ts_attn_fwd_split. */
 int ts_attn_bwd_ds_split(const ts_attn_problem* problem, ts_attn_rows q, ts_attn_rows out, ts_attn_rows dout,
                          const float* lse, int64_t lse_ld, float* rowstats, ts_attn_rows dq, const int64_t* span_ds,
                          const int64_t* visit_ds, int64_t ds_head, void* ds, int64_t ds_bytes,

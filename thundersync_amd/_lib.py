@@ -89,6 +89,8 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "ts_attn_fwd": (_INT, [ctypes.POINTER(AttnProblem), AttnRows, AttnRows, _P, _I64, _P]),
     "ts_attn_fwd_parts": (_INT, [ctypes.POINTER(AttnProblem), _I64]),
     "ts_attn_dq_parts": (_INT, [ctypes.POINTER(AttnProblem), ctypes.c_int32, _I64]),
+    "ts_attn_fwd_parts_workspace": (_I64, [ctypes.POINTER(AttnProblem), _INT]),
+    "ts_attn_dq_parts_workspace": (_I64, [ctypes.POINTER(AttnProblem), ctypes.c_int32, _INT]),
     "ts_attn_fwd_split": (_INT, [ctypes.POINTER(AttnProblem), AttnRows, AttnRows, _P, _I64, _INT, _P, _I64, _P]),
     "ts_attn_bwd_ds_split": (
         _INT,

@@ -599,9 +599,13 @@ def _gather(layout: AttnLayout, query: torch.Tensor, keys, values) -> list[int]:
     return out
 
 
-def _parts_workspace(parts: int, hq: int, q_rows: int, floats: int, device) -> torch.Tensor | None:
-    """fp32 rows for the partial sums of work items cut into ``parts`` (None for whole items)."""
-    return torch.empty(parts * hq * q_rows * floats, dtype=torch.float32, device=device) if parts > 1 else None
+def _parts_workspace(nbytes: int, device) -> torch.Tensor | None:
+    """Memory for the partial sums of work items cut into parts, None where the
+    device has none left (the items then stay whole)."""
+    try:
+        return torch.empty(nbytes, dtype=torch.uint8, device=device)
+    except torch.cuda.OutOfMemoryError:
+        return None
 
 
 def _attention_forward(query: torch.Tensor, layout: AttnLayout, scale: float, keys, values):
@@ -617,11 +621,14 @@ def _attention_forward(query: torch.Tensor, layout: AttnLayout, scale: float, ke
     check_tables(layout, problem, host, device)
     # few work items over many keys: each item's keys in several work-groups
     parts = lib.ts_attn_fwd_parts(ctypes.byref(problem), layout._description()["max_keys"])
-    work = _parts_workspace(parts, layout.hq, layout.q_rows, query.shape[2] + 2, device)
+    work = None
+    if parts > 1:
+        work = _parts_workspace(lib.ts_attn_fwd_parts_workspace(ctypes.byref(problem), parts), device)
+        parts = parts if work is not None else 1
     with operator_range("hip_attention_forward", rows=layout.q_rows, segments=len(layout.seg_q)):
         _lib.check(
             lib.ts_attn_fwd_split(ctypes.byref(problem), _rows(query), _rows(out), lse.data_ptr(), lse.shape[1],
-                                  parts, _lib.ptr(work), 0 if work is None else work.numel() * 4,
+                                  parts, _lib.ptr(work), 0 if work is None else work.numel(),
                                   _lib.stream_of(query)),
             lambda: f"ts_attn_fwd(rows={layout.q_rows}, hq={layout.hq}, hkv={layout.hkv})",
         )
@@ -694,13 +701,16 @@ def _attention_backward(query, out, lse, dout, layout: AttnLayout, scale: float,
                     sub.hq, sub.hkv, sub.runs = n * group, n, sub_runs.data_ptr()
                     check_tables(layout, sub, sub_host, device)
                 q_r, o_r, do_r, dq_r = (_head_rows(r, h0) for r in rows)
-                sums = _parts_workspace(parts, sub.hq, layout.q_rows, d, device)
+                sums = None
+                if parts > 1:
+                    sums = _parts_workspace(lib.ts_attn_dq_parts_workspace(ctypes.byref(sub), n_dq, parts), device)
+                    parts = parts if sums is not None else 1
                 _lib.check(
                     lib.ts_attn_bwd_ds_split(ctypes.byref(sub), q_r, o_r, do_r, lse.data_ptr() + h0 * lse.shape[1] * 4,
                                        lse.shape[1], rowstats.data_ptr() + h0 * lse.shape[1] * 8, dq_r,
                                        tabs["span"], tabs["visit"], tabs["head"], work.data_ptr(),
                                        work.numel() * 2, dq_list, n_dq, n_dq_long, parts, _lib.ptr(sums),
-                                       0 if sums is None else sums.numel() * 4, _lib.stream_of(query)),
+                                       0 if sums is None else sums.numel(), _lib.stream_of(query)),
                     lambda: f"ts_attn_bwd_ds(rows={layout.q_rows}, hq={layout.hq}, hkv={layout.hkv}, heads from {h0})",
                 )
             del work

@@ -72,7 +72,7 @@ int validate(const ts_attn_problem* p, const char* what) {
 // null), or storing dS in the dK/dV kernels and forming dQ = dS K from it
 int backward(const ts_attn_problem* problem, ts_attn_rows q, ts_attn_rows out, ts_attn_rows dout,
              const float* lse, int64_t lse_ld, float* rowstats, ts_attn_rows dq, const DsArgs* ds,
-             const char* what, void* stream, int dq_parts = 1, float* dq_part = nullptr) {
+             const char* what, void* stream, int dq_parts = 1, PartSums dq_part = PartSums{}) {
   int st = validate(problem, what);
   if (st != TS_OK) return st;
   const ts_attn_problem& P = *problem;
@@ -144,14 +144,24 @@ int parts_of(int64_t items, int64_t max_keys, const SplitModel& m) {
   return best;
 }
 
-int check_parts(const ts_attn_problem& P, int parts, const void* part, int64_t bytes, int64_t row_floats,
+// the partial sums of a launch over `n_items` work items of `pairs` (row, head) pairs a head chunk
+PartSums parts_of_items(const ts_attn_problem& P, int64_t n_items, int pairs, void* ptr) {
+  const int group = P.hq / P.hkv;
+  return part_sums(P, n_items * P.hkv * (group / heads_per_block(group)), pairs, ptr);
+}
+PartSums fwd_part_sums(const ts_attn_problem& P, void* ptr) { return parts_of_items(P, P.n_q_work, 128, ptr); }
+PartSums dq_part_sums(const ts_attn_problem& P, int64_t n_dq_work, void* ptr) {
+  return n_dq_work > 0 ? parts_of_items(P, n_dq_work, 256, ptr) : parts_of_items(P, P.n_q_work, 128, ptr);
+}
+
+int check_parts(const ts_attn_problem& P, int parts, const PartSums& part, int64_t bytes, int64_t row_floats,
                 const char* what) {
   TS_CHECK_ARG(parts >= 1 && parts < 65536 && (parts == 1 || ds_route(P.head_dim, P.hq / P.hkv)),
                "%s: %d parts (head dims 128 and 256 split their items)", what, parts);
-  TS_CHECK_ARG(parts == 1 || (part && (uint64_t)part % 16 == 0 &&
-                              bytes / 4 / row_floats >= (int64_t)parts * P.hq * P.q_rows),
-               "%s: a workspace of %lld bytes for %d parts of %d heads x %lld rows", what, (long long)bytes, parts, P.hq,
-               (long long)P.q_rows);
+  TS_CHECK_ARG(parts == 1 || (part.ptr && (uint64_t)part.ptr % 16 == 0 &&
+                              bytes / 4 / row_floats >= parts * part.rows),
+               "%s: a workspace of %lld bytes for %d parts of %lld rows", what, (long long)bytes, parts,
+               (long long)part.rows);
   return TS_OK;
 }
 
@@ -187,6 +197,18 @@ int ts_attn_dq_parts(const ts_attn_problem* problem, int32_t n_dq_work, int64_t 
                                                               : SplitModel{0.9, 32, 340, false});
 }
 
+int64_t ts_attn_fwd_parts_workspace(const ts_attn_problem* problem, int parts) {
+  using namespace ts::attn;
+  if (!problem || problem->hkv <= 0 || problem->hq % problem->hkv || parts <= 1) return 0;
+  return parts * fwd_part_sums(*problem, nullptr).rows * (problem->head_dim + 2) * (int64_t)sizeof(float);
+}
+
+int64_t ts_attn_dq_parts_workspace(const ts_attn_problem* problem, int32_t n_dq_work, int parts) {
+  using namespace ts::attn;
+  if (!problem || problem->hkv <= 0 || problem->hq % problem->hkv || parts <= 1) return 0;
+  return parts * dq_part_sums(*problem, n_dq_work, nullptr).rows * problem->head_dim * (int64_t)sizeof(float);
+}
+
 int ts_attn_fwd(const ts_attn_problem* problem, ts_attn_rows q, ts_attn_rows out, float* lse,
                 int64_t lse_ld, void* stream) {
   return ts_attn_fwd_split(problem, q, out, lse, lse_ld, 1, nullptr, 0, stream);
@@ -203,9 +225,10 @@ int ts_attn_fwd_split(const ts_attn_problem* problem, ts_attn_rows q, ts_attn_ro
                "with strides that are multiples of 8 elements");
   TS_CHECK_ARG(lse && lse_ld >= P.q_rows, "ts_attn_fwd: lse null or lse_ld %lld < rows %lld",
                (long long)lse_ld, (long long)P.q_rows);
-  st = check_parts(P, parts, workspace, workspace_bytes, P.head_dim + 2, "ts_attn_fwd");
+  const PartSums part = fwd_part_sums(P, workspace);
+  st = check_parts(P, parts, part, workspace_bytes, P.head_dim + 2, "ts_attn_fwd");
   if (st != TS_OK) return st;
-  return launch_fwd(P, q, out, lse, lse_ld, parts, (float*)workspace, (hipStream_t)stream);
+  return launch_fwd(P, q, out, lse, lse_ld, parts, part, (hipStream_t)stream);
 }
 
 int ts_attn_bwd(const ts_attn_problem* problem, ts_attn_rows q, ts_attn_rows out, ts_attn_rows dout,
@@ -288,9 +311,10 @@ int ts_attn_bwd_ds_split(const ts_attn_problem* problem, ts_attn_rows q, ts_attn
   TS_CHECK_ARG(!dq_work || (problem->head_dim == 128 && (problem->hq / problem->hkv) % 4 == 0),
                "%s: a dQ work list is for GQA groups that are a multiple of 4 at head dim 128", what);
   const DsArgs args{span_ds, visit_ds, ds_head, (uint64_t)ds, dq_work, n_dq_work, n_dq_long};
-  const int st = check_parts(*problem, dq_parts, workspace, workspace_bytes, problem->head_dim, what);
+  const PartSums part = dq_part_sums(*problem, dq_work ? n_dq_work : 0, workspace);
+  const int st = check_parts(*problem, dq_parts, part, workspace_bytes, problem->head_dim, what);
   if (st != TS_OK) return st;
-  return backward(problem, q, out, dout, lse, lse_ld, rowstats, dq, &args, what, stream, dq_parts, (float*)workspace);
+  return backward(problem, q, out, dout, lse, lse_ld, rowstats, dq, &args, what, stream, dq_parts, part);
 }
 
 int ts_attn_check_tables(const ts_attn_problem* problem, const ts_attn_segment* segs,

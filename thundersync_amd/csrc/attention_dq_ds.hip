@@ -89,7 +89,7 @@ template <int HD, int WV> constexpr int dq_ds_occupancy() {
 template <typename E, int HD, int GC, int WV = 4, bool SPLIT = false>
 __global__ __launch_bounds__(64 * WV, (dq_ds_occupancy<HD, WV>())) void dq_ds_kernel(ts_attn_problem P, DsArgs S,
                                                                                      ts_attn_rows dQ,
-                                                                                     float* __restrict__ part) {
+                                                                                     PartSums part) {
   static_assert(HD == 128 || HD == 256, "the K tile swizzle needs 16 or 32 chunks per row");
   constexpr int KT = dq_ds_tile_keys<HD>();      // keys per tile (64 or 32)
   constexpr int NKB = KT / 16;                   // 16-key dS blocks per tile
@@ -231,7 +231,9 @@ __global__ __launch_bounds__(64 * WV, (dq_ds_occupancy<HD, WV>())) void dq_ds_ke
     const int row = 32 * rb + 16 * ((j16 >> 2) & 1) + 4 * (2 * mbp + (j16 >> 3)) + (j16 & 3);
     if (row >= T) continue;
     if constexpr (SPLIT) {
-      float* prow = part + part_row(P, (int)blockIdx.y, h, seg.q_row0 + row) * HD + 4 * g4;
+      float* prow = part.ptr + 4 * g4 +
+                    HD * part_row<32 * WV>(P, part, (int)blockIdx.y, item * P.hkv * chunks + yb,
+                                           (row - q0) * GC + wave % GC, h, seg.q_row0 + row);
 #pragma unroll
       for (int mb = 0; mb < NMB; ++mb) *reinterpret_cast<f32x4*>(prow + 16 * mb) = acc[mb][mbp];
       continue;
@@ -249,7 +251,7 @@ __global__ __launch_bounds__(64 * WV, (dq_ds_occupancy<HD, WV>())) void dq_ds_ke
 // cover the work items' rows, as in fwd_merge_kernel
 template <typename E, int HD, int GC, int ROWS>
 __global__ __launch_bounds__(kThreads) void dq_merge_kernel(ts_attn_problem P, ts_attn_rows dQ,
-                                                            const float* __restrict__ part, int parts) {
+                                                            PartSums part, int parts) {
   constexpr int Q4 = HD / 4;  // threads per (row, head)
   const int chunks = P.hq / P.hkv / GC;
   const int heads = P.hkv * chunks;
@@ -258,13 +260,13 @@ __global__ __launch_bounds__(kThreads) void dq_merge_kernel(ts_attn_problem P, t
   const int q0 = uniform_table(P.q_work)[2 * item + 1];
   const ts_attn_segment seg = load_uniform(P.segs, seg_id);
   constexpr int kPairs = ROWS * GC / kMergeBlocks;
-  const int64_t step = (int64_t)P.hq * P.q_rows * HD;
+  const int64_t step = part.rows * HD;
 #pragma unroll 1
   for (int i = threadIdx.x / Q4; i < kPairs; i += kThreads / Q4) {
     const int pair = (int)blockIdx.y * kPairs + i;
     const int row = q0 + pair / GC, h = yb * GC + pair % GC, d = 4 * (threadIdx.x % Q4);
     if (row >= seg.q_len) break;
-    const float* x = part + part_row(P, 0, h, seg.q_row0 + row) * HD + d;
+    const float* x = part.ptr + part_row<ROWS * GC>(P, part, 0, (int)blockIdx.x, pair, h, seg.q_row0 + row) * HD + d;
     f32x4 v = *reinterpret_cast<const f32x4*>(x);
 #pragma unroll 4
     for (int p = 1; p < parts; ++p) v += *reinterpret_cast<const f32x4*>(x + p * step);
@@ -275,13 +277,13 @@ __global__ __launch_bounds__(kThreads) void dq_merge_kernel(ts_attn_problem P, t
 }
 
 template <typename E, int HD, int GC, int WV>
-void launch_dq_ds_items(const ts_attn_problem& P, const DsArgs& S, ts_attn_rows dq, int parts, float* part,
+void launch_dq_ds_items(const ts_attn_problem& P, const DsArgs& S, ts_attn_rows dq, int parts, PartSums part,
                         hipStream_t s) {
   if (P.n_q_work == 0) return;
   const unsigned grid = (unsigned)(P.n_q_work * P.hkv * (P.hq / P.hkv / GC));
   if (parts <= 1) {
     ts::TimedLaunch timed_("attention.dq_kernel", s);
-    hipLaunchKernelGGL((dq_ds_kernel<E, HD, GC, WV>), dim3(grid), dim3(64 * WV), 0, s, P, S, dq, nullptr);
+    hipLaunchKernelGGL((dq_ds_kernel<E, HD, GC, WV>), dim3(grid), dim3(64 * WV), 0, s, P, S, dq, part);
     return;
   }
   {
@@ -294,7 +296,7 @@ void launch_dq_ds_items(const ts_attn_problem& P, const DsArgs& S, ts_attn_rows 
 }
 
 template <typename E>
-void launch_dq_ds_t(const ts_attn_problem& P, const DsArgs& S, ts_attn_rows dq, int parts, float* part,
+void launch_dq_ds_t(const ts_attn_problem& P, const DsArgs& S, ts_attn_rows dq, int parts, PartSums part,
                     hipStream_t s) {
   const int gc = heads_per_block(P.hq / P.hkv);
   if (S.dq_work && P.head_dim == 128 && gc == 4) {
@@ -315,7 +317,7 @@ void launch_dq_ds_t(const ts_attn_problem& P, const DsArgs& S, ts_attn_rows dq, 
   }
 }
 
-int launch_dq_ds(const ts_attn_problem& P, const DsArgs& S, ts_attn_rows dq, int parts, float* part, hipStream_t s) {
+int launch_dq_ds(const ts_attn_problem& P, const DsArgs& S, ts_attn_rows dq, int parts, PartSums part, hipStream_t s) {
   if (P.dtype == kF16)
     launch_dq_ds_t<f16>(P, S, dq, parts, part, s);
   else

@@ -66,7 +66,7 @@ template <int HD> constexpr bool fwd_lazy_reference() { return HD % 128 == 0; }
 template <typename E, int NQB, int HD = D, int GC = 4, int KT = BK, bool SPLIT = false>
 __global__ __launch_bounds__(64 * 8 / NQB, (fwd_occupancy<NQB, HD, KT>())) void fwd_wave_kernel(
     ts_attn_problem P, ts_attn_rows Q, ts_attn_rows O, float* __restrict__ lse, int64_t lse_ld,
-    float* __restrict__ part) {
+    PartSums part) {
   constexpr int kWaves = 8 / NQB;
   constexpr int NKS = HD / 32, NMB = HD / 16;  // k-steps of S; 16-column blocks of O
   constexpr bool kLazy = fwd_lazy_reference<HD>();
@@ -268,12 +268,13 @@ __global__ __launch_bounds__(64 * 8 / NQB, (fwd_occupancy<NQB, HD, KT>())) void 
     const int row = qw + 16 * qb + j16;
     if (row >= T) continue;
     if constexpr (SPLIT) {
-      float* prow = part + part_row(P, (int)blockIdx.y, h, seg.q_row0 + row) * HD + 4 * g4;
+      const int64_t at = part_row<128>(P, part, (int)blockIdx.y, item * P.hkv * chunks + yb,
+                                       (row - q0) * GC + wave % GC, h, seg.q_row0 + row);
+      float* prow = part.ptr + at * HD + 4 * g4;
 #pragma unroll
       for (int mb = 0; mb < NMB; ++mb) *reinterpret_cast<f32x4*>(prow + 16 * mb) = acc[mb][qb];
       if (g4 == 0) {
-        float* st = part_stats<HD>(P, part, (int)gridDim.y) +
-                    2 * part_row(P, (int)blockIdx.y, h, seg.q_row0 + row);
+        float* st = part_stats<HD>(part, (int)gridDim.y) + 2 * at;
         st[0] = m[qb];
         st[1] = ls;
       }
@@ -298,7 +299,7 @@ __global__ __launch_bounds__(64 * 8 / NQB, (fwd_occupancy<NQB, HD, KT>())) void 
 template <typename E, int HD, int GC>
 __global__ __launch_bounds__(kThreads) void fwd_merge_kernel(ts_attn_problem P, ts_attn_rows O,
                                                              float* __restrict__ lse, int64_t lse_ld,
-                                                             const float* __restrict__ part, int parts) {
+                                                             PartSums part, int parts) {
   constexpr int NC = HD / 64;  // columns per lane (2 or 4)
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int chunks = P.hq / P.hkv / GC;
@@ -307,14 +308,14 @@ __global__ __launch_bounds__(kThreads) void fwd_merge_kernel(ts_attn_problem P, 
   const int seg_id = uniform_table(P.q_work)[2 * item];
   const int q0 = uniform_table(P.q_work)[2 * item + 1];
   const ts_attn_segment seg = load_uniform(P.segs, seg_id);
-  const float* stats = part_stats<HD>(P, part, parts);
+  const float* stats = part_stats<HD>(part, parts);
   constexpr int kPairs = 128 / kMergeBlocks;  // (row, head) pairs of a work-group
 #pragma unroll 1
   for (int i = wave; i < kPairs; i += kThreads / 64) {
     const int pair = (int)blockIdx.y * kPairs + i;
     const int row = q0 + pair / GC, h = yb * GC + pair % GC;
     if (row >= seg.q_len) break;
-    const int64_t at = part_row(P, 0, h, seg.q_row0 + row), step = (int64_t)P.hq * P.q_rows;
+    const int64_t at = part_row<128>(P, part, 0, (int)blockIdx.x, pair, h, seg.q_row0 + row), step = part.rows;
     float M = neg_inf();
     for (int p = 0; p < parts; ++p) M = fmaxf(M, stats[2 * (at + p * step)]);
     const float ref = M == neg_inf() ? 0.f : M;
@@ -325,7 +326,7 @@ __global__ __launch_bounds__(kThreads) void fwd_merge_kernel(ts_attn_problem P, 
     for (int p = 0; p < parts; ++p) {
       const float w = fast_exp2(stats[2 * (at + p * step)] - ref);
       L = fmaf(stats[2 * (at + p * step) + 1], w, L);
-      const float* x = part + (at + p * step) * HD + NC * lane;
+      const float* x = part.ptr + (at + p * step) * HD + NC * lane;
 #pragma unroll
       for (int c = 0; c < NC; ++c) acc[c] = fmaf(x[c], w, acc[c]);
     }
@@ -344,11 +345,11 @@ constexpr int kFwdRowsPerWave = 32;
 // whole items, or parts of them (head dims 128 and 256)
 template <typename E, int NQB, int HD, int GC, int KT>
 void launch_fwd_wave(const ts_attn_problem& P, dim3 grid, ts_attn_rows q, ts_attn_rows out, float* lse, int64_t lse_ld,
-                     int parts, float* part, hipStream_t s) {
+                     int parts, PartSums part, hipStream_t s) {
   if (parts <= 1) {
     ts::TimedLaunch timed_("attention.fwd_kernel", s);
     hipLaunchKernelGGL((fwd_wave_kernel<E, NQB, HD, GC, KT>), grid, dim3(64 * 8 / NQB), 0, s, P, q, out, lse, lse_ld,
-                       nullptr);
+                       part);
     return;
   }
   if constexpr (HD % 128 == 0) {
@@ -365,7 +366,7 @@ void launch_fwd_wave(const ts_attn_problem& P, dim3 grid, ts_attn_rows q, ts_att
 
 template <typename E, int NQB, int HD, int KT>
 void launch_fwd_hd(const ts_attn_problem& P, int gc, dim3 grid, ts_attn_rows q, ts_attn_rows out, float* lse,
-                   int64_t lse_ld, int parts, float* part, hipStream_t s) {
+                   int64_t lse_ld, int parts, PartSums part, hipStream_t s) {
   if (gc == 4) launch_fwd_wave<E, NQB, HD, 4, KT>(P, grid, q, out, lse, lse_ld, parts, part, s);
   else if (gc == 2) launch_fwd_wave<E, NQB, HD, 2, KT>(P, grid, q, out, lse, lse_ld, parts, part, s);
   else launch_fwd_wave<E, NQB, HD, 1, KT>(P, grid, q, out, lse, lse_ld, parts, part, s);
@@ -373,7 +374,7 @@ void launch_fwd_hd(const ts_attn_problem& P, int gc, dim3 grid, ts_attn_rows q, 
 
 template <typename E>
 int launch_fwd_t(const ts_attn_problem& P, ts_attn_rows q, ts_attn_rows out, float* lse, int64_t lse_ld, int parts,
-                 float* part, hipStream_t s) {
+                 PartSums part, hipStream_t s) {
   const int group = P.hq / P.hkv;
   const int gc = heads_per_block(group);
   const dim3 grid((unsigned)(P.n_q_work * P.hkv * (group / gc)));
@@ -394,7 +395,7 @@ int launch_fwd_t(const ts_attn_problem& P, ts_attn_rows q, ts_attn_rows out, flo
 }
 
 int launch_fwd(const ts_attn_problem& P, ts_attn_rows q, ts_attn_rows out, float* lse, int64_t lse_ld, int parts,
-               float* part, hipStream_t s) {
+               PartSums part, hipStream_t s) {
   return P.dtype == kF16 ? launch_fwd_t<f16>(P, q, out, lse, lse_ld, parts, part, s)
                          : launch_fwd_t<bf16>(P, q, out, lse, lse_ld, parts, part, s);
 }

@@ -307,13 +307,28 @@ __device__ __forceinline__ void part_of(int keys, int part, int parts, int& begi
 }
 
 // Partial sums of a launch whose items are cut into parts: fp32 rows
-// [parts][hq][q_rows][head dim], then (forward) (m, l) pairs [parts][hq][q_rows][2].
-__host__ __device__ inline int64_t part_row(const ts_attn_problem& P, int part, int h, int64_t row) {
-  return ((int64_t)part * P.hq + h) * P.q_rows + row;
+// [parts][rows][head dim], then (forward) (m, l) pairs [parts][rows][2].  A part's
+// rows are the launch's (query head, row) pairs or, where these are fewer, the
+// (item, head chunk, row, head) slots of its items -- segments may cover a small
+// share of a long query.
+struct PartSums {
+  float* ptr;
+  int64_t rows;     // of a part
+  int32_t by_item;
+};
+inline PartSums part_sums(const ts_attn_problem& P, int64_t groups, int pairs, void* ptr) {
+  const int64_t by_row = (int64_t)P.hq * P.q_rows, by_item = groups * pairs;
+  return PartSums{(float*)ptr, by_item < by_row ? by_item : by_row, by_item < by_row};
 }
-template <int HD, typename T>
-__device__ __forceinline__ T* part_stats(const ts_attn_problem& P, T* part, int parts) {
-  return part + part_row(P, parts, 0, 0) * HD;
+// `group`: the work item and head chunk, of PAIRS (row, head) pairs each
+template <int PAIRS>
+__device__ __forceinline__ int64_t part_row(const ts_attn_problem& P, const PartSums& S, int part, int group, int pair,
+                                            int h, int64_t row) {
+  return part * S.rows + (S.by_item ? (int64_t)group * PAIRS + pair : (int64_t)h * P.q_rows + row);
+}
+template <int HD>
+__device__ __forceinline__ float* part_stats(const PartSums& S, int parts) {
+  return S.ptr + parts * S.rows * HD;
 }
 constexpr int kMergeBlocks = 16;  // work-groups that merge one item's parts
 
@@ -434,9 +449,9 @@ inline int kv_block_keys(int group, int head_dim) { return group % 4 == 0 && hea
 
 // launchers (one per kernel family); each returns a TS_* status
 // `parts` > 1: each item's keys in that many work-groups, partial sums in
-// `part` (split_part_floats per part), merged by a second kernel
+// `part`, merged by a second kernel
 int launch_fwd(const ts_attn_problem& P, ts_attn_rows q, ts_attn_rows out, float* lse, int64_t lse_ld, int parts,
-               float* part, hipStream_t s);
+               PartSums part, hipStream_t s);
 int launch_delta(const ts_attn_problem& P, ts_attn_rows out, ts_attn_rows dout, const float* lse,
                  float* rowstats, int64_t lse_ld, hipStream_t s);
 int launch_dq(const ts_attn_problem& P, ts_attn_rows q, ts_attn_rows dout, const float* rowstats,
@@ -456,7 +471,7 @@ template <typename E, bool DS>
 void launch_dkdv256(dim3 grid, const ts_attn_problem& P, ts_attn_rows q, ts_attn_rows dout,
                     const float* rowstats, int64_t lse_ld, const DsArgs& S, hipStream_t s);
 // dQ = scale dS K from the workspace the dK/dV launch filled
-int launch_dq_ds(const ts_attn_problem& P, const DsArgs& ds, ts_attn_rows dq, int parts, float* part,
+int launch_dq_ds(const ts_attn_problem& P, const DsArgs& ds, ts_attn_rows dq, int parts, PartSums part,
                  hipStream_t s);
 
 // the dS route: head dims 128 and 256 (the DMA-staged dK/dV kernels), every
