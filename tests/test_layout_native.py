@@ -78,3 +78,30 @@ def test_run_table_and_one_piece_upload():
             assert runs[f"{name}_row_stride"][r] == row and runs[f"{name}_head_stride"][r] == head
         assert runs["len"][r] == run.length
         assert (runs["visit0"][r], runs["nvisit"][r]) == (tabs["visit0"][r], tabs["nvisit"][r])
+
+
+def test_arrays_outlive_the_call_that_reads_them(monkeypatch):
+    """A layout's description may be made again by another thread while a call fills its
+    run table: the arrays that the native code reads stay as long as it runs."""
+    import gc
+    import weakref
+
+    lay = list(layouts())[3]
+    tabs = lay.device_tables(CPU, 64)
+    lib = _lib.require_library()
+
+    class Library:
+        @staticmethod
+        def ts_attn_run_table(*args):
+            arrays = [weakref.ref(a) for a in lay._desc["arrays"]]
+            lay._desc = None
+            gc.collect()
+            assert all(a() is not None for a in arrays)
+            return lib.ts_attn_run_table(*args)
+
+        ts_hip_last_error = lib.ts_hip_last_error
+
+    monkeypatch.setattr(_lib, "_LIB", Library())
+    out = np.zeros(len(lay.runs), att.RUN_DTYPE)
+    lay._fill_runs(tabs, [0x10000, 256, 128] * 8, out)
+    assert out["len"].tolist() == [r.length for r in lay.runs]

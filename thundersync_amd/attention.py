@@ -292,7 +292,8 @@ class AttnLayout:
 
     def _fill_runs(self, tabs: dict, sources: Sequence[int], out: np.ndarray) -> None:
         """One call's run table into ``out`` (``sources``: ts_attn_run_table's)."""
-        p = self._description()["ptrs"]
+        d = self._description()  # held: `_desc` may be another thread's by the time the native code reads the arrays
+        p = d["ptrs"]
         src = array("q", sources)
         _lib.check(
             _lib.require_library().ts_attn_run_table(
