@@ -621,10 +621,10 @@ __global__ __launch_bounds__(kThreads) void zero_fill(T* __restrict__ out, int64
 // --------------------------------------------------------------------------
 struct Geometry {
   int lpr;  // lanes per row (vector path); 0 = scalar path
-  int nv;   // vectors per lane (1, 2, 4, 8 or 16)
+  int nv;   // vectors per lane (1, 2, 4, 8, 10, 12 or 16)
 };
 
-Geometry pick(int64_t width, int dtype) {
+Geometry pick(int64_t width, int elem_bytes) {
   Geometry g{0, 0};
   if (width % 8 != 0) return g;
   const int64_t nvec = width / 8;
@@ -632,15 +632,17 @@ Geometry pick(int64_t width, int dtype) {
   while (lpr > 4 && lpr > nvec) lpr >>= 1;
   const int64_t nv = (nvec + lpr - 1) / lpr;
   // vectors per lane the kernel is built for: powers of two and, between 8 and
-  // 16, 10 (widths up to 5120) and 12 (6144), which keep eight waves a block where
-  // 16 has registers for four (8192 rows: 5120 73 -> 54 us, 6144 83 -> 64); 12 that
-  // do not fill the row spill (5632: 87 us against 78 through 16)
+  // 16, 10 and 12, which keep eight waves a block where 16 has registers for four.
+  // 16-bit types: 10 for widths up to 5120, 12 for 6144 (8192 rows: 5120 73 -> 54 us,
+  // 6144 83 -> 64; 12 that do not fill the row spill: 5632 87 us against 78 through
+  // 16).  fp32: 10 for 5120 alone (2048 rows 39 -> 35 us, 8192 113 -> 110); its 10 that
+  // do not fill the row and its 12 spill (8192 rows: 4608 122 us against 105 through
+  // 16, 6144 228 against 135).
   int nvp = 1;
   while (nvp < nv) nvp <<= 1;
-  if (nvp == 16 && nv <= 10) nvp = 10;
-  if (nvp == 16 && nvec == 12 * kWave) nvp = 12;
+  if (nvp == 16 && (elem_bytes == 2 ? nv <= 10 : nvec == 10 * kWave)) nvp = 10;
+  if (nvp == 16 && elem_bytes == 2 && nvec == 12 * kWave) nvp = 12;
   if (nvp > 16) return g;  // wider than 8192: scalar path
-  (void)dtype;
   g.lpr = lpr;
   g.nv = nvp;
   return g;
@@ -653,7 +655,7 @@ int64_t bwd_parts(int64_t rows, int64_t width) {
   // 64 blocks of 32 rows 32 us, 256 of 8 20; 64 x 4096 26 -> 15); at most 256 blocks for rows
   // of 2048 and more elements -- one 8-wave block per CU is enough bytes in
   // flight there -- and up to 1024 for narrower rows, whose blocks carry less
-  const Geometry g = pick(width, 0);
+  const Geometry g = pick(width, 2);
   const int64_t pass = g.lpr > 16 ? 8 * (kWave / g.lpr) : 32;
   int64_t parts = (rows + pass - 1) / pass;
   const int64_t max_parts = width >= 2048 ? 256 : 1024;
@@ -717,7 +719,7 @@ int launch_fwd(const void* x, const void* w, void* y, float* rstd, int64_t rows,
 template <typename T>
 int launch_bwd(const void* dy, const void* x, const void* w, const float* rstd, void* dx,
                void* dw, float* part, int64_t rows, int width, hipStream_t s) {
-  const Geometry g = pick(width, 0);
+  const Geometry g = pick(width, sizeof(T));
   const int64_t parts = bwd_parts(rows, width);
   const int64_t slab = (rows + parts - 1) / parts;
   const int want_dx = dx != nullptr, want_dw = dw != nullptr;
@@ -739,20 +741,27 @@ int launch_bwd(const void* dy, const void* x, const void* w, const float* rstd, 
 #define TS_BWD(LPR, NV)                                                                      \
   if (!launched && g.lpr == LPR && g.nv == NV) {                                             \
     ts::TimedLaunch timed_("rmsnorm.rmsnorm_bwd_vec", s);                                    \
-    if (full)                                                                                \
+    if constexpr (NV != 12 && (NV != 10 || sizeof(T) == 2))                                  \
+      if (!full) {                                                                           \
+        hipLaunchKernelGGL((rmsnorm_bwd_vec<T, LPR, NV, false>), grid,                       \
+                           dim3(BwdShape<T, NV, false>::kThreads), lds, s,                   \
+                           (const T*)dy, (const T*)x, (const T*)w, rstd, (T*)dx, part, rows, \
+                           width, slab, want_dx, want_dw);                                   \
+        launched = true;                                                                     \
+      }                                                                                      \
+    if (full) {                                                                              \
       hipLaunchKernelGGL((rmsnorm_bwd_vec<T, LPR, NV, true>), grid,                          \
                          dim3(BwdShape<T, NV, true>::kThreads), lds, s,                      \
                          (const T*)dy, (const T*)x, (const T*)w, rstd, (T*)dx, part, rows,   \
                          width, slab, want_dx, want_dw);                                     \
-    else                                                                                     \
-      hipLaunchKernelGGL((rmsnorm_bwd_vec<T, LPR, NV, false>), grid,                         \
-                         dim3(BwdShape<T, NV, false>::kThreads), lds, s,                     \
-                         (const T*)dy, (const T*)x, (const T*)w, rstd, (T*)dx, part, rows,   \
-                         width, slab, want_dx, want_dw);                                     \
-    launched = true;                                                                         \
+      launched = true;                                                                       \
+    }                                                                                        \
   }
     TS_BWD(4, 1) TS_BWD(8, 1) TS_BWD(16, 1) TS_BWD(32, 1) TS_BWD(64, 1)
-    TS_BWD(4, 2) TS_BWD(8, 2) TS_BWD(16, 2) TS_BWD(32, 2) TS_BWD(64, 2) TS_BWD(64, 4) TS_BWD(64, 8) TS_BWD(64, 10) TS_BWD(64, 12) TS_BWD(64, 16)
+    TS_BWD(4, 2) TS_BWD(8, 2) TS_BWD(16, 2) TS_BWD(32, 2) TS_BWD(64, 2) TS_BWD(64, 4) TS_BWD(64, 8) TS_BWD(64, 10) TS_BWD(64, 16)
+    if constexpr (sizeof(T) == 2) {
+      TS_BWD(64, 12)
+    }
 #undef TS_BWD
     if (!launched) {
       set_error("ts_rmsnorm_bwd: no kernel for width %d", width);
