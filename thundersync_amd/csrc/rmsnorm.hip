@@ -650,14 +650,16 @@ Geometry pick(int64_t width, int elem_bytes) {
 
 int64_t bwd_parts(int64_t rows, int64_t width) {
   // at least one pass of the block's eight waves per block (8 rows, or 8 64 / LPR
-  // narrow ones up to 32): the partial rows, written and read once, are then at most a
-  // sixth of the kernel's traffic, and short launches fill the CUs (2048 x 4096:
-  // 64 blocks of 32 rows 32 us, 256 of 8 20; 64 x 4096 26 -> 15); at most 256 blocks for rows
+  // narrow ones up to 32) while the launch has at most a block per CU: short launches
+  // then fill the CUs (2048 x 4096: 64 blocks of 32 rows 32 us, 256 of 8 20; 64 x 4096
+  // 26 -> 15), and the partial rows, written and read once, are at most a sixth of the
+  // kernel's traffic.  Longer launches take 32 rows a block (16384 x 1024: 512 blocks
+  // 22.4 us and 6.2 for their sum, 1024 of 16 rows 26.4 and 7.0); at most 256 blocks for rows
   // of 2048 and more elements -- one 8-wave block per CU is enough bytes in
   // flight there -- and up to 1024 for narrower rows, whose blocks carry less
-  const Geometry g = pick(width, 2);
+  const Geometry g = pick(width, 2);  // lanes per row: the same for every type
   const int64_t pass = g.lpr > 16 ? 8 * (kWave / g.lpr) : 32;
-  int64_t parts = (rows + pass - 1) / pass;
+  int64_t parts = std::max(std::min<int64_t>((rows + pass - 1) / pass, 256), (rows + 31) / 32);
   const int64_t max_parts = width >= 2048 ? 256 : 1024;
   if (parts > max_parts) parts = max_parts;
   if (parts < 1) parts = 1;
