@@ -52,3 +52,17 @@ def test_backward(cuda, rows, width, dtype):
     slack_dw = 2.0 ** -24 * (rows + 8) * (gd * xd * r).abs().sum(0)
     assert bool(((dx.double() - want_dx).abs() <= unit * want_dx.abs() + slack_dx).all())
     assert bool(((dw.double() - want_dw).abs() <= unit * want_dw.abs() + slack_dw).all())
+
+
+@pytest.mark.parametrize("rows", [1024, 1025, 2048, 2049])
+@pytest.mark.parametrize("width", [6148, 7168])
+def test_forward_bytes_of_wide_fp32_rows(cuda, rows, width):
+    """fp32 rows of 32 vectors: launches of 257 to 512 blocks of four rows load the weight
+    after the reduction, the others beside the row."""
+    test_forward_bytes(cuda, rows, width, torch.float32)
+
+
+@pytest.mark.parametrize("rows,width", [(255 * 8, 512), (256 * 32, 512), (256 * 32 + 1, 1024), (2049, 1536)])
+def test_backward_of_narrow_rows(cuda, rows, width):
+    """Rows per block: one pass of its waves up to 256 blocks, 32 rows from there."""
+    test_backward(cuda, rows, width, torch.bfloat16)

@@ -245,7 +245,11 @@ template <typename T> __device__ __forceinline__ float primal(float w, float x, 
 // Non-temporal stores make that first launch 51.7 us in a stream of others, but a
 // pass by itself, forward and backward, 13 us longer (140 -> 153): the last-level
 // cache then takes no part of the output, which the next kernel would find there.
-template <typename T, bool VEC, int NV>
+// HOLD false loads the weight after the reduction: for fp32 rows of 32 vectors in
+// launches that its 186 registers (two blocks a CU) take in one round and the 308
+// of the other in two (2048 x 7168: 24.6 us against 27.2; but 64 rows 11.6 and 9.1,
+// 16384 rows 224 and 205).
+template <typename T, bool VEC, int NV, bool HOLD = true>
 __global__ __launch_bounds__(kThreads) void rmsnorm_fwd_lanes(
     const T* __restrict__ x, const T* __restrict__ w, T* __restrict__ y,
     float* __restrict__ rstd, int64_t rows, int width, int bw, float factor, float eps) {
@@ -263,8 +267,10 @@ __global__ __launch_bounds__(kThreads) void rmsnorm_fwd_lanes(
 #pragma unroll
     for (int k = 0; k < NV; ++k) v[k] = load4<T>(xr + min(sub + k * bw, nvec - 1) * 4);
     Raw4<T> wr[NV];
+    if constexpr (HOLD) {
 #pragma unroll
-    for (int k = 0; k < NV; ++k) wr[k] = load4<T>(w + min(sub + k * bw, nvec - 1) * 4);
+      for (int k = 0; k < NV; ++k) wr[k] = load4<T>(w + min(sub + k * bw, nvec - 1) * 4);
+    }
     float acc[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
@@ -287,7 +293,8 @@ __global__ __launch_bounds__(kThreads) void rmsnorm_fwd_lanes(
       if (vi < nvec) {
         float f[4], wv[4], o[4];
         unpack4<T>(v[k], f);
-        unpack4<T>(wr[k], wv);
+        if constexpr (HOLD) unpack4<T>(wr[k], wv);
+        else unpack4<T>(load4<T>(w + vi * 4), wv);
 #pragma unroll
         for (int i = 0; i < 4; ++i) o[i] = primal<T>(wv[i], f[i], r);
         store4<T>(yr + vi * 4, o);
@@ -699,6 +706,11 @@ int launch_fwd(const void* x, const void* w, void* y, float* rstd, int64_t rows,
       return check_launch("ts_rmsnorm_fwd");
     }
     const int loads = (width / 4 + c.bw - 1) / c.bw;
+    if (sizeof(T) == 4 && loads > 24 && loads <= 32 && grid.x > 256 && grid.x <= 512) {
+      hipLaunchKernelGGL((rmsnorm_fwd_lanes<T, true, 32, sizeof(T) != 4>), grid, dim3(kThreads), 0, s,
+                         (const T*)x, (const T*)w, (T*)y, rstd, rows, width, c.bw, factor, eps);
+      return check_launch("ts_rmsnorm_fwd");
+    }
 #define TS_FWD(NV)                                                                             \
   if (loads <= NV) {                                                                           \
     hipLaunchKernelGGL((rmsnorm_fwd_lanes<T, true, NV>), grid, dim3(kThreads), 0, s,           \
