@@ -48,7 +48,7 @@ def device_flags() -> list[str]:
 # written to VGPRs spare it per-tile copies out of the accumulation registers.
 FILE_FLAGS = {
     "attention_dq.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
-    # the one-wave-per-head dK/dV kernel: S and dP in VGPRs (MFMA results in
+    # the dK/dV kernel whose waves take steps of their own: S and dP in VGPRs (MFMA results in
     # VGPRs), its dK/dV accumulators in the accumulation registers through
     # inline assembly
     "attention_dkdv_wave.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],

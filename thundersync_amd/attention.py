@@ -86,10 +86,6 @@ def q_block_rows(hq: int, hkv: int) -> int:
     return 32 * 4 // heads_per_block(hq // hkv)
 
 
-# rows per item of the dS route's dQ pass at GQA groups that are a multiple of 4
-DQ_BLOCK_ROWS = 64
-
-
 def kv_block_keys(hq: int, hkv: int, head_dim: int = HEAD_DIM) -> int:
     """Keys per dK/dV work-group (mirror of ts_attn_kv_block): 64 at head dim
     256 and for GQA groups that are not a multiple of 4, else 48."""
@@ -113,13 +109,14 @@ DKDV256_MIN_ITEMS = 512
 # where there are many items of few.  A launch takes about
 #     start + round * rounds + step * max(tail * longest item's steps, steps a slot)
 # us, slots being the work-groups the device holds at once and rounds the items
-# over them: fitted to 186 launches (one sequence over a context, cohorts, packs; 16
+# over them: fitted to 266 launches (one sequence over a context, cohorts, packs; 16
 # to 9000 rows over up to 14000 keys) at head counts from 32/4 to 8/8, where the
-# choice costs 0.3 % on average and at most 13 % (24/8 heads, 8 sequences of 512 to
-# 2048 rows: 290 us dealt, 258 split).  By the average steps of an item alone it
-# cost 3.6 % and up to 79 %: dealt against split 146 / 101 us for 16 sequences of 256
-# to 1024 rows at 16/8, 130 / 103 for 256 rows over 8448 keys at 24/8, 31 / 41 for 4
-# sequences of 256 to 1024 rows at 8/8.
+# choice costs 0.4 % on average and at most 13 % (24/8 heads, 8 sequences of 512 to
+# 2048 rows: 290 us dealt, 258 split; outside them 133 rows over 1605 keys at 40/8,
+# just past one round of dealt items: 50 and 35).  By the average steps of an item
+# alone it cost 3.6 % and up to 79 %: dealt against split 146 / 101 us for 16
+# sequences of 256 to 1024 rows at 16/8, 130 / 103 for 256 rows over 8448 keys at
+# 24/8, 31 / 41 for 4 sequences of 256 to 1024 rows at 8/8.
 # (slots, start, round, step, tail) of the dealt and the key-split kernel
 DKDV_DEALT = (256, 4.0, 12.0, 0.46, 0.7)
 DKDV_SPLIT = (512, 10.0, 0.0, 1.8, 0.55)
@@ -429,7 +426,9 @@ class AttnLayout:
 # Otherwise only the items long enough to stretch the end of the launch when
 # started late -- a quarter or more of a slot's average share of the whole
 # launch -- and the rest run head by head, all XCDs streaming one head's rows
-# through the shared cache.  (ts_attn_layout_tables builds the lists.)
+# through the shared cache.  ts_attn_layout_tables builds the lists, by its own
+# copy of this constant (kOrderBand, attention_tables.hip); this one is for readers
+# of the lists.
 ORDER_BAND = 0.05
 
 

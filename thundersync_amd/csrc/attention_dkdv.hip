@@ -23,7 +23,7 @@ namespace attn {
 // zero dO row; at head dims 32, 64, 96 and 192 their P is also set to 0, which
 // holds beside a key with an infinite component too).  S = Q K^T and dP = dO V^T take the Q/dO rows as A operands;
 // dV^T += dO^T P and dK^T += Q^T dS take dO^T / Q^T from ds_read_b64_tr_b16
-// (the lane layout of the one-wave-per-head kernel).  A wave past the work
+// (the lane layout of the kernel with steps of its own for each wave).  A wave past the work
 // item's keys (kv_block 48) only issues its DMA share; only steps that cross
 // the diagonal are masked.
 //

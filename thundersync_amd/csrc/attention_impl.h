@@ -201,11 +201,6 @@ __device__ __forceinline__ int ds_store_offset(int lane) {
   return 64 * j16 + 16 * (g4 ^ ((j16 >> 1) & 2));
 }
 
-
-
-
-constexpr int kKV64 = BK * D;  // elements of one 64-key tile
-
 struct TileCursor {
   int sp;          // span index; == nspan at the end
   int kt0;         // first run-local key of the tile
@@ -460,8 +455,9 @@ int launch_dq(const ts_attn_problem& P, ts_attn_rows q, ts_attn_rows dout, const
 // (only where ds_route holds)
 int launch_dkdv(const ts_attn_problem& P, ts_attn_rows q, ts_attn_rows dout, const float* rowstats,
                 int64_t lse_ld, const DsArgs* ds, hipStream_t s);
-// the one-wave-per-head dK/dV kernel (groups that are a multiple of 4, head
-// dim 128; attention_dkdv_wave.hip), storing dS when DS
+// the dK/dV kernel whose waves take (query head, row block) steps of their own
+// (48-key work items at head dim 128, every group; attention_dkdv_wave.hip),
+// storing dS when DS
 template <typename E, bool DS>
 void launch_dkdv_wave(dim3 grid, const ts_attn_problem& P, ts_attn_rows q, ts_attn_rows dout,
                       const float* rowstats, int64_t lse_ld, const DsArgs& S, hipStream_t s);

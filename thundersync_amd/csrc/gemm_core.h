@@ -1,5 +1,6 @@
-// MFMA GEMM core for gfx950: one 256 x 256 work-group tile of C = A . B^T
-// (bf16 or fp16 operands E, fp32 accumulation), shared by the logprob and LoRA kernels.
+// MFMA GEMM core for gfx950: one work-group tile of C = A . B^T, 256 A rows by 256 B rows
+// (64 to 320 with the other shapes below; bf16 or fp16 operands E, fp32 accumulation),
+// shared by the logprob and LoRA kernels.
 //
 // 8 waves of 128 x 64 (two per SIMD, so one wave's memory instructions overlap
 // the other's MFMAs), v_mfma_f32_32x32x16_bf16.  K streams 32 at a time

@@ -16,11 +16,12 @@
 //             registers, rounds it to bf16 (the reference rounds dlogits to the
 //             hidden dtype before its VJP GEMM, fused_logprob.py:165, :295) and
 //             stores a [rows, V] bf16 block; a second GEMM multiplies it by
-//             W (given as W^T so both operands are K-contiguous) into dh.
+//             W, read in place (its rows are the contraction index), into dh,
+//             and for a trainable head a third by the hidden states into dW.
 //
-// GEMM core (gemm_core.h): 256 x 256 work-group tiles on
-// v_mfma_f32_32x32x16_bf16, K streamed through a 4-stage LDS ring by
-// buffer_load ... lds.
+// GEMM core (gemm_core.h): work-group tiles of 256 vocabulary rows (or hidden
+// dims) x 64 to 320 tokens on v_mfma_f32_32x32x16_bf16, K streamed through a
+// 4-stage LDS ring by buffer_load ... lds.
 #include <algorithm>
 #include <type_traits>
 
@@ -34,7 +35,7 @@ namespace lp {
 
 using namespace ts::gemm;
 
-constexpr int kThreads = 256;      // combine / transpose kernels
+constexpr int kThreads = 256;      // grad_hidden_reduce_kernel
 constexpr int BM = TM;   // vocab rows per forward partial
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
@@ -66,7 +67,6 @@ struct FwdArgs {
   int64_t ldh;
   const bf16* w;
   int64_t ldw;
-  const int64_t* target;
   int rows, dim, vocab;
   int n_ttiles, n_vtiles;
   float* part_m;   // [n_vtiles][rows]
@@ -621,7 +621,6 @@ int ts_logprob_fwd(const void* hidden, int64_t ld_hidden, const void* weight, in
   a.ldh = ld_hidden;
   a.w = (const ts::bf16*)weight;
   a.ldw = ld_weight;
-  a.target = target;
   a.rows = (int)rows;
   a.dim = (int)dim;
   a.vocab = (int)vocab;
