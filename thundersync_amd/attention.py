@@ -801,7 +801,9 @@ def _saved_gradients(ctx, dout: torch.Tensor):
     dq, dkeys, dvalues, ctx.keep_bwd = _attention_backward(query, out, lse, _pad_heads(dout, query.shape[-1]),
                                                            ctx.layout, ctx.scale, kv[:n], kv[n:])
     if query.shape[-1] != d:
-        dq, dkeys, dvalues = dq[..., :d], [g[..., :d] for g in dkeys], [g[..., :d] for g in dvalues]
+        # dense gradients that do not keep the padded ones
+        dq, *rest = (g[..., :d].clone() for g in (dq, *dkeys, *dvalues))
+        dkeys, dvalues = rest[:n], rest[n:]
     return dq, dkeys, dvalues
 
 
