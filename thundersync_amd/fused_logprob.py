@@ -92,7 +92,8 @@ def _rows_ok(t: torch.Tensor) -> torch.Tensor:
 
 
 def _unit_stride(t: torch.Tensor) -> torch.Tensor:
-    return t if t.stride(1) == 1 or t.shape[1] <= 1 else t.contiguous()
+    unit = t.stride(1) == 1 or t.shape[1] <= 1
+    return t if unit and (t.stride(0) >= t.shape[1] or t.shape[0] <= 1) else t.contiguous()
 
 
 def _forward_exact(hidden, weight, target, with_entropy):
