@@ -4,6 +4,8 @@ one-piece upload of a new layout with a call's run table."""
 
 from __future__ import annotations
 
+from pathlib import Path
+
 import numpy as np
 import pytest
 import torch
@@ -105,3 +107,32 @@ def test_arrays_outlive_the_call_that_reads_them(monkeypatch):
     out = np.zeros(len(lay.runs), att.RUN_DTYPE)
     lay._fill_runs(tabs, [0x10000, 256, 128] * 8, out)
     assert out["len"].tolist() == [r.length for r in lay.runs]
+
+
+def test_host_memory_is_an_error():
+    """Tables that do not fit the host's memory are an error of the call, not the process's end."""
+    import subprocess
+    import sys
+
+    code = """
+import resource, ctypes, sys
+from pathlib import Path
+
+import numpy as np
+from thundersync_amd import _lib, attention as att
+from thundersync_amd._abi import AttnLayoutDesc, AttnLayoutSizes
+lib = _lib.require_library()
+lay = att.chain_layout(1 << 29, [1 << 29], 32, 8)
+p = lay._description()["ptrs"]
+desc = AttnLayoutDesc(lay.q_rows, 1, 32, 8, 1, 1, 48, 0, p[0], p[1], p[2], p[3])
+sizes = AttnLayoutSizes()
+assert lib.ts_attn_layout_tables(ctypes.byref(desc), None, 0, None, ctypes.byref(sizes)) == 0
+run_visits, blob = np.zeros((1, 2), np.int32), np.zeros(sizes.bytes, np.uint8)  # pages come when they are written
+used = int(open("/proc/self/statm").read().split()[0]) * resource.getpagesize()
+resource.setrlimit(resource.RLIMIT_AS, (used + (64 << 20), resource.getrlimit(resource.RLIMIT_AS)[1]))
+status = lib.ts_attn_layout_tables(ctypes.byref(desc), blob.ctypes.data, sizes.bytes, run_visits.ctypes.data, ctypes.byref(sizes))
+sys.exit(0 if status != 0 else 3)
+"""
+    root = str(Path(__file__).resolve().parents[1])
+    done = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120, cwd=root)
+    assert done.returncode == 0, (done.returncode, done.stderr[-400:])

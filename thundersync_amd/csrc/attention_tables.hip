@@ -2,6 +2,7 @@
 // table, built in one pass each (a streamed chunk builds both on every call).
 #include <algorithm>
 #include <cmath>
+#include <exception>
 #include <vector>
 
 #include "attention_impl.h"
@@ -75,13 +76,8 @@ struct WorkList {
 
 int64_t align256(int64_t n) { return (n + 255) / 256 * 256; }
 
-}  // namespace attn
-}  // namespace ts
-
-extern "C" int ts_attn_layout_tables(const ts_attn_layout* layout, void* blob, int64_t blob_bytes, int32_t* run_visits,
-                                     ts_attn_layout_sizes* sizes) {
-  using namespace ts::attn;
-  const char* what = "ts_attn_layout_tables";
+int layout_tables(const ts_attn_layout* layout, void* blob, int64_t blob_bytes, int32_t* run_visits,
+                  ts_attn_layout_sizes* sizes, const char* what) {
   TS_CHECK_ARG(layout && sizes, "%s: null argument", what);
   const ts_attn_layout& L = *layout;
   TS_CHECK_ARG(L.hq > 0 && L.hkv > 0 && L.hq % L.hkv == 0 && L.kv_block > 0 && L.n_segs >= 0 && L.n_runs >= 0 &&
@@ -216,6 +212,20 @@ extern "C" int ts_attn_layout_tables(const ts_attn_layout* layout, void* blob, i
   z.ds_head = ds;
   *sizes = z;
   return TS_OK;
+}
+
+}  // namespace attn
+}  // namespace ts
+
+extern "C" int ts_attn_layout_tables(const ts_attn_layout* layout, void* blob, int64_t blob_bytes, int32_t* run_visits,
+                                     ts_attn_layout_sizes* sizes) {
+  const char* what = "ts_attn_layout_tables";
+  try {
+    return ts::attn::layout_tables(layout, blob, blob_bytes, run_visits, sizes, what);
+  } catch (const std::exception& e) {  // host memory
+    ts::set_error("%s: %s", what, e.what());
+    return TS_ERR_INVALID;
+  }
 }
 
 extern "C" int ts_attn_run_table(int32_t n_runs, const int32_t* run_len, const int32_t* run_source,
