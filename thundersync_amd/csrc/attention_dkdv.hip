@@ -27,11 +27,12 @@ namespace attn {
 // item's keys (kv_block 48) only issues its DMA share; only steps that cross
 // the diagonal are masked.
 //
-// Every wave reads the whole step from LDS for 16 of its keys, which bounds the
-// steps (16 KB of LDS reads a wave for 16 MFMAs at head dim 64).  Against
-// staging each step through registers between two barriers, with 48-key items
-// at groups of 4 (8 sequences of 512 to 2048 rows, us): head dim 64 at 16/8 heads
-// 184 -> 131, at 32/8 712 -> 300, 96 at 16/8 310 -> 167, 192 at 24/4 1222 -> 512.
+// Every wave reads the whole step from LDS for 16 of its keys (16 KB of LDS reads
+// a wave for 16 MFMAs at head dim 64, where the VALU is 46 % busy, LDS 31 % and the
+// matrix cores 25 %).  Against staging each step through registers between two
+// barriers, with 48-key items at groups of 4 (8 sequences of 512 to 2048 rows, us):
+// head dim 64 at 16/8 heads 197 -> 106, at 32/8 473 -> 237, 96 at 16/8 311 -> 143,
+// 192 at 24/4 1326 -> 564.
 // ---------------------------------------------------------------------------
 template <typename E, int HD, bool DS = false>
 __global__ __launch_bounds__(kThreads, 1) void dkdv_split_kernel(ts_attn_problem P, ts_attn_rows Q,

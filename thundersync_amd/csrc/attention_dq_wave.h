@@ -31,8 +31,8 @@ namespace attn {
 // the row's scores are low (dS past the element type's range, times its zero K
 // row: NaN).  Against
 // tiles passed through registers between two barriers (8 sequences of 512 to 2048
-// rows, us): head dim 64 at 16/8 heads 115 -> 71, 32 75 -> 48, 96 143 -> 98, 192 at
-// 24/4 647 -> 387.
+// rows, us): head dim 64 at 16/8 heads 87 -> 58, 32 62 -> 39, 96 108 -> 80, 192 at
+// 24/4 478 -> 299.
 // ---------------------------------------------------------------------------
 template <typename E, int NQB, int HD = D, int GC = 4, int NP = 1>
 __global__ __launch_bounds__(64 * 8 / (NQB * NP), 1) void dq_wave_kernel(ts_attn_problem P, ts_attn_rows Q, ts_attn_rows dO,
