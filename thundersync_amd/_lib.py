@@ -226,6 +226,16 @@ def dtype_code(dtype) -> int:
     return code
 
 
+def current_stream(device) -> int:
+    """The current HIP stream of ``device``, as an integer handle."""
+    import torch
+
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if raw is not None and device.index is not None:
+        return raw(device.index)
+    return torch.cuda.current_stream(device).cuda_stream
+
+
 def stream_of(tensor) -> int:
     """The current HIP stream of ``tensor``'s device, as an integer handle."""
     import torch

@@ -340,11 +340,16 @@ class AttnLayout:
                     base = dev.data_ptr()
                     tabs.update(
                         blob=dev, host=host, segs=base + sizes.segs, seg_spans=base + sizes.spans,
+                    if device.type == "cuda":
+                        tabs["stream"] = _lib.current_stream(device)
+                        tabs["streams"] = {tabs["stream"]}
                         run_visits_dev=base + sizes.visits, q_work=base + sizes.q_work, kv_work=base + sizes.kv_work,
                         dq_work=base + sizes.dq_work if sizes.n_dq_work else None,
                         span=base + sizes.span_ds, visit=base + sizes.visit_ds,
                     )
                     self._tables[key] = tabs
+        if device.type == "cuda":
+            _order_after_upload(tabs, device)
                     if sources is not None:
                         return tabs, (base + sizes.bytes, view[sizes.bytes : sizes.bytes + run_bytes], (dev, host))
         if sources is None:
@@ -428,6 +433,19 @@ class AttnLayout:
 # launch -- and the rest run head by head, all XCDs streaming one head's rows
 # through the shared cache.  ts_attn_layout_tables builds the lists, by its own
 # copy of this constant (kOrderBand, attention_tables.hip); this one is for readers
+def _order_after_upload(tabs: dict, device) -> None:
+    """Let the current stream read tables that another one uploads: it waits for
+    the upload (whose stream may not have run it yet), and the tables' memory is
+    its to read until it has.  Once per stream; a capture takes tables that its
+    stream has used before, or that are long there."""
+    if _lib.current_stream(device) in tabs["streams"] or torch.cuda.is_current_stream_capturing():
+        return
+    stream = torch.cuda.current_stream(device)
+    stream.wait_stream(torch.cuda.ExternalStream(tabs["stream"], device=device))
+    tabs["blob"].record_stream(stream)
+    tabs["streams"].add(_lib.current_stream(device))
+
+
 # of the lists.
 ORDER_BAND = 0.05
 
