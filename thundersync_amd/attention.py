@@ -117,18 +117,15 @@ DKDV256_MIN_ITEMS = 512
 # alone it cost 3.6 % and up to 79 %: dealt against split 146 / 101 us for 16
 # sequences of 256 to 1024 rows at 16/8, 130 / 103 for 256 rows over 8448 keys at
 # 24/8, 31 / 41 for 4 sequences of 256 to 1024 rows at 8/8.
-# (slots, start, round, step, tail) of the dealt and the key-split kernel
-DKDV_DEALT = (256, 4.0, 12.0, 0.46, 0.7)
-DKDV_SPLIT = (512, 10.0, 0.0, 1.8, 0.55)
-
-
-def _dkdv_us(kernel, items: int, group: int, mean_rows: float, most_rows: int) -> float:
-    """Estimated us of a dK/dV launch of `items` work items, each seen by
-    `mean_rows` query rows on average and `most_rows` at most."""
-    slots, start, per_round, step, tail = kernel
-    rounds = items / slots
-    work = max(tail * most_rows, mean_rows * rounds)
-    return start + per_round * (rounds if rounds > 1.0 else 1.0) + step * group * work / 32
+def _dealt_is_faster(items48: int, items64: int, group: int, mean: float, most: int) -> bool:
+    """Whether 48-key items are estimated to end sooner than 64-key ones, given
+    the items of either size and the query rows that an item sees, on average and
+    at most.  Dealt out: start 4, round 12, step 0.46 us, tail 0.7 over 256 slots;
+    key-split: 10, none, 1.8, 0.55 over 512."""
+    dealt, split = items48 / 256, items64 / 512  # rounds
+    steps = group / 32  # of a row
+    return (4.0 + 12.0 * max(dealt, 1.0) + 0.46 * steps * max(0.7 * most, mean * dealt)
+            < 10.0 + 1.8 * steps * max(0.55 * most, mean * split))
 
 
 # ---------------------------------------------------------------------------
@@ -230,8 +227,6 @@ class AttnLayout:
                 key_rows += length
                 items48 += (length + 47) // 48
                 items64 += (length + 63) // 64
-            # the GQA group, and the query rows that see a visited key, on average and at most
-            rows = (self.hq // self.hkv, self.visible_pairs() / max(key_rows, 1), max(users.values(), default=0))
             d = {
                 "arrays": arrays,
                 "ptrs": tuple(a.buffer_info()[0] if len(a) else None for a in arrays),
@@ -240,8 +235,9 @@ class AttnLayout:
                 "items64": items64,
                 # sources with rows that no visited run covers: their gradients are filled with zeros first
                 "uncovered": [i for i, n in enumerate(self.source_rows) if covered[i] != n],
-                "kv_block128": 48 if _dkdv_us(DKDV_DEALT, items48 * self.hkv, *rows)
-                < _dkdv_us(DKDV_SPLIT, items64 * self.hkv, *rows) else 64,
+                "kv_block128": 48 if _dealt_is_faster(
+                    items48 * self.hkv, items64 * self.hkv, self.hq // self.hkv,
+                    self.visible_pairs() / max(key_rows, 1), max(users.values(), default=0)) else 64,
                 "max_keys": max((kv for kv, (_, n) in zip(self.seg_kv, self.seg_q) if n), default=0),
                 "all_rows": sum(n for _, n in self.seg_q) == self.q_rows,
             }
@@ -340,20 +336,20 @@ class AttnLayout:
                     base = dev.data_ptr()
                     tabs.update(
                         blob=dev, host=host, segs=base + sizes.segs, seg_spans=base + sizes.spans,
-                    if device.type == "cuda":
-                        tabs["stream"] = _lib.current_stream(device)
-                        tabs["streams"] = {tabs["stream"]}
                         run_visits_dev=base + sizes.visits, q_work=base + sizes.q_work, kv_work=base + sizes.kv_work,
                         dq_work=base + sizes.dq_work if sizes.n_dq_work else None,
                         span=base + sizes.span_ds, visit=base + sizes.visit_ds,
                     )
+                    if device.type == "cuda":
+                        tabs["stream"] = _lib.current_stream(device)
+                        tabs["streams"] = {tabs["stream"]}
                     self._tables[key] = tabs
-        if device.type == "cuda":
-            _order_after_upload(tabs, device)
                     if sources is not None:
                         return tabs, (base + sizes.bytes, view[sizes.bytes : sizes.bytes + run_bytes], (dev, host))
         if sources is None:
             return tabs, None
+        if device.type == "cuda":
+            _order_after_upload(tabs, device)
         host = alloc(run_bytes)
         view = host.numpy()
         self._fill_runs(tabs, sources, view)
@@ -387,7 +383,7 @@ class AttnLayout:
     def call_kv_block(self, device, head_dim: int) -> int:
         """Keys per dK/dV work item of this package's own calls: kv_block_for's,
         except that at head dim 128 every GQA group takes either kernel, whichever
-        is estimated to end sooner (_dkdv_us), and at the head dims that only the
+        is estimated to end sooner (_dealt_is_faster), and at the head dims that only the
         key-split kernel takes, whose four waves hold 16 keys each, every group has
         64."""
         if head_dim == 256:
@@ -397,9 +393,9 @@ class AttnLayout:
         return self._description()["kv_block128"]
 
     def problem(self, device, runs_ptr: int, scale: float, dtype: torch.dtype = torch.bfloat16,
-                head_dim: int = HEAD_DIM, kv_block: int | None = None) -> AttnProblem:
+                head_dim: int = HEAD_DIM, kv_block: int | None = None, tables: dict | None = None) -> AttnProblem:
         kvb = self.kv_block_for(device, int(head_dim)) if kv_block is None else kv_block
-        t = self.device_tables(device, kvb)
+        t = tables or self.device_tables(device, kvb)
         return AttnProblem(
             t["segs"], t["seg_spans"], runs_ptr, t["run_visits_dev"], t["q_work"], t["kv_work"],
             t["n_q_work"], t["n_kv_work"], len(self.seg_q), len(self.runs), self.hq, self.hkv,
@@ -433,6 +429,10 @@ class AttnLayout:
 # launch -- and the rest run head by head, all XCDs streaming one head's rows
 # through the shared cache.  ts_attn_layout_tables builds the lists, by its own
 # copy of this constant (kOrderBand, attention_tables.hip); this one is for readers
+# of the lists.
+ORDER_BAND = 0.05
+
+
 def _order_after_upload(tabs: dict, device) -> None:
     """Let the current stream read tables that another one uploads: it waits for
     the upload (whose stream may not have run it yet), and the tables' memory is
@@ -444,10 +444,6 @@ def _order_after_upload(tabs: dict, device) -> None:
     stream.wait_stream(torch.cuda.ExternalStream(tabs["stream"], device=device))
     tabs["blob"].record_stream(stream)
     tabs["streams"].add(_lib.current_stream(device))
-
-
-# of the lists.
-ORDER_BAND = 0.05
 
 
 def _check_rows_tensor(t: torch.Tensor, name: str, heads: int, head_dim: int, max_row_stride: int = 1 << 24) -> None:
@@ -465,13 +461,13 @@ def _rows(t: torch.Tensor) -> AttnRows:
 
 
 def check_tables(layout: AttnLayout, problem: AttnProblem, run_table: np.ndarray | torch.Tensor,
-                 device: torch.device) -> None:
+                 device: torch.device, tables: dict | None = None) -> None:
     """Check the layout's tables for ``device`` and one call's run table on the
     host (ts_attn_check_tables) before the kernels read their device copies:
     spans tile every segment's keys, every visit is a span of its segment,
     the work lists hold every row and key block once, K/V/dK/dV addresses are
     aligned.  Raises RuntimeError naming the first inconsistency."""
-    tabs = layout.device_tables(device, problem.kv_block)
+    tabs = tables or layout.device_tables(device, problem.kv_block)
     runs = run_table.numpy() if isinstance(run_table, torch.Tensor) else run_table
     runs = np.ascontiguousarray(runs).view(np.uint8)
     if runs.size != len(layout.runs) * RUN_DTYPE.itemsize:
@@ -634,18 +630,19 @@ def _attention_forward(query: torch.Tensor, layout: AttnLayout, scale: float, ke
     out = torch.empty(query.shape, dtype=query.dtype, device=device)
     lse = torch.empty(layout.hq, max(layout.q_rows, 1), dtype=torch.float32, device=device)
     kvb = layout.call_kv_block(device, query.shape[2])
-    _, (runs, host, keep) = layout._upload(device, kvb, sources)
-    problem = layout.problem(device, runs, scale, query.dtype, query.shape[2], kvb)
-    check_tables(layout, problem, host, device)
+    tabs, (runs, host, keep) = layout._upload(device, kvb, sources)
+    problem = layout.problem(device, runs, scale, query.dtype, query.shape[2], kvb, tabs)
+    check_tables(layout, problem, host, device, tabs)
     # few work items over many keys: each item's keys in several work-groups
-    parts = lib.ts_attn_fwd_parts(ctypes.byref(problem), layout._description()["max_keys"])
+    at = ctypes.byref(problem)
+    parts = lib.ts_attn_fwd_parts(at, layout._description()["max_keys"])
     work = None
     if parts > 1:
-        work = _parts_workspace(lib.ts_attn_fwd_parts_workspace(ctypes.byref(problem), parts), device)
+        work = _parts_workspace(lib.ts_attn_fwd_parts_workspace(at, parts), device)
         parts = parts if work is not None else 1
     with operator_range("hip_attention_forward", rows=layout.q_rows, segments=len(layout.seg_q)):
         _lib.check(
-            lib.ts_attn_fwd_split(ctypes.byref(problem), _rows(query), _rows(out), lse.data_ptr(), lse.shape[1],
+            lib.ts_attn_fwd_split(at, _rows(query), _rows(out), lse.data_ptr(), lse.shape[1],
                                   parts, _lib.ptr(work), 0 if work is None else work.numel(),
                                   _lib.stream_of(query)),
             lambda: f"ts_attn_fwd(rows={layout.q_rows}, hq={layout.hq}, hkv={layout.hkv})",
@@ -681,8 +678,8 @@ def _attention_backward(query, out, lse, dout, layout: AttnLayout, scale: float,
     kvb = layout.call_kv_block(device, d)
     tabs, (runs, host, keep_runs) = layout._upload(device, kvb, sources)
     rowstats = torch.empty(layout.hq, max(layout.q_rows, 1), 2, dtype=torch.float32, device=device)
-    problem = layout.problem(device, runs, scale, query.dtype, d, kvb)
-    check_tables(layout, problem, host, device)
+    problem = layout.problem(device, runs, scale, query.dtype, d, kvb, tabs)
+    check_tables(layout, problem, host, device, tabs)
     keep = [keep_runs]
     ds = _ds_route(layout, query, lib)
     if ds is not None:
@@ -717,7 +714,7 @@ def _attention_backward(query, out, lse, dout, layout: AttnLayout, scale: float,
                     keep.append((sub_runs, sub_host))
                     sub = AttnProblem.from_buffer_copy(problem)
                     sub.hq, sub.hkv, sub.runs = n * group, n, sub_runs.data_ptr()
-                    check_tables(layout, sub, sub_host, device)
+                    check_tables(layout, sub, sub_host, device, tabs)
                 q_r, o_r, do_r, dq_r = (_head_rows(r, h0) for r in rows)
                 sums = None
                 if parts > 1:

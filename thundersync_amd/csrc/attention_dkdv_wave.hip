@@ -58,7 +58,7 @@ struct WaveCursor {
 // whose waves share each tile for 16 keys each with a barrier per step: C2-like
 // pack of 6 turns at 40/8 heads 1280 -> 900 us, 4096 rows over 8192 keys at
 // 40/8, 16/8 and 24/4 heads 1373 -> 1072, 573 -> 440 and 951 -> 651 us; items of
-// few steps keep the key-split kernel, attention.py _dkdv_us)  The K^T and V^T
+// few steps keep the key-split kernel, attention.py _dealt_is_faster)  The K^T and V^T
 // operands stay in registers.  Each wave streams its head's 32-row
 // Q/dO tiles and their 32 (lse * log2 e, delta) pairs into its own
 // double-buffered LDS region with buffer_load ... lds: the buffer resource of
