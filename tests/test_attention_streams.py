@@ -11,44 +11,83 @@ from thundersync_amd import _lib
 from thundersync_amd import attention as hip
 
 
-def test_another_stream_waits_once(monkeypatch):
-    """(CPU, streams that record what is asked of them.)"""
-    log = []
+class _Blob(torch.Tensor):
+    """A table tensor on the CPU that notes the streams it is recorded on."""
+
+    log: list
+
+    def record_stream(self, stream):
+        self.log.append(("record", stream.cuda_stream))
+
+
+@pytest.mark.parametrize("first, second", [(0, 7), (7, 0), (7, 9)])
+def test_another_stream_waits_once(monkeypatch, first, second):
+    """The tables' upload is what the other stream waits for, also when the
+    default stream, whose handle is 0, is either of the two.  (CPU, streams and
+    events that note what is asked of them; ExternalStream takes 0 for a stream
+    of its own, as torch's does.)"""
+    log, current, capturing = [], [first], [False]
 
     class Stream:
-        def __init__(self, name):
-            self.name, self.cuda_stream = name, name
+        def __init__(self, handle):
+            self.cuda_stream = handle
 
         def wait_stream(self, other):
-            log.append(("wait", self.name, other.name))
+            self.wait_event(other.cuda_stream)
 
-    class Blob:
-        def record_stream(self, stream):
-            log.append(("record", stream.name))
+        def wait_event(self, event):
+            log.append(("wait", self.cuda_stream, getattr(event, "stream", event)))
 
-    first, second, capturing = Stream("first"), Stream("second"), [False]
-    current = [first]
-    monkeypatch.setattr(_lib, "current_stream", lambda device: current[0].cuda_stream)
-    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: current[0])
+    class Event:
+        def record(self, stream):
+            self.stream = stream.cuda_stream
+
+    class Device:
+        type, index = "cuda", 0
+
+    class Host:
+        """What a layout's build takes for pinned memory."""
+
+        def __init__(self, n):
+            self.bytes = torch.zeros(n, dtype=torch.uint8)
+
+        def numpy(self):
+            return self.bytes.numpy()
+
+        def data_ptr(self):
+            return self.bytes.data_ptr()
+
+        def to(self, device, non_blocking):
+            blob = self.bytes.clone().as_subclass(_Blob)
+            blob.log = log
+            return blob
+
+    monkeypatch.setattr(_lib, "current_stream", lambda device: current[0])
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: Stream(current[0]))
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing[0])
-    monkeypatch.setattr(torch.cuda, "ExternalStream", lambda handle, device: {"first": first, "second": second}[handle])
-    tabs = {"stream": "first", "streams": {"first"}, "blob": Blob()}
-    device = torch.device("cuda:0")
-    hip._order_after_upload(tabs, device)
+    monkeypatch.setattr(torch.cuda, "ExternalStream", lambda handle, device=None: Stream(handle or "another"))
+    monkeypatch.setattr(torch.cuda, "Event", Event)
+    lay = hip.chain_layout(70, [300], 4, 1)
+    sources = [0x10000, 128, 128, 0x10000, 128, 128, 0, 0, 0, 0, 0, 0]
+    monkeypatch.setattr(torch, "empty", lambda n, dtype=None, pin_memory=False: Host(n))
+    upload = lambda: lay._upload(Device(), 64, sources)
+    upload()
+    upload()
     assert log == []
     current[0], capturing[0] = second, True
-    hip._order_after_upload(tabs, device)
+    upload()
     assert log == []
     capturing[0] = False
-    hip._order_after_upload(tabs, device)
-    hip._order_after_upload(tabs, device)
-    assert log == [("wait", "second", "first"), ("record", "second")]
+    upload()
+    upload()
+    assert log == [("wait", second, first), ("record", second)]
 
 
 @pytest.mark.gpu
-def test_two_streams(cuda):
+@pytest.mark.parametrize("default_first", [False, True])
+def test_two_streams(cuda, default_first):
     """The second stream's call is right though the first stream is still busy before the upload."""
-    print("two streams", flush=True)
+    print(f"two streams, default stream first: {default_first}", flush=True)
     g = torch.Generator().manual_seed(0)
     q, do = (torch.randn(70, 4, 128, generator=g).bfloat16() for _ in range(2))
     k, v = (torch.randn(300, 1, 128, generator=g).bfloat16() for _ in range(2))
@@ -58,7 +97,9 @@ def test_two_streams(cuda):
     busy = torch.randn(4096, 4096, device=cuda)
     torch.cuda.synchronize()
     results = []
-    for stream in (torch.cuda.Stream(), torch.cuda.Stream(), torch.cuda.current_stream()):
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    streams.insert(0 if default_first else 2, torch.cuda.current_stream())
+    for stream in streams:
         with torch.cuda.stream(stream):
             if not results:
                 for _ in range(20):

@@ -341,8 +341,11 @@ class AttnLayout:
                         span=base + sizes.span_ds, visit=base + sizes.visit_ds,
                     )
                     if device.type == "cuda":
-                        tabs["stream"] = _lib.current_stream(device)
-                        tabs["streams"] = {tabs["stream"]}
+                        tabs["streams"] = {_lib.current_stream(device)}
+                        tabs["uploaded"] = None
+                        if not torch.cuda.is_current_stream_capturing():
+                            tabs["uploaded"] = torch.cuda.Event()
+                            tabs["uploaded"].record(torch.cuda.current_stream(device))
                     self._tables[key] = tabs
                     if sources is not None:
                         return tabs, (base + sizes.bytes, view[sizes.bytes : sizes.bytes + run_bytes], (dev, host))
@@ -437,13 +440,17 @@ def _order_after_upload(tabs: dict, device) -> None:
     """Let the current stream read tables that another one uploads: it waits for
     the upload (whose stream may not have run it yet), and the tables' memory is
     its to read until it has.  Once per stream; a capture takes tables that its
-    stream has used before, or that are long there."""
-    if _lib.current_stream(device) in tabs["streams"] or torch.cuda.is_current_stream_capturing():
+    stream has used before, or that are long there.  The wait is on an event of
+    the upload: the uploading stream's handle would not do, being 0 for the
+    default stream, which torch.cuda.ExternalStream takes for no handle at all."""
+    handle = _lib.current_stream(device)
+    if handle in tabs["streams"] or torch.cuda.is_current_stream_capturing():
         return
     stream = torch.cuda.current_stream(device)
-    stream.wait_stream(torch.cuda.ExternalStream(tabs["stream"], device=device))
+    if tabs["uploaded"] is not None:  # None: a capture holds the upload
+        stream.wait_event(tabs["uploaded"])
     tabs["blob"].record_stream(stream)
-    tabs["streams"].add(_lib.current_stream(device))
+    tabs["streams"].add(handle)
 
 
 def _check_rows_tensor(t: torch.Tensor, name: str, heads: int, head_dim: int, max_row_stride: int = 1 << 24) -> None:
