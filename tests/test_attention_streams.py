@@ -1,5 +1,5 @@
-"""One layout used on several streams: its tables are uploaded by the first call's
-stream, and a call on another stream reads them after that."""
+"""One layout used on several streams: each reads the copy of its tables that it
+uploaded itself."""
 
 from __future__ import annotations
 
@@ -11,36 +11,12 @@ from thundersync_amd import _lib
 from thundersync_amd import attention as hip
 
 
-class _Blob(torch.Tensor):
-    """A table tensor on the CPU that notes the streams it is recorded on."""
-
-    log: list
-
-    def record_stream(self, stream):
-        self.log.append(("record", stream.cuda_stream))
-
-
 @pytest.mark.parametrize("first, second", [(0, 7), (7, 0), (7, 9)])
-def test_another_stream_waits_once(monkeypatch, first, second):
-    """The tables' upload is what the other stream waits for, also when the
-    default stream, whose handle is 0, is either of the two.  (CPU, streams and
-    events that note what is asked of them; ExternalStream takes 0 for a stream
-    of its own, as torch's does.)"""
-    log, current, capturing = [], [first], [False]
-
-    class Stream:
-        def __init__(self, handle):
-            self.cuda_stream = handle
-
-        def wait_stream(self, other):
-            self.wait_event(other.cuda_stream)
-
-        def wait_event(self, event):
-            log.append(("wait", self.cuda_stream, getattr(event, "stream", event)))
-
-    class Event:
-        def record(self, stream):
-            self.stream = stream.cuda_stream
+def test_each_stream_reads_its_own_upload(monkeypatch, first, second):
+    """A stream's tables are a copy that this stream uploads, once, also when the
+    default stream, whose handle is 0, is either of the two; a stream that
+    captures adds no copy.  (CPU, copies that note the stream they are made on.)"""
+    current, capturing, copies = [first], [False], []
 
     class Device:
         type, index = "cuda", 0
@@ -58,29 +34,36 @@ def test_another_stream_waits_once(monkeypatch, first, second):
             return self.bytes.data_ptr()
 
         def to(self, device, non_blocking):
-            blob = self.bytes.clone().as_subclass(_Blob)
-            blob.log = log
-            return blob
+            copies.append((current[0], self.bytes.numel(), self.bytes.clone()))
+            return copies[-1][2]
 
     monkeypatch.setattr(_lib, "current_stream", lambda device: current[0])
-    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: Stream(current[0]))
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing[0])
-    monkeypatch.setattr(torch.cuda, "ExternalStream", lambda handle, device=None: Stream(handle or "another"))
-    monkeypatch.setattr(torch.cuda, "Event", Event)
+    monkeypatch.setattr(torch, "empty", lambda n, dtype=None, pin_memory=False: Host(n))
     lay = hip.chain_layout(70, [300], 4, 1)
     sources = [0x10000, 128, 128, 0x10000, 128, 128, 0, 0, 0, 0, 0, 0]
-    monkeypatch.setattr(torch, "empty", lambda n, dtype=None, pin_memory=False: Host(n))
-    upload = lambda: lay._upload(Device(), 64, sources)
-    upload()
-    upload()
-    assert log == []
-    current[0], capturing[0] = second, True
-    upload()
-    assert log == []
-    capturing[0] = False
-    upload()
-    upload()
-    assert log == [("wait", second, first), ("record", second)]
+
+    def upload(stream, capture=False):
+        """A call's tables, and the streams that uploaded tables in it (a run table is smaller)."""
+        current[0], capturing[0] = stream, capture
+        copies.clear()
+        tabs, _ = lay._upload(Device(), 64, sources)
+        tables = [c for c in copies if c[1] > hip.RUN_DTYPE.itemsize]
+        assert all(c[2] is tabs["blob"] for c in tables)
+        return tabs, [c[0] for c in tables]
+
+    one, by = upload(first)
+    assert by == [first]
+    assert upload(first) == (one, [])
+    assert upload(second, capture=True) == (one, [])
+    two, by = upload(second)
+    assert by == [second] and two["blob"].data_ptr() != one["blob"].data_ptr()
+    assert torch.equal(two["blob"], one["blob"])
+    pointers = ("segs", "seg_spans", "run_visits_dev", "q_work", "kv_work", "dq_work", "span", "visit")
+    shift = two["blob"].data_ptr() - one["blob"].data_ptr()
+    assert [two[p] for p in pointers] == [one[p] and one[p] + shift for p in pointers]
+    assert two["array_ptrs"] == one["array_ptrs"]
+    assert upload(second) == (two, []) and upload(first) == (one, [])
 
 
 @pytest.mark.gpu

@@ -296,12 +296,18 @@ class AttnLayout:
         )
 
     def _upload(self, device: torch.device, kvb: int, sources: Sequence[int] | None):
-        """(tables, run table): the layout's tables on ``device``, built and
-        uploaded once per device and dK/dV item size, and, with ``sources``, one
-        call's run table as (device address, host bytes, tensors to keep).  Both
-        go through pinned memory without blocking, in one piece when the layout
-        is new."""
-        key = (device.type, device.index, kvb)
+        """(tables, run table): the layout's tables on ``device``, built once per
+        device and dK/dV item size and uploaded once per stream, and, with
+        ``sources``, one call's run table as (device address, host bytes, tensors
+        to keep).  Both go through pinned memory without blocking, in one piece
+        when the layout is new.  A stream reads the copy that it uploaded itself,
+        so no stream waits for another and the copy's memory is its own; a stream
+        that is capturing takes another's, if there is one, without a copy in the
+        graph.  (With an event recorded behind the upload for other streams to
+        wait on, a 48-row turn took 121 us; so 111.)"""
+        stream = _lib.current_stream(device) if device.type == "cuda" else 0
+        at = (device.type, device.index, kvb)
+        key = (*at, stream)
         run_bytes = len(self.runs) * RUN_DTYPE.itemsize if sources is not None else 0
 
         def alloc(n):
@@ -311,7 +317,12 @@ class AttnLayout:
         if tabs is None:
             with self._lock:
                 tabs = self._tables.get(key)
-                if tabs is None:
+                first = None if tabs else next((t for k, t in self._tables.items() if k[:3] == at), None)
+                if first is not None:
+                    tabs = first
+                    if not torch.cuda.is_current_stream_capturing():
+                        tabs = self._tables[key] = self._on_device(first, first["host"], first["sizes"], device)
+                elif tabs is None:
                     sizes, host, view, run_visits = self._build(kvb, alloc, run_bytes)
                     segs, spans, visits, q_work, kv_work, _ = self._views(sizes, view)
                     n = self._description()["n_spans"]
@@ -332,35 +343,33 @@ class AttnLayout:
                     }
                     if run_bytes:
                         self._fill_runs(tabs, sources, view[sizes.bytes :])
-                    dev = host.to(device, non_blocking=True)
-                    base = dev.data_ptr()
-                    tabs.update(
-                        blob=dev, host=host, segs=base + sizes.segs, seg_spans=base + sizes.spans,
-                        run_visits_dev=base + sizes.visits, q_work=base + sizes.q_work, kv_work=base + sizes.kv_work,
-                        dq_work=base + sizes.dq_work if sizes.n_dq_work else None,
-                        span=base + sizes.span_ds, visit=base + sizes.visit_ds,
-                    )
-                    if device.type == "cuda":
-                        tabs["streams"] = {_lib.current_stream(device)}
-                        tabs["uploaded"] = None
-                        if not torch.cuda.is_current_stream_capturing():
-                            tabs["uploaded"] = torch.cuda.Event()
-                            tabs["uploaded"].record(torch.cuda.current_stream(device))
-                    self._tables[key] = tabs
+                    tabs = self._tables[key] = self._on_device(tabs, host, sizes, device)
                     if sources is not None:
-                        return tabs, (base + sizes.bytes, view[sizes.bytes : sizes.bytes + run_bytes], (dev, host))
+                        dev = tabs["blob"]
+                        return tabs, (dev.data_ptr() + sizes.bytes,
+                                      view[sizes.bytes : sizes.bytes + run_bytes], (dev, host))
         if sources is None:
             return tabs, None
-        if device.type == "cuda":
-            _order_after_upload(tabs, device)
         host = alloc(run_bytes)
         view = host.numpy()
         self._fill_runs(tabs, sources, view)
         dev = host.to(device, non_blocking=True)
         return tabs, (dev.data_ptr(), view[:run_bytes], (dev, host))
 
+    @staticmethod
+    def _on_device(tabs: dict, host: torch.Tensor, sizes: AttnLayoutSizes, device: torch.device) -> dict:
+        """The tables with a copy of ``host`` that the current stream uploads."""
+        dev = host.to(device, non_blocking=True)
+        base = dev.data_ptr()
+        return dict(
+            tabs, blob=dev, host=host, sizes=sizes, segs=base + sizes.segs, seg_spans=base + sizes.spans,
+            run_visits_dev=base + sizes.visits, q_work=base + sizes.q_work, kv_work=base + sizes.kv_work,
+            dq_work=base + sizes.dq_work if sizes.n_dq_work else None,
+            span=base + sizes.span_ds, visit=base + sizes.visit_ds,
+        )
+
     def device_tables(self, device: torch.device, kv_block: int | None = None):
-        """The layout's integer tables on ``device``, uploaded once per device
+        """The layout's integer tables on ``device``, uploaded once per stream
         and dK/dV item size (pinned, non-blocking); `kv_block` None: the
         head-dim-128 size."""
         kvb = kv_block_keys(self.hq, self.hkv) if kv_block is None else int(kv_block)
@@ -434,23 +443,6 @@ class AttnLayout:
 # copy of this constant (kOrderBand, attention_tables.hip); this one is for readers
 # of the lists.
 ORDER_BAND = 0.05
-
-
-def _order_after_upload(tabs: dict, device) -> None:
-    """Let the current stream read tables that another one uploads: it waits for
-    the upload (whose stream may not have run it yet), and the tables' memory is
-    its to read until it has.  Once per stream; a capture takes tables that its
-    stream has used before, or that are long there.  The wait is on an event of
-    the upload: the uploading stream's handle would not do, being 0 for the
-    default stream, which torch.cuda.ExternalStream takes for no handle at all."""
-    handle = _lib.current_stream(device)
-    if handle in tabs["streams"] or torch.cuda.is_current_stream_capturing():
-        return
-    stream = torch.cuda.current_stream(device)
-    if tabs["uploaded"] is not None:  # None: a capture holds the upload
-        stream.wait_event(tabs["uploaded"])
-    tabs["blob"].record_stream(stream)
-    tabs["streams"].add(handle)
 
 
 def _check_rows_tensor(t: torch.Tensor, name: str, heads: int, head_dim: int, max_row_stride: int = 1 << 24) -> None:
