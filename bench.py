@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """Benchmark of the hot path on one MI355X; its last line is ONE JSON summary.
 
-Workloads (BASELINE.json configs, synthetic data drawn from fixed seeds):
+Workloads (synthetic data drawn from fixed seeds):
 
 * ``value``: C2 forest attention, forward + backward -- one shared
   2048-token prompt and 8 sibling completions of lengths U[256, 4096],
@@ -1108,7 +1108,7 @@ def main():
     out["device"] = {"name": props.name, "arch": getattr(props, "gcnArchName", ""),
                      "cus": props.multi_processor_count}
     out["peaks"] = dict(PEAKS)
-    # the full record first, then the one-line summary the driver reads last
+    # the full record first, then the one-line summary last
     print(json.dumps({"bench_detail": out}), flush=True)
     print(json.dumps(summary(out), separators=(",", ":")), flush=True)
 

@@ -1,5 +1,5 @@
 """CPU restatement of the reference's boundary-adjoint reduction and FP32
-ledger -- TEST INFRASTRUCTURE ONLY (the parity tests' checker and bench.py's
+ledger -- TEST INFRASTRUCTURE ONLY (the parity tests' oracle and bench.py's
 CPU baseline; the product never imports it).
 
 * :func:`reduce_sequential` -- engine/boundary_adjoint.py:156-180, the

@@ -1,5 +1,5 @@
 """CPU restatement of the reference's merged-weight LoRA linear -- TEST
-INFRASTRUCTURE ONLY (the parity tests' checker; the product never imports it).
+INFRASTRUCTURE ONLY (the parity tests' oracle; the product never imports it).
 
 * :func:`fused_forward` -- accel/fused_lora.py:29-33: ``x @ W_eff.T``.
 * :func:`fused_backward` -- accel/fused_lora.py:35-48: ``dx = g W_eff``,

@@ -1,6 +1,6 @@
 """Write tests/golden/forest_metadata.json from the reference's own builders.
 
-Run in the build container only (the reference is not on the GPU box):
+Run where the reference's source tree is:
 
     python tests/golden/make_forest_golden.py /root/reference/src
 

@@ -1,6 +1,6 @@
 """Write tests/golden/pack_layout.json from the reference's own ``_PackLayout``.
 
-Run in the build container only (the reference is not on the GPU box):
+Run where the reference's source tree is:
 
     python tests/golden/make_pack_golden.py /root/reference/src
 

@@ -1,9 +1,9 @@
 """Record stock-module RMSNorm bytes on the GPU as a data-only fixture.
 
-Run on a GPU box (it needs torch's GPU kernels, whose summation order and
+Run on an MI355X (it needs torch's GPU kernels, whose summation order and
 rsqrt rounding are what the fixture records):
 
-    python tests/golden/make_rmsnorm_golden.py gpurun_out/rmsnorm_device.npz
+    python tests/golden/make_rmsnorm_golden.py tests/golden/rmsnorm_device.npz
 
 For each case it draws ``hidden`` [rows, width] from a seeded CPU generator,
 runs transformers' stock ``Qwen3RMSNorm`` (the module the reference's swap

@@ -44,8 +44,7 @@ def test_traffic_table_entries_name_their_commit():
 
 
 def test_summary_line_keeps_every_secondary_in_a_short_line(monkeypatch):
-    """The summary line (the driver reads the last 2000 characters of the
-    output) carries the contract's keys, the roofline and CPU baseline, and
+    """The summary line (a log tail of 2000 characters has to hold it whole) carries the contract's keys, the roofline and CPU baseline, and
     one row per secondary workload."""
     out = {k: 1 for k in ("value", "n_gpus", "steps", "warmup", "ms_per_step")}
     out.update(metric=bench.METRIC, unit="TFLOP/s", higher_is_better=True, scaling="weak", vs_baseline=None,

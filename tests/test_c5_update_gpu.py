@@ -1,4 +1,4 @@
-"""One GRPO-shaped update at the C5 config's shapes.
+"""One GRPO-shaped update at the C5 workload's shapes.
 
 Two layers of the Qwen3-8B-shaped decoder (hidden 4096, 32 query / 8 KV
 heads, head dim 128, MLP 12288, vocab 151936, random-init bf16) with LoRA

@@ -14,7 +14,7 @@ and ``grpo_source_rms_norm_native_vjp``, bf16 modules only, Parameters kept,
 a module whose trials fail left as it is -- and marks the modules whose
 trials passed as :class:`NativeSourceRMSNorm`.
 
-The trials are this build's own:
+The trials are this package's own:
 
 * forward: for inputs shaped ``(1, 3, W)`` and ``(1, 3, 2, W)`` the HIP
   primal equals torch's stock operations on the device byte for byte, and
@@ -26,7 +26,7 @@ The trials are this build's own:
 Not bitwise against aten: the reference's bitwise trial compares aten's
 fused backward with Triton schedules written to reproduce its summation
 order; that order is not available in this image (torch ships the kernel's
-header, not its source), and this build's dW has its own fixed order.
+header, not its source), and the dW here has its own fixed order.
 """
 
 from __future__ import annotations
