@@ -179,16 +179,18 @@ __device__ __forceinline__ int acc_row(int i, int lane) { return 8 * (i >> 2) + 
   __shared__ __attribute__((aligned(16))) float sb1[stage_words<RB, KFB>()];
 
 // (max, sum exp(l - max), sum exp(l - max) (l - max)) of two disjoint sets of
-// logits.  A set whose maximum is -inf adds only its third sum: 0 when it is
-// empty, NaN when it holds logits of -inf (0 * -inf, as in the plain sum).
+// logits.  A set whose maximum is -inf adds only its sums: both 0 when it is
+// empty, the third NaN when it holds logits of -inf (0 * -inf, as in the plain
+// sum), both NaN when it holds a NaN, which no maximum shows.
 __device__ __forceinline__ void merge_stats(float& m, float& s, float& e, float mo, float so, float eo) {
   if (mo == neg_inf()) {
+    s += so;
     e += eo;
     return;
   }
   if (m == neg_inf()) {
     m = mo;
-    s = so;
+    s += so;
     e += eo;
     return;
   }
@@ -256,6 +258,12 @@ __global__ __launch_bounds__(kThreads, 2) void fwd_stats_kernel(const float* __r
               s += p;
               e += p * x;
             }
+      } else if (any) {
+#pragma unroll
+        for (int mi = 0; mi < 2; ++mi)
+#pragma unroll
+          for (int i = 0; i < 16; ++i)
+            if (64 * wm + 32 * mi + acc_row(i, lane) < left && acc[mi][nj][i] != neg_inf()) s = __builtin_nanf("");
       }
       merge_stats(sm[nj], ss[nj], se[nj], mx, s, e);
     }
