@@ -12,7 +12,7 @@ from thundersync_amd import fused_logprob as fl
 
 pytestmark = pytest.mark.gpu
 
-DTYPES = [torch.float32]
+DTYPES = [torch.bfloat16, torch.float16, torch.float32]
 
 
 @pytest.mark.parametrize("dtype", DTYPES)

@@ -42,13 +42,14 @@ constexpr float kLn2 = 0.6931471805599453f;
 __device__ __forceinline__ float neg_inf() { return -__builtin_huge_valf(); }
 
 // (max, sum exp(l - max), sum exp(l - max) (l - max)) of two disjoint sets of
-// logits, either of which may be empty (max = -inf)
+// logits, either of which may be empty (max = -inf, sums 0).  A set of logits of
+// -inf counts as empty; the sums of one that holds a NaN, which no maximum shows,
+// are NaN.
 __device__ __forceinline__ void merge_stats(float& m, float& s, float& e, float mo, float so, float eo) {
-  if (mo == neg_inf()) return;
-  if (m == neg_inf()) {
-    m = mo;
-    s = so;
-    e = eo;
+  if (mo == neg_inf() || m == neg_inf()) {
+    m = fmaxf(m, mo);
+    s += so;
+    e += eo;
     return;
   }
   const float mn = fmaxf(m, mo);
@@ -145,7 +146,13 @@ __global__ __launch_bounds__(kGemmThreads, 1) void fwd_stats_kernel(FwdArgs p) {
     // sum is taken back to natural-log units once
     float sum = 0.f, e = 0.f;
     const float m2 = m * kLog2e;
-    if (v0 + TM <= p.vocab) {
+    if (m == neg_inf()) {
+#pragma unroll
+      for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          if (acc[mi][ni][i] != neg_inf()) sum = e = __builtin_nanf("");
+    } else if (v0 + TM <= p.vocab) {
 #pragma unroll
       for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
@@ -155,7 +162,7 @@ __global__ __launch_bounds__(kGemmThreads, 1) void fwd_stats_kernel(FwdArgs p) {
           sum += q;
           e = fmaf(q, d2, e);
         }
-    } else if (m != neg_inf()) {
+    } else {
 #pragma unroll
       for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
