@@ -74,6 +74,7 @@ __global__ __launch_bounds__(64 * 8 / (NQB * NP), 1) void dq_wave_kernel(ts_attn
   }
   const int qw = qp + 16 * NQB * (wave / GC);  // this wave's first row
   const int last = min(qp + kPassRows, T) - 1;
+  const int w_last = min(qw + 16 * NQB, T) - 1;  // this wave's last row
   // Q / dO rows as B operands: reg[qb][ks] = row qw + 16 qb + j16, columns 32 ks + 8 g4 ..
   bf16x8 qreg[NQB][NKS], dreg[NQB][NKS];
   const int64_t row0 = seg.q_row0 + qw;
@@ -258,6 +259,11 @@ __global__ __launch_bounds__(64 * 8 / (NQB * NP), 1) void dq_wave_kernel(ts_attn
     if (nxt.sp < seg.nspan)
       issue_kv_tile<kWaves, HD>(wave, lane, nxt, bsel.value == 0 ? s_k1 : s_k0, bsel.value == 0 ? s_v1 : s_v0);
 
+    // as in the forward, at the narrow head dims: no tile past the wave's last visible key
+    if (HD % 128 != 0 && kpos + kt0 > off + w_last) {
+      cur = nxt;
+      return;
+    }
     if ((kpos + kt0 + BK - 1 > off + qw) | (kt0 + BK > run_len))
       tile_body(std::true_type{}, tk, tv, kpos, kt0, run_len);
     else

@@ -91,6 +91,7 @@ __global__ __launch_bounds__(64 * 8 / NQB, (fwd_occupancy<NQB, HD, KT>())) void 
   const int T = seg.q_len;
   const int off = seg.kv_len - seg.q_len;
   const int last = min(q0 + 16 * NQB * kWaves / GC, T) - 1;
+  const int w_last = min(qw + 16 * NQB, T) - 1;  // this wave's last row
   int begin = 0, stop = off + last + 1;
   if constexpr (SPLIT) part_of<KT>(stop, (int)blockIdx.y, (int)gridDim.y, begin, stop);
   const float c = P.scale * kLog2e;
@@ -124,6 +125,13 @@ __global__ __launch_bounds__(64 * 8 / NQB, (fwd_occupancy<NQB, HD, KT>())) void 
       issue_kv_tile<kWaves, HD, KT>(wave, lane, nxt, bsel.value == 0 ? s_k1 : s_k0, bsel.value == 0 ? s_v1 : s_v0);
 
     const bool masked = (kpos + kt0 + KT - 1 > off + qw) | (kt0 + KT > run_len);
+    // a tile that starts past the wave's last visible key adds nothing: at the
+    // narrow head dims it is passed over, so that an infinite or NaN component
+    // there (times a weight of 0) stays out of rows that do not see it
+    if (HD % 128 != 0 && kpos + kt0 > off + w_last) {
+      cur = nxt;
+      return;
+    }
     // two halves of 32 keys, each one online-softmax update:
     // S^T = K Q^T with sc[kb][qb] holding keys 32 ss + 16 kb + 4 g4 + i of column
     // 16 qb + j16, then O^T += V^T P^T with slot j <-> key 32 ss + 16 (j >> 2) + 4 g4 + (j & 3)
