@@ -30,3 +30,19 @@ def test_gradients_are_dense(cuda, dim):
     grads += torch.autograd.grad(out, [q, key, value, ks[0], vs[0]], torch.randn_like(out))
     for t in grads:
         assert t.is_contiguous() and t.untyped_storage().nbytes() == 2 * t.numel(), (t.shape, t.stride())
+
+
+@pytest.mark.parametrize("other", [32, 96])
+@pytest.mark.parametrize("which", ["key", "value"])
+@pytest.mark.parametrize("packed", [False, True])
+def test_another_head_dim_is_refused(cuda, packed, which, other):
+    """Keys or values whose head dim is not the query's raise (they were padded or cropped to it)."""
+    print(f"head dim 64 against {which} of {other}, packed: {packed}", flush=True)
+    dims = {"key": 64, "value": 64, which: other}
+    q = torch.zeros(1, 2, 4, 64, dtype=torch.bfloat16, device=cuda)
+    k, v = (torch.zeros(4, 2, dims[n], dtype=torch.bfloat16, device=cuda) for n in ("key", "value"))
+    with pytest.raises(ValueError, match="must be"):
+        if packed:
+            hip.PackedAttention.apply(q, k, v, 0.1, hip.pack_layout([4], [([], [])]))
+        else:
+            hip.ChunkedCausalAttention.apply(q, 0.1, 1, True, "auto", k, v)

@@ -800,7 +800,8 @@ def _save_attention(ctx, query: torch.Tensor, layout: AttnLayout, scale: float, 
     :func:`attention`."""
     d = query.shape[-1]
     dk = kernel_head_dim(d) or d
-    query, keys, values = _pad_heads(query, dk), [_pad_heads(k, dk) for k in keys], [_pad_heads(v, dk) for v in values]
+    if dk != d:  # else keys and values of another head dim are refused below
+        query, keys, values = _pad_heads(query, dk), [_pad_heads(k, dk) for k in keys], [_pad_heads(v, dk) for v in values]
     out, lse, ctx.keep = _attention_forward(query, layout, float(scale), keys, values)
     ctx.layout, ctx.scale = layout, float(scale)
     ctx.save_for_backward(query, out, lse, *keys, *values)
