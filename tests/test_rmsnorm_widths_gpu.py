@@ -62,6 +62,15 @@ def test_forward_bytes_of_wide_fp32_rows(cuda, rows, width):
     test_forward_bytes(cuda, rows, width, torch.float32)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("rows,width", [(6147, 2308), (8192, 3072), (6147, 3076), (4099, 4096), (8192, 4096), (8195, 4096),
+                                        (6145, 2048)])
+def test_forward_bytes_around_one_round(cuda, rows, width, dtype):
+    """Rows of 8 to 16 vectors a lane in launches that load the weight after the reduction
+    (one round of the CUs then), and just past them."""
+    test_forward_bytes(cuda, rows, width, dtype)
+
+
 @pytest.mark.parametrize("rows,width", [(255 * 8, 512), (256 * 32, 512), (256 * 32 + 1, 1024), (2049, 1536)])
 def test_backward_of_narrow_rows(cuda, rows, width):
     """Rows per block: one pass of its waves up to 256 blocks, 32 rows from there."""

@@ -245,10 +245,13 @@ template <typename T> __device__ __forceinline__ float primal(float w, float x, 
 // Non-temporal stores make that first launch 51.7 us in a stream of others, but a
 // pass by itself, forward and backward, 13 us longer (140 -> 153): the last-level
 // cache then takes no part of the output, which the next kernel would find there.
-// HOLD false loads the weight after the reduction: for fp32 rows of 32 vectors in
-// launches that its 186 registers (two blocks a CU) take in one round and the 308
-// of the other in two (2048 x 7168: 24.6 us against 27.2; but 64 rows 11.6 and 9.1,
-// 16384 rows 224 and 205).
+// HOLD false loads the weight after the reduction: fewer registers, so more blocks
+// a CU, for launches that are one round of it and would be two of the other
+// (fwd_lanes_kernel).  Held against not, us: bf16 8192 x 4096 (2048 blocks; 4 and 8 a
+// CU) 25.0 / 23.0 from cached rows and 39.8 / 38.1 from cold ones, 6144 x 3328 17.7 /
+// 16.9 and 27.1 / 25.8, fp32 6144 x 3072 25.4 / 23.9 and 43.4 / 40.5, 2048 x 7168 27.2
+// / 24.6; but 16384 x 4096 45.0 / 46.6 and 70 / 75, 2048 x 4096 10.4 / 11.5 and 15.2 / 18.2,
+// fp32 64 x 7168 9.1 / 11.6.
 template <typename T, bool VEC, int NV, bool HOLD = true>
 __global__ __launch_bounds__(kThreads) void rmsnorm_fwd_lanes(
     const T* __restrict__ x, const T* __restrict__ w, T* __restrict__ y,
@@ -685,11 +688,31 @@ int stream_cus(hipStream_t s) {
   return n;
 }
 
+// The forward's kernel for a launch of `blocks`: the weight loaded after the
+// reduction where the CUs take the launch in one round of it and not in one of the
+// kernel that holds the weight (rmsnorm_fwd_lanes).
+template <typename T, int NV>
+auto fwd_lanes_kernel(int64_t blocks, int cus) {
+  // (20 and 24 vectors, and 32 of a 16-bit type, gain up to 10 % from cached rows and
+  // lose as much from cold ones: they hold it always)
+  if constexpr ((NV >= 8 && NV <= 16) || (NV == 32 && sizeof(T) == 4)) {
+    auto per_cu = [](auto kernel) {
+      int n = 0;
+      return hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, kThreads, 0) == hipSuccess ? n : 0;
+    };
+    static const int held = per_cu(rmsnorm_fwd_lanes<T, true, NV, true>);
+    static const int loaded = per_cu(rmsnorm_fwd_lanes<T, true, NV, false>);
+    if (blocks > (int64_t)held * cus && blocks <= (int64_t)loaded * cus) return rmsnorm_fwd_lanes<T, true, NV, false>;
+  }
+  return rmsnorm_fwd_lanes<T, true, NV, true>;
+}
+
 template <typename T>
 int launch_fwd(const void* x, const void* w, void* y, float* rstd, int64_t rows, int width,
                float eps, hipStream_t s) {
   RowReduce c;
-  if (!torch_row_reduce(rows, width, stream_cus(s), c)) {
+  const int cus = stream_cus(s);
+  if (!torch_row_reduce(rows, width, cus, c)) {
     set_error("ts_rmsnorm_fwd: a single row of width %d is summed across work-groups by torch; "
               "that order is not reproduced", width);
     return TS_ERR_INVALID;
@@ -706,16 +729,12 @@ int launch_fwd(const void* x, const void* w, void* y, float* rstd, int64_t rows,
       return check_launch("ts_rmsnorm_fwd");
     }
     const int loads = (width / 4 + c.bw - 1) / c.bw;
-    if (sizeof(T) == 4 && loads > 24 && loads <= 32 && grid.x > 256 && grid.x <= 512) {
-      hipLaunchKernelGGL((rmsnorm_fwd_lanes<T, true, 32, sizeof(T) != 4>), grid, dim3(kThreads), 0, s,
-                         (const T*)x, (const T*)w, (T*)y, rstd, rows, width, c.bw, factor, eps);
-      return check_launch("ts_rmsnorm_fwd");
-    }
-#define TS_FWD(NV)                                                                             \
-  if (loads <= NV) {                                                                           \
-    hipLaunchKernelGGL((rmsnorm_fwd_lanes<T, true, NV>), grid, dim3(kThreads), 0, s,           \
-                       (const T*)x, (const T*)w, (T*)y, rstd, rows, width, c.bw, factor, eps); \
-    return check_launch("ts_rmsnorm_fwd");                                                     \
+#define TS_FWD(NV)                                                                               \
+  if (loads <= NV) {                                                                             \
+    const auto kernel = fwd_lanes_kernel<T, NV>(grid.x, cus);                                    \
+    hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, s, (const T*)x, (const T*)w, (T*)y,      \
+                       rstd, rows, width, c.bw, factor, eps);                                    \
+    return check_launch("ts_rmsnorm_fwd");                                                       \
   }
     TS_FWD(1) TS_FWD(2) TS_FWD(4) TS_FWD(8) TS_FWD(12) TS_FWD(16) TS_FWD(20) TS_FWD(24) TS_FWD(32)
 #undef TS_FWD
