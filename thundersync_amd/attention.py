@@ -304,7 +304,7 @@ class AttnLayout:
         so no stream waits for another and the copy's memory is its own; a stream
         that is capturing takes another's, if there is one, without a copy in the
         graph.  (With an event recorded behind the upload for other streams to
-        wait on, a 48-row turn took 121 us; so 111.)"""
+        wait on, a 48-row turn took 121 us; so 111 to 113.)"""
         stream = _lib.current_stream(device) if device.type == "cuda" else 0
         at = (device.type, device.index, kvb)
         key = (*at, stream)
